@@ -371,6 +371,7 @@ class memory:  # noqa: N801
     def __init__(self, handle, keepalive=None):
         self.h = handle
         self._keep = keepalive
+        self._np = None
 
     @staticmethod
     def allocate(eng, lay):
@@ -391,25 +392,28 @@ class memory:  # noqa: N801
         return _pointer(self)
 
     # numpy conveniences for plain layouts ----------------------------------------------------------
+    def _numpy_layout(self):
+        """(axis order, padded shape, slices of the logical part, element type, bytes); a memory's layout never changes"""
+        if self._np is None:
+            l = self.get_layout()
+            order, full, inner = _layout_shape(l)
+            dt = np.dtype(NP_OF[l.data_type])
+            self._np = order, full, inner, dt, int(np.prod(full)) * dt.itemsize
+        return self._np
+
     def write(self, array_bfyx):
         """Store a (b, f, y, x) array into the buffer, whatever its plain format and padding."""
-        l = self.get_layout()
-        order, full, inner = _layout_shape(l)
-        src = np.ascontiguousarray(array_bfyx, dtype=NP_OF[l.data_type]).transpose(["bfyx".index(c) for c in order])
+        order, full, inner, dt, nbytes = self._numpy_layout()
+        src = np.ascontiguousarray(array_bfyx, dtype=dt).transpose(["bfyx".index(c) for c in order])
         with self.pointer() as p:
-            buf = np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_uint8)), shape=(int(np.prod(full)) * src.itemsize,))
-            view = buf.view(src.dtype).reshape(full)
-            view[inner] = src
+            np.frombuffer((C.c_uint8 * nbytes).from_address(p), dt).reshape(full)[inner] = src
 
     def read(self):
         """The logical (b, f, y, x) contents of a plain-format buffer."""
-        l = self.get_layout()
-        order, full, inner = _layout_shape(l)
-        dt = np.dtype(NP_OF[l.data_type])
+        order, full, inner, dt, nbytes = self._numpy_layout()
         with self.pointer() as p:
-            buf = np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_uint8)), shape=(int(np.prod(full)) * dt.itemsize,))
-            view = buf.view(dt).reshape(full)[inner].copy()
-        return np.ascontiguousarray(view.transpose([order.index(c) for c in "bfyx"]))
+            view = np.frombuffer((C.c_uint8 * nbytes).from_address(p), dt).reshape(full)[inner]
+            return view.transpose([order.index(c) for c in "bfyx"]).copy("C")  # the one copy out of the locked buffer
 
     def __del__(self):
         if getattr(self, "h", None) and _lib is not None:
@@ -802,6 +806,7 @@ class network:  # noqa: N801
         carr, n, keep = (options or build_options())._c()
         self.h = _call("cldnn_build_network", eng.h, topo.h, carr, n)
         self._engine, self._topology = eng, topo
+        self._output_ids = None  # fixed by the build; encoded once
 
     def set_input_data(self, prim_id, mem):
         _call("cldnn_set_network_input", self.h, prim_id.encode(), mem.h)
@@ -832,8 +837,10 @@ class network:  # noqa: N801
         deps = (C.c_void_p * max(len(dependencies), 1))(*[e.h for e in dependencies])
         _call("cldnn_execute_network", self.h, deps, len(dependencies))
         out = {}
-        for name in self.get_output_ids():
-            o = _call("cldnn_get_network_output", self.h, name.encode())
+        if self._output_ids is None:
+            self._output_ids = [(name, name.encode()) for name in self.get_output_ids()]
+        for name, raw in self._output_ids:
+            o = _call("cldnn_get_network_output", self.h, raw)
             out[name] = network_output(event(o.event), memory(o.memory))
         return out
 

@@ -78,6 +78,24 @@ size_t tensor_elems(const cldnn_hip_tensor& t)
 
 using namespace chip;
 
+// A kernel reads a host image where it lies up to this size: at 150 KB that is 3.5 us instead of a copy in front of it (5 us
+// and a launch gap of 6); from a few MB on the host link is the time either way, and a copy leaves the tensor in HBM.
+enum { READ_IN_PLACE_BYTES = 4 << 20 };
+// A network's scores are written straight into host memory up to this size: 1000 scores cost the kernel nothing, the copy
+// back and its wait were 25 us.
+enum { WRITE_IN_PLACE_BYTES = 256 << 10 };
+
+void cldnn_hip_buffer_s::need_shadow()
+{
+    if (!shadow) CHIP_CHECK(hipHostMalloc(&shadow, bytes, hipHostMallocDefault));
+}
+
+void cldnn_hip_buffer_s::upload()
+{
+    engine->make_current();
+    CHIP_CHECK(hipMemcpyAsync(dev, shadow, bytes, hipMemcpyHostToDevice, engine->stream));
+}
+
 void cldnn_hip_engine_s::make_current() const { CHIP_CHECK(hipSetDevice(device)); }
 
 hipEvent_t cldnn_hip_engine_s::take_event()
@@ -265,8 +283,9 @@ void* cldnn_hip_buffer_lock(cldnn_hip_buffer b)
         std::lock_guard<std::mutex> g(b->lock_mutex);
         if (b->lock_count == 0) {
             b->engine->make_current();
-            if (!b->shadow) CHIP_CHECK(hipHostMalloc(&b->shadow, b->bytes, hipHostMallocDefault));
-            CHIP_CHECK(hipMemcpyAsync(b->shadow, b->dev, b->bytes, hipMemcpyDeviceToHost, b->engine->stream));
+            b->need_shadow();
+            if (b->newest != cldnn_hip_buffer_s::HOST)
+                CHIP_CHECK(hipMemcpyAsync(b->shadow, b->dev, b->bytes, hipMemcpyDeviceToHost, b->engine->stream));
             CHIP_CHECK(hipStreamSynchronize(b->engine->stream));
         }
         ++b->lock_count;
@@ -283,22 +302,115 @@ cldnn_hip_status cldnn_hip_buffer_unlock(cldnn_hip_buffer b)
         CHIP_REQUIRE(b->lock_count > 0, CLDNN_HIP_ERROR, "unlock without lock");
         if (--b->lock_count == 0) {
             b->engine->make_current();
-            CHIP_CHECK(hipMemcpyAsync(b->dev, b->shadow, b->bytes, hipMemcpyHostToDevice, b->engine->stream));
+            b->upload();
             CHIP_CHECK(hipStreamSynchronize(b->engine->stream));
+            b->newest = cldnn_hip_buffer_s::DEVICE;  // from here on the caller's kernels may write through the pointer
         }
     });
+}
+
+void* cldnn_hip_buffer_map(cldnn_hip_buffer b, cldnn_hip_event last_use)
+{
+    void* result = nullptr;
+    guarded([&] {
+        CHIP_REQUIRE(b, CLDNN_HIP_INVALID_ARG, "null buffer");
+        std::lock_guard<std::mutex> g(b->lock_mutex);
+        if (b->lock_count == 0) {
+            b->engine->make_current();
+            b->need_shadow();
+            if (b->newest == cldnn_hip_buffer_s::DEVICE) {
+                CHIP_CHECK(hipMemcpyAsync(b->shadow, b->dev, b->bytes, hipMemcpyDeviceToHost, b->engine->stream));
+                CHIP_CHECK(hipStreamSynchronize(b->engine->stream));
+                b->newest = cldnn_hip_buffer_s::BOTH;
+            } else if (last_use) {
+                // kernels and uploads in flight may still use the shadow.  An event that has been waited for already costs a
+                // microsecond here, the stream 25 (it sends a marker of its own through the queue)
+                const cldnn_hip_status st = cldnn_hip_event_wait(last_use);
+                if (st != CLDNN_HIP_SUCCESS) throw error(st, cldnn_hip_last_error());
+            } else {
+                CHIP_CHECK(hipStreamSynchronize(b->engine->stream));
+            }
+        }
+        ++b->lock_count;
+        result = b->shadow;
+    });
+    return result;
+}
+
+cldnn_hip_status cldnn_hip_buffer_unmap(cldnn_hip_buffer b)
+{
+    return guarded([&] {
+        CHIP_REQUIRE(b, CLDNN_HIP_INVALID_ARG, "null buffer");
+        std::lock_guard<std::mutex> g(b->lock_mutex);
+        CHIP_REQUIRE(b->lock_count > 0, CLDNN_HIP_ERROR, "unmap without map");
+        if (--b->lock_count == 0) b->newest = cldnn_hip_buffer_s::HOST, b->read_in_place = false;
+    });
+}
+
+void* cldnn_hip_buffer_use(cldnn_hip_buffer b, int32_t use)
+{
+    void* result = nullptr;
+    guarded([&] {
+        CHIP_REQUIRE(b, CLDNN_HIP_INVALID_ARG, "null buffer");
+        std::lock_guard<std::mutex> g(b->lock_mutex);
+        const bool host = b->newest == cldnn_hip_buffer_s::HOST;
+        result = b->dev;
+        switch (use) {
+        case CLDNN_HIP_USE_READ:
+        case CLDNN_HIP_USE_READ_ONCE:
+            if (!host) break;
+            if (use == CLDNN_HIP_USE_READ_ONCE && b->bytes <= READ_IN_PLACE_BYTES && !b->read_in_place) {
+                b->read_in_place = true;
+                result = b->shadow;
+                break;
+            }
+            b->upload();
+            b->newest = cldnn_hip_buffer_s::BOTH;
+            break;
+        case CLDNN_HIP_USE_UPDATE:
+            if (host) b->upload();
+            b->newest = cldnn_hip_buffer_s::DEVICE;
+            break;
+        case CLDNN_HIP_USE_WRITE: b->newest = cldnn_hip_buffer_s::DEVICE; break;
+        case CLDNN_HIP_USE_WRITE_FOR_HOST:
+            if (b->bytes > WRITE_IN_PLACE_BYTES) {
+                b->newest = cldnn_hip_buffer_s::DEVICE;
+                break;
+            }
+            b->engine->make_current();
+            b->need_shadow();
+            b->newest = cldnn_hip_buffer_s::HOST, b->read_in_place = false;
+            result = b->shadow;
+            break;
+        default: throw error(CLDNN_HIP_INVALID_ARG, "unknown use of a buffer");
+        }
+    });
+    return result;
 }
 
 cldnn_hip_status cldnn_hip_buffer_fill(cldnn_hip_buffer b, uint8_t pattern)
 {
     return guarded([&] {
         CHIP_REQUIRE(b, CLDNN_HIP_INVALID_ARG, "null buffer");
+        std::lock_guard<std::mutex> g(b->lock_mutex);
         b->engine->make_current();
         CHIP_CHECK(hipMemsetAsync(b->dev, pattern, b->bytes, b->engine->stream));
+        b->newest = cldnn_hip_buffer_s::DEVICE;
     });
 }
 
-void* cldnn_hip_buffer_device_ptr(cldnn_hip_buffer b) { return b ? b->dev : nullptr; }
+void* cldnn_hip_buffer_device_ptr(cldnn_hip_buffer b)
+{
+    if (!b) return nullptr;
+    void* result = nullptr;
+    guarded([&] {
+        std::lock_guard<std::mutex> g(b->lock_mutex);
+        if (b->newest == cldnn_hip_buffer_s::HOST) b->upload();
+        b->newest = cldnn_hip_buffer_s::DEVICE;  // the caller may write through it
+        result = b->dev;
+    });
+    return result;
+}
 size_t cldnn_hip_buffer_size(cldnn_hip_buffer b) { return b ? b->bytes : 0; }
 
 cldnn_hip_status cldnn_hip_buffer_write(cldnn_hip_buffer b, size_t offset, const void* host, size_t bytes)
@@ -306,9 +418,12 @@ cldnn_hip_status cldnn_hip_buffer_write(cldnn_hip_buffer b, size_t offset, const
     return guarded([&] {
         CHIP_REQUIRE(b && host, CLDNN_HIP_INVALID_ARG, "null argument");
         CHIP_REQUIRE(offset + bytes <= b->bytes, CLDNN_HIP_INVALID_ARG, "write beyond the end of the buffer");
+        std::lock_guard<std::mutex> g(b->lock_mutex);
         b->engine->make_current();
+        if (b->newest == cldnn_hip_buffer_s::HOST) b->upload();
         CHIP_CHECK(hipMemcpyAsync((char*)b->dev + offset, host, bytes, hipMemcpyHostToDevice, b->engine->stream));
         CHIP_CHECK(hipStreamSynchronize(b->engine->stream));
+        b->newest = cldnn_hip_buffer_s::DEVICE;
     });
 }
 
@@ -317,9 +432,12 @@ cldnn_hip_status cldnn_hip_buffer_read(cldnn_hip_buffer b, size_t offset, void* 
     return guarded([&] {
         CHIP_REQUIRE(b && host, CLDNN_HIP_INVALID_ARG, "null argument");
         CHIP_REQUIRE(offset + bytes <= b->bytes, CLDNN_HIP_INVALID_ARG, "read beyond the end of the buffer");
+        std::lock_guard<std::mutex> g(b->lock_mutex);
         b->engine->make_current();
-        CHIP_CHECK(hipMemcpyAsync(host, (const char*)b->dev + offset, bytes, hipMemcpyDeviceToHost, b->engine->stream));
+        if (b->newest != cldnn_hip_buffer_s::HOST)
+            CHIP_CHECK(hipMemcpyAsync(host, (const char*)b->dev + offset, bytes, hipMemcpyDeviceToHost, b->engine->stream));
         CHIP_CHECK(hipStreamSynchronize(b->engine->stream));
+        if (b->newest == cldnn_hip_buffer_s::HOST) std::memcpy(host, (const char*)b->shadow + offset, bytes);
     });
 }
 

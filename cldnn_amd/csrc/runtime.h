@@ -34,6 +34,13 @@ struct cldnn_hip_buffer_s {
     std::mutex lock_mutex;
     int lock_count = 0;
     void* shadow = nullptr;  // pinned host mirror, allocated on first lock
+    // which copy is current.  DEVICE also stands for "not known": whoever holds the device pointer may have written.
+    enum copy_state { DEVICE, HOST, BOTH };
+    copy_state newest = DEVICE;
+    bool read_in_place = false;  // since the host wrote the shadow a kernel has read it where it is
+
+    void need_shadow();
+    void upload();  // shadow -> device on the engine's stream, not waited for
 };
 
 struct cldnn_hip_event_s {

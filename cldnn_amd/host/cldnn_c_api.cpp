@@ -126,6 +126,17 @@ static void await_pending_run(cldnn_network_impl* net)
     HOST_REQUIRE(error.empty(), CLDNN_ERROR, "the postponed run of the network failed: " + error);
 }
 
+// How the launch of a node uses its output buffer.  Kernels write the logical elements only, so a buffer with padding or
+// rounded-up features is updated, not overwritten.  A result nobody in the network reads is on its way to the host.
+static int32_t use_of_output(const node* n)
+{
+    const cldnn_layout& l = n->out;
+    bool dense = l.format == cldnn_format_bfyx || l.format == cldnn_format_yxfb || l.format == cldnn_format_byxf;
+    for (int i = 0; i < 4; ++i) dense = dense && l.padding.lower_size.sizes[i] == 0 && l.padding.upper_size.sizes[i] == 0;
+    if (!dense || n->p->second_input_in_output) return CLDNN_HIP_USE_UPDATE;
+    return n->is_output && n->users.empty() ? CLDNN_HIP_USE_WRITE_FOR_HOST : CLDNN_HIP_USE_WRITE;
+}
+
 // Enqueue one run.  deferred_marker: the run was announced earlier (its outputs already carry that event) and is
 // submitted now that its user events are set.
 static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cldnn_event_impl* deferred_marker)
@@ -143,6 +154,9 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
     for (cldnn_hip_event ev : net->stream_events) cldnn_hip_event_release(ev);  // the previous run's; it has been waited for
     net->stream_events.clear();
     std::map<node*, cldnn_hip_event> joins;  // completion of the primitives on the second stream
+    if (eng->side)  // uploads go to the first stream: ahead of the events the second one waits for
+        for (auto& m : net->mem)
+            if (m.second) m.second->read_ptr();
     for (auto& u : prog->nodes) {
         node* n = u.get();
         prim& p = *n->p;
@@ -157,7 +171,7 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
             HOST_REQUIRE(it != net->mem.end() && it->second, CLDNN_ERROR, "no memory for primitive " + d->p->id);
             return it->second.get();
         };
-        cldnn_memory_impl* out = n->chain_unkept() ? nullptr : mem_of(n);
+        auto out_of = [&](node* d) { return mem_of(d)->use(use_of_output(d)); };
         // a primitive on the second stream starts when everything issued before it on the first has finished (its
         // inputs, and whatever used its output buffer before); its user waits for it
         cldnn_hip_engine where = eng->h;
@@ -178,9 +192,12 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
         const cldnn_hip_tensor ot = to_hip(n->out);
         switch (p.type) {
         case prim_type::reorder: {
-            cldnn_memory_impl* in = mem_of(n->deps[0]);
-            const cldnn_hip_tensor it = to_hip(n->deps[0]->out);
-            hip_check(cldnn_hip_reorder(eng->h, in->device_ptr(), &it, out->device_ptr(), &ot));
+            node* src = n->deps[0];
+            // an image that only this reorder reads need not be copied to the device first
+            const bool once = src->p->type == prim_type::input_layout && src->users.size() == 1;
+            const void* in = mem_of(src)->use(once ? CLDNN_HIP_USE_READ_ONCE : CLDNN_HIP_USE_READ);
+            const cldnn_hip_tensor it = to_hip(src->out);
+            hip_check(cldnn_hip_reorder(eng->h, in, &it, out_of(n), &ot));
             break;
         }
         case prim_type::concatenation: {
@@ -189,21 +206,19 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
             int at[4] = {0, 0, 0, 0};  // b, f, x, y
             for (size_t i = 0; i < p.inputs.size(); ++i) {
                 const cldnn_hip_tensor it = to_hip(n->deps[i]->out);
-                hip_check(cldnn_hip_copy_region(eng->h, mem_of(n->deps[i])->device_ptr(), &it, out->device_ptr(), &ot, at[0], at[1], at[3], at[2]));
+                hip_check(cldnn_hip_copy_region(eng->h, mem_of(n->deps[i])->read_ptr(), &it, mem_of(n)->use(CLDNN_HIP_USE_UPDATE), &ot, at[0], at[1], at[3], at[2]));
                 at[p.concat_axis] += n->deps[i]->out.size.sizes[p.concat_axis];
             }
             break;
         }
         case prim_type::pooling: {
-            cldnn_memory_impl* in = mem_of(n->deps[0]);
             cldnn_hip_pooling_desc pd = pooling_descriptor(n);
-            hip_check(cldnn_hip_pooling(eng->h, &pd, in->device_ptr(), out->device_ptr()));
+            hip_check(cldnn_hip_pooling(eng->h, &pd, mem_of(n->deps[0])->read_ptr(), out_of(n)));
             break;
         }
         case prim_type::activation: {
-            cldnn_memory_impl* in = mem_of(n->deps[0]);
             const cldnn_hip_tensor it = to_hip(n->deps[0]->out);
-            hip_check(cldnn_hip_activation(eng->h, in->device_ptr(), &it, out->device_ptr(), &ot, hip_activation_code(p.act_func),
+            hip_check(cldnn_hip_activation(eng->h, mem_of(n->deps[0])->read_ptr(), &it, out_of(n), &ot, hip_activation_code(p.act_func),
                                            p.act_a, p.act_b));
             break;
         }
@@ -215,7 +230,7 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
             d.mode = p.eltw_mode, d.n_inputs = (int32_t)count;
             for (size_t i = 0; i < count; ++i) {
                 d.inputs[i] = to_hip(n->deps[i]->out);
-                src[i] = mem_of(n->deps[i])->device_ptr();
+                src[i] = mem_of(n->deps[i])->read_ptr();
                 d.stride_x[i] = p.eltw_stride.empty() ? 1 : p.eltw_stride[i].sizes[2];
                 d.stride_y[i] = p.eltw_stride.empty() ? 1 : p.eltw_stride[i].sizes[3];
                 d.coefficients[i] = p.eltw_coefficients.empty() ? 1.0f : p.eltw_coefficients[i];
@@ -223,35 +238,35 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
             d.has_coefficients = !p.eltw_coefficients.empty();
             d.output = ot;
             const float* calib = nullptr;
-            if (!p.eltw_calib.empty()) calib = (const float*)mem_of(n->deps[count])->device_ptr();
+            if (!p.eltw_calib.empty()) calib = (const float*)mem_of(n->deps[count])->read_ptr();
             const bool int_data = n->deps[0]->out.data_type == cldnn_i8 || n->deps[0]->out.data_type == cldnn_u8;
             d.quantized = int_data && (calib || p.eltw_oqf != 1.0f);
             d.output_quantization_factor = p.eltw_oqf;
             d.activation = CLDNN_HIP_ACT_NONE;
             if (p.eltw_with_act) d.activation = p.eltw_slope == 0.0f ? CLDNN_HIP_ACT_RELU : CLDNN_HIP_ACT_RELU_SLOPE;
             d.m = p.eltw_slope;
-            hip_check(cldnn_hip_eltwise(eng->h, &d, src, calib, out->device_ptr()));
+            hip_check(cldnn_hip_eltwise(eng->h, &d, src, calib, out_of(n)));
             break;
         }
         case prim_type::convolution:
         case prim_type::fused_conv_eltwise: {
             if (n->chain_head) break;  // written by the launch of its chain's head
             if (n->sibling_head) break;  // written by the launch of the convolution it is paired with
-            cldnn_memory_impl* in = mem_of(n->deps[0]);
+            const void* in = mem_of(n->deps[0])->read_ptr();
             if (n->chain) {
                 void* outs[3] = {nullptr, nullptr, nullptr};
                 const void* eltws[3] = {nullptr, nullptr, nullptr};
                 for (size_t k = 0; k < n->chain_members.size(); ++k) {
                     node* m = n->chain_members[k];
-                    if (n->chain_keep[k]) outs[k] = mem_of(m)->device_ptr();
-                    if (m->p->type == prim_type::fused_conv_eltwise) eltws[k] = mem_of(m->deps[1])->device_ptr();
+                    if (n->chain_keep[k]) outs[k] = out_of(m);
+                    if (m->p->type == prim_type::fused_conv_eltwise) eltws[k] = mem_of(m->deps[1])->read_ptr();
                 }
-                hip_check(cldnn_hip_conv_chain_enqueue(n->chain, in->device_ptr(), outs, eltws));
+                hip_check(cldnn_hip_conv_chain_enqueue(n->chain, in, outs, eltws));
                 break;
             }
             const void* eltw = nullptr;
-            if (p.type == prim_type::fused_conv_eltwise && !p.second_input_in_output) eltw = mem_of(n->deps[1])->device_ptr();
-            hip_check(cldnn_hip_conv_enqueue(n->conv, in->device_ptr(), out->device_ptr(), eltw));
+            if (p.type == prim_type::fused_conv_eltwise && !p.second_input_in_output) eltw = mem_of(n->deps[1])->read_ptr();
+            hip_check(cldnn_hip_conv_enqueue(n->conv, in, out_of(n), eltw));
             break;
         }
         default: break;
@@ -272,21 +287,25 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
         }
         net->executed.push_back(p.id);
     }
-    if (deferred_marker) {
-        hip_check(cldnn_hip_event_record_deferred(deferred_marker->h));
-    } else {
-        // one marker for every output that has no event of its own (reference ocl_toolkit.cpp:170-178,197-230)
-        ref<cldnn_event_impl> marker;
-        for (auto& u : prog->nodes) {
-            node* n = u.get();
-            if (!n->is_output || net->events.count(n)) continue;
-            if (!marker) {
-                marker = ref<cldnn_event_impl>(new cldnn_event_impl(), false);
-                marker->engine = ref<cldnn_engine_impl>(eng, true);
-                hip_check(cldnn_hip_event_record(eng->h, &marker->h));
-            }
-            net->events[n] = marker;
+    {
+        std::lock_guard<std::mutex> g(eng->marking);
+        ref<cldnn_event_impl> marker(deferred_marker, true);
+        if (marker) {
+            hip_check(cldnn_hip_event_record_deferred(marker->h));
+        } else {
+            // one marker for every output that has no event of its own (reference ocl_toolkit.cpp:170-178,197-230)
+            marker = ref<cldnn_event_impl>(new cldnn_event_impl(), false);
+            marker->engine = ref<cldnn_engine_impl>(eng, true);
+            hip_check(cldnn_hip_event_record(eng->h, &marker->h));
+            for (auto& u : prog->nodes)
+                if (u->is_output && !net->events.count(u.get())) net->events[u.get()] = marker;
         }
+        net->run_end = marker;
+        for (auto& u : prog->nodes)
+            if (u->is_output || u->constant || u->p->type == prim_type::input_layout) {
+                auto it = net->mem.find(u.get());
+                if (it != net->mem.end() && it->second) it->second->last_use = marker;
+            }
     }
     if (eng->side) hip_check(cldnn_hip_engine_flush(eng->side));
     hip_check(cldnn_hip_engine_flush(eng->h));
@@ -1002,7 +1021,12 @@ void cldnn_set_network_input(cldnn_network network, cldnn_primitive_id id, cldnn
                      std::string("primitive ") + id + " is not an input");
         // the previous run must be over before its input is replaced (reference network.cpp:112-113)
         await_pending_run(network);
-        hip_check(cldnn_hip_engine_finish(prog->engine->h));
+        ref<cldnn_event_impl> run_end;
+        {
+            std::lock_guard<std::mutex> state(network->run_state);
+            run_end = network->run_end;
+        }
+        if (run_end) hip_check(cldnn_hip_event_wait(run_end->h));
         HOST_REQUIRE(same_layout(mem->layout, it->second->out), CLDNN_INVALID_ARG, "set_network_input: memory layout differs from the input's layout");
         network->mem[it->second] = on_engine(prog->engine.get(), mem);
         network->input_set[id] = true;
@@ -1174,7 +1198,12 @@ void* cldnn_lock_memory(cldnn_memory memory, cldnn_status* status)
     return guard<void*>(status, nullptr, [&]() -> void* {
         HOST_REQUIRE(memory, CLDNN_INVALID_ARG, "Memory should not be null.");
         if (memory->attached) return memory->attached;
-        void* p = cldnn_hip_buffer_lock(memory->buf);
+        ref<cldnn_event_impl> last;
+        {
+            std::lock_guard<std::mutex> g(memory->engine->marking);
+            last = memory->last_use;
+        }
+        void* p = cldnn_hip_buffer_map(memory->buf, last ? last->h : nullptr);
         if (!p) throw api_error(CLDNN_DEVICE_ERROR, cldnn_hip_last_error());
         return p;
     });
@@ -1184,7 +1213,7 @@ void cldnn_unlock_memory(cldnn_memory memory, cldnn_status* status)
 {
     guard_void(status, [&] {
         HOST_REQUIRE(memory, CLDNN_INVALID_ARG, "Memory should not be null.");
-        if (!memory->attached) hip_check(cldnn_hip_buffer_unlock(memory->buf));
+        if (!memory->attached) hip_check(cldnn_hip_buffer_unmap(memory->buf));
     });
 }
 

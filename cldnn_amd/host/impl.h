@@ -86,8 +86,15 @@ struct cldnn_engine_impl : host::refcounted {
     cldnn_hip_engine side = nullptr;  // second stream for primitives nothing waits for yet (enable_parallelisation)
     bool profiling = false;
     std::string tuning_cache_path = "cache.json";  // engine configuration; a tuning_config without a path of its own uses it
+    std::mutex marking;  // held while a run's last event is recorded and noted on the memories it used: same order in both
     bool memory_pool = true;  // networks share buffers between intermediate tensors whose lifetimes do not overlap
     ~cldnn_engine_impl() override;
+};
+
+struct cldnn_event_impl : host::refcounted {
+    host::ref<cldnn_engine_impl> engine;
+    cldnn_hip_event h = nullptr;
+    ~cldnn_event_impl() override;
 };
 
 struct cldnn_memory_impl : host::refcounted {
@@ -98,18 +105,17 @@ struct cldnn_memory_impl : host::refcounted {
     size_t attached_bytes = 0;
     host::ref<cldnn_memory_impl> view_of;  // a window into another memory's buffer (input of an in-place concatenation)
     size_t view_offset = 0;
+    host::ref<cldnn_event_impl> last_use;  // behind the last run that used it (inputs and outputs; engine->marking)
     ~cldnn_memory_impl() override;
-    void* device_ptr() const
+    cldnn_memory_impl* root() { return view_of ? view_of->root() : this; }
+    // the pointer for work enqueued next (CLDNN_HIP_USE_*); a window's write is a partial one
+    void* use(int32_t how)
     {
-        if (view_of) return (char*)view_of->device_ptr() + view_offset;
-        return buf ? cldnn_hip_buffer_device_ptr(buf) : nullptr;
+        if (view_of) return (char*)root()->use(how == CLDNN_HIP_USE_READ ? how : CLDNN_HIP_USE_UPDATE) + offset();
+        return buf ? cldnn_hip_buffer_use(buf, how) : nullptr;
     }
-};
-
-struct cldnn_event_impl : host::refcounted {
-    host::ref<cldnn_engine_impl> engine;
-    cldnn_hip_event h = nullptr;
-    ~cldnn_event_impl() override;
+    size_t offset() const { return view_of ? view_offset + view_of->offset() : 0; }
+    const void* read_ptr() { return use(CLDNN_HIP_USE_READ); }
 };
 
 namespace host {
@@ -252,6 +258,7 @@ struct cldnn_network_impl : host::refcounted {
     std::map<std::string, bool> input_set;
     std::vector<std::string> executed;
     std::vector<cldnn_hip_event> stream_events;  // fork / join events between the two streams of the last run
+    host::ref<cldnn_event_impl> run_end;  // behind everything the last submitted run enqueued
     bool has_run = false;
     size_t allocated_bytes = 0;  // device bytes of the buffers the network allocated for its primitives' outputs
     size_t pooled_tensors = 0;   // outputs that reuse the buffer of an earlier, finished tensor

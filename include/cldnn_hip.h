@@ -83,6 +83,22 @@ cldnn_hip_status cldnn_hip_buffer_retain(cldnn_hip_buffer b);
 cldnn_hip_status cldnn_hip_buffer_release(cldnn_hip_buffer b);
 void* cldnn_hip_buffer_lock(cldnn_hip_buffer b);     /* NULL on failure */
 cldnn_hip_status cldnn_hip_buffer_unlock(cldnn_hip_buffer b);
+/* The same for a buffer whose device pointer is only taken through cldnn_hip_buffer_use, so that the library knows which
+ * copy is current: map copies device -> shadow only if the device wrote since, and after the last unmap the shadow is the
+ * current copy until a use needs it on the device.  Both forms may be mixed on one buffer.
+ * last_use: an event recorded behind all work on the buffer, waited for instead of the stream (may be NULL). */
+void* cldnn_hip_buffer_map(cldnn_hip_buffer b, cldnn_hip_event last_use);  /* NULL on failure */
+cldnn_hip_status cldnn_hip_buffer_unmap(cldnn_hip_buffer b);
+enum {
+    CLDNN_HIP_USE_READ = 0,           /* the work enqueued next reads it */
+    CLDNN_HIP_USE_READ_ONCE = 1,      /* ... once, every byte at most once: may hand out the shadow itself */
+    CLDNN_HIP_USE_UPDATE = 2,         /* writes part of it */
+    CLDNN_HIP_USE_WRITE = 3,          /* overwrites all of it */
+    CLDNN_HIP_USE_WRITE_FOR_HOST = 4  /* overwrites all of it, and the host is the next reader: may hand out the shadow */
+};
+/* the pointer for that work (device-accessible; NULL on failure), to be enqueued on the buffer's engine before the next
+ * call on the buffer */
+void* cldnn_hip_buffer_use(cldnn_hip_buffer b, int32_t use);
 /* gpu_buffer::fill (reference src/gpu/memory_gpu.cpp:87-90) */
 cldnn_hip_status cldnn_hip_buffer_fill(cldnn_hip_buffer b, uint8_t pattern);
 void* cldnn_hip_buffer_device_ptr(cldnn_hip_buffer b);

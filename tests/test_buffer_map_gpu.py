@@ -1,0 +1,68 @@
+"""Which copy of a mapped buffer is current (cldnn_hip_buffer_map / _unmap / _use): every order of host writes and device
+uses gives the bytes written last, also where a kernel reads or writes the host copy in place."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from cldnn_amd import api as cl
+from cldnn_amd import hip
+
+pytestmark = pytest.mark.gpu
+READ, READ_ONCE, UPDATE, WRITE, WRITE_FOR_HOST = range(5)
+
+
+def mapped(buf):
+    p = hip.lib().cldnn_hip_buffer_map(buf.h, None)
+    assert p
+    return np.frombuffer((C.c_uint8 * buf.nbytes).from_address(p), np.uint8)
+
+
+def copy(eng, src, how_src, dst, how_dst):
+    L = hip.lib()
+    hip.check(L.cldnn_hip_reorder(eng.h, L.cldnn_hip_buffer_use(src.h, how_src), C.byref(src.tensor),
+                                  L.cldnn_hip_buffer_use(dst.h, how_dst), C.byref(dst.tensor)))
+
+
+@pytest.mark.parametrize("features", [1, 33, 16 * 5000], ids=["one_byte", "few", "beyond_the_in_place_limits"])
+@pytest.mark.parametrize("how_src", [READ, READ_ONCE])
+@pytest.mark.parametrize("how_dst", [WRITE, UPDATE, WRITE_FOR_HOST])
+def test_last_write_wins(features, how_src, how_dst):
+    eng, L = hip.Engine(0), hip.lib()
+    t = hip.Tensor.make(hip.U8, hip.BFYX, 1, features, 1, 61)
+    src, dst = hip.Buffer(eng, t), hip.Buffer(eng, t)
+    r = np.random.default_rng(features)
+    for turn in range(3):
+        data = r.integers(0, 256, src.nbytes, dtype=np.uint8)
+        mapped(src)[:] = data
+        hip.check(L.cldnn_hip_buffer_unmap(src.h))
+        for _ in range(2):  # the second read finds the device copy brought up to date
+            copy(eng, src, how_src, dst, how_dst)
+        m = mapped(dst)
+        assert np.array_equal(m, data)
+        m[0] ^= 255  # what the host changes in a result is seen by the next reader on the device
+        hip.check(L.cldnn_hip_buffer_unmap(dst.h))
+        copy(eng, dst, READ, src, WRITE)
+        data[0] ^= 255
+        assert np.array_equal(src.read_raw(), data)  # the copies of the plain entry points follow too
+        assert np.array_equal(dst.read_raw(), data)
+    for b in (src, dst):
+        b.close()
+    eng.close()
+
+
+def test_input_rewritten_and_reused_between_runs():
+    """one input memory: written once and run twice, then rewritten; two networks share it"""
+    eng = cl.engine()
+    F, DT = cl.format, cl.data_types
+    lay = cl.layout(DT.u8, F.bfyx, cl.tensor(2, 3, 9, 7))
+    nets = [cl.network(eng, cl.topology(cl.input_layout("x", lay), cl.reorder("y", "x", f, DT.f32))) for f in (F.bfyx, F.yxfb)]
+    r = np.random.default_rng(5)
+    mem = cl.memory.allocate(eng, lay)
+    for _ in range(3):
+        x = r.integers(0, 256, (2, 3, 7, 9), dtype=np.uint8)
+        mem.write(x)
+        for n in nets + nets:
+            n.set_input_data("x", mem)
+            assert np.array_equal(n.execute()["y"].get_memory().read(), x.astype(np.float32))
+        assert np.array_equal(mem.read(), x)
