@@ -250,6 +250,7 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
         c->fast = mfma_fast_epilogue(p, probe, calib_on ? calib : nullptr, eltw_calib, wqf, &c->fe);
     }
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE && e.fc) c->fast = false;  // the depthwise kernels have no short fully_connected form
+    if (impl == CLDNN_HIP_IMPL_DEPTHWISE && c->fe.f32) c->fast = false;  // nor a float one
     const bool dw_fast = impl == CLDNN_HIP_IMPL_DEPTHWISE && dw_fast_applies(p, c->fast);
     const bool xor_u8 = (impl == CLDNN_HIP_IMPL_MFMA || dw_fast) && p.in_dt == CLDNN_HIP_U8;
     for (int f = 0; f < p.OFM; ++f) {
@@ -287,7 +288,7 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
     if (impl == CLDNN_HIP_IMPL_MFMA) {
         int tile = d.tile_override > 0 ? d.tile_override - 1 : mfma_choose(p, c->engine->props.multiProcessorCount);
         CHIP_REQUIRE(tile >= 0 && tile < tile_config_count(), CLDNN_HIP_INVALID_ARG, "tile_override out of range");
-        c->mplan = mfma_plan(p, tile, c->engine->props.multiProcessorCount);
+        c->mplan = mfma_plan(p, tile, c->engine->props.multiProcessorCount, d.tile_override > 0);
         std::vector<int8_t> packed(c->mplan.packed_bytes);
         std::vector<int32_t> ktab(c->mplan.ktab_bytes / sizeof(int32_t));
         mfma_pack_weights(p, c->mplan, w8, packed.data(), ktab.data());
@@ -296,9 +297,9 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
         if (const size_t g = mfma_gather_bytes(p, c->mplan)) c->gather = upload(c, nullptr, 0, g);
         const TileConfig& tc = tile_config(tile);
         inf.tile_index = tile, inf.tile_pixels = tc.tile_pixels, inf.tile_ofm = tc.tile_ofm;
-        inf.grid = c->mplan.grid, inf.block = c->mplan.gemv ? 64 * c->mplan.gemv_waves : c->mplan.block, inf.lds_bytes = c->mplan.lds_bytes;
-        std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_%s<%s,%s,%s>", c->mplan.gemv ? "gemv" : c->mplan.halo ? "halo" : c->mplan.stream ? "stream" : (c->mplan.bdir ? "bdir" : (c->mplan.wsl ? "wsl" : "mfma")),
-                      tc.name, c->mplan.checked ? "checked" : "border", c->fast && !c->mplan.gemv ? "fast" : "generic");
+        inf.grid = c->mplan.grid, inf.block = c->mplan.ksplit ? 64 * c->mplan.ks_waves : c->mplan.block, inf.lds_bytes = c->mplan.lds_bytes;
+        std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_%s<%s,%s,%s>", c->mplan.gemv ? "gemv" : c->mplan.ksplit ? "ksplit" : c->mplan.halo ? "halo" : c->mplan.stream ? "stream" : (c->mplan.bdir ? "bdir" : (c->mplan.wsl ? "wsl" : "mfma")),
+                      tc.name, c->mplan.checked ? "checked" : "border", c->fast && !c->fe.f32 && !c->mplan.gemv ? "fast" : "generic");
     } else {
         c->dplan = dw_plan(p);
         std::vector<int8_t> packed(c->dplan.packed_bytes);

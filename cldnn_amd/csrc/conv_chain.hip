@@ -65,6 +65,7 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
         const ConvProblem& p = *st[k].p;
         const std::string at = "stage " + std::to_string(k) + ": ";
         if (!st[k].fast) return at + "needs the short int8 epilogue";
+        if (st[k].fe->f32) return at + "float output is not chained";
         if (st[k].fe->fc) return at + "the fully_connected form is not chained";
         const bool dw0 = k == 0 && st[0].dw_wmask != nullptr;
         if (p.groups != 1 && !dw0) return at + "grouped convolution";
@@ -100,7 +101,7 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
             if (k > 0) {
                 MfmaPlan mp{};
                 try {
-                    mp = mfma_plan(*st[k].p, ROW_P64_F64_FOR_DWCHAIN, cus);
+                    mp = mfma_plan(*st[k].p, ROW_P64_F64_FOR_DWCHAIN, cus, true);
                 } catch (const error& e) {
                     return "stage " + std::to_string(k) + ": " + e.what();
                 }
@@ -132,7 +133,7 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
     for (int k = 0; k < n; ++k) {
         ConvProblem q = *st[k].p;
         try {
-            mp[k] = mfma_plan(q, ROW_WSL_P64_FOR_CHAIN, cus);
+            mp[k] = mfma_plan(q, ROW_WSL_P64_FOR_CHAIN, cus, true);
         } catch (const error&) {
             // K beyond what that row keeps in LDS: only the K-step count is wanted here
             mp[k] = MfmaPlan{};
@@ -272,7 +273,7 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
         }
     }
     for (int k = pl.dw ? 1 : 0; k < pl.stages; ++k) {
-        const MfmaPlan mp = mfma_plan(*st[k].p, pl.dw ? ROW_P64_F64_FOR_DWCHAIN : ROW_WSL_P64_FOR_CHAIN, cus);
+        const MfmaPlan mp = mfma_plan(*st[k].p, pl.dw ? ROW_P64_F64_FOR_DWCHAIN : ROW_WSL_P64_FOR_CHAIN, cus, true);
         std::vector<int8_t> buf(mp.packed_bytes);
         std::vector<int32_t> ktab(mp.ktab_bytes / sizeof(int32_t));
         mfma_pack_weights(*st[k].p, mp, w[k], buf.data(), ktab.data());

@@ -334,6 +334,7 @@ void launch_halo_instance(hipStream_t s, const HaloArgs& h, int grid, int lds, i
     case EPI_KIND_FUSED: HALO_LAUNCH(EPI_KIND_FUSED) break;
     case EPI_KIND_LINEAR: HALO_LAUNCH(EPI_KIND_LINEAR) break;
     case EPI_KIND_FAST: HALO_LAUNCH(EPI_KIND_FAST) break;
+    case EPI_KIND_F32: HALO_LAUNCH(EPI_KIND_F32) break;
     default: HALO_LAUNCH(EPI_KIND_GENERIC) break;
     }
 #undef HALO_LAUNCH

@@ -16,7 +16,7 @@ void launch_bdir_f64(hipStream_t s, const MfmaArgs& a, int nt, int grid, int lds
 void launch_bdir_f128(hipStream_t s, const MfmaArgs& a, int nt, int grid, int lds, int epi);
 void launch_bdir_k2(hipStream_t s, const MfmaArgs& a, int nt, int grid, int lds, int epi);
 void launch_bdir_k4(hipStream_t s, const MfmaArgs& a, int nt, int grid, int lds, int epi);
-void launch_gemv(hipStream_t s, const MfmaArgs& a, int grid, int waves, int mtiles);
+void launch_ksplit(hipStream_t s, const MfmaArgs& a, int ft, int pt, int grid, bool lanes, int epi);
 size_t gemv_gather_bytes(int mtiles, int ksteps);
 size_t gemv_static_scratch_bytes();
 void* gemv_static_scratch(int device);
@@ -56,8 +56,8 @@ static const TileConfig g_tiles[] = {
     // first layers (at most 4 input features) read b_fs_yx_fsv4: a 16-byte fragment is 4 horizontal taps x 4 features;
     // streaming kernel
     {"stem_p32", 32, 64, 32},
-    // few pixels, long K (fully_connected): a workgroup owns one 16-feature fragment of a 64-feature tile and 16
-    // pixels; its waves split K and stream both operands straight from global memory
+    // few pixels, long K (fully_connected): split-K kernel on 16 pixels x 16 features of a 64-feature span, with the gather
+    // in front where the filter is wider than one tap
     {"gemv_p16_f16", 16, 64, 16},
     // first layers with several K-steps (a 7x7 filter): 64 pixels per wave, so the weights are fetched half as often
     {"stem_p64", 64, 64, 64},
@@ -65,8 +65,15 @@ static const TileConfig g_tiles[] = {
     // owns 64 positions x 128 features.  tile_pixels counts positions of the bordered input.
     {"halo_p256_f128", 256, 128, 64},   // 4 waves, two workgroups per CU
     {"halo_p512_f128", 512, 128, 64},   // 8 waves, one workgroup per CU (rows too long for two patches of 256 + halo in 80 KB)
+    // split-K kernel: weights packed for 64-feature spans, a workgroup takes fN features of one
+    {"ksplit_p16_f16", 16, 64, 16},
+    {"ksplit_p32_f16", 32, 64, 32},
+    {"ksplit_p64_f16", 64, 64, 64},
+    {"ksplit_p32_f32", 32, 64, 32},
+    {"ksplit_p32_f64", 32, 64, 32},
 };
-enum { FIRST_STREAM_ROW = 6, FIRST_BDIR_ROW = 8, FIRST_WSL_ROW = 14, FIRST_BDIRK_ROW = 17, STEM_ROW = 20, GEMV_ROW = 21, STEM_P64_ROW = 22, FIRST_HALO_ROW = 23 };
+static const struct { int ft, pt; } g_ksplit[] = {{1, 1}, {1, 2}, {1, 4}, {2, 2}, {4, 2}};
+enum { FIRST_STREAM_ROW = 6, FIRST_BDIR_ROW = 8, FIRST_WSL_ROW = 14, FIRST_BDIRK_ROW = 17, STEM_ROW = 20, GEMV_ROW = 21, STEM_P64_ROW = 22, FIRST_HALO_ROW = 23, FIRST_KSPLIT_ROW = 25 };
 enum { HALO_RING = 4, HALO_TAPS = 9 };
 enum { WSL_MAX_LDS = 160 * 1024 };
 enum { MFMA_SLACK_STEPS = 40 };  // >= weight look-ahead + activation look-ahead + 3
@@ -133,6 +140,37 @@ static int choose_lds_tile(const ConvProblem& p, int64_t m, int cus)
     return best;
 }
 
+// Microseconds of a split-K tile and of the best tile kernel at sizes where neither fills the chip twice, fitted to sweeps
+// of 43 layers (batch 1 to 32, 1x1 to 5x5; both within 15 %).  A split-K workgroup brings (features + pixels) * K bytes to
+// its CU at 115 bytes a nanosecond after a start of 0.9 us; a tile kernel walks its K-steps in 0.165 us each, two workgroups
+// per CU at the same speed, and its split form halves the walk.
+static double ksplit_us(int64_t m, int ofm, int ksteps, int cus, int ft, int pt)
+{
+    const double groups = (double)((m + 16 * pt - 1) / (16 * pt)) * ((ofm + 63) / 64) * (4 / ft);
+    const double rounds = groups <= cus ? 1.0 : std::max(1.5, groups / cus);  // a few groups more than CUs cost half a round
+    return 2.2 + rounds * (0.9 + 16.0 * (ft + pt) * 64 * ksteps / 115000.0);
+}
+static double tile_kernel_us(int64_t m, int ofm, int ksteps, int cus, bool direct)
+{
+    const double groups = (double)((m + 63) / 64) * ((ofm + 63) / 64);
+    return 3.3 + 0.165 * std::max(1.0, groups / (2 * cus)) * (direct && ksteps >= 32 && m < 4096 ? ksteps / 2 : ksteps);
+}
+// row of the split-K kernel that should beat the tile kernels by a tenth, or -1
+static int choose_ksplit(int64_t m, int ofm, int taps, int cb, int ksteps, bool border, int cus)
+{
+    // shorter walks gain less than a microsecond, and what is left of them is the launch
+    if (ksteps < (taps > 1 ? 10 : 5)) return -1;
+    const bool uniform = border && cb >= 4;
+    const int own_steps = uniform ? taps * ((cb + 3) / 4) : ksteps;
+    int best = -1;
+    double best_us = 0.9 * tile_kernel_us(m, ofm, ksteps, cus, border && cb % 4 == 0);
+    for (int i = 0; i < (int)(sizeof(g_ksplit) / sizeof(g_ksplit[0])); ++i) {
+        const double us = ksplit_us(m, ofm, own_steps, cus, g_ksplit[i].ft, g_ksplit[i].pt);
+        if (us < best_us) best_us = us, best = FIRST_KSPLIT_ROW + i;
+    }
+    return best;
+}
+
 int mfma_choose(const ConvProblem& p, int cus)
 {
     if (p.in_t.format == CLDNN_HIP_FMT_B_FS_YX_FSV4)
@@ -149,6 +187,9 @@ int mfma_choose(const ConvProblem& p, int cus)
     // a fragment or two of pixels and a long K (fully_connected): the weights are the traffic and the tile kernels
     // would occupy one workgroup per 64 features
     if (direct && m <= 32 && ksteps >= 16) return ROW_GEMV;
+    if (const int row = choose_ksplit(m, p.OFM, p.FY * p.FX, cb, ksteps, border, cus); row >= 0) return row;
+    // a few pixels and K <= 256: one round trip per wave and no barrier (3.0-3.4 us against 3.5-3.7 for the LDS tiles)
+    if (border && ksteps <= 4 && m < 4096 && !stream_fits) return ROW_STREAM_P16;
     if (ksteps <= 2 || !direct) {
         // one or two K-steps (or a first layer with three input features): bound by HBM bandwidth
         if (!direct && ksteps >= 3 && m >= 500000) return choose_lds_tile(p, m, cus);  // VGG conv1
@@ -212,7 +253,7 @@ static void wsl_depth(int ksteps, int* depth, int* padded)
     *depth = best_d, *padded = best_pad;
 }
 
-MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus)
+MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus, bool forced)
 {
     const TileConfig& tc = g_tiles[tile];
     MfmaPlan pl{};
@@ -223,9 +264,16 @@ MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus)
                  "b_fs_yx_fsv4 input goes with the first-layer row of the tile table and only with it");
     pl.stream = (tile >= FIRST_STREAM_ROW && tile < FIRST_BDIR_ROW) || pl.stem ? 1 : 0;
     pl.gemv = tile == GEMV_ROW ? 1 : 0;
-    pl.halo = tile >= FIRST_HALO_ROW ? 1 : 0;
+    pl.halo = tile >= FIRST_HALO_ROW && tile < FIRST_KSPLIT_ROW ? 1 : 0;
+    pl.ksplit = pl.gemv || tile >= FIRST_KSPLIT_ROW ? 1 : 0;
+    if (pl.ksplit) {
+        pl.ks_ft = pl.gemv ? 1 : g_ksplit[tile - FIRST_KSPLIT_ROW].ft;
+        pl.ks_pt = pl.gemv ? 1 : g_ksplit[tile - FIRST_KSPLIT_ROW].pt;
+        // 17 to 32 pixels: both fragments in one workgroup, so that every weight byte crosses to a CU once
+        if (pl.gemv && !forced && (int64_t)p.B * p.OH * p.OW > 16) pl.ks_pt = 2;
+    }
     pl.block = 256;
-    pl.bdir = ((tile >= FIRST_BDIR_ROW && tile < FIRST_WSL_ROW) || tile >= FIRST_BDIRK_ROW) && !pl.stem && !pl.gemv && !pl.halo ? 1 : 0;
+    pl.bdir = ((tile >= FIRST_BDIR_ROW && tile < FIRST_WSL_ROW) || tile >= FIRST_BDIRK_ROW) && !pl.stem && !pl.ksplit && !pl.halo ? 1 : 0;
     pl.wsl = tile >= FIRST_WSL_ROW && tile < FIRST_BDIRK_ROW ? 1 : 0;
     CHIP_REQUIRE(!(pl.stream && pl.checked), CLDNN_HIP_INVALID_ARG,
                  "the streaming kernel needs an input whose physical zero border covers the convolution's padding");
@@ -234,7 +282,11 @@ MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus)
                               "the first-layer kernel takes at most 4 input features and no horizontal dilation");
     CHIP_REQUIRE(!(pl.bdir || pl.wsl || pl.gemv || pl.halo) || (!pl.checked && pl.cb % 4 == 0), CLDNN_HIP_INVALID_ARG,
                  "the direct-activation kernels need a zero border covering the padding and input features in multiples of 64");
-    pl.kchunks = pl.stem ? p.FY * ((p.FX + 3) / 4) : p.FY * p.FX * pl.cb;  // first layer: a chunk is 4 horizontal taps
+    if (pl.ksplit) {
+        pl.ks_lanes = pl.checked || pl.cb < 4 ? 1 : 0;
+        pl.shifted = !pl.ks_lanes && pl.cb % 4 != 0 ? 1 : 0;
+    }
+    pl.kchunks = pl.shifted ? p.FY * p.FX * ((pl.cb + 3) / 4 * 4) : pl.stem ? p.FY * ((p.FX + 3) / 4) : p.FY * p.FX * pl.cb;  // first layer: a chunk is 4 horizontal taps
     pl.ksteps = (pl.kchunks + 3) / 4;
     if (pl.stream) {
         CHIP_REQUIRE(pl.ksteps <= 8, CLDNN_HIP_INVALID_ARG, "the streaming kernel handles at most 8 K-steps (K <= 512)");
@@ -251,7 +303,7 @@ MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus)
     // K order.  With the taps innermost, consecutive K-steps of a wave read the same cache lines of the input shifted
     // by one pixel (or one row), so most activation loads of a 3x3 filter hit in the CU's L1 instead of going to L2.
     // The weights-stationary and streaming kernels walk the taps with counters in (tap, slice) order.
-    pl.tap_minor = !pl.stream && !pl.wsl && pl.cb % 4 == 0 && p.FY * p.FX > 1 ? 1 : 0;
+    pl.tap_minor = pl.shifted || (!pl.stream && !pl.wsl && !pl.ks_lanes && pl.cb % 4 == 0 && p.FY * p.FX > 1) ? 1 : 0;
     if (pl.halo) {
         const cldnn_hip_tensor& t = p.in_t;
         CHIP_REQUIRE(p.FY * p.FX == HALO_TAPS && p.sy == 1 && p.sx == 1 && p.groups == 1, CLDNN_HIP_INVALID_ARG,
@@ -280,7 +332,7 @@ MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus)
     if (pl.halo) pl.mtiles = pl.halo_ptiles;
     // which operand do the eight dies share out?  the larger one (it is then read from memory once, not 8 times)
     const int64_t w_bytes = (int64_t)p.OFM * (p.IFM / p.groups) * p.FY * p.FX, in_bytes = (int64_t)p.B * p.IFM * p.IH * p.IW;
-    pl.by_features = !pl.stream && !pl.wsl && !pl.gemv && !pl.halo && w_bytes > in_bytes && (p.OFM + tc.tile_ofm - 1) / tc.tile_ofm >= 8 ? 1 : 0;
+    pl.by_features = !pl.stream && !pl.wsl && !pl.ksplit && !pl.halo && w_bytes > in_bytes && (p.OFM + tc.tile_ofm - 1) / tc.tile_ofm >= 8 ? 1 : 0;
     int64_t grid = pl.by_features ? (int64_t)((pl.ofm_tiles + 7) / 8) * 8 * pl.mtiles : (int64_t)((pl.mtiles + 7) / 8) * 8 * pl.ofm_tiles;
     if (pl.stream) grid = ((int64_t)pl.mtiles * pl.ofm_tiles + 3) / 4;  // one wave per (pixel tile, span)
     pl.lds_bytes = pl.stream ? 0 : (pl.bdir ? 3 * 4 * tc.tile_ofm * 16 : 2 * 4 * (tc.tile_ofm + tc.tile_pixels) * 16);
@@ -311,12 +363,19 @@ MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus)
         pl.halo_parts = parts;
         grid = (int64_t)parts * pl.ofm_tiles;
     }
-    if (pl.gemv) {
-        // one workgroup per 16-feature fragment and 16 pixels; 4, 8 or 16 waves split K, at least eight steps (one
-        // look-ahead window) each
-        grid = (int64_t)pl.mtiles * pl.ofm_tiles * 4;
-        pl.gemv_waves = pl.ksteps >= 128 ? 16 : (pl.ksteps >= 64 ? 8 : 4);
-        pl.lds_bytes = 16 * 1024;
+    if (pl.ksplit) {
+        // 16 waves where each still gets two or three K-steps, fewer otherwise: a wave with one step costs its start and its
+        // share of the sums; 64 KB of LDS hold the partial tiles of 64 / (fragments per tile) waves
+        const int frags = pl.ks_ft * pl.ks_pt;
+        pl.ks_waves = pl.ksteps >= 32 ? 16 : (pl.ksteps >= 8 ? 8 : 4);
+        pl.ks_waves = std::max(std::min(pl.ks_waves, 64 / frags), frags);
+        pl.ks_per = (pl.ksteps + pl.ks_waves - 1) / pl.ks_waves;
+        const int64_t ftiles = (int64_t)pl.ofm_tiles * (4 / pl.ks_ft);
+        pl.mtiles = (int)((pl.m_total + 16 * pl.ks_pt - 1) / (16 * pl.ks_pt));
+        pl.by_features = w_bytes > in_bytes && ftiles >= 8 ? 1 : (pl.mtiles >= 8 && !pl.gemv ? 0 : 2);
+        if (pl.gemv) pl.by_features = 2;
+        grid = pl.by_features == 1 ? (ftiles + 7) / 8 * 8 * pl.mtiles : (pl.by_features == 0 ? (int64_t)((pl.mtiles + 7) / 8) * 8 * ftiles : ftiles * pl.mtiles);
+        pl.lds_bytes = pl.ks_waves * frags * 1024;
     }
     CHIP_REQUIRE(grid < (1ll << 31), CLDNN_HIP_UNSUPPORTED_SIZE, "convolution too large for one launch");
     pl.grid = (int)grid;
@@ -362,7 +421,12 @@ void mfma_pack_weights(const ConvProblem& p, const MfmaPlan& pl, const int8_t* w
     // k-chunk -> (tap, feature slice): tap-major with the slices innermost, or groups of 4 slices with the taps innermost
     const int taps = p.FY * p.FX;
     auto chunk_tap = [&](int kc) { return pl.tap_minor ? (kc / 4) % taps : kc / pl.cb; };
-    auto chunk_slice = [&](int kc) { return pl.tap_minor ? (kc / 4) / taps * 4 + kc % 4 : kc % pl.cb; };
+    auto chunk_slice = [&](int kc) {
+        if (pl.shifted) return std::min((kc / 4) / taps * 4, pl.cb - 4) + kc % 4;
+        return pl.tap_minor ? (kc / 4) / taps * 4 + kc % 4 : kc % pl.cb;
+    };
+    // a slice that the step before has multiplied already
+    auto chunk_repeated = [&](int kc) { return pl.shifted && chunk_slice(kc) < (kc / 4) / taps * 4; };
     for (int kc = 0; kc < (pl.ksteps + MFMA_SLACK_STEPS) * 4; ++kc) {
         if (kc >= pl.kchunks) {
             ktab[kc] = pl.checked ? (int32_t)0x80000000 : 0;  // padding chunk: zero weights
@@ -377,6 +441,7 @@ void mfma_pack_weights(const ConvProblem& p, const MfmaPlan& pl, const int8_t* w
         const int nt = f / BN;
         const int row = row_of(f);
         for (int kc = 0; kc < pl.kchunks; ++kc) {
+            if (chunk_repeated(kc)) continue;
             const int tap = chunk_tap(kc), cb = chunk_slice(kc);
             const int ks = kc / 4, kq = kc % 4;
             int8_t* dst = packed + ((((size_t)nt * pl.ksteps + ks) * 4 + kq) * BN + row) * 16;
@@ -408,6 +473,19 @@ bool mfma_fast_epilogue(const ConvProblem& p, const Epilogue& e, const float* ca
         F.fc = 1;
     } else if (e.bias) {
         return false;  // an int32 bias is folded into the accumulator start; a float bias takes the long path
+    }
+    if (e.out_dt == CLDNN_HIP_F32) {
+        if (e.fc || e.fused || e.split_f > 0 || e.mode != MODE_Q) return false;
+        if (!(e.act == CLDNN_HIP_ACT_NONE || e.act == CLDNN_HIP_ACT_RELU || e.act == CLDNN_HIP_ACT_CLAMP)) return false;
+        bool unit = e.iqf == 1.0f;
+        if (wqf)
+            for (int f = 0; f < p.OFM && unit; ++f) unit = wqf[f] == 1.0f;
+        F.f32 = 1;
+        F.has_wqf = wqf && !unit ? 1 : 0;
+        F.iqf = e.iqf;
+        F.act = e.act, F.act_m = e.act_m, F.act_n = e.act_n;
+        *out = F;
+        return true;
     }
     if (!(e.out_dt == CLDNN_HIP_S8 || e.out_dt == CLDNN_HIP_U8)) return false;
     if (e.split_f > 0) {
@@ -492,7 +570,7 @@ bool mfma_fast_epilogue(const ConvProblem& p, const Epilogue& e, const float* ca
 // a filter of one tap puts the 16 pixels' bytes of a K-step side by side already
 size_t mfma_gather_bytes(const ConvProblem& p, const MfmaPlan& pl)
 {
-    return pl.gemv && p.FY * p.FX > 1 ? gemv_gather_bytes(pl.mtiles, pl.ksteps) : 0;
+    return pl.gemv && p.FY * p.FX > 1 ? gemv_gather_bytes(pl.mtiles * pl.ks_pt, pl.ksteps) : 0;
 }
 
 size_t mfma_static_scratch_bytes() { return gemv_static_scratch_bytes(); }
@@ -552,8 +630,9 @@ void launch_conv_mfma(hipStream_t s, const ConvProblem& p, const MfmaPlan& pl, c
     if (fast && !raw) {
         a.fe = *fast;
         kind = EPI_KIND_FAST;
+        if (fast->f32) kind = EPI_KIND_F32;
         // the branch-free forms
-        if (!fast->has_wqf && epi.calib && !fast->fc) {
+        else if (!fast->has_wqf && epi.calib && !fast->fc) {
             if (!fast->fused && fast->relu_folded) kind = EPI_KIND_RELU;
             if (!fast->fused && fast->act == CLDNN_HIP_ACT_NONE) kind = EPI_KIND_LINEAR;
             if (fast->fused && fast->act == CLDNN_HIP_ACT_NONE && fast->eltw_relu_folded && epi.eltw_calib && !fast->conv_sat)
@@ -581,7 +660,13 @@ void launch_conv_mfma(hipStream_t s, const ConvProblem& p, const MfmaPlan& pl, c
             h.tap[k] = h.halo_lo + ((k / p.FX) * p.dy - p.py) * h.Wp + ((k % p.FX) * p.dx - p.px);
         launch_halo(s, h, pl.tile - FIRST_HALO_ROW, pl.halo_pl, pl.grid, pl.lds_bytes, kind);
     }
-    else if (pl.gemv) launch_gemv(s, a, pl.grid, pl.gemv_waves, pl.mtiles);  // element-wise epilogue only
+    else if (pl.ksplit) {
+        a.ofm_tiles = pl.ofm_tiles * (4 / pl.ks_ft);
+        a.div_ofm_tiles = make_div((uint32_t)a.ofm_tiles);
+        a.kwaves = pl.ks_waves, a.kper = pl.ks_per, a.checked = pl.checked, a.dil_y = p.dy, a.dil_x = p.dx;
+        a.div_taps = make_div((uint32_t)(p.FY * p.FX));
+        launch_ksplit(s, a, pl.ks_ft, pl.ks_pt, pl.grid, pl.ks_lanes != 0, kind);
+    }
     else if (pl.stream) launch_stream(s, a, tc.wave_pixels / 16, pl.grid, kind);
     else if (pl.bdir && tc.kgroups == 2) launch_bdir_k2(s, a, tc.wave_pixels / 16, pl.grid, pl.lds_bytes, kind);
     else if (pl.bdir && tc.kgroups == 4) launch_bdir_k4(s, a, tc.wave_pixels / 16, pl.grid, pl.lds_bytes, kind);

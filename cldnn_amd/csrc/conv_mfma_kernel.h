@@ -74,7 +74,10 @@ struct MfmaArgs {
     // instructions with four trips between the vector and the scalar unit, before its first load is requested
     FastDiv div_mtiles, div_ofm_tiles;
     uint32_t xor_mask;  // 0x80808080 for u8 activations, 0 for s8
-    const v4i* bpk;     // small-batch kernel: scratch for the activations in fragment order (nullptr: read them in place)
+    const v4i* bpk;     // split-K kernel: scratch for the activations in fragment order (nullptr: read them in place)
+    // split-K kernel: waves per workgroup, K-steps per wave, bounds checks (input without a border)
+    int32_t kwaves, kper, checked, dil_y, dil_x;
+    FastDiv div_taps;
     FastEpi fe;
     Epilogue epi;
 };
@@ -91,8 +94,11 @@ struct MfmaArgs {
 //   SUMLIN clamp((sat(round(acc * cal)) + residual) * ecal, lo, hi)    (residual sum without activation, the rounded
 //                                                                      convolution result optionally saturated first, unit
 //                                                                      wqf; a MobileNet projection; chain kernels)
+//   F32    act(acc * wqf) * cal as a float                             (the output layer of a detector; what the element-wise
+//                                                                      form made of it ran 6 to 10 times as long: sixteen
+//                                                                      4-byte stores and three dozen instructions a value)
 enum { EPI_KIND_GENERIC = 0, EPI_KIND_FAST = 1, EPI_KIND_RELU = 2, EPI_KIND_FUSED = 3, EPI_KIND_LINEAR = 4, EPI_KIND_CLAMPQ = 5,
-       EPI_KIND_SUMLIN = 6 };
+       EPI_KIND_SUMLIN = 6, EPI_KIND_F32 = 7 };
 template <int EPI> struct epi_is_short { static constexpr bool value = EPI != EPI_KIND_GENERIC; };
 
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() also drains every outstanding
@@ -414,41 +420,58 @@ __device__ __forceinline__ v4i epilogue_fast16(const Args& a, const v4i (&acc)[4
     return packed;
 }
 
+// float output: the long form's operations for a plain convolution, in its order (x * 1.0f == x where a factor is absent)
+template <class Args>
+__device__ __forceinline__ float epilogue_f32(const Args& a, float x, float wq, float cal)
+{
+    const FastEpi& F = a.fe;
+    if (F.has_wqf) {
+        x = x * wq;
+        x = x * F.iqf;
+    }
+    if (F.act == CLDNN_HIP_ACT_RELU) x = fmaxf(0.0f, x);
+    else if (F.act == CLDNN_HIP_ACT_CLAMP) x = fmaxf(F.act_m, fminf(F.act_n, x));
+    return x * cal;
+}
+
 // per-lane requantisation factors of the 16 features a lane finishes
 struct LaneScales {
     float wq[16], cal[16], ecal[16];
 };
 
+// factors of the four features [f0, f0 + 4) into entries [4 * d, 4 * d + 4)
 template <int EPI, class Args>
-__device__ __forceinline__ void load_scales(const Args& a, int f0, LaneScales& sc)
+__device__ __forceinline__ void load_scales4(const Args& a, int f0, LaneScales& sc, int d = 0)
 {
+    const Epilogue& e = a.epi;
     if constexpr (EPI == EPI_KIND_RELU || EPI == EPI_KIND_FUSED || EPI == EPI_KIND_LINEAR) {
         // these kinds are only chosen when the vectors they read exist
-        const Epilogue& e = a.epi;
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            const float4 c4 = *reinterpret_cast<const float4*>(e.calib + f0 + d * 4);
-            sc.cal[d * 4 + 0] = c4.x, sc.cal[d * 4 + 1] = c4.y, sc.cal[d * 4 + 2] = c4.z, sc.cal[d * 4 + 3] = c4.w;
-            if constexpr (EPI == EPI_KIND_FUSED) {
-                const float4 e4 = *reinterpret_cast<const float4*>(e.eltw_calib + f0 + d * 4);
-                sc.ecal[d * 4 + 0] = e4.x, sc.ecal[d * 4 + 1] = e4.y, sc.ecal[d * 4 + 2] = e4.z, sc.ecal[d * 4 + 3] = e4.w;
-            }
+        const float4 c4 = *reinterpret_cast<const float4*>(e.calib + f0);
+        sc.cal[d * 4 + 0] = c4.x, sc.cal[d * 4 + 1] = c4.y, sc.cal[d * 4 + 2] = c4.z, sc.cal[d * 4 + 3] = c4.w;
+        if constexpr (EPI == EPI_KIND_FUSED) {
+            const float4 e4 = *reinterpret_cast<const float4*>(e.eltw_calib + f0);
+            sc.ecal[d * 4 + 0] = e4.x, sc.ecal[d * 4 + 1] = e4.y, sc.ecal[d * 4 + 2] = e4.z, sc.ecal[d * 4 + 3] = e4.w;
         }
-    } else if constexpr (EPI == EPI_KIND_FAST) {
-        const Epilogue& e = a.epi;
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            float4 c4 = {1.f, 1.f, 1.f, 1.f}, w4 = c4, e4 = c4;
-            if (e.calib) c4 = *reinterpret_cast<const float4*>(e.calib + f0 + d * 4);
-            else if (e.oqf_on) c4 = make_float4(e.oqf, e.oqf, e.oqf, e.oqf);
-            if (a.fe.has_wqf) w4 = *reinterpret_cast<const float4*>(e.wqf + f0 + d * 4);
-            if (a.fe.has_ecal) e4 = *reinterpret_cast<const float4*>(e.eltw_calib + f0 + d * 4);
-            if (a.fe.fc) e4 = *reinterpret_cast<const float4*>((const float*)e.bias + f0 + d * 4);  // never fused: the slot is free
-            sc.cal[d * 4 + 0] = c4.x, sc.cal[d * 4 + 1] = c4.y, sc.cal[d * 4 + 2] = c4.z, sc.cal[d * 4 + 3] = c4.w;
-            sc.wq[d * 4 + 0] = w4.x, sc.wq[d * 4 + 1] = w4.y, sc.wq[d * 4 + 2] = w4.z, sc.wq[d * 4 + 3] = w4.w;
+    } else if constexpr (EPI == EPI_KIND_FAST || EPI == EPI_KIND_F32) {
+        float4 c4 = {1.f, 1.f, 1.f, 1.f}, w4 = c4, e4 = c4;
+        if (e.calib) c4 = *reinterpret_cast<const float4*>(e.calib + f0);
+        else if (e.oqf_on) c4 = make_float4(e.oqf, e.oqf, e.oqf, e.oqf);
+        if (a.fe.has_wqf) w4 = *reinterpret_cast<const float4*>(e.wqf + f0);
+        sc.cal[d * 4 + 0] = c4.x, sc.cal[d * 4 + 1] = c4.y, sc.cal[d * 4 + 2] = c4.z, sc.cal[d * 4 + 3] = c4.w;
+        sc.wq[d * 4 + 0] = w4.x, sc.wq[d * 4 + 1] = w4.y, sc.wq[d * 4 + 2] = w4.z, sc.wq[d * 4 + 3] = w4.w;
+        if constexpr (EPI == EPI_KIND_FAST) {
+            if (a.fe.has_ecal) e4 = *reinterpret_cast<const float4*>(e.eltw_calib + f0);
+            if (a.fe.fc) e4 = *reinterpret_cast<const float4*>((const float*)e.bias + f0);  // never fused: the slot is free
             sc.ecal[d * 4 + 0] = e4.x, sc.ecal[d * 4 + 1] = e4.y, sc.ecal[d * 4 + 2] = e4.z, sc.ecal[d * 4 + 3] = e4.w;
         }
     }
+}
+
+template <int EPI, class Args>
+__device__ __forceinline__ void load_scales(const Args& a, int f0, LaneScales& sc)
+{
+#pragma unroll
+    for (int d = 0; d < 4; ++d) load_scales4<EPI>(a, f0 + d * 4, sc, d);
 }
 
 // Finish the 16 features [f0, f0+16) of one pixel held in acc[.][nt] and store them.
@@ -459,7 +482,20 @@ __device__ __forceinline__ void finish_pixel(const MfmaArgs& a, const v4i (&acc)
                                              uint32_t oy, uint32_t ox)
 {
     const Epilogue& e = a.epi;
-    if constexpr (EPI != EPI_KIND_GENERIC) {
+    if constexpr (EPI == EPI_KIND_F32) {
+        float* dst = (float*)a.out + obase;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = epilogue_f32(a, (float)acc[d][nt][i], sc.wq[d * 4 + i], sc.cal[d * 4 + i]);
+            if (valid >= d * 4 + 4) *reinterpret_cast<float4*>(dst + d * 4) = make_float4(v[0], v[1], v[2], v[3]);
+            else
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (d * 4 + i < valid) dst[d * 4 + i] = v[i];
+        }
+    } else if constexpr (EPI != EPI_KIND_GENERIC) {
         const v4i packed = epilogue_fast16<NT, EPI>(a, acc, nt, sc.wq, sc.cal, sc.ecal, ev4, valid);
         *reinterpret_cast<v4i*>((int8_t*)a.out + obase) = packed;
     } else {
@@ -1281,6 +1317,7 @@ void launch_mfma_instance(hipStream_t s, const MfmaArgs& a, int grid, int lds, i
     case EPI_KIND_FUSED: hipLaunchKernelGGL((conv_mfma_kernel<BM, BN, WP, CHECKED, EPI_KIND_FUSED>), g, b, lds, s, a); break;
     case EPI_KIND_LINEAR: hipLaunchKernelGGL((conv_mfma_kernel<BM, BN, WP, CHECKED, EPI_KIND_LINEAR>), g, b, lds, s, a); break;
     case EPI_KIND_FAST: hipLaunchKernelGGL((conv_mfma_kernel<BM, BN, WP, CHECKED, EPI_KIND_FAST>), g, b, lds, s, a); break;
+    case EPI_KIND_F32: hipLaunchKernelGGL((conv_mfma_kernel<BM, BN, WP, CHECKED, EPI_KIND_F32>), g, b, lds, s, a); break;
     default: hipLaunchKernelGGL((conv_mfma_kernel<BM, BN, WP, CHECKED, EPI_KIND_GENERIC>), g, b, lds, s, a); break;
     }
 }
@@ -1304,6 +1341,7 @@ void launch_bdir_instance(hipStream_t s, const MfmaArgs& a, int grid, int lds, i
     case EPI_KIND_FUSED: BDIR_LAUNCH(EPI_KIND_FUSED) break;
     case EPI_KIND_LINEAR: BDIR_LAUNCH(EPI_KIND_LINEAR) break;
     case EPI_KIND_FAST: BDIR_LAUNCH(EPI_KIND_FAST) break;
+    case EPI_KIND_F32: BDIR_LAUNCH(EPI_KIND_F32) break;
     default: BDIR_LAUNCH(EPI_KIND_GENERIC) break;
     }
 #undef BDIR_LAUNCH
@@ -1328,6 +1366,7 @@ void launch_wsl_instance(hipStream_t s, const MfmaArgs& a, int grid, int lds, in
     case EPI_KIND_FUSED: WSL_LAUNCH(EPI_KIND_FUSED) break;
     case EPI_KIND_LINEAR: WSL_LAUNCH(EPI_KIND_LINEAR) break;
     case EPI_KIND_FAST: WSL_LAUNCH(EPI_KIND_FAST) break;
+    case EPI_KIND_F32: WSL_LAUNCH(EPI_KIND_F32) break;
     default: WSL_LAUNCH(EPI_KIND_GENERIC) break;
     }
 #undef WSL_LAUNCH
@@ -1342,6 +1381,7 @@ void launch_stream_instance(hipStream_t s, const MfmaArgs& a, int grid, int epi)
     case EPI_KIND_FUSED: hipLaunchKernelGGL((conv_stream_kernel<NT, KS, EPI_KIND_FUSED>), g, b, 0, s, a); break;
     case EPI_KIND_LINEAR: hipLaunchKernelGGL((conv_stream_kernel<NT, KS, EPI_KIND_LINEAR>), g, b, 0, s, a); break;
     case EPI_KIND_FAST: hipLaunchKernelGGL((conv_stream_kernel<NT, KS, EPI_KIND_FAST>), g, b, 0, s, a); break;
+    case EPI_KIND_F32: hipLaunchKernelGGL((conv_stream_kernel<NT, KS, EPI_KIND_F32>), g, b, 0, s, a); break;
     default: hipLaunchKernelGGL((conv_stream_kernel<NT, KS, EPI_KIND_GENERIC>), g, b, 0, s, a); break;
     }
 }

@@ -44,13 +44,17 @@ struct MfmaPlan {
     int stream;          // 1: streaming kernel (no LDS), 0: LDS-staged tile kernel
     int bdir;            // 1: direct-activation tile kernel (weights through LDS, activations into registers)
     int stem;            // 1: first-layer row (b_fs_yx_fsv4 input, streaming kernel)
-    int by_features;     // 1: accelerator dies split the feature tiles (weights larger than activations)
+    int by_features;     // 1: accelerator dies split the feature tiles (weights larger than activations); 2: tiles counted off
     int wsl;             // 1: weights-stationary persistent kernel (weight tile resident in LDS)
     int wsl_depth;       // its activation look-ahead in K-steps
     int wsl_parts;       // pixel-range partitions per feature tile (multiple of 8)
     int wsl_tpp;         // pixel tiles per partition
-    int gemv;            // 1: few pixels, long K: 16-feature fragments, waves split K (no LDS in the loop)
-    int gemv_waves;      // its waves per workgroup
+    int ksplit;          // 1: few output tiles: small tiles, the waves of a workgroup split K (conv_ksplit_kernel.h)
+    int gemv;            // 1: its row for at most 4096 pixels, which gathers the activations of a filter wider than one tap
+    int ks_ft, ks_pt;    // its tile in 16-feature and 16-pixel fragments
+    int ks_waves, ks_per;  // its waves per workgroup, K-steps per wave
+    int ks_lanes;        // 1: lanes find their own taps (fewer than four slices, or no border)
+    int shifted;         // 1: feature slices not in fours: the last K-step of a tap starts at the last four slices
     int halo;            // 1: nine-tap stride-1 kernel with both operands staged in LDS by direct loads (conv_halo_kernel.h)
     int halo_patch_len;  // its patch length in positions per slice (multiple of 64)
     int halo_parts;      // its workgroups per feature tile (multiple of 8)
@@ -72,7 +76,8 @@ struct MfmaPlan {
 };
 // table lookup: row of the tile table for a problem
 int mfma_choose(const ConvProblem& p, int cus);
-MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus);
+// forced: the row was named by the caller (tuning, tests) and is taken as the table describes it
+MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus, bool forced);
 // host-side packing: weights [OFM][IFM][FY][FX] s8 -> MFMA operand stream, ktab -> per-kchunk tap table
 void mfma_pack_weights(const ConvProblem& p, const MfmaPlan& plan, const int8_t* w, int8_t* packed, int32_t* ktab);
 struct MfmaBuffers {
@@ -85,8 +90,9 @@ size_t mfma_gather_bytes(const ConvProblem& p, const MfmaPlan& pl);  // 0 when t
 // mfma_static_scratch returns its device address on `device`, which must be the current device.
 size_t mfma_static_scratch_bytes();
 void* mfma_static_scratch(int device);
-// parameters of the short epilogue (int8 output, float requantisation)
+// parameters of the short epilogue (int8 output in the float-requantisation mode, or float output)
 struct FastEpi {
+    int32_t f32;          // float output: act(acc * wqf * iqf) * factor, nothing rounded
     int32_t has_wqf;      // multiply by wqf[f] and iqf
     int32_t act;          // CLDNN_HIP_ACT_NONE / RELU / CLAMP
     float act_m, act_n;

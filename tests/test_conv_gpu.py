@@ -859,3 +859,39 @@ def test_reference_differential_recipe_with_iota_data(eng, fmt, k, F, stride, ou
     if with_bias and fmt != "bfyx":
         assert info.impl == hip.IMPL_MFMA, info.kernel_name  # the quantized form runs on the matrix-core kernels
     assert_same(ro, go)
+
+
+@pytest.mark.parametrize("row", ["ksplit_p16_f16", "ksplit_p32_f16", "ksplit_p64_f16", "ksplit_p32_f32", "ksplit_p32_f64"])
+@pytest.mark.parametrize("shape", [
+    # B IFM H W OFM filter stride border
+    (1, 16, 1, 1, 1, 1, 1, True),       # one pixel, one feature, one K-step: waves without steps
+    (1, 100, 5, 13, 67, 3, 1, True),    # 65 pixels; seven slices: the last step of a tap starts at slice three
+    (3, 72, 4, 4, 130, 3, 2, True),     # five slices, stride 2
+    (1, 40, 7, 5, 20, 5, 1, True),      # three slices: lanes find their own taps
+    (2, 80, 6, 3, 33, 3, 1, False),     # no border: taps checked
+    (1, 1600, 3, 11, 48, 3, 1, True),   # 225 K-steps: the loop behind the look-ahead, with a remainder
+], ids=lambda s: "x".join(map(str, s[:7])) + ("" if s[7] else "_checked"))
+def test_split_k_rows(eng, row, shape):
+    B, IFM, H, W, OFM, F, st, border = shape
+    x, w, bias, wqf, calib = problem(91, B, IFM, H, W, OFM, F, F)
+    pad = F // 2
+    tile = tile_names().index(row) + 1
+    kw = dict(stride=(st, st), pad=(pad, pad))
+    for out_dt, act in (("s8", ("relu", 0, 0)), ("f32", ("clamp", -2.0, 9.0e5)), ("f32", ("none", 0, 0)), ("u8", ("relu_slope", 0.5, 0))):
+        (ro, ra), (go, ga, info) = both(eng, x, w, bias, wqf, calib, fmt="fs_b_yx_fsv16", tile=tile, in_pad=(pad, pad) if border else (0, 0),
+                                        out_dt=out_dt, act=act[0], act_m=act[1], act_n=act[2], **kw)
+        assert b"conv_ksplit<" + row.encode() in info.kernel_name and (pad == 0 or (b"checked" in info.kernel_name) == (not border))
+        np.testing.assert_array_equal(ga, ra)
+        assert_same(ro, go)
+
+
+@pytest.mark.parametrize("OFM", [1, 16, 35, 126])
+def test_float_output_of_every_row(eng, OFM):
+    """float results leave through the short float epilogue: partly filled slices and groups of four, factors present and absent"""
+    x, w, bias, wqf, calib = problem(92, 2, 64, 9, 9, OFM, 3, 3)
+    for kw in (dict(wqf=wqf, calib=calib), dict(wqf=wqf * np.float32(0.37), calib=None, iqf=0.5, act="relu"), dict(wqf=wqf, calib=-calib, act="relu")):
+        wq, ca = kw.pop("wqf"), kw.pop("calib")
+        ref = rc.conv(x, w, bias, wqf=wq, calib=ca, pad=(1, 1), out_dt="f32", **kw)
+        for tile in [0] + [t for t in tiles() if not tile_names()[t - 1].startswith(("stem", "stream"))]:
+            got = hip.conv_forward(eng, x, w, bias, wq, ca, fmt="fs_b_yx_fsv16", in_pad=(1, 1), pad=(1, 1), out_dt="f32", tile=tile, **kw)
+            assert_same(ref, got)
