@@ -484,7 +484,7 @@ cldnn_hip_status cldnn_hip_conv_chain_create(cldnn_hip_engine e, int32_t count, 
             CHIP_CHECK(hipStreamSynchronize(e->stream));
             cldnn_hip_conv_info& inf = ch->info;
             inf.impl = CLDNN_HIP_IMPL_MFMA, inf.tile_index = -1, inf.tile_pixels = 64 * (ch->plan.dw ? 4 : ch->plan.nt), inf.tile_ofm = 64;
-            inf.grid = ch->plan.grid, inf.block = 256, inf.lds_bytes = ch->plan.lds_bytes;
+            inf.grid = ch->plan.grid, inf.block = 64 * ch->plan.waves, inf.lds_bytes = ch->plan.lds_bytes;
             std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "%s", ch->plan.name);
             // algorithmic work of the chain: every stage's operations; bytes of what has to cross the memory interface,
             // i.e. without the intermediate tensors that are neither kept nor re-read

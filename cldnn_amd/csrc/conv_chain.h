@@ -22,6 +22,8 @@ struct ChainPlan {
     int stages;
     int dw;                    // 1: the first stage is a depthwise 3x3 on the vector ALU (granules of 64 pixels), the LDS
                                // image holds the units and vectors of the later stages only
+    int coop;                  // 1: its form for small planes, a workgroup's waves share a granule (conv_dwcoop_kernel.h)
+    int waves;                 // waves per workgroup
     int nt;                    // 16-pixel fragments per wave and granule
     int depth;                 // activation look-ahead of stage 0 in K-steps
     int ksteps0;               // K-steps of stage 0 (padded to a multiple of depth)
@@ -30,6 +32,7 @@ struct ChainPlan {
     int unit0[3], kstride[3];  // LDS image: first 4 KB unit and units per span of every stage
     int vec0[3];               // first dword of every stage's per-feature vectors behind the weights
     int units;
+    int img_bytes;             // weights and per-feature vectors on the device
     int lds_bytes;
     int grid;
     int granules;

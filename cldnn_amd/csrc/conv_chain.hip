@@ -1,11 +1,12 @@
 // Host side of the convolution chain kernel: eligibility, LDS image of the weights, launch.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 #include <string>
 #include <vector>
 
-#include "conv_dwchain_kernel.h"
+#include "conv_dwcoop_kernel.h"
 
 namespace chip {
 
@@ -90,9 +91,10 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
         // ---- depthwise first stage: lane = pixel on the vector ALU, 64-pixel granules, later stages resident in LDS
         if (p0.FY != 3 || p0.FX != 3) return "stage 0: the depthwise stage of a chain is 3x3";
         if (st[0].fe->fused) return "stage 0: a fused depthwise stage is not chained";
-        if (pl.sp[1] != 1) return "stage 1: the projection behind a depthwise stage has at most 64 features";
+        if (pl.sp[1] > 3) return "stage 1: the projection behind a depthwise stage has at most 192 features";
         pl.dw = 1;
         // 32-pixel granules; 16-pixel ones where that still leaves waves without work (14x14 and 7x7 planes)
+        pl.waves = 4;
         pl.nt = pl.m_total / 32 >= (int64_t)cus * 8 ? 2 : 1;
         pl.granules = (int)((pl.m_total + 16 * pl.nt - 1) / (16 * pl.nt));
         pl.units = 0;
@@ -112,7 +114,28 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
             vec += 4 * pl.sp[k] * 64;
         }
         pl.ksteps0 = pl.sp[0];  // K-steps the depthwise stage delivers to stage 1
-        pl.lds_bytes = pl.sp[0] * 9 * 1024 + pl.units * 4096 + vec * 4;  // diagonal-weight table, units, vectors
+        pl.img_bytes = pl.sp[0] * 9 * 1024 + pl.units * 4096 + vec * 4;  // diagonal-weight table, units, vectors
+        pl.lds_bytes = pl.img_bytes;
+        // Small planes: the waves of a workgroup share a granule.  Up to three granules per CU that beats one granule per
+        // wave with the weights in LDS (14x14 at batch 32; 28x28 at batch 32, with six per CU, reads the weights from L2 too
+        // often: 15.3 us against 12.4), from two K-steps on (a single one occupies one wave of four).
+        const bool block = pl.epi[0] == EPI_KIND_CLAMPQ && (pl.epi[1] == EPI_KIND_LINEAR || pl.epi[1] == EPI_KIND_SUMLIN)
+                           && (n < 3 || pl.epi[2] == EPI_KIND_CLAMPQ) && !st[1].fe->split_valid;
+        const bool small = (pl.m_total + 15) / 16 <= 3ll * cus;
+        if (pl.sp[1] > 1 && !(block && small))
+            return "stage 1: a projection of more than 64 features is chained in the forms of a MobileNet block and on small planes only";
+        if (block && small && pl.ksteps0 >= 2) {
+            pl.coop = 1, pl.nt = 1;
+            pl.waves = pl.ksteps0 <= 8 ? std::max(4, pl.ksteps0) : std::min(8, (pl.ksteps0 + 1) / 2);
+            pl.granules = (int)((pl.m_total + 15) / 16);
+            pl.lds_bytes = (pl.waves * 4 + 1) * pl.sp[1] * 1024 + vec * 4;
+            const int per_cu = std::max(1, std::min((pl.sp[1] == 1 ? 12 : 8) / pl.waves, CHAIN_MAX_LDS / pl.lds_bytes));
+            pl.grid = std::min(cus * per_cu / 8 * 8, (pl.granules + 7) / 8 * 8);
+            std::snprintf(pl.name, sizeof(pl.name), "conv_dwchain<%d stages,p16 shared by %d waves,mid %d,spans %d-%d>", n, pl.waves, p0.OFM, pl.sp[1],
+                          n > 2 ? pl.sp[2] : 0);
+            *out = pl;
+            return std::string();
+        }
         if (pl.lds_bytes > CHAIN_MAX_LDS) return "the weights of the chain (" + std::to_string(pl.lds_bytes / 1024) + " KiB) do not fit into LDS";
         // workgroups a CU holds at once: by LDS, and by registers (16-pixel granules: 137-167 registers = three waves per
         // SIMD; 32-pixel granules: 206-239 = two).  The grid is what is resident, so that no workgroup waits for a slot.
@@ -126,7 +149,7 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
         *out = pl;
         return std::string();
     }
-    pl.nt = 2;
+    pl.nt = 2, pl.waves = 4;
     pl.granules = (int)((pl.m_total + 16 * pl.nt - 1) / (16 * pl.nt));
     // K-steps of every stage as the weights-stationary row packs them
     MfmaPlan mp[3]{};
@@ -153,7 +176,7 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
             vec += 4 * pl.sp[k] * 64;
         }
         pl.depth = mp[0].wsl_depth, pl.ksteps0 = mp[0].ksteps;
-        pl.lds_bytes = pl.units * 4096 + vec * 4;
+        pl.lds_bytes = pl.img_bytes = pl.units * 4096 + vec * 4;
         if (mp[0].wsl_depth > 0 && pl.lds_bytes <= CHAIN_MAX_LDS && find_instance(pl)) {
             const int per_cu = pl.lds_bytes * 2 <= CHAIN_MAX_LDS ? 2 : 1;
             int grid = cus * per_cu / 8 * 8;
@@ -172,7 +195,7 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
     return "no compiled instance for this chain shape";
 }
 
-size_t chain_packed_bytes(const ChainPlan& pl) { return (size_t)pl.lds_bytes + 4096; }
+size_t chain_packed_bytes(const ChainPlan& pl) { return (size_t)pl.img_bytes + 4096; }
 
 static void fill_stage(ChainStage& c, const ChainStageIn& in, const ChainPlan& pl, int k, void* out, const void* eltw)
 {
@@ -190,6 +213,54 @@ static void fill_stage(ChainStage& c, const ChainStageIn& in, const ChainPlan& p
     c.epi = *in.epi;
 }
 
+static void launch_dwcoop(hipStream_t s, const ChainStageIn* st, const ChainPlan& pl, const void* packed_dev, const void* in,
+                          void* const* outs, const void* const* eltws)
+{
+    const ConvProblem& p0 = *st[0].p;
+    const ConvProblem& p1 = *st[1].p;
+    DwCoopArgs a{};
+    a.in = (const int8_t*)in, a.img = (const int8_t*)packed_dev, a.eltw = eltws ? (const int8_t*)eltws[1] : nullptr;
+    a.unit_bytes = pl.sp[0] * 9 * 1024;
+    a.vec_bytes = a.unit_bytes + pl.units * 4096;
+    a.vec_quads = (pl.img_bytes - a.vec_bytes) / 16;
+    a.el_off = (int32_t)p1.eltw_p.off, a.el_pb = (int32_t)p1.eltw_p.pb, a.el_pf = (int32_t)p1.eltw_p.pf;
+    a.el_py = (int32_t)p1.eltw_p.py * p1.esy, a.el_px = 16 * p1.esx;
+    a.M = (uint32_t)pl.m_total;
+    a.OHW = p0.OH * p0.OW, a.OW = p0.OW;
+    a.div_ohw = make_fast_div((uint32_t)a.OHW), a.div_ow = make_fast_div((uint32_t)a.OW);
+    a.in_off = (int32_t)p0.in_p.off - p0.py * (int32_t)p0.in_p.py - p0.px * 16;
+    a.in_pb = (int32_t)p0.in_p.pb, a.in_pf = (int32_t)p0.in_p.pf;
+    a.row = p0.sy * (int32_t)p0.in_p.py, a.col = p0.sx * 16, a.tap_dy = (int32_t)p0.in_p.py;
+    a.CB = (p0.OFM + 15) / 16, a.KS = pl.sp[0], a.SP2 = pl.stages > 2 ? pl.sp[2] : 0, a.waves = pl.waves;
+    a.gpw = pl.granules / pl.grid, a.grem = pl.granules % pl.grid;
+    a.div_parts = make_fast_div((uint32_t)pl.grid);
+    const FastEpi &f0 = *st[0].fe, &f1 = *st[1].fe;
+    const bool sum = pl.epi[1] == EPI_KIND_SUMLIN;
+    CHIP_REQUIRE(!sum || a.eltw, CLDNN_HIP_INVALID_ARG, "fused stage of a chain without its second input");
+    a.clamp_m0 = f0.act_m, a.clamp_n0 = f0.act_n;
+    a.lo1 = f1.lo, a.hi1 = f1.hi, a.eltw_u8 = f1.eltw_u8;
+    a.conv_lo = f1.conv_sat ? f1.conv_lo : -INFINITY, a.conv_hi = f1.conv_sat ? f1.conv_hi : INFINITY;
+    if (pl.stages > 2) a.clamp_m2 = st[2].fe->act_m, a.clamp_n2 = st[2].fe->act_n;
+    for (int k = 0; k < pl.stages; ++k) {
+        const ConvProblem& p = *st[k].p;
+        CoopStage& c = a.st[k];
+        c.out = (int8_t*)outs[k];
+        c.off = (int32_t)p.out_p.off, c.pb = (int32_t)p.out_p.pb, c.pf = (int32_t)p.out_p.pf, c.py = (int32_t)p.out_p.py;
+        c.ofm = p.OFM, c.xor_mask = p.in_dt == CLDNN_HIP_U8 ? 0x80808080u : 0u;
+        c.unit0 = pl.unit0[k], c.kstride = pl.kstride[k], c.vec0 = pl.vec0[k];
+    }
+#define DWCOOP_LAUNCH(SP1)                                                                    \
+    {                                                                                         \
+        if (pl.stages > 2 && sum) launch_dwcoop_instance<SP1, true, true>(s, a, pl.grid, pl.lds_bytes);   \
+        else if (pl.stages > 2) launch_dwcoop_instance<SP1, true, false>(s, a, pl.grid, pl.lds_bytes);    \
+        else if (sum) launch_dwcoop_instance<SP1, false, true>(s, a, pl.grid, pl.lds_bytes);  \
+        else launch_dwcoop_instance<SP1, false, false>(s, a, pl.grid, pl.lds_bytes);          \
+    }
+    if (pl.sp[1] == 1) DWCOOP_LAUNCH(1) else if (pl.sp[1] == 2) DWCOOP_LAUNCH(2) else DWCOOP_LAUNCH(3)
+#undef DWCOOP_LAUNCH
+    CHIP_CHECK(hipGetLastError());
+}
+
 static void launch_dwchain(hipStream_t s, const ChainStageIn* st, const ChainPlan& pl, const void* packed_dev, const void* in,
                            void* const* outs, const void* const* eltws)
 {
@@ -199,7 +270,7 @@ static void launch_dwchain(hipStream_t s, const ChainStageIn* st, const ChainPla
     a.img = (const v4i*)packed_dev;
     a.dw_quads = pl.sp[0] * 9 * 64;
     a.units = pl.units;
-    a.vec_quads = (pl.lds_bytes - a.dw_quads * 16 - pl.units * 4096) / 16;
+    a.vec_quads = (pl.img_bytes - a.dw_quads * 16 - pl.units * 4096) / 16;
     a.granules = pl.granules;
     a.gpw = pl.granules / (pl.grid * 4), a.grem = pl.granules % (pl.grid * 4);
     a.div_waves = make_fast_div((uint32_t)pl.grid * 4u);
@@ -251,7 +322,7 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
                         const int ch = ks * 64 + 16 * (l16 >> 2) + 4 * mt + (l16 & 3);
                         int32_t v = 0;
                         if (kq == (l16 >> 2) && ch < p0.OFM) v = (int32_t)((uint32_t)(uint8_t)w[0][(size_t)ch * 9 + tap] << (8 * (l16 & 3)));
-                        dia[((ks * 9 + tap) * 4 + mt) * 64 + lane] = v;
+                        dia[pl.coop ? ((ks * 9 + tap) * 64 + lane) * 4 + mt : ((ks * 9 + tap) * 4 + mt) * 64 + lane] = v;
                     }
     }
     packed += dw_bytes;
@@ -284,6 +355,7 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
 void launch_conv_chain(hipStream_t s, const ChainStageIn* st, const ChainPlan& pl, const void* packed_dev, const void* in,
                        void* const* outs, const void* const* eltws)
 {
+    if (pl.coop) return launch_dwcoop(s, st, pl, packed_dev, in, outs, eltws);
     if (pl.dw) return launch_dwchain(s, st, pl, packed_dev, in, outs, eltws);
     const ConvProblem& p0 = *st[0].p;
     ChainArgs a{};

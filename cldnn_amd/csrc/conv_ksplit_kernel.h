@@ -175,6 +175,12 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
             if (d < rest) mma(ra[d], rb[d]);
     }
 
+    step_fence();
+#pragma unroll
+    for (int f = 0; f < FT; ++f)
+#pragma unroll
+        for (int p = 0; p < PT; ++p) mfma_settle(acc[f][p]);
+
     // ---- partial sums; wave w < FT * PT finishes fragment (w % FT, w / FT)
     constexpr int TILE = FT * PT * 64;
     extern __shared__ __align__(16) unsigned char smem[];

@@ -114,6 +114,11 @@ __device__ __forceinline__ void lds_barrier()
 // look-ahead queue once per loop iteration.
 __device__ __forceinline__ void step_fence() { __builtin_amdgcn_sched_barrier(0); }
 
+// Accumulators may be read from here on.  The compiler inserts the idle slots between a matrix instruction and a reader of
+// its result, but where the last one stands under a branch of its own it has been seen to count them along the longer path
+// only.
+__device__ __forceinline__ void mfma_settle(v4i& acc) { asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc)); }
+
 // Instruction order inside one K-step: after each of the M matrix instructions (16 clocks in the matrix pipe, 4 to
 // issue) the scheduler is told to place a share of the step's other work -- R LDS reads, W LDS writes, V global
 // loads, VALU register work -- so that it issues in the shadow of the matrix pipe instead of in front of it.  The

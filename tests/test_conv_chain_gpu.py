@@ -293,3 +293,54 @@ def test_depthwise_chain_with_the_blocks_sum_on_the_projection(eng, saturate, el
     xin.close(), ebuf.close()
     for b in bufs:
         b.close()
+
+
+@pytest.mark.parametrize("mid,proj,stride,stages,hw", [(576, 96, 1, 3, (7, 9)), (576, 160, 2, 3, (9, 9)), (960, 160, 1, 3, (7, 7)), (960, 192, 1, 2, (5, 3)),
+                                                        (80, 24, 1, 3, (1, 1)), (576, 72, 1, 3, (41, 53))],
+                         ids=["14x14_like", "two_rounds_s2", "7x7_like", "two_stages", "one_pixel", "several_granules_a_group"])
+@pytest.mark.parametrize("in_dt,saturate", [(np.uint8, None), (np.int8, 0), (np.uint8, 1)], ids=["u8", "s8_sum", "u8_sum_saturated"])
+def test_depthwise_chain_on_small_planes(eng, mid, proj, stride, stages, hw, in_dt, saturate):
+    """waves that share a granule: one to three spans of projection, more K-steps and spans than waves, a last granule that
+    is not full, with and without the block's sum, against the oracle's separate convolutions"""
+    r = np.random.default_rng(mid + proj)
+    B = 5 if hw == (41, 53) else 3
+    H, W = hw
+    OH, OW = (H + 2 - 3) // stride + 1, (W + 2 - 3) // stride + 1
+    lo, hi = (0, 256) if in_dt == np.uint8 else (-128, 128)
+    x = r.integers(lo, hi, (B, mid, H, W)).astype(in_dt)
+    xin = hip.upload(eng, x, "fs_b_yx_fsv16", (1, 1))
+    e = r.integers(-128, 128, (B, proj, OH, OW)).astype(np.int8)
+    ecal = r.uniform(0.5, 1.0, proj).astype(np.float32)
+    ebuf = hip.upload(eng, e, "fs_b_yx_fsv16", (0, 1))
+    spec, refs, bufs = [], [], []
+    prev_t, ref_in = xin.tensor, x
+    for k, (ofm, ifm_g, fk, act, groups) in enumerate([(mid, 1, 3, "relu6", mid), (proj, mid, 1, "none", 1), (2 * proj + 8, proj, 1, "relu6", 1)][:stages]):
+        w, bias, wqf, calib, akw = relu6_layer(r, ofm, ifm_g, fk, act)
+        s = stride if k == 0 else 1
+        kw = dict(stride=(s, s), pad=(fk // 2,) * 2, groups=groups, bias_dt=hip.I32, has_wqf=True, has_calib=True, **akw)
+        okw = dict(stride=(s, s), pad=(fk // 2,) * 2, groups=groups, out_dt="s8", **akw)
+        summed = k == 1 and saturate is not None
+        if summed:
+            kw.update(eltw_t=ebuf.tensor, eltw_act="none", has_eltw_calib=True, conv_saturate=saturate)
+        d = hip.conv_desc(prev_t, w.shape, "s8", out_pad=(1, 1), **kw)
+        spec.append((d, w, bias, wqf, calib, ecal if summed else None))
+        bufs.append(hip.Buffer(eng, d.output))
+        if summed and saturate:
+            refs.append(rc.eltwise([e, rc.conv(ref_in, w, bias, wqf=wqf, calib=calib, **okw)], "sum", calib=ecal))
+        elif summed:
+            refs.append(rc.conv(ref_in, w, bias, wqf=wqf, calib=calib, eltw=e, eltw_act="none", eltw_calib=ecal, **okw))
+        else:
+            refs.append(rc.conv(ref_in, w, bias, wqf=wqf, calib=calib, **okw))
+        ref_in, prev_t = refs[-1], hip.Tensor.make(hip.S8, hip.FS_B_YX_FSV16, B, ofm, OH, OW)
+    for keep in ([False] * (stages - 1) + [True], None):
+        ch = hip.ConvChain(eng, spec, keep)
+        assert b"conv_dwchain" in ch.info().kernel_name and b"shared" in ch.info().kernel_name
+        ch.enqueue(xin, [b if keep is None or keep[k] else None for k, b in enumerate(bufs)], [None, ebuf, None])
+        eng.finish()
+        for k in range(stages):
+            if keep is None or keep[k]:
+                bad = np.argwhere(hip.download(eng, bufs[k]) != refs[k])
+                assert bad.size == 0, "stage %d: %d differ, first at %s" % (k, len(bad), bad[0])
+        ch.close()
+    for b in bufs + [xin, ebuf]:
+        b.close()
