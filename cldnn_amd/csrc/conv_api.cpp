@@ -25,6 +25,7 @@ struct cldnn_hip_conv_s {
     // device allocations
     void* w_raw = nullptr;    // dense weights (reference kernel)
     void* w_packed = nullptr; // MFMA / depthwise operand stream
+    void* w_rows = nullptr;   // depthwise rows kernel
     void* w_masked = nullptr; // depthwise 3x3 kernel: one weight byte per dword
     void* ktab = nullptr;
     void* gather = nullptr;   // scratch of the small-batch kernel (activations in fragment order)
@@ -251,8 +252,9 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
     }
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE && e.fc) c->fast = false;  // the depthwise kernels have no short fully_connected form
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE && c->fe.f32) c->fast = false;  // nor a float one
-    const bool dw_fast = impl == CLDNN_HIP_IMPL_DEPTHWISE && dw_fast_applies(p, c->fast);
-    const bool xor_u8 = (impl == CLDNN_HIP_IMPL_MFMA || dw_fast) && p.in_dt == CLDNN_HIP_U8;
+    const bool dw_fast = impl == CLDNN_HIP_IMPL_DEPTHWISE && p.FY == 3 && p.FX == 3 && dw_fast_applies(p, c->fast);
+    if (impl == CLDNN_HIP_IMPL_DEPTHWISE) c->dplan = dw_plan(p, c->fast, c->engine->props.multiProcessorCount);
+    const bool xor_u8 = (impl == CLDNN_HIP_IMPL_MFMA || dw_fast || c->dplan.rows) && p.in_dt == CLDNN_HIP_U8;
     for (int f = 0; f < p.OFM; ++f) {
         int64_t s = 0;
         if (xor_u8)
@@ -301,7 +303,6 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
         std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_%s<%s,%s,%s>", c->mplan.gemv ? "gemv" : c->mplan.ksplit ? "ksplit" : c->mplan.halo ? "halo" : c->mplan.stream ? "stream" : (c->mplan.bdir ? "bdir" : (c->mplan.wsl ? "wsl" : "mfma")),
                       tc.name, c->mplan.checked ? "checked" : "border", c->fast && !c->fe.f32 && !c->mplan.gemv ? "fast" : "generic");
     } else {
-        c->dplan = dw_plan(p);
         std::vector<int8_t> packed(c->dplan.packed_bytes);
         dw_pack_weights(p, w8, packed.data());
         c->w_packed = upload(c, packed.data(), packed.size());
@@ -310,9 +311,15 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
             dw_mask_weights(p, w8, masked.data());
             c->w_masked = upload(c, masked.data(), c->dplan.mask_bytes);
         }
-        inf.grid = c->dplan.grid * ((p.OFM + 15) / 16), inf.block = c->dplan.block, inf.lds_bytes = dw_fast ? 0 : p.FY * p.FX * 16;
-        std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "%s<%s>", dw_fast ? "conv_dw3x3_kernel" : "conv_dw_kernel",
-                      p.in_dt == CLDNN_HIP_U8 ? "u8" : "s8");
+        if (c->dplan.rows) {
+            std::vector<int32_t> rows(c->dplan.row_bytes / 4);
+            dw_row_weights(p, w8, rows.data());
+            c->w_rows = upload(c, rows.data(), c->dplan.row_bytes);
+        }
+        inf.grid = c->dplan.rows ? c->dplan.grid_rows : c->dplan.grid * ((p.OFM + 15) / 16);
+        inf.block = c->dplan.block, inf.lds_bytes = dw_fast || c->dplan.rows ? 0 : p.FY * p.FX * 16;
+        std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "%s<%s%s>", dw_fast ? "conv_dw3x3_kernel" : c->dplan.rows ? "conv_dw_rows_kernel" : "conv_dw_kernel",
+                      c->dplan.rows && dw_fast ? "rows," : "", p.in_dt == CLDNN_HIP_U8 ? "u8" : "s8");
     }
 }
 
@@ -397,7 +404,7 @@ static void run(cldnn_hip_conv c, const void* in, void* out, const void* eltw, i
         break;
     }
     case CLDNN_HIP_IMPL_DEPTHWISE:
-        launch_conv_dw(s, p, c->dplan, (const int8_t*)c->w_packed, (const int32_t*)c->w_masked,
+        launch_conv_dw(s, p, c->dplan, (const int8_t*)c->w_packed, (const int32_t*)c->w_masked, (const int32_t*)c->w_rows,
                        (const int32_t*)(raw ? c->acc_init_raw : c->acc_init), c->epi, c->fast ? &c->fe : nullptr, in, eltw, out,
                        raw);
         break;

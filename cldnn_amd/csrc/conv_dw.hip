@@ -1,11 +1,9 @@
-// Depthwise quantized convolution (groups == input features == output features) on
-// fs_b_yx_fsv16.  Not a contraction over features, so no matrix cores: the kernel is a
-// stencil bound by HBM bandwidth.  One lane owns the 16 features of one output pixel:
-// every tap is one coalesced 128-bit load (a wave covers 64 consecutive pixels = 1 KiB),
-// the per-slice weights [tap][16] sit in LDS, and the int8 result leaves as one 128-bit store.
+// Depthwise quantized convolution (groups == input features == output features) on fs_b_yx_fsv16.
 //
-// Two kernels: conv_dw3x3_kernel for the case every MobileNet layer is (3x3 filter, input with a zero border,
-// int8 output through the short requantisation epilogue), and conv_dw_kernel for everything else.
+// Three kernels.  conv_dw_rows_kernel runs 3x3 (stride 1) and 5x5 filters on the matrix cores; conv_dw3x3_kernel takes the
+// other 3x3 layers with dot-product instructions; both need an input with a zero border and
+// the short requantisation epilogue.  conv_dw_kernel is everything else: one lane owns the 16 features of one output pixel,
+// every tap is one coalesced 128-bit load and the per-slice weights [tap][16] sit in LDS.
 #include "conv_mfma_kernel.h"
 
 #include <cstring>
@@ -16,6 +14,7 @@ struct DwArgs {
     const int8_t* in;
     const int8_t* wpk;        // [fs][tap][16]
     const int32_t* wmask;     // [fs][tap][16] dwords: weight of feature c alone in byte c % 4 (3x3 kernel)
+    const v4i* wrows;         // [fs][row of the filter][block of 4 positions][lane] (rows kernel)
     const int32_t* acc_init;  // [fs*16]
     void* out;
     const void* eltw;
@@ -27,6 +26,11 @@ struct DwArgs {
     int in_u8;
     uint32_t xor_mask;
     FastDiv div_ohw, div_ow;
+    // rows kernel: OW4 groups of four output pixels in a row, OH * OW4 in an image, `chunks` workgroups to a feature slice
+    uint32_t OW4, OHW4, groups, chunks, works;
+    int rounds;
+    uint32_t in_last;  // offset of the last 16 bytes of the input
+    FastDiv div_ohw4, div_ow4, div_chunks;
     FastEpi fe;
     Epilogue epi;
 };
@@ -171,14 +175,124 @@ __global__ void __launch_bounds__(256) conv_dw3x3_kernel(DwArgs a)
     *reinterpret_cast<v4i*>((int8_t*)a.out + obase) = packed;
 }
 
-DwPlan dw_plan(const ConvProblem& p)
+// Depthwise on the matrix cores: FY rows of the filter, NB blocks of four input positions to a row.
+//
+// The sixteen columns of a v_mfma_i32_16x16x64_i8 are sixteen groups of four neighbouring output pixels of a row.  The 64
+// values of its contraction are four input positions (lane / 16) of the slice's 16 features, one 128-bit load per lane.  Its
+// rows are chosen so that four products (p = 0..3) leave in lane (group, q) the features 4p..4p+3 of output pixel q of its
+// group: row (q, i) of product p holds the taps of feature 4p + i that pixel q sees in these four positions.  So every
+// input byte is loaded once for four outputs (the dot-product kernel loads nine or twenty-five), a lane ends with all 16
+// features of its pixel, and the row operands have one dword each that is not zero: the table holds those alone.
+//
+// 3x3, stride 1: 6 loads and 24 products for 64 pixels of a slice, against 9 loads and 144 dot products; 5x5: 10 and 40
+// against 25 and 400.  At that rate memory is the bound of large planes; a wave keeps its table in registers for `rounds`
+// sets of 64 pixels and requests the next set before it finishes the present one.  Small planes are bound by the launch and
+// the latency of one set.
+// 32 x 576 x 14x14, 3x3: 6.3 -> 5.0 us (1.4 us at the rate of a large copy and about 3 of launch); 8 x 512 x 28x28, 5x5:
+// 30.8 -> 6.0; 32 x 64 x 112x112, 5x5: 137 -> 24 (10.3 at the rate of a large copy), 3x3: 18.9 -> 17.9.
+template <int FY, int NB, int EPI>
+__global__ void __launch_bounds__(256, 2) conv_dw_rows_kernel(DwArgs a)
+{
+    constexpr int S = FY * NB;
+    // neighbouring chunks of a plane on one XCD (the grid is a multiple of 8): the rows they share are in its L2
+    const uint32_t work = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (work >= a.works) return;
+    const uint32_t fs = a.div_chunks.div(work), chunk = work - fs * a.chunks;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, f0 = (int)fs * 16;
+
+    v4i w[S];
+    const v4i* wt = a.wrows + (size_t)fs * S * 64 + lane;
+#pragma unroll
+    for (int s = 0; s < S; ++s) w[s] = wt[s * 64];
+
+    const uint32_t in_py = (uint32_t)a.in_p.py, tap_py = in_py * (uint32_t)a.dy;
+    int8_t* out = (int8_t*)a.out + (a.out_p.off + (int64_t)fs * a.out_p.pf);
+    const int8_t* el = (const int8_t*)a.eltw + (a.eltw_p.off + (int64_t)fs * a.eltw_p.pf);
+    const uint32_t in_slice = (uint32_t)(a.in_p.off + (int64_t)fs * a.in_p.pf);
+    LaneScales sc;
+    load_scales<EPI>(a, f0, sc);
+    v4i init[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) init[p] = *reinterpret_cast<const v4i*>(a.acc_init + f0 + p * 4);
+
+    v4i x[S], ev4 = {0, 0, 0, 0};
+    uint32_t opos = 0;
+    bool ok = false;
+    auto request = [&](int r) {
+        const uint32_t g = ((chunk * (uint32_t)a.rounds + (uint32_t)r) * 4u + (uint32_t)wave) * 16u + (uint32_t)(lane & 15);
+        const bool real = g < a.groups;
+        const uint32_t gg = real ? g : 0;
+        const uint32_t b = a.div_ohw4.div(gg), t = gg - b * a.OHW4, oy = a.div_ow4.div(t), ox0 = (t - oy * a.OW4) * 4u;
+        const uint32_t src = in_slice + b * (uint32_t)a.in_p.pb + (uint32_t)((int)oy * a.sy - a.py) * in_py
+                             + (uint32_t)(((int)ox0 * a.sx - a.px) * 16) + (uint32_t)q * 16u;
+#pragma unroll
+        for (int j = 0; j < FY; ++j)
+#pragma unroll
+            for (int n = 0; n < NB; ++n)  // (positions past the row belong to pixels that do not exist, or to no tap)
+                x[j * NB + n] = *reinterpret_cast<const v4i*>(a.in + min(src + (uint32_t)j * tap_py + (uint32_t)n * 64u, a.in_last));
+        const uint32_t ox = ox0 + (uint32_t)q;
+        ok = real && ox < (uint32_t)a.OW;
+        opos = b * (uint32_t)a.out_p.pb + oy * (uint32_t)a.out_p.py + ox * 16u;
+        if constexpr (EPI == EPI_KIND_FAST)
+            if (a.fe.fused && ok)
+                ev4 = *reinterpret_cast<const v4i*>(el + (b * (uint32_t)a.eltw_p.pb + oy * (uint32_t)(a.esy * (int)a.eltw_p.py) + ox * (uint32_t)(a.esx * 16)));
+    };
+    request(0);
+    for (int r = 0; r < a.rounds; ++r) {
+        v4i acc[4][1];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) acc[p][0] = init[p];
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            v4i xs = x[s];
+            asm volatile("" : "+v"(w[s]));  // the row operands are made here: made once for all rounds they take four times the registers
+#pragma unroll
+            for (int d = 0; d < 4; ++d) xs[d] ^= (int)a.xor_mask;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                v4i row = {0, 0, 0, 0};
+                row[p] = w[s][p];
+                acc[p][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(row, xs, acc[p][0], 0, 0, 0);
+            }
+        }
+        const v4i e = ev4;
+        const uint32_t at = opos;
+        const bool store = ok;
+        if (r + 1 < a.rounds) request(r + 1);
+        const v4i packed = epilogue_fast16<1, EPI>(a, acc, 0, sc.wq, sc.cal, sc.ecal, e, a.C - f0);
+        if (store) *reinterpret_cast<v4i*>(out + at) = packed;
+    }
+}
+
+// blocks of four positions that four neighbouring outputs see in a row
+static int dw_row_blocks(const ConvProblem& p)
+{
+    return (3 * p.sx + (p.FX - 1) * p.dx + 1 + 3) / 4;
+}
+
+DwPlan dw_plan(const ConvProblem& p, bool fast_epilogue, int cus)
 {
     DwPlan pl{};
     pl.block = 256;
+    const int nb = dw_row_blocks(p);
+    // 5x5 at strides 1 and 2, 3x3 at stride 1.  At stride 2 four outputs of a 3x3 row see nine positions, three blocks: that is
+    // as many loads as the dot products have taps (16 x 256 x 56x56: 7.0 us against 5.2), so those layers keep them.
+    if (dw_fast_applies(p, fast_epilogue) && ((p.FY == 3 && nb == 2) || (p.FY == 5 && (nb == 2 || nb == 3)))) {
+        pl.rows = 1;
+        pl.row_bytes = (size_t)((p.OFM + 15) / 16) * p.FY * nb * 1024;
+        const int64_t groups = (int64_t)p.B * p.OH * ((p.OW + 3) / 4), slices = (p.OFM + 15) / 16;
+        // sets of 64 pixels to a wave: one or two, so that the chip holds many waves (16 x 256 x 56x56, 5x5 at stride 2: 11.2 us
+        // with one, 10.4 with two, 12.5 with four), four 3x3 sets where there are 48 waves to a CU all the same
+        const int64_t sets = (groups + 15) / 16, per_cu = sets * slices / cus;
+        pl.rounds = p.FY == 5 ? (per_cu >= 8 ? 2 : 1) : per_cu >= 192 ? 4 : per_cu >= 96 ? 2 : 1;
+        pl.chunks = (int)((sets + 4 * pl.rounds - 1) / (4 * pl.rounds));
+        pl.works = (int)(pl.chunks * slices);
+        pl.grid_rows = (pl.works + 7) / 8 * 8;
+    }
     const int64_t m = (int64_t)p.B * p.OH * p.OW;
     const int64_t gx = (m + pl.block - 1) / pl.block;
     CHIP_REQUIRE(gx < (1ll << 31), CLDNN_HIP_UNSUPPORTED_SIZE, "convolution too large for one launch");
-    pl.grid = (int)gx;
+    pl.grid = (int)gx;  // of the accumulator probe as well
     pl.packed_bytes = (size_t)((p.OFM + 15) / 16) * p.FY * p.FX * 16;
     pl.mask_bytes = pl.packed_bytes * 4;
     return pl;
@@ -204,14 +318,44 @@ void dw_mask_weights(const ConvProblem& p, const int8_t* w, int32_t* masked)
                 (int32_t)((uint32_t)(uint8_t)w[(size_t)c * taps + t] << (8 * (c % 4)));
 }
 
-// the 3x3 kernel applies when: 3x3 filter, zero border covering the padding, short epilogue, 32-bit offsets
-bool dw_fast_applies(const ConvProblem& p, bool fast_epilogue)
+// rows [fs][filter row][block][lane] of four dwords: lane (row (q, i), position k) holds in dword p the weight with which
+// feature 4p + i of output pixel q takes position 4 * block + k, in byte i
+void dw_row_weights(const ConvProblem& p, const int8_t* w, int32_t* rows)
 {
-    return fast_epilogue && p.FY == 3 && p.FX == 3 && conv_border_covers(p) && tensor_elems(p.in_t) < (1ull << 31)
-           && tensor_elems(p.out_t) < (1ull << 31) && (int64_t)p.B * p.OH * p.OW < (1ll << 31);
+    const int nb = dw_row_blocks(p);
+    size_t at = 0;
+    for (int s = 0; s < (p.OFM + 15) / 16; ++s)
+        for (int j = 0; j < p.FY; ++j)
+            for (int n = 0; n < nb; ++n)
+                for (int lane = 0; lane < 64; ++lane)
+                    for (int d = 0; d < 4; ++d, ++at) {
+                        const int q = (lane % 16) / 4, i = lane % 4, c = s * 16 + d * 4 + i, t = 4 * n + lane / 16 - q * p.sx;
+                        rows[at] = 0;
+                        if (c < p.OFM && t >= 0 && t % p.dx == 0 && t / p.dx < p.FX)
+                            rows[at] = (int32_t)((uint32_t)(uint8_t)w[((size_t)c * p.FY + j) * p.FX + t / p.dx] << (8 * i));
+                    }
 }
 
-void launch_conv_dw(hipStream_t s, const ConvProblem& p, const DwPlan& pl, const int8_t* packed, const int32_t* masked,
+// what the two fast kernels ask for: zero border covering the padding, short epilogue, 32-bit offsets
+bool dw_fast_applies(const ConvProblem& p, bool fast_epilogue)
+{
+    return fast_epilogue && conv_border_covers(p) && tensor_elems(p.in_t) < (1ull << 31) && tensor_elems(p.out_t) < (1ull << 31)
+           && (p.eltw_t.b <= 0 || tensor_elems(p.eltw_t) < (1ull << 31)) && (int64_t)p.B * p.OH * (p.OW + 3) < (1ll << 31);
+}
+
+template <int FY, int NB>
+static void launch_rows(hipStream_t s, const DwPlan& pl, const DwArgs& a)
+{
+    const dim3 g(pl.grid_rows), b(256);
+    const FastEpi& f = a.fe;
+    const bool plain = a.epi.calib && !f.fused;
+    if (plain && f.has_wqf && f.iqf_one && f.clamp_folded) hipLaunchKernelGGL((conv_dw_rows_kernel<FY, NB, EPI_KIND_CLAMPQ>), g, b, 0, s, a);
+    else if (plain && !f.has_wqf && f.relu_folded) hipLaunchKernelGGL((conv_dw_rows_kernel<FY, NB, EPI_KIND_RELU>), g, b, 0, s, a);
+    else if (plain && !f.has_wqf && f.act == CLDNN_HIP_ACT_NONE) hipLaunchKernelGGL((conv_dw_rows_kernel<FY, NB, EPI_KIND_LINEAR>), g, b, 0, s, a);
+    else hipLaunchKernelGGL((conv_dw_rows_kernel<FY, NB, EPI_KIND_FAST>), g, b, 0, s, a);
+}
+
+void launch_conv_dw(hipStream_t s, const ConvProblem& p, const DwPlan& pl, const int8_t* packed, const int32_t* masked, const int32_t* rows,
                     const int32_t* acc_init, const Epilogue& epi, const FastEpi* fast, const void* in, const void* eltw,
                     void* out, int32_t* raw)
 {
@@ -225,9 +369,21 @@ void launch_conv_dw(hipStream_t s, const ConvProblem& p, const DwPlan& pl, const
     a.M = (int64_t)p.B * p.OH * p.OW;
     a.epi = epi;
     const dim3 grid(pl.grid, (p.OFM + 15) / 16);
+    if (fast) a.fe = *fast;
+    a.xor_mask = p.in_dt == CLDNN_HIP_U8 ? 0x80808080u : 0u;
+    if (pl.rows && !raw) {
+        a.wrows = (const v4i*)rows, a.OW4 = (uint32_t)(p.OW + 3) / 4, a.OHW4 = (uint32_t)p.OH * a.OW4, a.groups = (uint32_t)p.B * a.OHW4;
+        a.chunks = (uint32_t)pl.chunks, a.works = (uint32_t)pl.works, a.rounds = pl.rounds;
+        a.in_last = (uint32_t)tensor_elems(p.in_t) - 16u;
+        a.div_ohw4 = make_fast_div(a.OHW4), a.div_ow4 = make_fast_div(a.OW4), a.div_chunks = make_fast_div(a.chunks);
+        const int nb = dw_row_blocks(p);
+        if (p.FY == 3) launch_rows<3, 2>(s, pl, a);
+        else if (nb == 2) launch_rows<5, 2>(s, pl, a);
+        else launch_rows<5, 3>(s, pl, a);
+        CHIP_CHECK(hipGetLastError());
+        return;
+    }
     if (fast && masked && !raw) {
-        a.fe = *fast;
-        a.xor_mask = p.in_dt == CLDNN_HIP_U8 ? 0x80808080u : 0u;
         a.div_ohw = make_fast_div((uint32_t)a.OHW), a.div_ow = make_fast_div((uint32_t)a.OW);
         const bool plain = !fast->has_wqf && epi.calib && !fast->fused;
         if (plain && fast->relu_folded) hipLaunchKernelGGL(conv_dw3x3_kernel<EPI_KIND_RELU>, grid, dim3(256), 0, s, a);

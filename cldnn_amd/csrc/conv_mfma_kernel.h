@@ -469,6 +469,10 @@ __device__ __forceinline__ void load_scales4(const Args& a, int f0, LaneScales& 
             if (a.fe.fc) e4 = *reinterpret_cast<const float4*>((const float*)e.bias + f0);  // never fused: the slot is free
             sc.ecal[d * 4 + 0] = e4.x, sc.ecal[d * 4 + 1] = e4.y, sc.ecal[d * 4 + 2] = e4.z, sc.ecal[d * 4 + 3] = e4.w;
         }
+    } else if constexpr (EPI == EPI_KIND_CLAMPQ) {
+        const float4 c4 = *reinterpret_cast<const float4*>(e.calib + f0), w4 = *reinterpret_cast<const float4*>(e.wqf + f0);
+        sc.cal[d * 4 + 0] = c4.x, sc.cal[d * 4 + 1] = c4.y, sc.cal[d * 4 + 2] = c4.z, sc.cal[d * 4 + 3] = c4.w;
+        sc.wq[d * 4 + 0] = w4.x, sc.wq[d * 4 + 1] = w4.y, sc.wq[d * 4 + 2] = w4.z, sc.wq[d * 4 + 3] = w4.w;
     }
 }
 

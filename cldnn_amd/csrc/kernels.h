@@ -131,13 +131,17 @@ struct DwPlan {
     int grid, block;
     size_t packed_bytes;
     size_t mask_bytes;  // masked weight dwords of the 3x3 kernel
+    int rows;           // the matrix-core kernel: its grid, workgroups to a slice, workgroups in all, sets of 64 pixels to a wave
+    int grid_rows, chunks, works, rounds;
+    size_t row_bytes;
 };
-DwPlan dw_plan(const ConvProblem& p);
+DwPlan dw_plan(const ConvProblem& p, bool fast_epilogue, int cus);
 void dw_pack_weights(const ConvProblem& p, const int8_t* w, int8_t* packed);
 void dw_mask_weights(const ConvProblem& p, const int8_t* w, int32_t* masked);
+void dw_row_weights(const ConvProblem& p, const int8_t* w, int32_t* rows);
 bool dw_fast_applies(const ConvProblem& p, bool fast_epilogue);
 bool conv_border_covers(const ConvProblem& p);
-void launch_conv_dw(hipStream_t s, const ConvProblem& p, const DwPlan& plan, const int8_t* packed, const int32_t* masked,
+void launch_conv_dw(hipStream_t s, const ConvProblem& p, const DwPlan& plan, const int8_t* packed, const int32_t* masked, const int32_t* rows,
                     const int32_t* acc_init, const Epilogue& epi, const FastEpi* fast, const void* in, const void* eltw,
                     void* out, int32_t* raw);
 

@@ -895,3 +895,28 @@ def test_float_output_of_every_row(eng, OFM):
         for tile in [0] + [t for t in tiles() if not tile_names()[t - 1].startswith(("stem", "stream"))]:
             got = hip.conv_forward(eng, x, w, bias, wq, ca, fmt="fs_b_yx_fsv16", in_pad=(1, 1), pad=(1, 1), out_dt="f32", tile=tile, **kw)
             assert_same(ref, got)
+
+
+@pytest.mark.parametrize("shape", [(2, 40, 9, 5, 3, 1, 1), (1, 16, 3, 1, 3, 1, 1), (3, 72, 13, 15, 5, 1, 1), (1, 33, 11, 6, 5, 1, 1), (2, 48, 14, 17, 5, 2, 1),
+                                   (1, 32, 12, 11, 3, 1, 2), (4, 336, 112, 61, 3, 1, 1), (2, 336, 56, 61, 5, 1, 1)],
+                         ids=["ragged", "one_pixel", "5x5_ragged", "5x5", "5x5_stride_2", "dilated", "several_sets", "5x5_several_sets"])
+@pytest.mark.parametrize("form", ["linear", "fused", "clamp"])
+@pytest.mark.parametrize("in_dt", [np.uint8, np.int8], ids=["u8", "s8"])
+def test_depthwise_rows(eng, shape, form, in_dt):
+    """depthwise on the matrix cores: row lengths that are no multiple of four, rows that end at the end of the input,
+    features that do not fill a slice, several sets of pixels to a wave, the residual of the run-time form"""
+    B, C, H, W, F, s, dil = shape
+    x, w, bias, wqf, calib = problem(31, B, C, H, W, C, F, F, in_dt, groups=C)
+    r = np.random.default_rng(5)
+    pad = dil * (F // 2)
+    kw = dict(stride=(s, s), pad=(pad, pad), dilation=(dil, dil), groups=C, out_dt="s8", act="none")
+    wqf, calib = np.ones(C, np.float32), (40.0 / (F * 147.4 * 73.3) * r.uniform(0.5, 2, C)).astype(np.float32)
+    if form == "clamp":
+        wqf, calib = (3.0 / (F * 147.4 * 73.3) * r.uniform(0.5, 2, C)).astype(np.float32), np.full(C, 127 / 6, np.float32)
+        kw.update(act="clamp", act_m=0.0, act_n=6.0)
+    if form == "fused":
+        OH, OW = ((n + 2 * pad - dil * (F - 1) - 1) // s + 1 for n in (H, W))
+        kw.update(eltw=r.integers(-128, 128, (B, C, OH, OW)).astype(np.int8), eltw_act="relu", eltw_calib=r.uniform(0.5, 1, C).astype(np.float32))
+    ref, (got, info) = both(eng, x, w, bias, wqf, calib, fmt="fs_b_yx_fsv16", in_pad=(pad, pad), acc=False, **kw)
+    assert b"rows" in info.kernel_name
+    assert_same(ref, got)
