@@ -28,6 +28,7 @@ struct cldnn_hip_conv_s {
     void* w_rows = nullptr;   // depthwise rows kernel
     void* w_masked = nullptr; // depthwise 3x3 kernel: one weight byte per dword
     void* ktab = nullptr;
+    void* origin = nullptr;   // grouped: where the input of each span of 64 output features starts
     void* gather = nullptr;   // scratch of the small-batch kernel (activations in fragment order)
     void* acc_init = nullptr;      // int32: offset correction + int32 bias
     void* acc_init_raw = nullptr;  // int32: offset correction only (accumulator probe)
@@ -188,11 +189,10 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
     const bool stem = d.input.format == CLDNN_HIP_FMT_B_FS_YX_FSV4 && d.output.format == CLDNN_HIP_FMT_FS_B_YX_FSV16
                       && (!d.fused || p.eltw_t.format == CLDNN_HIP_FMT_FS_B_YX_FSV16) && d.ifm <= 4 && d.groups == 1
                       && d.dilation_x == 1 && conv_border_covers(p) && (p.FY * ((p.FX + 3) / 4) + 3) / 4 <= 8;
-    // Grouped (not depthwise) convolutions run on the same matrix-core kernels as one dense convolution whose weight
-    // matrix is block-diagonal: feature f only has weights for the input features of its own group, the rest are zero.
-    // That is the arithmetic of the reference's per-group launches (fused_conv_eltwise_gpu_ref.cl:108-112,134-136) in one
-    // launch; the zero blocks cost matrix-core time that these layers do not miss (they are bound by launch and memory),
-    // and dense weights of more than 64 MiB stay on the one-thread-per-output kernel.
+    // Grouped (not depthwise) convolutions run on the same matrix-core kernels as a dense convolution, in one launch: a tile
+    // of 64 output features reads the input features of its groups, and a feature has zero weights for those of the others.
+    // That is the arithmetic of the reference's per-group launches (fused_conv_eltwise_gpu_ref.cl:108-112,134-136).
+    // Layers whose dense weights would be more than 64 MiB stay on the one-thread-per-output kernel.
     const bool grouped = d.groups > 1 && !depthwise;
     const bool grouped_dense = grouped && blocked && (size_t)d.ofm * d.ifm * d.fy * d.fx <= ((size_t)64 << 20);
     int impl = d.impl;
@@ -277,12 +277,31 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
 
     std::vector<int8_t> dense;
     if (impl == CLDNN_HIP_IMPL_MFMA && grouped) {
-        // [ofm][ifm / groups][fy][fx] -> block-diagonal [ofm][ifm][fy][fx]
-        const size_t taps = (size_t)p.FY * p.FX, ofm_g = (size_t)p.OFM / p.groups;
-        dense.assign((size_t)p.OFM * p.IFM * taps, 0);
+        // [ofm][ifm / groups][fy][fx] -> [ofm][features its span of 64 reads][fy][fx].  The groups of a span read a run of
+        // input features; every span gets as many slices as the longest run, starting where its own does.  One run of all
+        // features (a block-diagonal matrix) when a row of the table is asked for: some of its tiles are wider than a span.
+        const int taps = p.FY * p.FX, ofm_g = p.OFM / p.groups, all = (p.IFM + 15) / 16, spans = (p.OFM + 63) / 64;
+        auto first_feature = [&](int span) { return span * 64 / ofm_g * (int)ifm_g; };
+        int count = 0;
+        for (int sp = 0; sp < spans; ++sp) {
+            const int last = (std::min(sp * 64 + 64, p.OFM) - 1) / ofm_g * (int)ifm_g + (int)ifm_g - 1;
+            count = std::max(count, last / 16 - first_feature(sp) / 16 + 1);
+        }
+        // slices in fours for the kernels that want them so, where that costs at most a third
+        if (count % 4 && (count + 3) / 4 * 4 * 3 <= count * 4) count = (count + 3) / 4 * 4;
+        count = d.tile_override > 0 ? all : std::min(count, all);
+        std::vector<int32_t> origin(spans);
+        for (int sp = 0; sp < spans; ++sp) origin[sp] = std::min(first_feature(sp) / 16, all - count);
+        const int width = count < all ? count * 16 : p.IFM;
+        dense.assign((size_t)p.OFM * width * taps, 0);
         for (int f = 0; f < p.OFM; ++f) {
-            const size_t g = (size_t)f / ofm_g;
-            std::memcpy(&dense[((size_t)f * p.IFM + g * ifm_g) * taps], w8 + (size_t)f * ifm_g * taps, (size_t)ifm_g * taps);
+            const size_t at = (size_t)(f / ofm_g) * ifm_g - (size_t)origin[f / 64] * 16;
+            std::memcpy(&dense[((size_t)f * width + at) * taps], w8 + (size_t)f * ifm_g * taps, (size_t)ifm_g * taps);
+        }
+        if (count < all) {
+            for (int32_t& o : origin) o *= (int32_t)p.in_p.pf;
+            c->origin = upload(c, origin.data(), origin.size() * 4);
+            p.IFM = width, p.by_span = 1;
         }
         w8 = dense.data();
         p.groups = 1;  // from here on the problem is the dense one (the algorithmic work above counts the real weights)
@@ -300,7 +319,7 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
         const TileConfig& tc = tile_config(tile);
         inf.tile_index = tile, inf.tile_pixels = tc.tile_pixels, inf.tile_ofm = tc.tile_ofm;
         inf.grid = c->mplan.grid, inf.block = c->mplan.ksplit ? 64 * c->mplan.ks_waves : c->mplan.block, inf.lds_bytes = c->mplan.lds_bytes;
-        std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_%s<%s,%s,%s>", c->mplan.gemv ? "gemv" : c->mplan.ksplit ? "ksplit" : c->mplan.halo ? "halo" : c->mplan.stream ? "stream" : (c->mplan.bdir ? "bdir" : (c->mplan.wsl ? "wsl" : "mfma")),
+        std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_%s<%s,%s,%s>", c->mplan.gemv ? "gemv" : c->mplan.ksplit ? "ksplit" : c->mplan.halo ? "halo" : c->mplan.stream ? "stream" : (c->mplan.bdir ? "bdir" : (c->mplan.wsl ? "wsl" : c->mplan.direct ? "mfma_direct" : "mfma")),
                       tc.name, c->mplan.checked ? "checked" : "border", c->fast && !c->fe.f32 && !c->mplan.gemv ? "fast" : "generic");
     } else {
         std::vector<int8_t> packed(c->dplan.packed_bytes);
@@ -387,7 +406,7 @@ static void run(cldnn_hip_conv c, const void* in, void* out, const void* eltw, i
         launch_conv_ref(s, p, c->epi, in, c->w_raw, eltw, out, raw);
         break;
     case CLDNN_HIP_IMPL_MFMA: {
-        MfmaBuffers wb{(const int8_t*)c->w_packed, (const int32_t*)c->ktab, c->gather};
+        MfmaBuffers wb{(const int8_t*)c->w_packed, (const int32_t*)c->ktab, c->gather, (const int32_t*)c->origin};
         if (static_scratch) {
             // the gather scratch comes from the array inside the code object instead of the object's own allocation
             const size_t need = mfma_gather_bytes(p, c->mplan);

@@ -72,12 +72,13 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
 
     uint32_t boff[PT];
     int iy0[PT], ix0[PT];
+    const int origin = a.in_off + span_origin(a, span);
 #pragma unroll
     for (int pt = 0; pt < PT; ++pt) {
         const uint32_t m = (uint32_t)(ptile * PT + pt) * 16 + l16;
         const PixelPos pp = pixel_pos(a, m < a.M ? m : 0);  // pixels past the end read pixel 0
         iy0[pt] = (int)pp.oy * a.sy - a.py, ix0[pt] = (int)pp.ox * a.sx - a.px;
-        boff[pt] = (uint32_t)(a.in_off + (int)pp.b * a.in_pb + iy0[pt] * a.in_py + ix0[pt] * 16 + (ADDR == ADDR_UNIFORM ? kq * a.in_pf : 0));
+        boff[pt] = (uint32_t)(origin + (int)pp.b * a.in_pb + iy0[pt] * a.in_py + ix0[pt] * 16 + (ADDR == ADDR_UNIFORM ? kq * a.in_pf : 0));
     }
 
     // (group of four slices, filter row, filter column) of the next step to request; taps innermost

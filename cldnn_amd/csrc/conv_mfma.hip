@@ -14,6 +14,7 @@ DECL_TILE(0) DECL_TILE(1) DECL_TILE(2) DECL_TILE(3) DECL_TILE(4) DECL_TILE(5)
 void launch_stream(hipStream_t s, const MfmaArgs& a, int nt, int grid, int epi);
 void launch_bdir_f64(hipStream_t s, const MfmaArgs& a, int nt, int grid, int lds, int epi);
 void launch_bdir_f128(hipStream_t s, const MfmaArgs& a, int nt, int grid, int lds, int epi);
+void launch_direct(hipStream_t s, const MfmaArgs& a, int ofm, int nt, int grid, int lds, int epi);
 void launch_bdir_k2(hipStream_t s, const MfmaArgs& a, int nt, int grid, int lds, int epi);
 void launch_bdir_k4(hipStream_t s, const MfmaArgs& a, int nt, int grid, int lds, int epi);
 void launch_ksplit(hipStream_t s, const MfmaArgs& a, int ft, int pt, int grid, bool lanes, int epi);
@@ -171,7 +172,76 @@ static int choose_ksplit(int64_t m, int ofm, int taps, int cb, int ksteps, bool 
     return best;
 }
 
+static int choose_row(const ConvProblem& p, int cus);
+static int choose_row(const ConvProblem& p, int cus);
+static void wsl_depth(int ksteps, int* depth, int* padded);
+// Microseconds of a row on an arbitrary shape with a border: start + K-steps * time of a step + output bytes.  A step takes
+// its latency (`step`) or, with several workgroups on a CU, its throughput (`load` times the workgroups per CU), whichever
+// is longer.  Fitted to timings of 270 layers drawn over 1 to 150 images, 3 to 480 K-steps and 8 to 1016 features
+// (within 10-14 % rms).  The table in choose_row was swept over the layers of three networks; picking by these costs
+// instead takes a layer drawn from that range from 11 % above its best row to 5 % (slices in fours), and from 9 % to 3 %.
+struct RowCost {
+    int row;
+    double start, step, load, per_mb;
+};
+static const RowCost g_row_costs[] = {
+    {ROW_BDIR_P64_F64, 3.94, 0.117, 0.099, 0.66},  {ROW_BDIR_P128_F64, 4.42, 0.150, 0.154, 0.65},
+    {ROW_BDIR_P256_F64, 5.05, 0.231, 0.249, 0.57}, {ROW_BDIR_P128_F128, 4.44, 0.252, 0.241, 0.58},
+    {ROW_BDIR_P256_F128, 5.35, 0.391, 0.383, 0.51}, {ROW_WSL_P64, 4.15, 0.126, 0.113, 0.30},
+    {ROW_WSL_P128, 4.09, 0.197, 0.178, 0.43}, {ROW_BDIR_K2_P128_F64, 5.54, 0.062, 0.188, 1.23}, {ROW_BDIR_K2_P64_F64, 4.82, 0.028, 0.139, 1.21},
+    // run by the direct-activation kernel with an offset per chunk
+    {ROW_P64_F64, 3.83, 0.145, 0.097, 0.69},   {ROW_P128_F64, 4.44, 0.173, 0.148, 0.72}, {ROW_P256_F64, 5.30, 0.235, 0.238, 0.65},
+    {ROW_P64_F128, 4.47, 0.200, 0.177, 0.76},  {ROW_P128_F128, 4.40, 0.260, 0.231, 0.72}, {ROW_P256_F128, 5.45, 0.417, 0.354, 0.66},
+};
+static double row_us(const RowCost& c, const ConvProblem& p, int64_t m, int ksteps, int cus)
+{
+    const TileConfig& tc = g_tiles[c.row];
+    const double wgs = (double)((m + tc.tile_pixels - 1) / tc.tile_pixels) * ((p.OFM + tc.tile_ofm - 1) / tc.tile_ofm) / cus;
+    const double busy = wgs > 4.0 ? wgs : 0.5 * (wgs + std::max(1.0, std::ceil(wgs - 0.05)));  // part of the last round is idle
+    const double load = c.load * busy, step = std::cbrt(c.step * c.step * c.step + load * load * load);
+    const double mb = (double)m * p.OFM * (p.out_dt == CLDNN_HIP_F32 ? 4 : p.eltw_t.b > 0 ? 2 : 1) / 1e6;
+    return c.start + ksteps * step + c.per_mb * mb;
+}
+// the cheapest row of the same kind (slices in fours or not), if it beats `row` clearly
+static int cheaper_row(const ConvProblem& p, int row, int cus)
+{
+    const int64_t m = (int64_t)p.B * p.OH * p.OW;
+    const int cb = (p.IFM + 15) / 16, ksteps = (p.FY * p.FX * cb + 3) / 4;
+    auto cost = [](int r) {
+        for (const RowCost& c : g_row_costs)
+            if (c.row == r) return &c;
+        return (const RowCost*)nullptr;
+    };
+    const bool fours = cb % 4 == 0;
+    // (layers of more pixels than the fit covers are in the table's sweeps: they stay with it)
+    if (m > 131072 || !border_covers(p) || !cost(row) || (row < FIRST_STREAM_ROW) == fours) return row;
+    // (the split-K rows are the ones the fit describes worst: an eighth there)
+    double best = (g_tiles[row].kgroups > 1 ? 0.88 : 0.95) * row_us(*cost(row), p, m, ksteps, cus);
+    for (const RowCost& c : g_row_costs) {
+        if ((c.row < FIRST_STREAM_ROW) == fours || (p.by_span && g_tiles[c.row].tile_ofm > 64)) continue;
+        int depth, padded;
+        if (c.row >= FIRST_WSL_ROW && (wsl_depth(ksteps, &depth, &padded), padded * 4096 > WSL_MAX_LDS)) continue;
+        if (const double us = row_us(c, p, m, ksteps, cus); us < best) best = us, row = c.row;
+    }
+    return row;
+}
+
 int mfma_choose(const ConvProblem& p, int cus)
+{
+    const int row = cheaper_row(p, choose_row(p, cus), cus);
+    if (!p.by_span || g_tiles[row].tile_ofm <= 64) return row;
+    // spans of a grouped layer start at slices of their own: tiles of one span
+    switch (row) {
+    case ROW_P128_F128: return ROW_P128_F64;
+    case ROW_P64_F128: return ROW_P64_F64;
+    case ROW_P256_F128: return ROW_P256_F64;
+    case ROW_BDIR_P64_F128: return ROW_BDIR_P64_F64;
+    case ROW_BDIR_P128_F128: return ROW_BDIR_P128_F64;
+    default: return ROW_BDIR_P256_F64;
+    }
+}
+
+static int choose_row(const ConvProblem& p, int cus)
 {
     if (p.in_t.format == CLDNN_HIP_FMT_B_FS_YX_FSV4)
         return p.FY * ((p.FX + 3) / 4) > 8 ? ROW_STEM_P64 : ROW_STEM_P32;  // more than two K-steps of four 4-tap chunks
@@ -186,7 +256,7 @@ int mfma_choose(const ConvProblem& p, int cus)
 
     // a fragment or two of pixels and a long K (fully_connected): the weights are the traffic and the tile kernels
     // would occupy one workgroup per 64 features
-    if (direct && m <= 32 && ksteps >= 16) return ROW_GEMV;
+    if (direct && !p.by_span && m <= 32 && ksteps >= 16) return ROW_GEMV;
     if (const int row = choose_ksplit(m, p.OFM, p.FY * p.FX, cb, ksteps, border, cus); row >= 0) return row;
     // a few pixels and K <= 256: one round trip per wave and no barrier (3.0-3.4 us against 3.5-3.7 for the LDS tiles)
     if (border && ksteps <= 4 && m < 4096 && !stream_fits) return ROW_STREAM_P16;
@@ -211,7 +281,7 @@ int mfma_choose(const ConvProblem& p, int cus)
         // 256 and more features: 64 pixels x 128 features per wave, two waves per SIMD (3x3 at 56x56 with 128 / 256 input features)
         if (p.OFM >= 256 && p.OFM % 128 == 0) return ROW_BDIR_P256_F128;
         if (ksteps <= 18) return p.OFM <= 128 ? ROW_WSL_P128 : ROW_WSL_P64;  // 3x3 at 56x56 .. 224x224 with 64 / 128 input features
-        return p.OFM >= 128 ? ROW_P256_F128 : ROW_BDIR_P256_F64;
+        return p.OFM >= 128 ? ROW_BDIR_P256_F128 : ROW_BDIR_P256_F64;
     }
     const int64_t grid_p128_f64 = ((m + 127) / 128) * ((p.OFM + 63) / 64);
     if (m >= 8192) {
@@ -294,6 +364,8 @@ MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus, bool forced)
         while (ks < pl.ksteps) ks *= 2;  // compile-time K-step counts: 1, 2, 4, 8 (zero-weight padding chunks)
         pl.ksteps = ks;
     }
+    // feature slices that do not come in fours: the table's LDS-staged tiles run on the direct-activation kernel
+    pl.direct = tile < FIRST_STREAM_ROW && !forced && !pl.checked && pl.cb % 4 != 0 ? 1 : 0;
     if (tc.kgroups > 1) pl.ksteps = (pl.ksteps + tc.kgroups - 1) / tc.kgroups * tc.kgroups;  // zero-weight padding steps
     if (pl.wsl) {
         wsl_depth(pl.ksteps, &pl.wsl_depth, &pl.ksteps);
@@ -303,7 +375,7 @@ MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus, bool forced)
     // K order.  With the taps innermost, consecutive K-steps of a wave read the same cache lines of the input shifted
     // by one pixel (or one row), so most activation loads of a 3x3 filter hit in the CU's L1 instead of going to L2.
     // The weights-stationary and streaming kernels walk the taps with counters in (tap, slice) order.
-    pl.tap_minor = pl.shifted || (!pl.stream && !pl.wsl && !pl.ks_lanes && pl.cb % 4 == 0 && p.FY * p.FX > 1) ? 1 : 0;
+    pl.tap_minor = pl.shifted || pl.direct || (!pl.stream && !pl.wsl && !pl.ks_lanes && pl.cb % 4 == 0 && p.FY * p.FX > 1) ? 1 : 0;
     if (pl.halo) {
         const cldnn_hip_tensor& t = p.in_t;
         CHIP_REQUIRE(p.FY * p.FX == HALO_TAPS && p.sy == 1 && p.sx == 1 && p.groups == 1, CLDNN_HIP_INVALID_ARG,
@@ -335,7 +407,7 @@ MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus, bool forced)
     pl.by_features = !pl.stream && !pl.wsl && !pl.ksplit && !pl.halo && w_bytes > in_bytes && (p.OFM + tc.tile_ofm - 1) / tc.tile_ofm >= 8 ? 1 : 0;
     int64_t grid = pl.by_features ? (int64_t)((pl.ofm_tiles + 7) / 8) * 8 * pl.mtiles : (int64_t)((pl.mtiles + 7) / 8) * 8 * pl.ofm_tiles;
     if (pl.stream) grid = ((int64_t)pl.mtiles * pl.ofm_tiles + 3) / 4;  // one wave per (pixel tile, span)
-    pl.lds_bytes = pl.stream ? 0 : (pl.bdir ? 3 * 4 * tc.tile_ofm * 16 : 2 * 4 * (tc.tile_ofm + tc.tile_pixels) * 16);
+    pl.lds_bytes = pl.stream ? 0 : (pl.bdir || pl.direct ? 3 * 4 * tc.tile_ofm * 16 : 2 * 4 * (tc.tile_ofm + tc.tile_pixels) * 16);
     if (tc.kgroups > 1)  // per-group weight buffers, later reused for the partial sums of groups 1..
         pl.lds_bytes = std::max(tc.kgroups * pl.lds_bytes, (tc.kgroups - 1) * (tc.tile_ofm / 16) * (tc.wave_pixels / 16) * 4096);
     if (pl.wsl) {
@@ -420,8 +492,13 @@ void mfma_pack_weights(const ConvProblem& p, const MfmaPlan& pl, const int8_t* w
     }
     // k-chunk -> (tap, feature slice): tap-major with the slices innermost, or groups of 4 slices with the taps innermost
     const int taps = p.FY * p.FX;
-    auto chunk_tap = [&](int kc) { return pl.tap_minor ? (kc / 4) % taps : kc / pl.cb; };
+    const int fours = pl.cb / 4 * 4 * taps, left = std::max(1, pl.cb % 4);  // direct: chunks of whole groups; slices of the last one
+    auto chunk_tap = [&](int kc) {
+        if (pl.direct && kc >= fours) return (kc - fours) / left;
+        return pl.tap_minor ? (kc / 4) % taps : kc / pl.cb;
+    };
     auto chunk_slice = [&](int kc) {
+        if (pl.direct && kc >= fours) return pl.cb / 4 * 4 + (kc - fours) % left;
         if (pl.shifted) return std::min((kc / 4) / taps * 4, pl.cb - 4) + kc % 4;
         return pl.tap_minor ? (kc / 4) / taps * 4 + kc % 4 : kc % pl.cb;
     };
@@ -640,6 +717,7 @@ void launch_conv_mfma(hipStream_t s, const ConvProblem& p, const MfmaPlan& pl, c
         }
     }
     a.bpk = (const v4i*)wb.gather;
+    a.origin = wb.origin;
     if (pl.halo) {
         HaloArgs h{};
         h.m = a;
@@ -668,6 +746,7 @@ void launch_conv_mfma(hipStream_t s, const ConvProblem& p, const MfmaPlan& pl, c
         launch_ksplit(s, a, pl.ks_ft, pl.ks_pt, pl.grid, pl.ks_lanes != 0, kind);
     }
     else if (pl.stream) launch_stream(s, a, tc.wave_pixels / 16, pl.grid, kind);
+    else if (pl.direct) launch_direct(s, a, tc.tile_ofm, tc.tile_pixels / 64, pl.grid, pl.lds_bytes, kind);
     else if (pl.bdir && tc.kgroups == 2) launch_bdir_k2(s, a, tc.wave_pixels / 16, pl.grid, pl.lds_bytes, kind);
     else if (pl.bdir && tc.kgroups == 4) launch_bdir_k4(s, a, tc.wave_pixels / 16, pl.grid, pl.lds_bytes, kind);
     else if (pl.bdir && tc.tile_ofm == 64) launch_bdir_f64(s, a, tc.wave_pixels / 16, pl.grid, pl.lds_bytes, kind);

@@ -78,6 +78,7 @@ struct MfmaArgs {
     // split-K kernel: waves per workgroup, K-steps per wave, bounds checks (input without a border)
     int32_t kwaves, kper, checked, dil_y, dil_x;
     FastDiv div_taps;
+    const int32_t* origin;  // grouped: byte offset of the first input slice that each span of 64 output features reads
     FastEpi fe;
     Epilogue epi;
 };
@@ -179,6 +180,13 @@ typedef const int32_t __attribute__((address_space(4))) * const_i32_ptr;
 __device__ __forceinline__ int32_t scalar_table_load(const int32_t* table, int index)
 {
     return ((const_i32_ptr)(uintptr_t)table)[index];
+}
+
+// where the input of a feature tile starts (MfmaArgs.origin; 0 for dense layers)
+template <class Args>
+__device__ __forceinline__ int32_t span_origin(const Args& a, int span)
+{
+    return a.origin ? scalar_table_load(a.origin, span) : 0;
 }
 
 __device__ __forceinline__ float rha(float v) { return truncf(v + copysignf(0.49999997f, v)); }
@@ -551,7 +559,7 @@ __device__ __forceinline__ void fetch_arguments(const MfmaArgs& a)
     asm volatile("" ::"s"(a.div_cb.mul), "s"(a.div_cb.shift), "s"(a.div_cb.one), "s"(a.div_fx.mul), "s"(a.div_fx.shift),
                  "s"(a.div_fx.one), "s"(a.div_mtiles.mul), "s"(a.div_mtiles.shift), "s"(a.div_mtiles.one), "s"(a.div_ofm_tiles.mul),
                  "s"(a.div_ofm_tiles.shift), "s"(a.div_ofm_tiles.one), "s"(a.xor_mask), "s"(a.wsl_parts), "s"(a.wsl_tpp), "s"(a.FY),
-                 "s"(a.epi.calib), "s"(a.epi.eltw_calib), "s"(a.epi.wqf), "s"(a.fe.hi), "s"(a.fe.lo));
+                 "s"(a.epi.calib), "s"(a.epi.eltw_calib), "s"(a.epi.wqf), "s"(a.fe.hi), "s"(a.fe.lo), "s"(a.origin));
 }
 
 __device__ __forceinline__ PixelPos pixel_pos(const MfmaArgs& a, uint32_t m)
@@ -626,7 +634,7 @@ __global__ void __launch_bounds__(256) conv_mfma_kernel(MfmaArgs a)
         const PixelPos pp = pixel_pos(a, ld_valid ? m0 + lp : 0);
         iy0 = (int)pp.oy * a.sy - a.py;
         ix0 = (int)pp.ox * a.sx - a.px;
-        pix_off = a.in_off + (int)pp.b * a.in_pb + iy0 * a.in_py + ix0 * 16;
+        pix_off = a.in_off + span_origin(a, ntile) + (int)pp.b * a.in_pb + iy0 * a.in_py + ix0 * 16;
     }
     const v4i* wsrc = a.wpk + (size_t)ntile * a.ksteps * (4 * BN) + t;
 
@@ -742,7 +750,13 @@ __global__ void __launch_bounds__(256) conv_mfma_kernel(MfmaArgs a)
 // reads per 4*NT MFMAs (the LDS-staged 64x64 tile: 5 reads per 4 MFMAs), so the LDS pipe stops being the bound.
 #define BDIR_PREFETCH_DISTANCE(loads) ((loads) <= 3 ? 8 : ((loads) <= 4 ? 6 : 4))
 
-template <int BN, int NT, int KG, int EPI>
+//
+// LANES: feature slices that do not come in fours, or fewer than four.  The four chunks of a K-step are then any four
+// (tap, slice) pairs: a step reads four table entries and each lane picks its own.  Seven vector instructions a step,
+// against 8 to 64 matrix instructions of four times their length; the LDS-staged kernel, which had these shapes before,
+// moves every activation through LDS.
+// 5 x 142 -> 638, 61x61, 5x5: 112 us there, 50 here; 12 x 213 -> 178, 36x42, 3x3: 24.6 and 13.9.
+template <int BN, int NT, int KG, bool LANES, int EPI>
 __global__ void __launch_bounds__(256 * KG) conv_bdir_kernel(MfmaArgs a)
 {
     fetch_arguments(a);
@@ -793,12 +807,13 @@ __global__ void __launch_bounds__(256 * KG) conv_bdir_kernel(MfmaArgs a)
 
     // byte offset of (pixel, slice kq) of each of the lane's pixels; pixels past the end read pixel 0
     uint32_t boff[NT];
+    const int origin = a.in_off + span_origin(a, ntile);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         const uint32_t m = m0 + nt * 16 + l16;
         const PixelPos pp = pixel_pos(a, m < a.M ? m : 0);
-        boff[nt] = (uint32_t)(a.in_off + (int)pp.b * a.in_pb + ((int)pp.oy * a.sy - a.py) * a.in_py
-                              + ((int)pp.ox * a.sx - a.px) * 16 + kq * a.in_pf);
+        boff[nt] = (uint32_t)(origin + (int)pp.b * a.in_pb + ((int)pp.oy * a.sy - a.py) * a.in_py
+                              + ((int)pp.ox * a.sx - a.px) * 16 + (LANES ? 0 : kq * a.in_pf));
     }
     const int steps = a.ksteps / KG;  // the host pads the K-steps to a multiple of KG
     const int step0 = grp * steps;
@@ -816,6 +831,16 @@ __global__ void __launch_bounds__(256 * KG) conv_bdir_kernel(MfmaArgs a)
         for (int q = 0; q < A_LOADS; ++q) xa[q] = wsrc[(size_t)ks * (4 * BN) + q * 256];
     };
     auto load_b = [&](int ks, v4i (&xb)[NT]) {
+        if constexpr (LANES) {
+            int e[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) e[c] = scalar_table_load(a.ktab, (step0 + ks) * 4 + c);
+            const int lo = kq & 1 ? e[1] : e[0], hi = kq & 1 ? e[3] : e[2];
+            const uint32_t off = (uint32_t)(kq & 2 ? hi : lo);
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) xb[nt] = *reinterpret_cast<const v4i*>(a.in + (boff[nt] + off));
+            return;
+        }
         // the four k-chunks of a step are one tap and four consecutive slices: one uniform offset per step
         const int8_t* base = a.in + scalar_table_load(a.ktab, (step0 + ks) * 4);
 #pragma unroll
@@ -1101,13 +1126,14 @@ __global__ void __launch_bounds__(256) conv_wsl_kernel(MfmaArgs a)
         int ob[NT], eb[NT];
         PixelPos pos[NT];
     };
+    const int origin = a.in_off + span_origin(a, ntile);
     auto setup = [&](int tile, TileRefs& r) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             const uint32_t m = ((uint32_t)tile * 4 + (uint32_t)wave) * WP + nt * 16 + l16;
             const bool ok = tile < t_end && m < a.M;
             const PixelPos pp = pixel_pos(a, ok ? m : 0);
-            r.boff[nt] = (uint32_t)(a.in_off + (int)pp.b * a.in_pb + ((int)pp.oy * a.sy - a.py) * a.in_py
+            r.boff[nt] = (uint32_t)(origin + (int)pp.b * a.in_pb + ((int)pp.oy * a.sy - a.py) * a.in_py
                                     + ((int)pp.ox * a.sx - a.px) * 16 + kq * a.in_pf);
             const int o = a.out_off + (int)pp.b * a.out_pb + fs * a.out_pf + (int)pp.oy * a.out_py + (int)pp.ox * 16;
             r.ob[nt] = ok && live ? o : -1;
@@ -1244,6 +1270,7 @@ __global__ void __launch_bounds__(256) conv_stream_kernel(MfmaArgs a)
     }
 
     // ---- requests
+    const int origin = a.in_off + span_origin(a, span);
     v4i fb[KS][NT], ev[NT], fa[KS][4], init[4];
     int ob[NT], eb[NT];
     PixelPos pos[NT];
@@ -1253,14 +1280,14 @@ __global__ void __launch_bounds__(256) conv_stream_kernel(MfmaArgs a)
         const uint32_t mm = m < a.M ? m : a.M - 1;
         int pix, o, e;
         if (a.linear) {  // dense tensors, 1x1 / stride 1: pixel m sits at m * 16, no division needed
-            pix = a.in_off + (int)mm * 16;
+            pix = origin + (int)mm * 16;
             o = a.out_off + fs * a.out_pf + (int)mm * 16;
             e = a.el_off + fs * a.el_pf + (int)mm * 16;
             pos[nt] = PixelPos{0, 0, 0};
         } else {
             const PixelPos pp = pixel_pos(a, mm);
             pos[nt] = pp;
-            pix = a.in_off + (int)pp.b * a.in_pb + ((int)pp.oy * a.sy - a.py) * a.in_py + ((int)pp.ox * a.sx - a.px) * a.px_bytes;
+            pix = origin + (int)pp.b * a.in_pb + ((int)pp.oy * a.sy - a.py) * a.in_py + ((int)pp.ox * a.sx - a.px) * a.px_bytes;
             o = a.out_off + (int)pp.b * a.out_pb + fs * a.out_pf + (int)pp.oy * a.out_py + (int)pp.ox * 16;
             e = a.el_off + (int)pp.b * a.el_pb + fs * a.el_pf + (int)(pp.oy * a.esy) * a.el_py + (int)(pp.ox * a.esx) * 16;
         }
@@ -1331,7 +1358,7 @@ void launch_mfma_instance(hipStream_t s, const MfmaArgs& a, int grid, int lds, i
     }
 }
 
-template <int BN, int NT, int KG>
+template <int BN, int NT, int KG, bool LANES = false>
 void launch_bdir_instance(hipStream_t s, const MfmaArgs& a, int grid, int lds, int epi)
 {
     const dim3 g(grid), b(256 * KG);
@@ -1340,10 +1367,10 @@ void launch_bdir_instance(hipStream_t s, const MfmaArgs& a, int grid, int lds, i
     {                                                                                                           \
         static std::once_flag allowed;                                                                          \
         std::call_once(allowed, [] {                                                                            \
-            CHIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bdir_kernel<BN, NT, KG, KIND>),  \
+            CHIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_bdir_kernel<BN, NT, KG, LANES, KIND>),  \
                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));            \
         });                                                                                                     \
-        hipLaunchKernelGGL((conv_bdir_kernel<BN, NT, KG, KIND>), g, b, lds, s, a);                              \
+        hipLaunchKernelGGL((conv_bdir_kernel<BN, NT, KG, LANES, KIND>), g, b, lds, s, a);                              \
     }
     switch (epi) {
     case EPI_KIND_RELU: BDIR_LAUNCH(EPI_KIND_RELU) break;

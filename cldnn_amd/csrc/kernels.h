@@ -11,6 +11,7 @@ struct ConvProblem {
     int in_dt, w_dt, out_dt, eltw_dt;
     cldnn_hip_tensor in_t, out_t, eltw_t;
     Pitch in_p, out_p, eltw_p;
+    int by_span;  // grouped: IFM counts the features that a span of 64 outputs reads, from an origin of its own
 };
 
 // ---- layout-agnostic kernels (kernels_ref.hip)
@@ -54,6 +55,7 @@ struct MfmaPlan {
     int ks_ft, ks_pt;    // its tile in 16-feature and 16-pixel fragments
     int ks_waves, ks_per;  // its waves per workgroup, K-steps per wave
     int ks_lanes;        // 1: lanes find their own taps (fewer than four slices, or no border)
+    int direct;          // 1: a row of the LDS-staged kernel run by the direct-activation kernel with an offset per chunk
     int shifted;         // 1: feature slices not in fours: the last K-step of a tap starts at the last four slices
     int halo;            // 1: nine-tap stride-1 kernel with both operands staged in LDS by direct loads (conv_halo_kernel.h)
     int halo_patch_len;  // its patch length in positions per slice (multiple of 64)
@@ -84,6 +86,7 @@ struct MfmaBuffers {
     const int8_t* packed;
     const int32_t* ktab;
     void* gather = nullptr;  // small-batch kernel with a filter wider than one tap: mfma_gather_bytes() of scratch
+    const int32_t* origin = nullptr;  // grouped: byte offset of the first input slice of each span of 64 output features
 };
 size_t mfma_gather_bytes(const ConvProblem& p, const MfmaPlan& pl);  // 0 when the plan needs no scratch
 // The same scratch without an allocation: a fixed-size array inside the loaded code object, one copy per device.

@@ -1059,7 +1059,8 @@ static bool compile_siblings(cldnn_program_impl* prog, node* a)
         if (st == CLDNN_HIP_SUCCESS) {
             cldnn_hip_conv_info info{};
             hip_check(cldnn_hip_conv_get_info(c, &info));
-            if (!std::strstr(info.kernel_name, "generic")) {
+            // (the row for a few pixels has one name for all its epilogues, the short ones included)
+            if (!std::strstr(info.kernel_name, "generic") || std::strstr(info.kernel_name, "conv_gemv")) {
                 a->conv = c, a->conv_info = info;
                 return true;
             }

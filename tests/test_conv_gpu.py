@@ -920,3 +920,40 @@ def test_depthwise_rows(eng, shape, form, in_dt):
     ref, (got, info) = both(eng, x, w, bias, wqf, calib, fmt="fs_b_yx_fsv16", in_pad=(pad, pad), acc=False, **kw)
     assert b"rows" in info.kernel_name
     assert_same(ref, got)
+
+
+@pytest.mark.parametrize("shape", [(8, 150, 33, 35, 70, 3, 1), (9, 20, 40, 41, 130, 5, 1), (7, 330, 30, 31, 260, 3, 1), (5, 80, 59, 61, 648, 3, 2), (20, 36, 63, 64, 200, 5, 1),
+                                   (30, 600, 40, 40, 24, 1, 1)],
+                         ids=["10_slices", "2_slices_5x5", "21_slices", "5_slices_s2", "3_slices_wide_tiles", "38_slices_1x1"])
+@pytest.mark.parametrize("out", ["s8", "f32", "fused"])
+def test_direct_activations_without_slices_in_fours(eng, shape, out):
+    """feature slices that are no multiple of four: a K-step takes any four chunks, lanes look up their own"""
+    B, IFM, H, W, OFM, F, s = shape
+    x, w, bias, wqf, calib = problem(61, B, IFM, H, W, OFM, F, F, np.uint8 if out == "s8" else np.int8)
+    pad = F // 2
+    kw = dict(stride=(s, s), pad=(pad, pad), out_dt="f32" if out == "f32" else "s8", act="none")
+    if out == "fused":
+        OH, OW = ((n + 2 * pad - F) // s + 1 for n in (H, W))
+        r = np.random.default_rng(6)
+        kw.update(eltw=r.integers(-128, 128, (B, OFM, OH, OW)).astype(np.int8), eltw_act="relu", eltw_calib=r.uniform(0.5, 1, OFM).astype(np.float32))
+    got, info = hip.conv_forward(eng, x, w, bias, wqf, calib, fmt="fs_b_yx_fsv16", in_pad=(pad, pad), want_info=True, **kw)
+    assert b"conv_mfma_direct" in info.kernel_name, info.kernel_name
+    images = [0, B - 1]
+    if out == "fused":
+        kw["eltw"] = kw["eltw"][images]
+    assert_same(rc.conv(x[images], w, bias, wqf=wqf, calib=calib, **kw), got[images])
+
+
+@pytest.mark.parametrize("shape", [(2, 236, 20, 21, 144, 3, 4), (1, 68, 10, 69, 28, 3, 4), (8, 512, 40, 52, 88, 3, 8), (3, 512, 25, 25, 512, 3, 4), (2, 96, 9, 9, 384, 3, 2),
+                                   (1, 512, 6, 6, 128, 3, 32), (2, 192, 14, 14, 192, 1, 3)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("border", [True, False], ids=["border", "checked"])
+def test_grouped_spans_read_the_features_of_their_groups(eng, shape, border):
+    """groups that straddle spans of 64 outputs and slices of 16 inputs, runs that end at the last slice"""
+    B, IFM, H, W, OFM, F, G = shape
+    x, w, bias, wqf, calib = problem(62, B, IFM, H, W, OFM, F, F, groups=G)
+    pad = F // 2
+    kw = dict(pad=(pad, pad), groups=G, out_dt="s8", act="relu")
+    (ro, ra), (go, ga, info) = both(eng, x, w, bias, wqf, calib, fmt="fs_b_yx_fsv16", in_pad=(pad, pad) if border else (0, 0), **kw)
+    assert info.impl == hip.IMPL_MFMA
+    np.testing.assert_array_equal(ga, ra)
+    assert_same(ro, go)
