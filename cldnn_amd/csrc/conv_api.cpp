@@ -181,7 +181,13 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
     }
 
     // ---- kernel family
-    const bool blocked = d.input.format == CLDNN_HIP_FMT_FS_B_YX_FSV16 && d.output.format == CLDNN_HIP_FMT_FS_B_YX_FSV16
+    // a classifier's scores (one output pixel per image): the split-K kernel finishes four features at a time and can write
+    // them as plain bfyx or yxfb, which saves the layout change after it
+    const cldnn_hip_tensor& o = d.output;
+    p.plain_out = d.input.format == CLDNN_HIP_FMT_FS_B_YX_FSV16 && (o.format == CLDNN_HIP_FMT_BFYX || o.format == CLDNN_HIP_FMT_YXFB) && o.y == 1 && o.x == 1 && o.f % 4 == 0
+                  && is_int8(o.dtype) && !d.fused && d.groups == 1 && d.tile_override == 0 && o.pad_lo_b + o.pad_hi_b == 0
+                  && o.pad_lo_f + o.pad_hi_f + o.pad_lo_y + o.pad_hi_y + o.pad_lo_x + o.pad_hi_x == 0;
+    const bool blocked = d.input.format == CLDNN_HIP_FMT_FS_B_YX_FSV16 && (o.format == CLDNN_HIP_FMT_FS_B_YX_FSV16 || p.plain_out)
                          && (!d.fused || p.eltw_t.format == CLDNN_HIP_FMT_FS_B_YX_FSV16);
     const bool int_path = in8 && p.w_dt == CLDNN_HIP_S8 && e.mode != MODE_NAT;
     const bool depthwise = d.groups > 1 && d.groups == d.ifm && d.groups == d.ofm;

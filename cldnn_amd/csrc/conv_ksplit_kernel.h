@@ -197,7 +197,7 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
     const bool finisher = wave < FT * PT;
     const bool live = finisher && m < a.M && f0 < a.OFM;
     const PixelPos pp = pixel_pos(a, live ? m : 0);
-    const int obase = a.out_off + (int)pp.b * a.out_pb + (fb >> 4) * a.out_pf + (int)pp.oy * a.out_py + (int)pp.ox * 16 + (f0 & 15);
+    const int obase = a.out_off + (int)pp.b * a.out_pb + (fb >> 4) * a.out_pf + (int)pp.oy * a.out_py + (int)pp.ox * 16 + (f0 & 15) * a.out_f;
     const int ebase = a.el_off + (int)pp.b * a.el_pb + (fb >> 4) * a.el_pf + (int)(pp.oy * a.esy) * a.el_py + (int)(pp.ox * a.esx) * 16 + (f0 & 15);
     // what the epilogue reads, requested in front of the barrier
     v4i init = {0, 0, 0, 0};
@@ -234,7 +234,7 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
             }
             float ev = 0.f;
             if (e.fused) ev = load_as_float(a.eltw, e.eltw_dt, ebase + i);
-            store_out(a.out, e.out_dt, obase + i, epilogue_generic(e, sum[i], f0 + i, ev));
+            store_out(a.out, e.out_dt, obase + i * a.out_f, epilogue_generic(e, sum[i], f0 + i, ev));
         }
     } else if constexpr (EPI == EPI_KIND_F32) {
         float v[4];
@@ -247,7 +247,11 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
     } else {
         v4i acc4[4][1] = {{sum}, {v4i{0, 0, 0, 0}}, {v4i{0, 0, 0, 0}}, {v4i{0, 0, 0, 0}}};
         const v4i packed = epilogue_fast16<1, EPI>(a, acc4, 0, sc.wq, sc.cal, sc.ecal, ev4, valid);
-        *reinterpret_cast<int*>((int8_t*)a.out + obase) = packed[0];
+        int8_t* dst = (int8_t*)a.out + obase;
+        if (a.out_f == 1) *reinterpret_cast<int*>(dst) = packed[0];
+        else  // images innermost: the lanes next to this one write the bytes beside these
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dst[i * a.out_f] = (int8_t)(packed[0] >> (8 * i));
     }
 }
 

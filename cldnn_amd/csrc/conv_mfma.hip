@@ -256,6 +256,14 @@ static int choose_row(const ConvProblem& p, int cus)
 
     // a fragment or two of pixels and a long K (fully_connected): the weights are the traffic and the tile kernels
     // would occupy one workgroup per 64 features
+    if (p.plain_out && !(direct && m <= 32 && ksteps >= 16)) {
+        int best = FIRST_KSPLIT_ROW;
+        const int own_steps = border && cb >= 4 ? p.FY * p.FX * ((cb + 3) / 4) : ksteps;
+        auto us = [&](int row) { return ksplit_us(m, p.OFM, own_steps, cus, g_ksplit[row - FIRST_KSPLIT_ROW].ft, g_ksplit[row - FIRST_KSPLIT_ROW].pt); };
+        for (int row = FIRST_KSPLIT_ROW; row < tile_config_count(); ++row)
+            if (us(row) < us(best)) best = row;
+        return best;
+    }
     if (direct && !p.by_span && m <= 32 && ksteps >= 16) return ROW_GEMV;
     if (const int row = choose_ksplit(m, p.OFM, p.FY * p.FX, cb, ksteps, border, cus); row >= 0) return row;
     // a few pixels and K <= 256: one round trip per wave and no barrier (3.0-3.4 us against 3.5-3.7 for the LDS tiles)
@@ -342,6 +350,7 @@ MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus, bool forced)
         // 17 to 32 pixels: both fragments in one workgroup, so that every weight byte crosses to a CU once
         if (pl.gemv && !forced && (int64_t)p.B * p.OH * p.OW > 16) pl.ks_pt = 2;
     }
+    CHIP_REQUIRE(!p.plain_out || pl.ksplit, CLDNN_HIP_INVALID_ARG, "only the split-K kernel writes plain layouts");
     pl.block = 256;
     pl.bdir = ((tile >= FIRST_BDIR_ROW && tile < FIRST_WSL_ROW) || tile >= FIRST_BDIRK_ROW) && !pl.stem && !pl.ksplit && !pl.halo ? 1 : 0;
     pl.wsl = tile >= FIRST_WSL_ROW && tile < FIRST_BDIRK_ROW ? 1 : 0;
@@ -673,7 +682,8 @@ void launch_conv_mfma(hipStream_t s, const ConvProblem& p, const MfmaPlan& pl, c
     a.div_mtiles = make_div((uint32_t)a.mtiles), a.div_ofm_tiles = make_div((uint32_t)a.ofm_tiles);
     a.sy = p.sy, a.sx = p.sx, a.py = p.py, a.px = p.px, a.esy = p.esy, a.esx = p.esx;
     a.in_off = (int32_t)p.in_p.off, a.in_pb = (int32_t)p.in_p.pb, a.in_pf = (int32_t)p.in_p.pf, a.in_py = (int32_t)p.in_p.py;
-    a.out_off = (int32_t)p.out_p.off, a.out_pb = (int32_t)p.out_p.pb, a.out_pf = (int32_t)p.out_p.pf;
+    a.out_off = (int32_t)p.out_p.off, a.out_pb = (int32_t)p.out_p.pb, a.out_pf = (int32_t)p.out_p.pf * (p.plain_out ? 16 : 1);
+    a.out_f = p.plain_out ? (int32_t)p.out_p.pf : 1;
     a.out_py = (int32_t)p.out_p.py;
     a.el_off = (int32_t)p.eltw_p.off, a.el_pb = (int32_t)p.eltw_p.pb, a.el_pf = (int32_t)p.eltw_p.pf;
     a.el_py = (int32_t)p.eltw_p.py;

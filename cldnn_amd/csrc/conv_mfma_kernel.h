@@ -78,6 +78,7 @@ struct MfmaArgs {
     // split-K kernel: waves per workgroup, K-steps per wave, bounds checks (input without a border)
     int32_t kwaves, kper, checked, dil_y, dil_x;
     FastDiv div_taps;
+    int32_t out_f;          // split-K kernel: bytes between neighbouring features of the output
     const int32_t* origin;  // grouped: byte offset of the first input slice that each span of 64 output features reads
     FastEpi fe;
     Epilogue epi;

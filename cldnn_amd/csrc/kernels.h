@@ -11,6 +11,7 @@ struct ConvProblem {
     int in_dt, w_dt, out_dt, eltw_dt;
     cldnn_hip_tensor in_t, out_t, eltw_t;
     Pitch in_p, out_p, eltw_p;
+    int plain_out;  // one output pixel per image, written as bfyx or yxfb; split-K kernel
     int by_span;  // grouped: IFM counts the features that a span of 64 outputs reads, from an origin of its own
 };
 

@@ -192,6 +192,7 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
         const cldnn_hip_tensor ot = to_hip(n->out);
         switch (p.type) {
         case prim_type::reorder: {
+            if (n->written_by) break;
             node* src = n->deps[0];
             // an image that only this reorder reads need not be copied to the device first
             const bool once = src->p->type == prim_type::input_layout && src->users.size() == 1;
@@ -266,7 +267,7 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
             }
             const void* eltw = nullptr;
             if (p.type == prim_type::fused_conv_eltwise && !p.second_input_in_output) eltw = mem_of(n->deps[1])->read_ptr();
-            hip_check(cldnn_hip_conv_enqueue(n->conv, in, out_of(n), eltw));
+            hip_check(cldnn_hip_conv_enqueue(n->conv, in, out_of(n->writes_for ? n->writes_for : n), eltw));
             break;
         }
         default: break;
@@ -927,6 +928,7 @@ cldnn_network cldnn_allocate_network(cldnn_program program, cldnn_status* status
                 continue;
             }
             if (n->chain_unkept()) continue;  // never written: the next member of the chain takes it in registers
+            if (n->writes_for) continue;  // writes its reader's buffer
             if (n->sibling_head) continue;  // a window into the pair's buffer, made when the pair's first node came up
             if (n->concat_in_place || n->concat_into) {
                 // an in-place concatenation owns one buffer of its own (outside the pool); its inputs, which come earlier

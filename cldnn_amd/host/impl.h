@@ -207,6 +207,10 @@ struct node {
     // two results share one buffer (the second is its contiguous tail: feature slices are the outermost axis).
     node* sibling = nullptr;
     node* sibling_head = nullptr;
+    // a classifier whose only reader changes its layout: `writes_for` (on the convolution) is that reorder, whose tensor the
+    // convolution writes itself; `written_by` (on the reorder) is the convolution.  The convolution has no buffer.
+    node* writes_for = nullptr;
+    node* written_by = nullptr;
     cldnn_padding unpaired_padding{};  // the output padding this node had before it took the wider border of its pair
     // member of a chain whose result stays in registers: it has no buffer and nobody but the next member reads it
     bool chain_unkept() const

@@ -957,3 +957,29 @@ def test_grouped_spans_read_the_features_of_their_groups(eng, shape, border):
     assert info.impl == hip.IMPL_MFMA
     np.testing.assert_array_equal(ga, ra)
     assert_same(ro, go)
+
+
+@pytest.mark.parametrize("shape", [(1, 2048, 1, 1, 1000), (40, 2048, 1, 1, 1000), (3, 100, 1, 1, 12), (2, 512, 7, 7, 4096), (20, 48, 5, 3, 68), (300, 64, 1, 1, 132)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("form", ["relu", "fc", "element"])
+@pytest.mark.parametrize("out_fmt", [hip.BFYX, hip.YXFB], ids=["bfyx", "yxfb"])
+def test_scores_written_in_plain_layouts(eng, shape, form, out_fmt):
+    """one output pixel per image, blocked input, plain output: the split-K kernel writes four features at a time"""
+    B, IFM, H, W, OFM = shape
+    x, w, bias, wqf, calib = problem(71, B, IFM, H, W, OFM, H, W, np.int8)
+    kw = dict(out_dt="s8", act="relu" if form == "relu" else "none")
+    if form == "element":
+        kw.update(act="relu_slope", act_m=0.25)
+    if form == "fc":
+        kw.update(fc=True)
+        bias = (bias.astype(np.float32) * 1e-3).astype(np.float32)
+    ref = rc.conv(x, w, bias, wqf=wqf, calib=calib, **kw)
+    xin = hip.upload(eng, x, "fs_b_yx_fsv16")
+    args = {k: v for k, v in kw.items() if k != "out_dt"}
+    d = hip.conv_desc(xin.tensor, w.shape, "s8", out_fmt=out_fmt, bias_dt=hip.F32 if form == "fc" else hip.I32, has_wqf=True, has_calib=True, **args)
+    c = hip.Conv(eng, d, w, bias, wqf, calib)
+    assert c.info().impl == hip.IMPL_MFMA
+    out = hip.Buffer(eng, d.output)
+    c.enqueue(xin, out)
+    eng.finish()
+    assert_same(ref, hip.download(eng, out))

@@ -257,3 +257,26 @@ def test_api_conv_pool_conv_network(cl_eng, optimize):
     np.testing.assert_array_equal(outs["pool1"].get_memory().read(), p1)
     np.testing.assert_array_equal(outs["pool5"].get_memory().read(), p5)
     assert p5.shape == (2, 96, 1, 1) and p5.any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [np.uint8, np.int8], ids=["u8", "s8"])
+@pytest.mark.parametrize("shape", [
+    (2, 16, 7, 9, "max", (2, 2), (2, 2), (0, 0)), (1, 37, 12, 5, "max", (2, 2), (1, 2), (1, 1)), (2, 50, 8, 11, "max", (3, 3), (2, 1), (2, 1)),
+    (3, 40, 7, 7, "max", (7, 7), (1, 1), (0, 0)), (2, 19, 6, 5, "average", (4, 4), (2, 2), (2, 3)), (2, 33, 6, 5, "average_no_padding", (4, 5), (1, 1), (3, 2)),
+    (1, 64, 16, 16, "average", (16, 16), (1, 1), (0, 0)), (1, 20, 17, 16, "average", (17, 16), (1, 1), (0, 0)), (2, 24, 8, 9, "average_no_padding", (8, 9), (1, 1), (0, 0)),
+    (1, 16, 9, 9, "max", (3, 3), (4, 4), (3, 3))],
+    ids=lambda s: "x".join(str(v) for v in s[:4]) + "_" + s[4] + "_" + "x".join(map(str, s[5])))
+def test_gpu_pooling_windows(eng, shape, dt):
+    """bytes compared in 16-bit lanes and windows shared by sixteen lanes: taps outside the input, partly filled slices,
+    16, 64, 72, 256 and 272 taps, extreme values, windows with no tap inside"""
+    from cldnn_amd import hip
+    B, F, H, W, mode, size, stride, pad = shape
+    r = np.random.default_rng(12)
+    lo, hi = (0, 255) if dt == np.uint8 else (-128, 127)
+    x = r.integers(lo, hi + 1, (B, F, H, W)).astype(dt)
+    x[r.random(x.shape) < 0.2] = lo
+    x[r.random(x.shape) < 0.2] = hi
+    x[0, 0], x[-1, -1] = lo, hi
+    out = hip.pool_forward(eng, x, mode, size, stride, pad, fmt="fs_b_yx_fsv16", in_pad=(1, 2), out_pad=(0, 1))
+    np.testing.assert_array_equal(out, rc.pool(x, mode, size, stride, pad))
