@@ -126,6 +126,7 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
             return "stage 1: a projection of more than 64 features is chained in the forms of a MobileNet block and on small planes only";
         if (block && small && pl.ksteps0 >= 2) {
             pl.coop = 1, pl.nt = 1;
+            pl.img_bytes = pl.sp[0] * DWCOOP_KS_BYTES + pl.units * 4096 + vec * 4;
             pl.waves = pl.ksteps0 <= 8 ? std::max(4, pl.ksteps0) : std::min(8, (pl.ksteps0 + 1) / 2);
             pl.granules = (int)((pl.m_total + 15) / 16);
             pl.lds_bytes = (pl.waves * 4 + 1) * pl.sp[1] * 1024 + vec * 4;
@@ -220,7 +221,7 @@ static void launch_dwcoop(hipStream_t s, const ChainStageIn* st, const ChainPlan
     const ConvProblem& p1 = *st[1].p;
     DwCoopArgs a{};
     a.in = (const int8_t*)in, a.img = (const int8_t*)packed_dev, a.eltw = eltws ? (const int8_t*)eltws[1] : nullptr;
-    a.unit_bytes = pl.sp[0] * 9 * 1024;
+    a.unit_bytes = pl.sp[0] * DWCOOP_KS_BYTES;
     a.vec_bytes = a.unit_bytes + pl.units * 4096;
     a.vec_quads = (pl.img_bytes - a.vec_bytes) / 16;
     a.el_off = (int32_t)p1.eltw_p.off, a.el_pb = (int32_t)p1.eltw_p.pb, a.el_pf = (int32_t)p1.eltw_p.pf;
@@ -308,8 +309,17 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
                         int8_t* packed)
 {
     std::memset(packed, 0, chain_packed_bytes(pl));
-    const size_t dw_bytes = pl.dw ? (size_t)pl.sp[0] * 9 * 1024 : 0;
-    if (pl.dw) {
+    const size_t dw_bytes = pl.dw ? (size_t)pl.sp[0] * (pl.coop ? DWCOOP_KS_BYTES : 9 * 1024) : 0;
+    if (pl.coop) {
+        // byte mt of dword (K-step, lane % 16, tap): feature 64 ks + 16 (l16 / 4) + 4 mt + l16 % 4
+        for (int ks = 0; ks < pl.sp[0]; ++ks)
+            for (int l16 = 0; l16 < 16; ++l16)
+                for (int tap = 0; tap < 9; ++tap)
+                    for (int mt = 0; mt < 4; ++mt) {
+                        const int ch = ks * 64 + 16 * (l16 >> 2) + 4 * mt + (l16 & 3);
+                        if (ch < st[0].p->OFM) packed[((ks * 16 + l16) * 12 + tap) * 4 + mt] = w[0][(size_t)ch * 9 + tap];
+                    }
+    } else if (pl.dw) {
         // diagonal-weight dwords [K-step][tap][fragment][lane]: lane (kq, l16) of fragment mt carries the weight of feature
         // 64 ks + 16 (l16 / 4) + 4 mt + l16 % 4 in byte l16 % 4 when kq == l16 / 4, else zero
         const ConvProblem& p0 = *st[0].p;
@@ -322,7 +332,7 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
                         const int ch = ks * 64 + 16 * (l16 >> 2) + 4 * mt + (l16 & 3);
                         int32_t v = 0;
                         if (kq == (l16 >> 2) && ch < p0.OFM) v = (int32_t)((uint32_t)(uint8_t)w[0][(size_t)ch * 9 + tap] << (8 * (l16 & 3)));
-                        dia[pl.coop ? ((ks * 9 + tap) * 64 + lane) * 4 + mt : ((ks * 9 + tap) * 4 + mt) * 64 + lane] = v;
+                        dia[((ks * 9 + tap) * 4 + mt) * 64 + lane] = v;
                     }
     }
     packed += dw_bytes;

@@ -19,11 +19,16 @@
 // time: 164 registers (64-feature projection) let a CU hold twelve waves, which is worth more than the look-ahead (221
 // registers: 20 us instead of 15 for 28x28 at batch 32).
 //
-// The diagonal-weight table is laid out [K-step][tap][lane][4 fragments] here: one 16-byte load per tap.
+// The depthwise weights are a dword per tap and lane here, the four features of the lane's rows of the diagonal, [K-step][lane
+// % 16][12 taps]; a byte permute moves each into its fragment.  The table of the other kernel has them spread out: 9 KB a
+// K-step instead of 768 bytes, and with a granule or two on the chip what one CU fetches is the time (touching the 1x1
+// weights' lines early, to have them nearer, made 7x7 blocks slower: 12.4 -> 15.4 us).
 #pragma once
 #include "conv_dwchain_kernel.h"
 
 namespace chip {
+
+enum { DWCOOP_KS_BYTES = 16 * 12 * 4 };
 
 struct CoopStage {
     int8_t* out;                          // nullptr: the result stays in registers
@@ -86,9 +91,16 @@ __global__ void __launch_bounds__(512) conv_dwcoop_kernel(DwCoopArgs a)
     if (g_begin >= g_end) return;  // the whole workgroup
 
     // everything is addressed as a uniform pointer and a 32-bit lane offset (a pointer per lane costs two registers a load)
-    const uint32_t lane16 = (uint32_t)lane * 16, row16 = (uint32_t)(kq * 64 + l16) * 16;
+    const uint32_t row16 = (uint32_t)(kq * 64 + l16) * 16;
     auto unit = [&](int u, int mt) { return *reinterpret_cast<const v4i*>(a.img + (size_t)(a.unit_bytes + u * 4096 + mt * 256) + row16); };
-    v4i xb[9], dw[9], u1[SP1 * 4], u2[SP1 * 4];
+    v4i xb[9], dw[3], u1[SP1 * 4], u2[SP1 * 4];
+    // fragment mt of the diagonal: byte mt of a tap's dword moves to byte l16 % 4 in the lanes of the diagonal, zeros elsewhere
+    unsigned sel[4];
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+        const int sh = 8 * (l16 & 3);
+        sel[mt] = kq == (l16 >> 2) ? (0x0c0c0c0cu & ~(0xffu << sh)) | ((unsigned)mt << sh) : 0x0c0c0c0cu;
+    }
     uint32_t boff = 0, b = 0, oy = 0, ox = 0;
     bool ok = false;
     auto locate = [&](int g) {
@@ -113,12 +125,10 @@ __global__ void __launch_bounds__(512) conv_dwcoop_kernel(DwCoopArgs a)
         }
         const int slice = ks * 4 + kq;  // a slice past the end reads slice 0, its diagonal weights are zero
         const uint32_t off = boff + (uint32_t)((slice < a.CB ? slice : 0) * a.in_pf);
-        const int8_t* dia = a.img + (size_t)ks * (9 * 1024);
 #pragma unroll
-        for (int t = 0; t < 9; ++t) {
-            xb[t] = *reinterpret_cast<const v4i*>(a.in + ((t / 3) * a.tap_dy + (t % 3) * 16) + off);
-            dw[t] = *reinterpret_cast<const v4i*>(dia + t * 1024 + lane16);
-        }
+        for (int t = 0; t < 9; ++t) xb[t] = *reinterpret_cast<const v4i*>(a.in + ((t / 3) * a.tap_dy + (t % 3) * 16) + off);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) dw[q] = *reinterpret_cast<const v4i*>(a.img + ((size_t)ks * DWCOOP_KS_BYTES + q * 16) + (uint32_t)(l16 * 48));
     };
     auto request1 = [&](int ks) {
 #pragma unroll
@@ -155,6 +165,17 @@ __global__ void __launch_bounds__(512) conv_dwcoop_kernel(DwCoopArgs a)
     lds_barrier();
 
     for (int g = g_begin; g < g_end; ++g) {
+        int ev_early[SP1];  // the residual of the fragments this wave will finish
+        if constexpr (SUM) {
+#pragma unroll
+            for (int u = 0; u < SP1; ++u) {
+                const int i = wave + u * W, sp = i >> 2, mt = i & 3;
+                ev_early[u] = 0;
+                if (i < SP1 * 4 && sp * 64 + kq * 16 < s1.ofm)
+                    ev_early[u] = *reinterpret_cast<const int*>(a.eltw + (uint32_t)(a.el_off + (int)b * a.el_pb + kq * a.el_pf + (int)oy * a.el_py + (int)ox * a.el_px
+                                                                                     + sp * 4 * a.el_pf + mt * 4));
+            }
+        }
         v4i acc1[SP1 * 4];
 #pragma unroll
         for (int i = 0; i < SP1 * 4; ++i) acc1[i] = v4i{0, 0, 0, 0};
@@ -171,7 +192,7 @@ __global__ void __launch_bounds__(512) conv_dwcoop_kernel(DwCoopArgs a)
 #pragma unroll
                 for (int mt = 0; mt < 4; ++mt) {
                     v4i fa = {0, 0, 0, 0};
-                    fa[mt] = dw[t][mt];
+                    fa[mt] = (int)__builtin_amdgcn_perm(0u, (unsigned)dw[t >> 2][t & 3], sel[mt]);
                     acc0[mt][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa, x, acc0[mt][0], 0, 0, 0);
                 }
                 step_fence();  // a diagonal fragment is four registers: without it all 36 are made at once
@@ -200,15 +221,15 @@ __global__ void __launch_bounds__(512) conv_dwcoop_kernel(DwCoopArgs a)
         lds_barrier();
 
         // ---------------- projection: fragment i = (span, mt) of the sum, four features of a lane
-        for (int i = wave; i < SP1 * 4; i += W) {
+#pragma unroll
+        for (int u = 0; u < SP1; ++u) {  // (at least four waves)
+            const int i = wave + u * W;
+            if (i >= SP1 * 4) break;
             const int sp = i >> 2, mt = i & 3;
             const int fb = sp * 64 + kq * 16, f0 = fb + mt * 4;
             const uint32_t lane_at = (uint32_t)(sp * 4 * s1.pf + mt * 4);
             v4i ev = {0, 0, 0, 0};
-            if constexpr (SUM)
-                if (fb < s1.ofm)
-                    ev[0] = *reinterpret_cast<const int*>(a.eltw + (uint32_t)(a.el_off + (int)b * a.el_pb + kq * a.el_pf + (int)oy * a.el_py + (int)ox * a.el_px
-                                                                              + sp * 4 * a.el_pf + mt * 4));
+            if constexpr (SUM) ev[0] = ev_early[u];
             float cal[16] = {}, ecal[16] = {};
             auto vec4 = [&](int at, float(&dst)[16]) {
                 const v4i q = *reinterpret_cast<const v4i*>(V + at);
