@@ -6,6 +6,7 @@
 #include <string>
 #include <vector>
 
+#include "conv_coop_kernel.h"
 #include "conv_dwcoop_kernel.h"
 
 namespace chip {
@@ -37,12 +38,10 @@ struct Instance {
 #define CHAIN_INSTANCE(NT, D, SP0, SP1, SP2, E0, E1, E2) \
     {NT, D, SP0, SP1, SP2, E0, E1, E2, &launch_chain_instance<NT, D, SP0, SP1, SP2, E0, E1, E2>}
 // What is compiled: the tails of ResNet bottlenecks with 64 mid features (3x3 -> expansion [+ residual] -> next
-// reduction), with and without the third stage, residual fused or not.
+// reduction), residual fused or not.
 const Instance g_instances[] = {
     CHAIN_INSTANCE(2, 3, 1, 4, 1, EPI_KIND_RELU, EPI_KIND_FUSED, EPI_KIND_RELU),
-    CHAIN_INSTANCE(2, 3, 1, 4, 0, EPI_KIND_RELU, EPI_KIND_FUSED, EPI_KIND_RELU),
     CHAIN_INSTANCE(2, 3, 1, 4, 1, EPI_KIND_RELU, EPI_KIND_RELU, EPI_KIND_RELU),
-    CHAIN_INSTANCE(2, 3, 1, 4, 0, EPI_KIND_RELU, EPI_KIND_RELU, EPI_KIND_RELU),
 };
 
 const Instance* find_instance(const ChainPlan& pl)
@@ -176,6 +175,23 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
             pl.vec0[k] = vec;
             vec += 4 * pl.sp[k] * 64;
         }
+        // The weights in the registers of eight waves that share a granule: chains of two stages, and of three up to two
+        // granules per CU (with more, one granule per wave needs fewer instructions a pixel; conv_coop_kernel.h).
+        const bool block = p0.FY == 3 && p0.FX == 3 && pl.sp[0] == 1 && p0.IFM == 64 && pl.sp[1] == 4 && (n < 3 || pl.sp[2] == 1)
+                           && pl.epi[0] == EPI_KIND_RELU && (pl.epi[1] == EPI_KIND_RELU || pl.epi[1] == EPI_KIND_FUSED)
+                           && (n < 3 || pl.epi[2] == EPI_KIND_RELU);
+        const int granules = (int)((pl.m_total + 15) / 16);
+        if (block && (n == 2 || granules <= 2 * cus)) {
+            pl.coop = 1, pl.nt = 1, pl.waves = 8;
+            pl.granules = granules;
+            pl.img_bytes = pl.units * 4096 + vec * 4;
+            pl.lds_bytes = (n > 2 ? 2 : 1) * 32 * 1024 + 1024 + vec * 4;
+            pl.grid = std::min(cus * 2 / 8 * 8, (granules + 7) / 8 * 8);
+            std::snprintf(pl.name, sizeof(pl.name), "conv_chain<%d stages,p16 shared by 8 waves,spans %d-%d-%d,epi %d-%d-%d>", n, pl.sp[0], pl.sp[1], n > 2 ? pl.sp[2] : 0,
+                          pl.epi[0], pl.epi[1], n > 2 ? pl.epi[2] : -1);
+            *out = pl;
+            return std::string();
+        }
         pl.depth = mp[0].wsl_depth, pl.ksteps0 = mp[0].ksteps;
         pl.lds_bytes = pl.img_bytes = pl.units * 4096 + vec * 4;
         if (mp[0].wsl_depth > 0 && pl.lds_bytes <= CHAIN_MAX_LDS && find_instance(pl)) {
@@ -262,6 +278,43 @@ static void launch_dwcoop(hipStream_t s, const ChainStageIn* st, const ChainPlan
     CHIP_CHECK(hipGetLastError());
 }
 
+static void launch_coop(hipStream_t s, const ChainStageIn* st, const ChainPlan& pl, const void* packed_dev, const void* in,
+                        void* const* outs, const void* const* eltws)
+{
+    const ConvProblem& p0 = *st[0].p;
+    const ConvProblem& p1 = *st[1].p;
+    CoopConvArgs a{};
+    a.in = (const int8_t*)in, a.img = (const int8_t*)packed_dev, a.eltw = eltws ? (const int8_t*)eltws[1] : nullptr;
+    a.vec_bytes = pl.units * 4096;
+    a.vec_quads = (pl.img_bytes - a.vec_bytes) / 16;
+    a.el_off = (int32_t)p1.eltw_p.off, a.el_pb = (int32_t)p1.eltw_p.pb, a.el_pf = (int32_t)p1.eltw_p.pf;
+    a.el_py = (int32_t)p1.eltw_p.py * p1.esy, a.el_px = 16 * p1.esx;
+    a.M = (uint32_t)pl.m_total;
+    a.OHW = p0.OH * p0.OW, a.OW = p0.OW;
+    a.div_ohw = make_fast_div((uint32_t)a.OHW), a.div_ow = make_fast_div((uint32_t)a.OW);
+    a.in_off = (int32_t)p0.in_p.off - p0.py * (int32_t)p0.in_p.py - p0.px * 16;
+    a.in_pb = (int32_t)p0.in_p.pb, a.in_pf = (int32_t)p0.in_p.pf;
+    a.row = p0.sy * (int32_t)p0.in_p.py, a.col = p0.sx * 16, a.tap_dy = (int32_t)p0.in_p.py;
+    a.gpw = pl.granules / pl.grid, a.grem = pl.granules % pl.grid;
+    a.div_parts = make_fast_div((uint32_t)pl.grid);
+    const bool sum = pl.epi[1] == EPI_KIND_FUSED;
+    CHIP_REQUIRE(!sum || a.eltw, CLDNN_HIP_INVALID_ARG, "fused stage of a chain without its second input");
+    for (int k = 0; k < pl.stages; ++k) {
+        const ConvProblem& p = *st[k].p;
+        CoopConvStage& c = a.st[k];
+        c.out = (int8_t*)outs[k];
+        c.off = (int32_t)p.out_p.off, c.pb = (int32_t)p.out_p.pb, c.pf = (int32_t)p.out_p.pf, c.py = (int32_t)p.out_p.py;
+        c.xor_mask = p.in_dt == CLDNN_HIP_U8 ? 0x80808080u : 0u;
+        c.unit0 = pl.unit0[k], c.kstride = pl.kstride[k], c.vec0 = pl.vec0[k];
+        c.hi = st[k].fe->hi, c.eltw_u8 = st[k].fe->eltw_u8;
+    }
+    if (pl.stages > 2 && sum) launch_coop_instance<true, true>(s, a, pl.grid, pl.lds_bytes);
+    else if (pl.stages > 2) launch_coop_instance<true, false>(s, a, pl.grid, pl.lds_bytes);
+    else if (sum) launch_coop_instance<false, true>(s, a, pl.grid, pl.lds_bytes);
+    else launch_coop_instance<false, false>(s, a, pl.grid, pl.lds_bytes);
+    CHIP_CHECK(hipGetLastError());
+}
+
 static void launch_dwchain(hipStream_t s, const ChainStageIn* st, const ChainPlan& pl, const void* packed_dev, const void* in,
                            void* const* outs, const void* const* eltws)
 {
@@ -310,7 +363,7 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
 {
     std::memset(packed, 0, chain_packed_bytes(pl));
     const size_t dw_bytes = pl.dw ? (size_t)pl.sp[0] * (pl.coop ? DWCOOP_KS_BYTES : 9 * 1024) : 0;
-    if (pl.coop) {
+    if (pl.coop && pl.dw) {
         // byte mt of dword (K-step, lane % 16, tap): feature 64 ks + 16 (l16 / 4) + 4 mt + l16 % 4
         for (int ks = 0; ks < pl.sp[0]; ++ks)
             for (int l16 = 0; l16 < 16; ++l16)
@@ -365,6 +418,7 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
 void launch_conv_chain(hipStream_t s, const ChainStageIn* st, const ChainPlan& pl, const void* packed_dev, const void* in,
                        void* const* outs, const void* const* eltws)
 {
+    if (pl.coop && !pl.dw) return launch_coop(s, st, pl, packed_dev, in, outs, eltws);
     if (pl.coop) return launch_dwcoop(s, st, pl, packed_dev, in, outs, eltws);
     if (pl.dw) return launch_dwchain(s, st, pl, packed_dev, in, outs, eltws);
     const ConvProblem& p0 = *st[0].p;

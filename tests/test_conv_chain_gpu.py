@@ -344,3 +344,26 @@ def test_depthwise_chain_on_small_planes(eng, mid, proj, stride, stages, hw, in_
         ch.close()
     for b in bufs + [xin, ebuf]:
         b.close()
+
+
+@pytest.mark.parametrize("hw", [(1, 1), (17, 15), (46, 41)], ids=["one_pixel", "ragged", "several_granules"])
+@pytest.mark.parametrize("in_dt", [np.uint8, np.int8], ids=["u8", "s8"])
+@pytest.mark.parametrize("stages,fused", [(3, True), (2, True), (3, False), (2, False)], ids=["3fused", "2fused", "3plain", "2plain"])
+def test_bottleneck_chain_with_weights_in_registers(eng, hw, in_dt, stages, fused):
+    """eight waves to a granule: a last granule that is not full, workgroups with several granules, every result kept"""
+    mid, B = 64, 3 if hw[0] < 40 or stages == 3 else 8
+    for keep in ([False] + [True] * (stages - 1), [True] * stages):
+        xin, spec, bufs, refs = bottleneck_tail(eng, 21, B, hw[0], hw[1], mid, stages, fused, in_dt, out_pad=(1, 1))
+        ch = hip.ConvChain(eng, spec, keep)
+        assert b"shared by 8 waves" in ch.info().kernel_name
+        ch.enqueue(xin, [b if keep[k] else None for k, (b, _) in enumerate(bufs)], [e for _, e in bufs])
+        eng.finish()
+        for k in range(stages):
+            if keep[k]:
+                bad = np.argwhere(hip.download(eng, bufs[k][0]) != refs[k])
+                assert bad.size == 0, "stage %d: %d differ, first at %s" % (k, len(bad), bad[0])
+        ch.close(), xin.close()
+        for b, e in bufs:
+            b.close()
+            if e is not None:
+                e.close()
