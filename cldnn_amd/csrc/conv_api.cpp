@@ -716,6 +716,24 @@ cldnn_hip_status cldnn_hip_conv_accumulators(cldnn_hip_conv c, const void* input
     });
 }
 
+cldnn_hip_status cldnn_hip_conv_pool_output(cldnn_hip_conv c, const cldnn_hip_pooling_desc* d)
+{
+    return guarded([&] {
+        CHIP_REQUIRE(c && d, CLDNN_HIP_INVALID_ARG, "null argument");
+        ConvProblem& p = c->p;
+        const cldnn_hip_tensor &i = d->input, &o = d->output;
+        CHIP_REQUIRE(i.b == p.B && i.f == p.OFM && i.y == p.OH && i.x == p.OW && i.dtype == p.out_dt && o.b == p.B && o.f == p.OFM && o.dtype == p.out_dt,
+                     CLDNN_HIP_DIMENSION_MISMATCH, "the pooling does not read this convolution's result");
+        const bool halves = d->mode == CLDNN_HIP_POOL_MAX && d->size_y == 2 && d->size_x == 2 && d->stride_y == 2 && d->stride_x == 2 && d->pad_y == 0
+                            && d->pad_x == 0 && o.y * 2 == p.OH && o.x * 2 == p.OW && o.format == CLDNN_HIP_FMT_FS_B_YX_FSV16;
+        CHIP_REQUIRE(halves && !p.pooled && c->impl == CLDNN_HIP_IMPL_MFMA && c->fast && mfma_can_pool(p, c->mplan, c->fe, c->epi)
+                         && tensor_elems(o) < (1ull << 31),
+                     CLDNN_HIP_UNSUPPORTED_FORMAT, "this convolution cannot pool its own result");
+        c->info.bytes -= (int64_t)p.B * p.OFM * p.OH * p.OW / 4 * 3;
+        p.pooled = 1, p.out_t = o, p.out_p = make_pitch(o);
+    });
+}
+
 cldnn_hip_status cldnn_hip_conv_get_info(cldnn_hip_conv c, cldnn_hip_conv_info* info)
 {
     return guarded([&] {

@@ -75,8 +75,8 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
     const int origin = a.in_off + span_origin(a, span);
 #pragma unroll
     for (int pt = 0; pt < PT; ++pt) {
-        const uint32_t m = (uint32_t)(ptile * PT + pt) * 16 + l16;
-        const PixelPos pp = pixel_pos(a, m < a.M ? m : 0);  // pixels past the end read pixel 0
+        bool ok;
+        const PixelPos pp = pixel_at<EPI, PT>(a, (uint32_t)ptile * PT * 16, pt, l16, ok);  // pixels past the end read pixel 0
         iy0[pt] = (int)pp.oy * a.sy - a.py, ix0[pt] = (int)pp.ox * a.sx - a.px;
         boff[pt] = (uint32_t)(origin + (int)pp.b * a.in_pb + iy0[pt] * a.in_py + ix0[pt] * 16 + (ADDR == ADDR_UNIFORM ? kq * a.in_pf : 0));
     }
@@ -192,11 +192,13 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
         for (int f = 0; f < FT; ++f) part[wave * TILE + (p * FT + f) * 64 + lane] = acc[f][p];
 
     const int ff = wave % FT, fp = wave / FT;
-    const uint32_t m = (uint32_t)(ptile * PT + fp) * 16 + l16;
     const int fb = span * 64 + kq * 16, f0 = fb + (q0 + ff) * 4;
-    const bool finisher = wave < FT * PT;
-    const bool live = finisher && m < a.M && f0 < a.OFM;
-    const PixelPos pp = pixel_pos(a, live ? m : 0);
+    constexpr bool PAIR = EPI == EPI_KIND_POOL && PT > 1;  // fragments 2k and 2k + 1 are two rows of the same windows
+    const bool finisher = wave < FT * PT && !(PAIR && (fp & 1));
+    bool inside;
+    PixelPos pp = pixel_at<EPI, PT>(a, (uint32_t)ptile * PT * 16, finisher ? fp : 0, l16, inside);
+    const bool live = finisher && inside && f0 < a.OFM;
+    if constexpr (EPI == EPI_KIND_POOL) pp.oy >>= 1, pp.ox >>= 1;
     const int obase = a.out_off + (int)pp.b * a.out_pb + (fb >> 4) * a.out_pf + (int)pp.oy * a.out_py + (int)pp.ox * 16 + (f0 & 15) * a.out_f;
     const int ebase = a.el_off + (int)pp.b * a.el_pb + (fb >> 4) * a.el_pf + (int)(pp.oy * a.esy) * a.el_py + (int)(pp.ox * a.esx) * 16 + (f0 & 15);
     // what the epilogue reads, requested in front of the barrier
@@ -209,7 +211,7 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
     }
     if (live) {
         init = *reinterpret_cast<const v4i*>(a.acc_init + f0);
-        load_scales4<EPI>(a, f0, sc);
+        load_scales4<EPI == EPI_KIND_POOL ? EPI_KIND_RELU : EPI>(a, f0, sc);
         bool residual = EPI == EPI_KIND_FUSED;
         if constexpr (EPI == EPI_KIND_FAST) residual = a.fe.fused != 0;
         if (residual) ev4[0] = *reinterpret_cast<const int*>((const int8_t*)a.eltw + ebase);
@@ -223,6 +225,20 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
         sum[0] += o[0], sum[1] += o[1], sum[2] += o[2], sum[3] += o[3];
     }
     const int valid = a.OFM - f0;
+    if constexpr (PAIR) {
+        v4i low = init;
+        for (int w = 0; w < a.kwaves; ++w) {
+            const v4i o = src[w * TILE + FT * 64];
+            low[0] += o[0], low[1] += o[1], low[2] += o[2], low[3] += o[3];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[i] = max_dpp<0xb1>(max(sum[i], low[i]));
+        if (l16 & 1) return;  // the first of the window's lanes stores its four features
+    } else if constexpr (EPI == EPI_KIND_POOL) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[i] = max_of_window(sum[i]);
+        if (l16 & 3) return;
+    }
     if constexpr (EPI == EPI_KIND_GENERIC) {
         const Epilogue& e = a.epi;
 #pragma unroll
@@ -246,7 +262,7 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
             for (int i = 0; i < valid; ++i) dst[i] = v[i];
     } else {
         v4i acc4[4][1] = {{sum}, {v4i{0, 0, 0, 0}}, {v4i{0, 0, 0, 0}}, {v4i{0, 0, 0, 0}}};
-        const v4i packed = epilogue_fast16<1, EPI>(a, acc4, 0, sc.wq, sc.cal, sc.ecal, ev4, valid);
+        const v4i packed = epilogue_fast16<1, EPI == EPI_KIND_POOL ? EPI_KIND_RELU : EPI>(a, acc4, 0, sc.wq, sc.cal, sc.ecal, ev4, valid);
         int8_t* dst = (int8_t*)a.out + obase;
         if (a.out_f == 1) *reinterpret_cast<int*>(dst) = packed[0];
         else  // images innermost: the lanes next to this one write the bytes beside these
@@ -266,6 +282,7 @@ void launch_ksplit_instance(hipStream_t s, const MfmaArgs& a, int grid, int epi)
     case EPI_KIND_LINEAR: hipLaunchKernelGGL((conv_ksplit_kernel<FT, PT, ADDR, EPI_KIND_LINEAR>), g, b, lds, s, a); break;
     case EPI_KIND_FAST: hipLaunchKernelGGL((conv_ksplit_kernel<FT, PT, ADDR, EPI_KIND_FAST>), g, b, lds, s, a); break;
     case EPI_KIND_F32: hipLaunchKernelGGL((conv_ksplit_kernel<FT, PT, ADDR, EPI_KIND_F32>), g, b, lds, s, a); break;
+    case EPI_KIND_POOL: hipLaunchKernelGGL((conv_ksplit_kernel<FT, PT, ADDR, EPI_KIND_POOL>), g, b, lds, s, a); break;
     default: hipLaunchKernelGGL((conv_ksplit_kernel<FT, PT, ADDR, EPI_KIND_GENERIC>), g, b, lds, s, a); break;
     }
 }

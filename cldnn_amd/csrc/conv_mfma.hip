@@ -653,6 +653,12 @@ bool mfma_fast_epilogue(const ConvProblem& p, const Epilogue& e, const float* ca
     return true;
 }
 
+bool mfma_can_pool(const ConvProblem& p, const MfmaPlan& pl, const FastEpi& f, const Epilogue& e)
+{
+    const bool relu = !f.has_wqf && e.calib && !f.fc && !f.fused && !f.f32 && f.relu_folded;
+    return relu && (pl.bdir || pl.direct || pl.wsl || (pl.ksplit && !pl.gemv)) && p.OH % 2 == 0 && p.OW % 2 == 0 && !p.plain_out;
+}
+
 // a filter of one tap puts the 16 pixels' bytes of a K-step side by side already
 size_t mfma_gather_bytes(const ConvProblem& p, const MfmaPlan& pl)
 {
@@ -725,6 +731,12 @@ void launch_conv_mfma(hipStream_t s, const ConvProblem& p, const MfmaPlan& pl, c
             if (fast->fused && fast->act == CLDNN_HIP_ACT_NONE && fast->eltw_relu_folded && epi.eltw_calib && !fast->conv_sat)
                 kind = EPI_KIND_FUSED;
         }
+    }
+    if (p.pooled && !raw) {
+        kind = EPI_KIND_POOL;
+        if ((pl.ksplit ? pl.ks_pt : tc.wave_pixels / 16) > 1) a.OHW /= 2;  // columns of row pairs, or windows (see pixel_at)
+        else a.OHW /= 4, a.OW /= 2;
+        a.div_ohw = make_div((uint32_t)a.OHW), a.div_ow = make_div((uint32_t)a.OW);
     }
     a.bpk = (const v4i*)wb.gather;
     a.origin = wb.origin;

@@ -11,6 +11,7 @@ struct ConvProblem {
     int in_dt, w_dt, out_dt, eltw_dt;
     cldnn_hip_tensor in_t, out_t, eltw_t;
     Pitch in_p, out_p, eltw_p;
+    int pooled;     // the output tensor holds the maxima over 2x2 windows of the OH x OW result
     int plain_out;  // one output pixel per image, written as bfyx or yxfb; split-K kernel
     int by_span;  // grouped: IFM counts the features that a span of 64 outputs reads, from an origin of its own
 };
@@ -129,6 +130,9 @@ bool mfma_fast_epilogue(const ConvProblem& p, const Epilogue& e, const float* ca
 void launch_conv_mfma(hipStream_t s, const ConvProblem& p, const MfmaPlan& plan, const MfmaBuffers& wb,
                       const int32_t* acc_init, const Epilogue& epi, const FastEpi* fast, const void* in, const void* eltw,
                       void* out, int32_t* raw);
+
+// can the plan's kernel pool its result (2x2 windows) as it writes it?
+bool mfma_can_pool(const ConvProblem& p, const MfmaPlan& pl, const FastEpi& fast, const Epilogue& epi);
 
 // ---- depthwise bandwidth kernel on fs_b_yx_fsv16 (conv_dw.hip)
 struct DwPlan {

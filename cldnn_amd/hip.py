@@ -180,6 +180,7 @@ SIGNATURES = {
     "cldnn_hip_conv_chain_get_info": (C.c_int32, [C.c_void_p, C.POINTER(ConvInfo)]),
     "cldnn_hip_conv_accumulators": (C.c_int32, [C.c_void_p, C.c_void_p, C.c_void_p]),
     "cldnn_hip_conv_get_info": (C.c_int32, [C.c_void_p, C.POINTER(ConvInfo)]),
+    "cldnn_hip_conv_pool_output": (C.c_int32, [C.c_void_p, C.POINTER(PoolingDesc)]),
     "cldnn_hip_conv_out_extent": (C.c_int32, [C.c_int32] * 5),
     "cldnn_hip_pooling": (C.c_int32, [C.c_void_p, C.POINTER(PoolingDesc), C.c_void_p, C.c_void_p]),
     "cldnn_hip_pooling_out_extent": (C.c_int32, [C.c_int32] * 4),

@@ -213,6 +213,7 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
             break;
         }
         case prim_type::pooling: {
+            if (n->written_by) break;
             cldnn_hip_pooling_desc pd = pooling_descriptor(n);
             hip_check(cldnn_hip_pooling(eng->h, &pd, mem_of(n->deps[0])->read_ptr(), out_of(n)));
             break;

@@ -207,8 +207,9 @@ struct node {
     // two results share one buffer (the second is its contiguous tail: feature slices are the outermost axis).
     node* sibling = nullptr;
     node* sibling_head = nullptr;
-    // a classifier whose only reader changes its layout: `writes_for` (on the convolution) is that reorder, whose tensor the
-    // convolution writes itself; `written_by` (on the reorder) is the convolution.  The convolution has no buffer.
+    // a convolution that does its only reader's work as it writes (the change of a classifier's layout, a 2x2 max pooling):
+    // `writes_for` (on the convolution) is that reader, whose tensor it writes; `written_by` (on the reader) is the
+    // convolution.  The convolution has no buffer.
     node* writes_for = nullptr;
     node* written_by = nullptr;
     cldnn_padding unpaired_padding{};  // the output padding this node had before it took the wider border of its pair

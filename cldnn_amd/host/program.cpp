@@ -983,6 +983,12 @@ static node* plain_reader(const cldnn_program_impl* prog, const node* n)
     return n->out.size.sizes[2] == 1 && n->out.size.sizes[3] == 1 ? r : nullptr;
 }
 
+static bool only_pooled(const node* n)
+{
+    return n->p->type == prim_type::convolution && !n->is_output && !n->side_stream && !n->concat_into && n->users.size() == 1
+           && n->users[0]->p->type == prim_type::pooling && !n->users[0]->concat_into;
+}
+
 static void compile_conv(cldnn_program_impl* prog, node* n)
 {
     conv_build cb;
@@ -1010,6 +1016,11 @@ static void compile_conv(cldnn_program_impl* prog, node* n)
     apply_tuning(prog, d, wv.data(), bias_ptr, wqf_ptr, calib_ptr, (const float*)eltw_calib);
     hip_check(cldnn_hip_conv_create(n->side_stream ? prog->engine->side : prog->engine->h, &d, wv.data(), bias_ptr, wqf_ptr, calib_ptr,
                                     (const float*)eltw_calib, &n->conv));
+    // a max pooling behind it that nobody else reads past
+    if (prog->optimize_data && only_pooled(n)) {
+        const cldnn_hip_pooling_desc pd = pooling_descriptor(n->users[0]);
+        if (cldnn_hip_conv_pool_output(n->conv, &pd) == CLDNN_HIP_SUCCESS) n->writes_for = n->users[0], n->users[0]->written_by = n;
+    }
     hip_check(cldnn_hip_conv_get_info(n->conv, &n->conv_info));
 }
 

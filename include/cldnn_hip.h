@@ -363,6 +363,10 @@ typedef struct {
     char kernel_name[96];
 } cldnn_hip_conv_info;
 cldnn_hip_status cldnn_hip_conv_get_info(cldnn_hip_conv c, cldnn_hip_conv_info* info);
+/* From now on the convolution writes what the pooling `d` (which reads its result) would: the launch and the tensor in
+ * between are saved.  Maximum over 2x2 windows at stride 2 without padding, even sizes, a relu convolution on a kernel that
+ * can do it; CLDNN_HIP_UNSUPPORTED_FORMAT otherwise, and the convolution stays as it was. */
+cldnn_hip_status cldnn_hip_conv_pool_output(cldnn_hip_conv c, const cldnn_hip_pooling_desc* d);
 
 /* ------------------------------------------------------------------ convolution chain
  * Two or three convolution / fused_conv_eltwise nodes of which every one after the first is a 1x1 / stride-1 /

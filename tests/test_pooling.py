@@ -280,3 +280,41 @@ def test_gpu_pooling_windows(eng, shape, dt):
     x[0, 0], x[-1, -1] = lo, hi
     out = hip.pool_forward(eng, x, mode, size, stride, pad, fmt="fs_b_yx_fsv16", in_pad=(1, 2), out_pad=(0, 1))
     np.testing.assert_array_equal(out, rc.pool(x, mode, size, stride, pad))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,row", [((1, 512, 14, 14, 64, 3), "ksplit"), ((2, 64, 34, 30, 70, 3), None), ((8, 128, 56, 56, 128, 3), "bdir"), ((9, 256, 56, 56, 264, 1), None),
+                                       ((4, 64, 112, 114, 64, 3), None), ((12, 100, 42, 40, 130, 3), "direct"), ((24, 256, 42, 40, 256, 3), None),
+                                       ((16, 512, 14, 14, 512, 3), "bdir_k2")], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+@pytest.mark.parametrize("out_dt", ["s8", "u8"])
+def test_convolution_that_pools_its_own_result(eng, shape, row, out_dt):
+    """relu convolution and the 2x2 max pooling behind it in one launch, on every kernel family that does it"""
+    import ctypes as C
+    from cldnn_amd import hip
+    B, IFM, H, W, OFM, F = shape
+    r = np.random.default_rng(31)
+    x = r.integers(0, 256, (B, IFM, H, W)).astype(np.uint8)
+    w = r.integers(-127, 128, (OFM, IFM, F, F)).astype(np.int8)
+    bias = r.integers(-1000, 1001, OFM).astype(np.int32)
+    calib = (60.0 / (np.sqrt(IFM * F * F) * 147.4 * 73.3) * r.uniform(0.5, 2.0, OFM)).astype(np.float32)
+    pad = (F // 2, F // 2)
+    xin = hip.upload(eng, x, "fs_b_yx_fsv16", pad)
+    d = hip.conv_desc(xin.tensor, w.shape, out_dt, pad=pad, bias_dt=hip.I32, has_wqf=True, has_calib=True, act="relu")
+    c = hip.Conv(eng, d, w, bias, np.ones(OFM, np.float32), calib)
+    if row:
+        assert row in c.info().kernel_name.decode(), c.info().kernel_name
+    pd = hip.PoolingDesc()
+    pd.input = d.output
+    pd.output = hip.Tensor.make(d.output.dtype, d.output.format, B, OFM, H // 2, W // 2, 1, 1)
+    pd.mode, pd.size_y, pd.size_x, pd.stride_y, pd.stride_x = hip.POOL_MAX, 2, 2, 2, 2
+    assert hip.lib().cldnn_hip_conv_pool_output(c.h, C.byref(pd)) == 0
+    out = hip.Buffer(eng, pd.output)
+    c.enqueue(xin, out)
+    eng.finish()
+    images = [0, B - 1]
+    ref = rc.pool(rc.conv(x[images], w, bias, wqf=np.ones(OFM, np.float32), calib=calib, pad=pad, out_dt=out_dt, act="relu"), "max", (2, 2), (2, 2), (0, 0))
+    np.testing.assert_array_equal(hip.download(eng, out)[images], ref)
+    assert hip.lib().cldnn_hip_conv_pool_output(c.h, C.byref(pd)) == -6  # once
+    pd.size_y = 3
+    plain = hip.Conv(eng, d, w, bias, np.ones(OFM, np.float32), calib)
+    assert hip.lib().cldnn_hip_conv_pool_output(plain.h, C.byref(pd)) == -6  # other windows: unchanged
