@@ -20,8 +20,7 @@ struct ChainStageIn {
 
 struct ChainPlan {
     int stages;
-    int dw;                    // 1: the first stage is a depthwise 3x3 on the vector ALU (granules of 64 pixels), the LDS
-                               // image holds the units and vectors of the later stages only
+    int dw;                    // 1: the first stage is a depthwise 3x3
     int coop;                  // 1: its form for small planes, a workgroup's waves share a granule (conv_dwcoop_kernel.h)
     int waves;                 // waves per workgroup
     int nt;                    // 16-pixel fragments per wave and granule
@@ -29,6 +28,7 @@ struct ChainPlan {
     int ksteps0;               // K-steps of stage 0 (padded to a multiple of depth)
     int sp[3];                 // 64-feature spans per stage
     int epi[3];                // epilogue kind per stage
+    int u32[3];                // units of 32 features per stage (depthwise form with one granule per wave)
     int unit0[3], kstride[3];  // LDS image: first 4 KB unit and units per span of every stage
     int vec0[3];               // first dword of every stage's per-feature vectors behind the weights
     int units;

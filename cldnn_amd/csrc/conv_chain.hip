@@ -87,15 +87,13 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
     if (p0.dy != 1 || p0.dx != 1) return "stage 0: dilation";
     pl.m_total = (int64_t)p0.B * p0.OH * p0.OW;
     if (st[0].dw_wmask) {
-        // ---- depthwise first stage: lane = pixel on the vector ALU, 64-pixel granules, later stages resident in LDS
+        // ---- depthwise first stage: granules of 16 pixels
         if (p0.FY != 3 || p0.FX != 3) return "stage 0: the depthwise stage of a chain is 3x3";
         if (st[0].fe->fused) return "stage 0: a fused depthwise stage is not chained";
         if (pl.sp[1] > 3) return "stage 1: the projection behind a depthwise stage has at most 192 features";
         pl.dw = 1;
-        // 32-pixel granules; 16-pixel ones where that still leaves waves without work (14x14 and 7x7 planes)
-        pl.waves = 4;
-        pl.nt = pl.m_total / 32 >= (int64_t)cus * 8 ? 2 : 1;
-        pl.granules = (int)((pl.m_total + 16 * pl.nt - 1) / (16 * pl.nt));
+        pl.waves = 4, pl.nt = 1;
+        pl.granules = (int)((pl.m_total + 15) / 16);
         pl.units = 0;
         int vec = 0;
         for (int k = 0; k < n; ++k) {
@@ -113,14 +111,13 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
             vec += 4 * pl.sp[k] * 64;
         }
         pl.ksteps0 = pl.sp[0];  // K-steps the depthwise stage delivers to stage 1
-        pl.img_bytes = pl.sp[0] * 9 * 1024 + pl.units * 4096 + vec * 4;  // diagonal-weight table, units, vectors
-        pl.lds_bytes = pl.img_bytes;
-        // Small planes: the waves of a workgroup share a granule.  Up to three granules per CU that beats one granule per
-        // wave with the weights in LDS (14x14 at batch 32; 28x28 at batch 32, with six per CU, reads the weights from L2 too
-        // often: 15.3 us against 12.4), from two K-steps on (a single one occupies one wave of four).
+        // Small planes: the waves of a workgroup share a granule.  Up to two granules per CU that beats one granule per wave with
+        // the weights in LDS (14x14, 384 mid features: 6.5 us against 14.9 at batch 16, 11.2 against 14.9 at batch 32, but 20
+        // against 17 at batch 64) and separate launches where that form does not apply, from two K-steps on (a single one
+        // occupies one wave of four).
         const bool block = pl.epi[0] == EPI_KIND_CLAMPQ && (pl.epi[1] == EPI_KIND_LINEAR || pl.epi[1] == EPI_KIND_SUMLIN)
                            && (n < 3 || pl.epi[2] == EPI_KIND_CLAMPQ) && !st[1].fe->split_valid;
-        const bool small = (pl.m_total + 15) / 16 <= 3ll * cus;
+        const bool small = (pl.m_total + 15) / 16 <= 2ll * cus;
         if (pl.sp[1] > 1 && !(block && small))
             return "stage 1: a projection of more than 64 features is chained in the forms of a MobileNet block and on small planes only";
         if (block && small && pl.ksteps0 >= 2) {
@@ -136,10 +133,14 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
             *out = pl;
             return std::string();
         }
+        // units of 32 features (conv_dwchain_kernel.h)
+        for (int k = 0; k < n; ++k) pl.u32[k] = (st[k].p->OFM + 31) / 32;
+        pl.units = pl.u32[0] + 2 * ((pl.u32[0] + 1) / 2 * pl.u32[1] + (n > 2 ? pl.u32[2] : 0));  // kilobytes of weights
+        pl.lds_bytes = pl.img_bytes = pl.units * 1024 + vec * 4;
         if (pl.lds_bytes > CHAIN_MAX_LDS) return "the weights of the chain (" + std::to_string(pl.lds_bytes / 1024) + " KiB) do not fit into LDS";
-        // workgroups a CU holds at once: by LDS, and by registers (16-pixel granules: 137-167 registers = three waves per
-        // SIMD; 32-pixel granules: 206-239 = two).  The grid is what is resident, so that no workgroup waits for a slot.
-        const int per_cu = std::min(pl.nt == 1 ? 3 : 2, CHAIN_MAX_LDS / pl.lds_bytes);
+        // workgroups a CU holds at once: by LDS, and by registers (128 with a projection of 32 features, 142 with 64, 256 in
+        // the run-time form).  The grid is what is resident, so that no workgroup waits for a slot.
+        const int per_cu = std::min(!block ? 2 : (pl.u32[1] == 1 ? 4 : 3), CHAIN_MAX_LDS / pl.lds_bytes);
         int grid = cus * per_cu / 8 * 8;
         const int wanted = ((pl.granules + 3) / 4 + 7) / 8 * 8;  // at least one granule per wave
         if (grid > wanted) grid = wanted;
@@ -322,38 +323,43 @@ static void launch_dwchain(hipStream_t s, const ChainStageIn* st, const ChainPla
     DwChainArgs a{};
     a.in = (const int8_t*)in;
     a.img = (const v4i*)packed_dev;
-    a.dw_quads = pl.sp[0] * 9 * 64;
-    a.units = pl.units;
-    a.vec_quads = (pl.img_bytes - a.dw_quads * 16 - pl.units * 4096) / 16;
-    a.granules = pl.granules;
+    a.quads = pl.img_bytes / 16;
+    a.U0 = pl.u32[0], a.KS = (a.U0 + 1) / 2, a.U2 = pl.stages > 2 ? pl.u32[2] : 0;
+    a.w1 = a.U0 * 64, a.w2 = a.w1 + a.KS * pl.u32[1] * 128, a.vec = a.w2 + a.U2 * 128;
+    a.n0 = pl.sp[0] * 64, a.n1 = pl.sp[1] * 64, a.n2 = pl.stages > 2 ? pl.sp[2] * 64 : 0;
     a.gpw = pl.granules / (pl.grid * 4), a.grem = pl.granules % (pl.grid * 4);
     a.div_waves = make_fast_div((uint32_t)pl.grid * 4u);
     a.M = (uint32_t)pl.m_total;
     a.OHW = p0.OH * p0.OW, a.OW = p0.OW;
     a.div_ohw = make_fast_div((uint32_t)a.OHW), a.div_ow = make_fast_div((uint32_t)a.OW);
-    a.sy = p0.sy, a.sx = p0.sx, a.py = p0.py, a.px = p0.px;
-    a.in_off = (int32_t)p0.in_p.off, a.in_pb = (int32_t)p0.in_p.pb, a.in_pf = (int32_t)p0.in_p.pf, a.in_py = (int32_t)p0.in_p.py;
-    a.tap_dy = p0.dy * (int32_t)p0.in_p.py, a.tap_dx = p0.dx * 16;
+    a.in_off = (int32_t)p0.in_p.off - p0.py * (int32_t)p0.in_p.py - p0.px * 16;
+    a.in_pb = (int32_t)p0.in_p.pb, a.in_pf = (int32_t)p0.in_p.pf;
+    a.row = p0.sy * (int32_t)p0.in_p.py, a.col = p0.sx * 16, a.tap_dy = (int32_t)p0.in_p.py;
     a.CB = (p0.OFM + 15) / 16;
-    a.KS = (a.CB + 3) / 4;
-    a.SP2 = pl.stages > 2 ? pl.sp[2] : 0;
     for (int k = 0; k < pl.stages; ++k) fill_stage(a.st[k], st[k], pl, k, outs[k], eltws ? eltws[k] : nullptr);
     // the branch-free epilogue forms of a MobileNet block (clamp on the dequantised value, linear projection, clamp), else
     // the run-time form for every stage
     constexpr int CQ = EPI_KIND_CLAMPQ, LIN = EPI_KIND_LINEAR, SUM = EPI_KIND_SUMLIN, ANY = EPI_KIND_FAST;
     const bool ends = pl.epi[0] == CQ && (pl.stages < 3 || pl.epi[2] == CQ);
     const bool block = ends && pl.epi[1] == LIN, block_sum = ends && pl.epi[1] == SUM;  // projection without / with the block's sum
-#define DWCHAIN_LAUNCH(NT, HAS2)                                                                           \
-    {                                                                                                      \
-        if (block) launch_dwchain_instance<NT, 1, HAS2, CQ, LIN, CQ>(s, a, pl.grid, pl.lds_bytes);         \
-        else if (block_sum) launch_dwchain_instance<NT, 1, HAS2, CQ, SUM, CQ>(s, a, pl.grid, pl.lds_bytes); \
-        else launch_dwchain_instance<NT, 1, HAS2, ANY, ANY, ANY>(s, a, pl.grid, pl.lds_bytes);             \
+    bool flip = false;
+    for (int k = 0; k < pl.stages; ++k) flip = flip || st[k].p->in_dt == CLDNN_HIP_U8;
+#define DWCHAIN_LAUNCH(P1, HAS2, FLIP)                                                                          \
+    {                                                                                                           \
+        if (block) launch_dwchain_instance<P1, HAS2, FLIP, CQ, LIN, CQ>(s, a, pl.grid, pl.lds_bytes);           \
+        else if (block_sum) launch_dwchain_instance<P1, HAS2, FLIP, CQ, SUM, CQ>(s, a, pl.grid, pl.lds_bytes);  \
+        else launch_dwchain_instance<P1, HAS2, true, ANY, ANY, ANY>(s, a, pl.grid, pl.lds_bytes);               \
     }
-    if (pl.nt == 2) {
-        if (pl.stages > 2) DWCHAIN_LAUNCH(2, true) else DWCHAIN_LAUNCH(2, false)
-    } else {
-        if (pl.stages > 2) DWCHAIN_LAUNCH(1, true) else DWCHAIN_LAUNCH(1, false)
+#define DWCHAIN_STAGES(P1, FLIP)                          \
+    {                                                     \
+        if (pl.stages > 2) DWCHAIN_LAUNCH(P1, true, FLIP) \
+        else DWCHAIN_LAUNCH(P1, false, FLIP)              \
     }
+    if (pl.u32[1] == 1 && flip) DWCHAIN_STAGES(1, true)
+    else if (pl.u32[1] == 1) DWCHAIN_STAGES(1, false)
+    else if (flip) DWCHAIN_STAGES(2, true)
+    else DWCHAIN_STAGES(2, false)
+#undef DWCHAIN_STAGES
 #undef DWCHAIN_LAUNCH
     CHIP_CHECK(hipGetLastError());
 }
@@ -362,7 +368,6 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
                         int8_t* packed)
 {
     std::memset(packed, 0, chain_packed_bytes(pl));
-    const size_t dw_bytes = pl.dw ? (size_t)pl.sp[0] * (pl.coop ? DWCOOP_KS_BYTES : 9 * 1024) : 0;
     if (pl.coop && pl.dw) {
         // byte mt of dword (K-step, lane % 16, tap): feature 64 ks + 16 (l16 / 4) + 4 mt + l16 % 4
         for (int ks = 0; ks < pl.sp[0]; ++ks)
@@ -372,25 +377,35 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
                         const int ch = ks * 64 + 16 * (l16 >> 2) + 4 * mt + (l16 & 3);
                         if (ch < st[0].p->OFM) packed[((ks * 16 + l16) * 12 + tap) * 4 + mt] = w[0][(size_t)ch * 9 + tap];
                     }
+        packed += (size_t)pl.sp[0] * DWCOOP_KS_BYTES;
     } else if (pl.dw) {
-        // diagonal-weight dwords [K-step][tap][fragment][lane]: lane (kq, l16) of fragment mt carries the weight of feature
-        // 64 ks + 16 (l16 / 4) + 4 mt + l16 % 4 in byte l16 % 4 when kq == l16 / 4, else zero
-        const ConvProblem& p0 = *st[0].p;
-        int32_t* dia = reinterpret_cast<int32_t*>(packed);
-        for (int ks = 0; ks < pl.sp[0]; ++ks)
-            for (int tap = 0; tap < 9; ++tap)
-                for (int mt = 0; mt < 4; ++mt)
-                    for (int lane = 0; lane < 64; ++lane) {
-                        const int kq = lane >> 4, l16 = lane & 15;
-                        const int ch = ks * 64 + 16 * (l16 >> 2) + 4 * mt + (l16 & 3);
-                        int32_t v = 0;
-                        if (kq == (l16 >> 2) && ch < p0.OFM) v = (int32_t)((uint32_t)(uint8_t)w[0][(size_t)ch * 9 + tap] << (8 * (l16 & 3)));
-                        dia[((ks * 9 + tap) * 4 + mt) * 64 + lane] = v;
+        // feature of row r of fragment mt in a unit, and of byte b of lane kq in (half h of) a K-step
+        auto row = [](int r, int mt) { return 16 * ((r >> 2) & 1) + 8 * (r >> 3) + 4 * mt + (r & 3); };
+        auto col = [](int kq, int b) { return 32 * (b >> 3) + 16 * (kq & 1) + 8 * (kq >> 1) + (b & 7); };
+        const int mid = st[0].p->OFM;
+        for (int u = 0; u < pl.u32[0]; ++u)
+            for (int lane = 0; lane < 64; ++lane)
+                for (int s5 = 0; s5 < DWCHAIN_STEPS; ++s5)
+                    for (int mt = 0; mt < 2; ++mt) {
+                        const int ch = u * 32 + row(lane & 15, mt), tap = 2 * s5 + (lane >> 5);
+                        if (ch < mid && tap < 9) packed[((size_t)u * 64 + lane) * 16 + (s5 >> 1) * 4 + 2 * (s5 & 1) + mt] = w[0][(size_t)ch * 9 + tap];
                     }
+        int8_t* at = packed + (size_t)pl.u32[0] * 1024;
+        for (int k = 1; k < pl.stages; ++k) {
+            const int ofm = st[k].p->OFM, ifm = st[k].p->IFM, ksteps = (pl.u32[k - 1] + 1) / 2;
+            for (int ks = 0; ks < ksteps; ++ks)
+                for (int u = 0; u < pl.u32[k]; ++u)
+                    for (int mt = 0; mt < 2; ++mt)
+                        for (int lane = 0; lane < 64; ++lane)
+                            for (int b = 0; b < 16; ++b, ++at) {
+                                const int f = u * 32 + row(lane & 15, mt), c = ks * 64 + col(lane >> 4, b);
+                                if (f < ofm && c < ifm) *at = w[k][(size_t)f * ifm + c];
+                            }
+        }
     }
-    packed += dw_bytes;
+    const size_t unit_bytes = (size_t)pl.units * (pl.dw && !pl.coop ? 1024 : 4096);
     // per-feature vectors behind the weight units: per stage init, calib, eltw_calib, wqf, spans * 64 entries each
-    int32_t* v = reinterpret_cast<int32_t*>(packed + (size_t)pl.units * 4096);
+    int32_t* v = reinterpret_cast<int32_t*>(packed + unit_bytes);
     const float one = 1.0f;
     int32_t one_bits;
     std::memcpy(&one_bits, &one, 4);
@@ -406,6 +421,7 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
             if (src[kind]) std::memcpy(dst, src[kind], (size_t)ofm * 4);
         }
     }
+    if (pl.dw && !pl.coop) return;
     for (int k = pl.dw ? 1 : 0; k < pl.stages; ++k) {
         const MfmaPlan mp = mfma_plan(*st[k].p, pl.dw ? ROW_P64_F64_FOR_DWCHAIN : ROW_WSL_P64_FOR_CHAIN, cus, true);
         std::vector<int8_t> buf(mp.packed_bytes);

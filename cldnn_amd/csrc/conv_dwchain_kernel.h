@@ -3,52 +3,57 @@
 //     depthwise 3x3 (mid -> mid)  ->  1x1 projection (mid -> few)  ->  1x1 expansion of the next block (few -> 6 few).
 // The depthwise result (as large as the expanded tensor it reads) and the projection's input never touch memory.
 //
-// The depthwise stage runs on the MATRIX cores, which the 1x1 stages leave almost idle, so that the vector ALU is
-// free for the three requantisation epilogues (they are what bounds these layers).  One v_mfma_i32_16x16x64_i8 per
-// filter tap and 16-feature fragment: B is what the dense kernels feed anyway -- lane (kq, l16) holds the 16 features
-// of slice kq of pixel l16, shifted by the tap -- and A is DIAGONAL: row r of fragment mt stands for feature
-// 16 * (r / 4) + 4 * mt + r % 4 of the K-step's 64 features (the row order that leaves a lane with 16 consecutive
-// features), and its only non-zero weight sits at exactly that feature's k position.  In register terms the lane
-// (kq, l16) of such an A fragment is one dword (weight << 8 * (l16 % 4), or zero unless kq == l16 / 4) in slot mt of
-// four; the host precomputes that dword per (K-step, tap, fragment, lane) and the kernel keeps the table in LDS.
-// Nine taps times four fragments give the 64 depthwise features of a K-step for 16 pixels; their requantised, packed
-// result is the B fragment of the projection's K-step, and from there on the chain is the dense one.
+// What bounds these layers is the vector ALU: the requantisation of three tensors.  So the depthwise stage runs on the
+// matrix cores, and everything is laid out in units of 32 features, not the dense kernels' spans of 64: a unit costs a lane
+// eight values, and 16, 24, 32, 96 or 144 features fill 1, 1, 1, 3 and 5 of them (in spans of 64 they are 64, 64, 64, 128
+// and 192 features' work).
 //
-// Work split as in the dense chain: persistent workgroups of four independent waves, granules of 16 * NT pixels, the
-// activation taps requested D steps ahead (also across granules), all weights and per-feature vectors in LDS.
+// A unit is two slices of 16 features and two fragments of a v_mfma_i32_16x16x64_i8.  Row (q, i) of fragment mt stands for
+// feature 16 (q % 2) + 8 (q / 2) + 4 mt + i of the unit, so lane (q, l16) ends with eight consecutive features of its pixel:
+// half q / 2 of slice q % 2.  Two units side by side are the 64 values of a K-step of the next stage (lane q: eight bytes of
+// the first, eight of the second; the host lays its weights out for that order; an absent second unit is zeros).
+//
+// Depthwise: the 64 values a product sums over are the unit's two slices at TWO taps (lane q: slice q % 2, tap 2 s + q / 2),
+// so nine taps are five products per fragment.  The weight operand has one byte per row and tap that is not zero; a lane
+// reads the ten bytes of its row (a 16-byte piece, 1 KB per unit in LDS) and a byte permute puts each in its place.
+//
+// Work split as in the dense chain: persistent workgroups of four independent waves, granules of 16 pixels, the
+// activations of the next unit (also across granules) requested while the present one is multiplied, all weights and
+// per-feature vectors in LDS.
+// MobileNet v2 at batch 32, before (spans of 64, one tap per product) and now: 112x112 32-16-96 43.7 -> 28.6 us, 112x112
+// 96-24-144 25.0 -> 18.6, 56x56 144-24-144 30.2 -> 21.2, 28x28 192-32-192 12.9 -> 10.0.
 #pragma once
+#include <type_traits>
+
 #include "conv_chain_kernel.h"
 
 namespace chip {
 
+enum { DWCHAIN_STEPS = 5 };  // pairs of taps
+
 struct DwChainArgs {
     const int8_t* in;
-    const v4i* img;            // LDS image: diagonal-weight dwords [KS][9][4][64], units of stage 1 [SP1][KS], units of
-                               // stage 2 [SP2][SP1], per-feature vectors of stages 0, 1, 2
-    int32_t dw_quads;          // 16-byte pieces of the diagonal-weight table (KS * 9 * 64)
-    int32_t units, vec_quads;
-    int32_t granules;          // ceil(M / (16 * NT))
+    const v4i* img;            // LDS image: depthwise weights [U0][64], fragments of stage 1 [KS][P1][2], of stage 2 [U2][2], vectors
+    int32_t quads;             // its 16-byte pieces
+    int32_t w1, w2, vec;       // where the fragments and the vectors start, in pieces
     int32_t gpw, grem;         // granules / waves of the grid and the remainder
     FastDiv div_waves;         // wave w starts at granule w * gpw + (w * grem) / waves = floor(w * granules / waves)
     uint32_t M;
     int32_t OHW, OW;
     FastDiv div_ohw, div_ow;
-    int32_t sy, sx, py, px;
-    int32_t in_off, in_pb, in_pf, in_py;  // bytes
-    int32_t tap_dy, tap_dx;
-    int32_t CB;                // 16-feature slices of the depthwise stage
-    int32_t KS;                // K-steps of stage 1 = ceil(CB / 4)
-    int32_t SP2;               // 64-feature spans of stage 2 (0: two stages)
+    int32_t in_off, in_pb, in_pf, row, col, tap_dy;  // bytes; in_off: of tap (0, 0) of output pixel (0, 0); row / col: of one output row / pixel
+    int32_t CB, U0, KS, U2;    // slices and units of the depthwise stage, K-steps of stage 1, units of stage 2 (0: two stages)
+    int32_t n0, n1, n2;        // entries of the stages' vectors
     ChainStage st[CHAIN_MAX_STAGES];
 };
 
-// EPI0 / EPI1 / EPI2: epilogue kinds of the three stages, fixed at compile time where the stages have one of the
-// branch-free forms (a MobileNet block: CLAMPQ, LINEAR, CLAMPQ), else the run-time form FAST for all of them
-template <int NT, int SP1, bool HAS2, int EPI0, int EPI1, int EPI2>
-__global__ void __launch_bounds__(256) conv_dwchain_kernel(DwChainArgs a)
+// P1: units of the projection.  FLIP: some stage reads u8 (see the dense kernels' xor).  EPI0 / EPI1 / EPI2: epilogue kinds of
+// the three stages, fixed at compile time where the stages have one of the branch-free forms (a MobileNet block: CLAMPQ,
+// LINEAR, CLAMPQ), else the run-time form FAST for all of them
+template <int P1, bool HAS2, bool FLIP, int EPI0, int EPI1, int EPI2>
+__global__ void __launch_bounds__(256, EPI0 == EPI_KIND_FAST ? 2 : (P1 == 1 ? 4 : 3)) conv_dwchain_kernel(DwChainArgs a)
 {
-    constexpr int WP = NT * 16;
-    constexpr int D = 3;  // look-ahead in taps; the nine taps of a K-step are three rounds
+    constexpr int S = DWCHAIN_STEPS;
     const int t = threadIdx.x;
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -59,20 +64,17 @@ __global__ void __launch_bounds__(256) conv_dwchain_kernel(DwChainArgs a)
     const ChainStage& s2 = a.st[2];
 
     extern __shared__ __align__(16) unsigned char smem[];
-    const int32_t* ldsD = reinterpret_cast<const int32_t*>(smem);                         // [KS][9][4][64] dwords
-    v4i* ldsW = reinterpret_cast<v4i*>(smem + (size_t)a.dw_quads * 16);                    // [units][4][64]
-    const int32_t* ldsV = reinterpret_cast<const int32_t*>(smem + (size_t)a.dw_quads * 16 + (size_t)a.units * 4096);
+    v4i* lds = reinterpret_cast<v4i*>(smem);
+    const int32_t* V = reinterpret_cast<const int32_t*>(lds + a.vec);
     {
-        v4i* dst = reinterpret_cast<v4i*>(smem);
-        const int total = a.dw_quads + a.units * 256 + a.vec_quads;
         constexpr int BATCH = 8;
-        for (int i = t; i < total; i += BATCH * 256) {
+        for (int i = t; i < a.quads; i += BATCH * 256) {
             v4i r[BATCH];
 #pragma unroll
-            for (int u = 0; u < BATCH; ++u) r[u] = a.img[min(i + u * 256, total - 1)];
+            for (int u = 0; u < BATCH; ++u) r[u] = a.img[min(i + u * 256, a.quads - 1)];
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
-                if (i + u * 256 < total) dst[i + u * 256] = r[u];
+                if (i + u * 256 < a.quads) lds[i + u * 256] = r[u];
         }
     }
 
@@ -86,211 +88,185 @@ __global__ void __launch_bounds__(256) conv_dwchain_kernel(DwChainArgs a)
         return;
     }
 
-    const v4i xm0 = {(int)s0.xor_mask, (int)s0.xor_mask, (int)s0.xor_mask, (int)s0.xor_mask};
-    const v4i xm1 = {(int)s1.xor_mask, (int)s1.xor_mask, (int)s1.xor_mask, (int)s1.xor_mask};
-    const v4i xm2 = {(int)s2.xor_mask, (int)s2.xor_mask, (int)s2.xor_mask, (int)s2.xor_mask};
+    // byte 2 (s % 2) + mt of the row's weights goes to byte l16 % 4 of dword 2 h + mt, h = l16 / 8, in the lanes of the row's slice
+    unsigned sel[2][2][2];  // [s % 2][mt][h]
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int sh = 8 * (l16 & 3);
+                const bool mine = (kq & 1) == ((l16 >> 2) & 1) && h == (l16 >> 3);
+                sel[e][mt][h] = mine ? (0x0c0c0c0cu & ~(0xffu << sh)) | ((unsigned)(2 * e + mt) << sh) : 0x0c0c0c0cu;
+            }
+    uint32_t tap_off[S];  // of the lane's tap in step s; the tenth tap has no weight and reads the ninth
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int tap = min(2 * s + (kq >> 1), 8), ty = (tap * 11) >> 5;
+        tap_off[s] = (uint32_t)(ty * a.tap_dy + (tap - ty * 3) * 16);
+    }
 
     struct Refs {
-        uint32_t boff[NT];  // byte offset of the lane's pixel at tap (0, 0), slice 0
-        int o0[NT], o1[NT], e1[NT], o2[NT];
+        uint32_t boff;  // byte offset of the lane's pixel at tap (0, 0), slice 0
+        int o0, o1, e1, o2;
     };
     auto setup = [&](int g, Refs& r) {
+        const uint32_t m = (uint32_t)g * 16 + l16;
+        const bool ok = g < g_end && m < a.M;
+        const uint32_t mm = ok ? m : 0;
+        const uint32_t b = a.div_ohw.div(mm);
+        const uint32_t rr = mm - b * a.OHW;
+        const uint32_t oy = a.div_ow.div(rr), ox = rr - oy * a.OW;
+        r.boff = (uint32_t)(a.in_off + (int)b * a.in_pb + (int)oy * a.row + (int)ox * a.col);
+        auto at = [&](const ChainStage& st) {
+            return st.out_off + (int)b * st.out_pb + (kq & 1) * st.out_pf + (int)oy * st.out_py + (int)ox * 16 + (kq >> 1) * 8;
+        };
+        r.o0 = ok && s0.out ? at(s0) : -1;
+        r.o1 = ok && s1.out ? at(s1) : -1;
+        r.o2 = HAS2 && ok && s2.out ? at(s2) : -1;
+        r.e1 = s1.el_off + (int)b * s1.el_pb + (kq & 1) * s1.el_pf + (int)oy * s1.el_py + (int)ox * s1.el_px + (kq >> 1) * 8;
+    };
+    v4i rb[S];
+    auto load_step = [&](const Refs& r, uint32_t slice_off, int s) { rb[s] = *reinterpret_cast<const v4i*>(a.in + (r.boff + (slice_off + tap_off[s]))); };
+    // a slice past the end (an odd number of them) reads the last one, its weights are zero
+    auto slice_of = [&](int u) { return (uint32_t)(min(2 * u + (kq & 1), a.CB - 1) * a.in_pf); };
+    auto flip = [](const v4i& v, uint32_t mask) {
+        if constexpr (!FLIP) return v;
+        else return v ^ v4i{(int)mask, (int)mask, (int)mask, (int)mask};
+    };
+    auto flip2 = [](const int2& v, uint32_t mask) {
+        if constexpr (!FLIP) return v;
+        else return make_int2(v.x ^ (int)mask, v.y ^ (int)mask);
+    };
+    auto fragment = [&](int i) { return lds[i * 64 + lane]; };
+    // the lane's eight values of a vector
+    auto vec8 = [&](int at, float(&dst)[16]) {
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const uint32_t m = (uint32_t)g * WP + nt * 16 + l16;
-            const bool ok = g < g_end && m < a.M;
-            const PixelPos pp = [&] {
-                PixelPos q;
-                const uint32_t mm = ok ? m : 0;
-                q.b = a.div_ohw.div(mm);
-                const uint32_t rr = mm - q.b * a.OHW;
-                q.oy = a.div_ow.div(rr);
-                q.ox = rr - q.oy * a.OW;
-                return q;
-            }();
-            r.boff[nt] = (uint32_t)(a.in_off + (int)pp.b * a.in_pb + ((int)pp.oy * a.sy - a.py) * a.in_py + ((int)pp.ox * a.sx - a.px) * 16);
-            auto at = [&](const ChainStage& st) {
-                return st.out_off + (int)pp.b * st.out_pb + kq * st.out_pf + (int)pp.oy * st.out_py + (int)pp.ox * 16;
-            };
-            r.o0[nt] = ok && s0.out ? at(s0) : -1;
-            r.o1[nt] = ok && s1.out ? at(s1) : -1;
-            r.o2[nt] = HAS2 && ok && s2.out ? at(s2) : -1;
-            r.e1[nt] = s1.el_off + (int)pp.b * s1.el_pb + kq * s1.el_pf + (int)pp.oy * s1.el_py + (int)pp.ox * s1.el_px;
+        for (int d = 0; d < 2; ++d) {
+            const v4i q = *reinterpret_cast<const v4i*>(V + at + d * 4);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dst[d * 4 + i] = __int_as_float(q[i]);
         }
     };
-    // walk over the (K-step, tap) sequence of the activation requests: the lane's slice of K-step ks is 4 * ks + kq; a
-    // slice past the end (a partly filled last K-step) reads slice 0, its diagonal weights are zero
-    struct Walk {
-        int ks, fy, fx;
+    // eight features of the lane's pixel: f0 is the first, `valid` of them exist
+    auto finish = [&](auto kind, const ChainStage& st, int n, int f0, const v4i(&acc)[2], const int2& ev, int valid) {
+        constexpr int EPI = decltype(kind)::value;
+        float cal[16], ecal[16] = {}, wq[16] = {};
+        vec8(st.vec0 + n + f0, cal);
+        if constexpr (EPI == EPI_KIND_FUSED || EPI == EPI_KIND_SUMLIN || EPI == EPI_KIND_FAST) vec8(st.vec0 + 2 * n + f0, ecal);
+        if constexpr (EPI == EPI_KIND_CLAMPQ || EPI == EPI_KIND_FAST) vec8(st.vec0 + 3 * n + f0, wq);
+        const v4i none = {0, 0, 0, 0}, acc4[4][1] = {{acc[0]}, {acc[1]}, {none}, {none}}, ev4 = {ev.x, ev.y, 0, 0};
+        const v4i p = epilogue_fast16<1, EPI>(st, acc4, 0, wq, cal, ecal, ev4, valid);
+        return make_int2(p[0], p[1]);
     };
-    auto walk_reset = [](Walk& w) { w.ks = 0, w.fy = 0, w.fx = 0; };
-    auto walk_advance = [&](Walk& w) {
-        if (++w.fx == 3) {
-            w.fx = 0;
-            if (++w.fy == 3) w.fy = 0, ++w.ks;
-        }
-    };
-    auto load_b = [&](const Refs& r, const Walk& w, v4i (&xb)[NT]) {
-        const int ks = w.ks < a.KS ? w.ks : 0;
-        const int slice = ks * 4 + kq;
-        const int8_t* base = a.in + ((slice < a.CB ? slice : 0) * a.in_pf + w.fy * a.tap_dy + w.fx * a.tap_dx);
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) xb[nt] = *reinterpret_cast<const v4i*>(base + r.boff[nt]);
-    };
-    auto unit = [&](const ChainStage& st, int span, int ks) { return ldsW + (size_t)(st.unit0 + span * st.kstride + ks) * 256; };
+    const std::integral_constant<int, EPI0> kind0{};
+    const std::integral_constant<int, EPI1> kind1{};
+    const std::integral_constant<int, EPI2> kind2{};
+    const int lf = 16 * (kq & 1) + 8 * (kq >> 1);  // the lane's first feature in a unit
+    auto exists = [&](int u, const ChainStage& st) { return u * 32 + 16 * (kq & 1) < st.OFM; };  // its slice
+    auto store = [&](const ChainStage& st, int at, int u, const int2& v) { *reinterpret_cast<int2*>((int8_t*)st.out + at + u * 2 * st.out_pf) = v; };
+    const int2 zero2 = make_int2(0, 0);
 
     Refs cur, nxt;
-    v4i rb[D][NT];
-    Walk walk;
     setup(g_begin, cur);
-    walk_reset(walk);
+    {
+        const uint32_t so = slice_of(0);
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-        load_b(cur, walk, rb[d]);
-        walk_advance(walk);
+        for (int s = 0; s < S; ++s) load_step(cur, so, s);
     }
-    __syncthreads();  // table, weights and vectors are in LDS; no barrier after this point
+    __syncthreads();  // weights and vectors are in LDS; no barrier after this point
 
     for (int g = g_begin; g < g_end; ++g) {
         setup(g + 1, nxt);
         // residual of the projection (a fused sum): requested now, used after the whole depthwise stage
-        v4i ev1[SP1][NT];
+        int2 ev1[P1];
+        v4i acc1[P1][2];
 #pragma unroll
-        for (int sp = 0; sp < SP1; ++sp)
+        for (int p = 0; p < P1; ++p) {
+            ev1[p] = zero2;
+            if constexpr (chain_reads_residual<EPI1>())
+                if (s1.fe.fused && exists(p, s1)) ev1[p] = *reinterpret_cast<const int2*>((const int8_t*)s1.eltw + cur.e1 + p * 2 * s1.el_pf);
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                ev1[sp][nt] = v4i{0, 0, 0, 0};
-                if constexpr (chain_reads_residual<EPI1>())
-                    if (s1.fe.fused && sp * 64 + kq * 16 < s1.OFM)
-                        ev1[sp][nt] = *reinterpret_cast<const v4i*>((const int8_t*)s1.eltw + cur.e1[nt] + sp * 4 * s1.el_pf);
-            }
-        v4i acc1[SP1 * 4][NT];
-#pragma unroll
-        for (int sp = 0; sp < SP1; ++sp)
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt) {
-                const v4i init = *reinterpret_cast<const v4i*>(ldsV + s1.vec0 + sp * 64 + kq * 16 + mt * 4);
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) acc1[sp * 4 + mt][nt] = init;
-            }
+            for (int mt = 0; mt < 2; ++mt) acc1[p][mt] = *reinterpret_cast<const v4i*>(V + s1.vec0 + p * 32 + lf + mt * 4);
+        }
 
-        for (int ks = 0; ks < a.KS; ++ks) {
-            // ---------------- stage 0: 64 depthwise features of the granule's pixels
-            v4i acc0[4][NT];
+        for (int k = 0; k < a.KS; ++k) {
+            v4i bf0 = {0, 0, 0, 0};
 #pragma unroll
-            for (int mt = 0; mt < 4; ++mt) {
-                const v4i init = *reinterpret_cast<const v4i*>(ldsV + s0.vec0 + ks * 64 + kq * 16 + mt * 4);
+            for (int h = 0; h < 2; ++h) {
+                const int u = 2 * k + h;
+                if (u >= a.U0) break;
+                // ---------------- stage 0: a unit of the granule's pixels
+                v4i acc0[2];
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt) acc0[mt][nt] = init;
-            }
-            const bool last_ks = ks + 1 == a.KS;
+                for (int mt = 0; mt < 2; ++mt) acc0[mt] = *reinterpret_cast<const v4i*>(V + s0.vec0 + u * 32 + lf + mt * 4);
+                const v4i w = fragment(u);
+                const bool last = u + 1 == a.U0;
+                const uint32_t so = slice_of(last ? 0 : u + 1);
 #pragma unroll
-            for (int t0 = 0; t0 < 9; t0 += D) {
-                if (last_ks && t0 + D == 9) walk_reset(walk);  // the last round requests the next granule's first taps
+                for (int s = 0; s < S; ++s) {
 #pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    const int tap = t0 + d;
-                    const int32_t* dia = ldsD + ((ks * 9 + tap) * 4) * 64 + lane;
-#pragma unroll
-                    for (int mt = 0; mt < 4; ++mt) {
+                    for (int mt = 0; mt < 2; ++mt) {
                         v4i fa = {0, 0, 0, 0};
-                        fa[mt] = dia[mt * 64];
 #pragma unroll
-                        for (int nt = 0; nt < NT; ++nt)
-                            acc0[mt][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa, rb[d][nt] ^ xm0, acc0[mt][nt], 0, 0, 0);
+                        for (int hh = 0; hh < 2; ++hh) fa[2 * hh + mt] = (int)__builtin_amdgcn_perm(0u, (unsigned)w[s >> 1], sel[s & 1][mt][hh]);
+                        acc0[mt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa, flip(rb[s], s0.xor_mask), acc0[mt], 0, 0, 0);
                     }
-                    load_b(last_ks && t0 + D == 9 ? nxt : cur, walk, rb[d]);
-                    walk_advance(walk);
+                    load_step(last ? nxt : cur, so, s);
                     step_fence();
                 }
-            }
-            // requantise: the packed results are the B fragment of stage 1's K-step ks
-            const int f0 = ks * 64 + kq * 16;
-            LaneScales sc;
-            chain_scales<EPI0>(s0, ldsV, a.KS, f0, sc);
-            v4i bf0[NT];
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const v4i none = {0, 0, 0, 0};
-                v4i packed = epilogue_fast16<NT, EPI0>(s0, acc0, nt, sc.wq, sc.cal, sc.ecal, none, 16);
-                if (f0 >= s0.OFM) packed = v4i{0, 0, 0, 0};
-                else if (cur.o0[nt] >= 0) *reinterpret_cast<v4i*>((int8_t*)s0.out + cur.o0[nt] + ks * 4 * s0.out_pf) = packed;
-                bf0[nt] = packed ^ xm1;
+                // requantise: the packed results are half of the B fragment of stage 1's K-step k
+                int2 p = finish(kind0, s0, a.n0, u * 32 + lf, acc0, zero2, 16);
+                if (!exists(u, s0)) p = zero2;
+                else if (cur.o0 >= 0) store(s0, cur.o0, u, p);
+                p = flip2(p, s1.xor_mask);
+                bf0[2 * h] = p.x, bf0[2 * h + 1] = p.y;
             }
             // ---------------- stage 1 accumulates this K-step
 #pragma unroll
-            for (int sp = 0; sp < SP1; ++sp)
+            for (int p = 0; p < P1; ++p)
 #pragma unroll
-                for (int mt = 0; mt < 4; ++mt) {
-                    const v4i fa = unit(s1, sp, ks)[kq * 64 + mt * 16 + l16];
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt)
-                        acc1[sp * 4 + mt][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa, bf0[nt], acc1[sp * 4 + mt][nt], 0, 0, 0);
-                }
+                for (int mt = 0; mt < 2; ++mt)
+                    acc1[p][mt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lds[a.w1 + ((k * P1 + p) * 2 + mt) * 64 + lane], bf0, acc1[p][mt], 0, 0, 0);
         }
 
-        // ---------------- stage 1 epilogue: the packed results are the B fragments of stage 2 (K-step = span)
-        v4i bf1[SP1][NT];
+        // ---------------- stage 1 epilogue: the packed results are the B fragment of stage 2
+        v4i bf1 = {0, 0, 0, 0};
 #pragma unroll
-        for (int sp = 0; sp < SP1; ++sp) {
-            const int f0 = sp * 64 + kq * 16;
-            LaneScales sc;
-            chain_scales<EPI1>(s1, ldsV, SP1, f0, sc);
-            const v4i(&acc_sp)[4][NT] = *reinterpret_cast<const v4i(*)[4][NT]>(&acc1[sp * 4]);
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                v4i packed = epilogue_fast16<NT, EPI1>(s1, acc_sp, nt, sc.wq, sc.cal, sc.ecal, ev1[sp][nt], s1.OFM - f0);
-                if (f0 >= s1.OFM) packed = v4i{0, 0, 0, 0};
-                else if (cur.o1[nt] >= 0) *reinterpret_cast<v4i*>((int8_t*)s1.out + cur.o1[nt] + sp * 4 * s1.out_pf) = packed;
-                bf1[sp][nt] = packed ^ xm2;
-            }
+        for (int p = 0; p < P1; ++p) {
+            int2 r = finish(kind1, s1, a.n1, p * 32 + lf, acc1[p], ev1[p], s1.OFM - p * 32 - lf);
+            if (!exists(p, s1)) r = zero2;
+            else if (cur.o1 >= 0) store(s1, cur.o1, p, r);
+            r = flip2(r, s2.xor_mask);
+            bf1[2 * p] = r.x, bf1[2 * p + 1] = r.y;
         }
 
-        // ---------------- stage 2, span by span
+        // ---------------- stage 2, unit by unit
         if constexpr (HAS2) {
-            for (int sp = 0; sp < a.SP2; ++sp) {
-                const int f0 = sp * 64 + kq * 16;
-                v4i acc2[4][NT];
+            for (int u = 0; u < a.U2; ++u) {
+                const int f0 = u * 32 + lf;
+                v4i acc2[2];
 #pragma unroll
-                for (int mt = 0; mt < 4; ++mt) {
-                    const v4i init = *reinterpret_cast<const v4i*>(ldsV + s2.vec0 + f0 + mt * 4);
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt) acc2[mt][nt] = init;
-                }
-#pragma unroll
-                for (int ks = 0; ks < SP1; ++ks)
-#pragma unroll
-                    for (int mt = 0; mt < 4; ++mt) {
-                        const v4i fa = unit(s2, sp, ks)[kq * 64 + mt * 16 + l16];
-#pragma unroll
-                        for (int nt = 0; nt < NT; ++nt)
-                            acc2[mt][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa, bf1[ks][nt], acc2[mt][nt], 0, 0, 0);
-                    }
-                if (f0 >= s2.OFM) continue;
-                LaneScales sc;
-                chain_scales<EPI2>(s2, ldsV, a.SP2, f0, sc);
-                const v4i none = {0, 0, 0, 0};
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    if (cur.o2[nt] < 0) continue;
-                    const v4i packed = epilogue_fast16<NT, EPI2>(s2, acc2, nt, sc.wq, sc.cal, sc.ecal, none, s2.OFM - f0);
-                    *reinterpret_cast<v4i*>((int8_t*)s2.out + cur.o2[nt] + sp * 4 * s2.out_pf) = packed;
-                }
+                for (int mt = 0; mt < 2; ++mt)
+                    acc2[mt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lds[a.w2 + (u * 2 + mt) * 64 + lane], bf1, *reinterpret_cast<const v4i*>(V + s2.vec0 + f0 + mt * 4), 0, 0, 0);
+                const int2 r = finish(kind2, s2, a.n2, f0, acc2, zero2, s2.OFM - f0);
+                if (cur.o2 >= 0 && exists(u, s2)) store(s2, cur.o2, u, r);
             }
         }
         cur = nxt;
     }
 }
 
-template <int NT, int SP1, bool HAS2, int EPI0, int EPI1, int EPI2>
+template <int P1, bool HAS2, bool FLIP, int EPI0, int EPI1, int EPI2>
 void launch_dwchain_instance(hipStream_t s, const DwChainArgs& a, int grid, int lds)
 {
     static std::once_flag allowed;
     std::call_once(allowed, [] {
-        CHIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_dwchain_kernel<NT, SP1, HAS2, EPI0, EPI1, EPI2>),
+        CHIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_dwchain_kernel<P1, HAS2, FLIP, EPI0, EPI1, EPI2>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     });
-    hipLaunchKernelGGL((conv_dwchain_kernel<NT, SP1, HAS2, EPI0, EPI1, EPI2>), dim3(grid), dim3(256), lds, s, a);
+    hipLaunchKernelGGL((conv_dwchain_kernel<P1, HAS2, FLIP, EPI0, EPI1, EPI2>), dim3(grid), dim3(256), lds, s, a);
 }
 
 }  // namespace chip

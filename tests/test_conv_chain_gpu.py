@@ -296,15 +296,18 @@ def test_depthwise_chain_with_the_blocks_sum_on_the_projection(eng, saturate, el
 
 
 @pytest.mark.parametrize("mid,proj,stride,stages,hw", [(576, 96, 1, 3, (7, 9)), (576, 160, 2, 3, (9, 9)), (960, 160, 1, 3, (7, 7)), (960, 192, 1, 2, (5, 3)),
-                                                        (80, 24, 1, 3, (1, 1)), (576, 72, 1, 3, (41, 53))],
-                         ids=["14x14_like", "two_rounds_s2", "7x7_like", "two_stages", "one_pixel", "several_granules_a_group"])
+                                                        (80, 24, 1, 3, (1, 1)), (576, 72, 1, 3, (41, 53)),
+                                                        (32, 16, 1, 3, (93, 91)), (96, 24, 2, 3, (185, 181)), (144, 40, 1, 2, (97, 87)), (48, 64, 1, 3, (92, 95)), (208, 32, 1, 3, (91, 94))],
+                         ids=["14x14_like", "two_rounds_s2", "7x7_like", "two_stages", "one_pixel", "several_granules_a_group", "large_one_unit", "large_s2",
+                              "large_two_stages", "large_odd_slices", "large_odd_units"])
 @pytest.mark.parametrize("in_dt,saturate", [(np.uint8, None), (np.int8, 0), (np.uint8, 1)], ids=["u8", "s8_sum", "u8_sum_saturated"])
 def test_depthwise_chain_on_small_planes(eng, mid, proj, stride, stages, hw, in_dt, saturate):
     """waves that share a granule: one to three spans of projection, more K-steps and spans than waves, a last granule that
-    is not full, with and without the block's sum, against the oracle's separate convolutions"""
+    is not full; and large planes with a granule per wave: odd numbers of slices and of 32-feature units; with and without
+    the block's sum, against the oracle's separate convolutions"""
     r = np.random.default_rng(mid + proj)
-    B = 5 if hw == (41, 53) else 3
     H, W = hw
+    B = 3 if H * W < 4000 else 1
     OH, OW = (H + 2 - 3) // stride + 1, (W + 2 - 3) // stride + 1
     lo, hi = (0, 256) if in_dt == np.uint8 else (-128, 128)
     x = r.integers(lo, hi, (B, mid, H, W)).astype(in_dt)
@@ -334,7 +337,7 @@ def test_depthwise_chain_on_small_planes(eng, mid, proj, stride, stages, hw, in_
         ref_in, prev_t = refs[-1], hip.Tensor.make(hip.S8, hip.FS_B_YX_FSV16, B, ofm, OH, OW)
     for keep in ([False] * (stages - 1) + [True], None):
         ch = hip.ConvChain(eng, spec, keep)
-        assert b"conv_dwchain" in ch.info().kernel_name and b"shared" in ch.info().kernel_name
+        assert b"conv_dwchain" in ch.info().kernel_name and (b"shared" in ch.info().kernel_name) == (B * OH * OW <= 8192)
         ch.enqueue(xin, [b if keep is None or keep[k] else None for k, b in enumerate(bufs)], [None, ebuf, None])
         eng.finish()
         for k in range(stages):
