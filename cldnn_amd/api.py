@@ -269,6 +269,7 @@ def lib():
         for name, (res, args) in SIGNATURES.items():
             f = getattr(l, name)
             f.restype, f.argtypes = res, args
+        l.cldnn_hip_transpose_bytes.restype, l.cldnn_hip_transpose_bytes.argtypes = None, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_size_t]
         _lib = l
     return _lib
 
@@ -368,10 +369,10 @@ class engine:  # noqa: N801
 class memory:  # noqa: N801
     """cldnn::memory (reference api/CPP/memory.hpp:40-180)."""
 
-    def __init__(self, handle, keepalive=None):
+    def __init__(self, handle, keepalive=None, known=None):
         self.h = handle
         self._keep = keepalive
-        self._np = None
+        self._known = {} if known is None else known
 
     @staticmethod
     def allocate(eng, lay):
@@ -394,12 +395,12 @@ class memory:  # noqa: N801
     # numpy conveniences for plain layouts ----------------------------------------------------------
     def _numpy_layout(self):
         """(axis order, padded shape, slices of the logical part, element type, bytes); a memory's layout never changes"""
-        if self._np is None:
+        if not self._known:
             l = self.get_layout()
             order, full, inner = _layout_shape(l)
             dt = np.dtype(NP_OF[l.data_type])
-            self._np = order, full, inner, dt, int(np.prod(full)) * dt.itemsize
-        return self._np
+            self._known["numpy"] = order, full, inner, dt, int(np.prod(full)) * dt.itemsize
+        return self._known["numpy"]
 
     def write(self, array_bfyx):
         """Store a (b, f, y, x) array into the buffer, whatever its plain format and padding."""
@@ -412,8 +413,13 @@ class memory:  # noqa: N801
         """The logical (b, f, y, x) contents of a plain-format buffer."""
         order, full, inner, dt, nbytes = self._numpy_layout()
         with self.pointer() as p:
+            # the one copy out of the locked buffer; the bytes of [feature][batch] go 16 x 16 at a time
+            if order == "yxfb" and nbytes == inner[2].stop * inner[3].stop > inner[2].stop:
+                out = np.empty((full[3], full[2], 1, 1), dt)
+                lib().cldnn_hip_transpose_bytes(p, out.ctypes.data, full[2], full[3])
+                return out
             view = np.frombuffer((C.c_uint8 * nbytes).from_address(p), dt).reshape(full)[inner]
-            return view.transpose([order.index(c) for c in "bfyx"]).copy("C")  # the one copy out of the locked buffer
+            return view.transpose([order.index(c) for c in "bfyx"]).copy("C")
 
     def __del__(self):
         if getattr(self, "h", None) and _lib is not None:
@@ -806,7 +812,8 @@ class network:  # noqa: N801
         carr, n, keep = (options or build_options())._c()
         self.h = _call("cldnn_build_network", eng.h, topo.h, carr, n)
         self._engine, self._topology = eng, topo
-        self._output_ids = None  # fixed by the build; encoded once
+        self._outputs = None  # fixed by the build: names, encoded names, what is known of the layouts
+        self._output_layouts = {}  # so are the layouts
 
     def set_input_data(self, prim_id, mem):
         _call("cldnn_set_network_input", self.h, prim_id.encode(), mem.h)
@@ -837,11 +844,11 @@ class network:  # noqa: N801
         deps = (C.c_void_p * max(len(dependencies), 1))(*[e.h for e in dependencies])
         _call("cldnn_execute_network", self.h, deps, len(dependencies))
         out = {}
-        if self._output_ids is None:
-            self._output_ids = [(name, name.encode()) for name in self.get_output_ids()]
-        for name, raw in self._output_ids:
+        if self._outputs is None:
+            self._outputs = [(name, name.encode(), {}) for name in self.get_output_ids()]
+        for name, raw, known in self._outputs:
             o = _call("cldnn_get_network_output", self.h, raw)
-            out[name] = network_output(event(o.event), memory(o.memory))
+            out[name] = network_output(event(o.event), memory(o.memory, known=known))
         return out
 
     def __del__(self):

@@ -3,6 +3,7 @@
 #include "kernels.h"
 #include "runtime.h"
 
+#include <algorithm>
 #include <chrono>
 #include <cstring>
 #include <thread>
@@ -120,6 +121,49 @@ void cldnn_hip_engine_s::give_event(hipEvent_t ev)
     event_pool.push_back(ev);
 }
 
+uint64_t cldnn_hip_engine_s::mark()
+{
+    std::lock_guard<std::mutex> g(mark_mutex);  // numbers go into the stream in order
+    CHIP_CHECK(hipStreamWriteValue64(stream, reached, marks + 1, 0));
+    return ++marks;
+}
+
+// A launched kernel and its end, waited for here: 8.7 us; by hipStreamSynchronize 11.7 and behind 48 launches 20 us more than
+// here; by an event 11.5.  Runs take microseconds to a few milliseconds: the processor is offered to others after the first
+// hundred microseconds, and given up after 20 ms.
+void cldnn_hip_engine_s::wait_for(uint64_t m) const
+{
+    using clock = std::chrono::steady_clock;
+    const clock::time_point begin = clock::now();
+    for (;;) {
+        for (int i = 0; i < 64; ++i)
+            if (has_reached(m)) return;
+        const clock::duration waited = clock::now() - begin;
+        if (waited > std::chrono::milliseconds(20)) break;
+        if (waited > std::chrono::microseconds(100)) std::this_thread::yield();
+    }
+    make_current();
+    CHIP_CHECK(hipStreamSynchronize(stream));
+}
+
+// the end of an event's work, which has been submitted
+static void wait_for_end(const cldnn_hip_event_s& ev)
+{
+    if (ev.mark) ev.engine->wait_for(ev.mark);
+    if (ev.stop) CHIP_CHECK(hipEventSynchronize(ev.stop));
+}
+
+// an event behind the work enqueued so far.  With profiling it is a HIP event, which carries a time.
+static void record_end(cldnn_hip_event_s& ev)
+{
+    if (ev.engine->profiling) {
+        ev.stop = ev.engine->take_event();
+        CHIP_CHECK(hipEventRecord(ev.stop, ev.engine->stream));
+    } else {
+        ev.mark = ev.engine->mark();
+    }
+}
+
 extern "C" {
 
 const char* cldnn_hip_last_error(void) { return g_last_error.c_str(); }
@@ -149,8 +193,12 @@ cldnn_hip_status cldnn_hip_engine_create(uint32_t device, uint32_t enable_profil
             e->make_current();
             CHIP_CHECK(hipGetDeviceProperties(&e->props, e->device));
             CHIP_CHECK(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
+            CHIP_CHECK(hipHostMalloc((void**)&e->reached, sizeof(*e->reached), hipHostMallocDefault));
+            *e->reached = 0;
             e->static_scratch = mfma_static_scratch(e->device);
         } catch (...) {
+            if (e->reached) (void)hipHostFree(e->reached);
+            if (e->stream) (void)hipStreamDestroy(e->stream);
             delete e;
             throw;
         }
@@ -175,6 +223,7 @@ cldnn_hip_status cldnn_hip_engine_release(cldnn_hip_engine e)
             (void)hipStreamSynchronize(e->stream);
             for (hipEvent_t ev : e->event_pool) (void)hipEventDestroy(ev);
             (void)hipStreamDestroy(e->stream);
+            (void)hipHostFree(e->reached);
             delete e;
         }
     });
@@ -216,7 +265,7 @@ cldnn_hip_status cldnn_hip_engine_finish(cldnn_hip_engine e)
     return guarded([&] {
         CHIP_REQUIRE(e, CLDNN_HIP_INVALID_ARG, "null engine");
         e->make_current();
-        CHIP_CHECK(hipStreamSynchronize(e->stream));
+        e->wait_for(e->mark());
     });
 }
 
@@ -441,6 +490,37 @@ cldnn_hip_status cldnn_hip_buffer_read(cldnn_hip_buffer b, size_t offset, void* 
     });
 }
 
+// 16 x 16 bytes: four rounds, in each of which rows r and r + 8 are interleaved
+static void transpose_16x16(const uint8_t* src, size_t src_ld, uint8_t* dst, size_t dst_ld)
+{
+    typedef uint8_t bytes16 __attribute__((vector_size(16)));
+    bytes16 a[16], b[16];
+    for (int i = 0; i < 16; ++i) std::memcpy(&a[i], src + i * src_ld, 16);
+    for (int round = 0; round < 4; ++round) {
+        for (int i = 0; i < 8; ++i) {
+            b[2 * i] = __builtin_shufflevector(a[i], a[i + 8], 0, 16, 1, 17, 2, 18, 3, 19, 4, 20, 5, 21, 6, 22, 7, 23);
+            b[2 * i + 1] = __builtin_shufflevector(a[i], a[i + 8], 8, 24, 9, 25, 10, 26, 11, 27, 12, 28, 13, 29, 14, 30, 15, 31);
+        }
+        for (int i = 0; i < 16; ++i) a[i] = b[i];
+    }
+    for (int i = 0; i < 16; ++i) std::memcpy(dst + i * dst_ld, &a[i], 16);
+}
+
+void cldnn_hip_transpose_bytes(const void* src, void* dst, size_t rows, size_t cols)
+{
+    const uint8_t* s = (const uint8_t*)src;
+    uint8_t* d = (uint8_t*)dst;
+    for (size_t r = 0; r < rows; r += 16)
+        for (size_t c = 0; c < cols; c += 16) {
+            if (r + 16 <= rows && c + 16 <= cols) {
+                transpose_16x16(s + r * cols + c, cols, d + c * rows + r, rows);
+                continue;
+            }
+            for (size_t i = r; i < std::min(r + 16, rows); ++i)
+                for (size_t j = c; j < std::min(c + 16, cols); ++j) d[j * rows + i] = s[i * cols + j];
+        }
+}
+
 // ------------------------------------------------------------------------------------------ events
 static cldnn_hip_event new_event(cldnn_hip_engine e, bool user)
 {
@@ -490,8 +570,8 @@ cldnn_hip_status cldnn_hip_event_record(cldnn_hip_engine e, cldnn_hip_event* out
         CHIP_REQUIRE(e && out, CLDNN_HIP_INVALID_ARG, "null argument");
         cldnn_hip_event ev = new_event(e, false);
         *out = ev;
-        ev->stop = e->take_event();
-        CHIP_CHECK(hipEventRecord(ev->stop, e->stream));
+        e->make_current();
+        record_end(*ev);
     });
 }
 
@@ -506,21 +586,33 @@ cldnn_hip_status cldnn_hip_event_create_deferred(cldnn_hip_engine e, cldnn_hip_e
     });
 }
 
+static bool submission_pending(cldnn_hip_event ev)
+{
+    if (!ev->deferred) return false;
+    std::lock_guard<std::mutex> g(ev->deferred_mutex);
+    return ev->deferred_pending;
+}
+
 cldnn_hip_status cldnn_hip_event_record_deferred(cldnn_hip_event ev)
 {
     return guarded([&] {
         CHIP_REQUIRE(ev && ev->deferred, CLDNN_HIP_INVALID_ARG, "not a deferred event");
-        hipError_t r = hipSuccess;
-        {
-            std::lock_guard<std::mutex> g(ev->deferred_mutex);
-            CHIP_REQUIRE(ev->deferred_pending, CLDNN_HIP_ERROR, "deferred event recorded twice");
-            ev->engine->make_current();
-            ev->stop = ev->engine->take_event();
-            r = hipEventRecord(ev->stop, ev->engine->stream);
-            ev->deferred_pending = false;  // also after a failed record: nobody may wait for ever
-        }
-        ev->deferred_cv.notify_all();
-        CHIP_CHECK(r);
+        // also after a failed record: nobody may wait for ever
+        struct submitted {
+            cldnn_hip_event ev;
+            ~submitted()
+            {
+                {
+                    std::lock_guard<std::mutex> g(ev->deferred_mutex);
+                    ev->deferred_pending = false;
+                }
+                ev->deferred_cv.notify_all();
+            }
+        };
+        CHIP_REQUIRE(submission_pending(ev), CLDNN_HIP_ERROR, "deferred event recorded twice");
+        submitted release{ev};
+        ev->engine->make_current();
+        record_end(*ev);
     });
 }
 
@@ -530,13 +622,6 @@ static void await_submission(cldnn_hip_event ev)
     if (!ev->deferred) return;
     std::unique_lock<std::mutex> g(ev->deferred_mutex);
     ev->deferred_cv.wait(g, [&] { return !ev->deferred_pending; });
-}
-
-static bool submission_pending(cldnn_hip_event ev)
-{
-    if (!ev->deferred) return false;
-    std::lock_guard<std::mutex> g(ev->deferred_mutex);
-    return ev->deferred_pending;
 }
 
 cldnn_hip_status cldnn_hip_event_retain(cldnn_hip_event ev)
@@ -584,7 +669,7 @@ cldnn_hip_status cldnn_hip_event_wait(cldnn_hip_event ev)
             while (!ev->user_set.load()) std::this_thread::sleep_for(std::chrono::microseconds(50));
         } else {
             await_submission(ev);
-            if (ev->stop) CHIP_CHECK(hipEventSynchronize(ev->stop));
+            wait_for_end(*ev);
         }
         fire_handlers(ev);
     });
@@ -594,7 +679,9 @@ int32_t cldnn_hip_event_is_set(cldnn_hip_event ev)
 {
     if (!ev) return 0;
     if (ev->user) return ev->user_set.load() ? 1 : 0;
-    if (submission_pending(ev) || !ev->stop) return 0;
+    if (submission_pending(ev)) return 0;
+    if (ev->mark) return ev->engine->has_reached(ev->mark) ? 1 : 0;
+    if (!ev->stop) return 0;
     hipError_t r = hipEventQuery(ev->stop);
     if (r == hipSuccess) return 1;
     (void)hipGetLastError();
@@ -632,7 +719,7 @@ cldnn_hip_status cldnn_hip_event_add_handler(cldnn_hip_event ev, cldnn_hip_event
             std::thread([ev] {
                 (void)hipSetDevice(ev->engine->device);
                 await_submission(ev);
-                if (ev->stop) (void)hipEventSynchronize(ev->stop);
+                guarded([&] { wait_for_end(*ev); });
                 fire_handlers(ev);
                 cldnn_hip_event_release(ev);
             }).detach();
@@ -666,9 +753,16 @@ cldnn_hip_status cldnn_hip_engine_wait_events(cldnn_hip_engine e, const cldnn_hi
                 while (!ev->user_set.load()) std::this_thread::sleep_for(std::chrono::microseconds(50));
             } else {
                 await_submission(ev);
-                if (ev->stop && ev->engine != e) CHIP_CHECK(hipStreamWaitEvent(e->stream, ev->stop, 0));
+                if (ev->engine == e) continue;  // the single in-order stream already orders the work
+                if (ev->mark && !ev->engine->has_reached(ev->mark)) {
+                    // a stream waits for HIP events only: for one behind the mark
+                    hipEvent_t behind = ev->engine->take_event();
+                    CHIP_CHECK(hipEventRecord(behind, ev->engine->stream));
+                    CHIP_CHECK(hipStreamWaitEvent(e->stream, behind, 0));
+                    ev->engine->give_event(behind);
+                }
+                if (ev->stop) CHIP_CHECK(hipStreamWaitEvent(e->stream, ev->stop, 0));
             }
-            // same engine: the single in-order stream already orders the work
         }
     });
 }

@@ -21,8 +21,17 @@ struct cldnn_hip_engine_s {
     // cldnn_hip_conv_enqueue_static_scratch only launches
     void* static_scratch = nullptr;
 
+    // A mark is a number the stream writes into pinned host memory when everything before it is done; waiting for it is
+    // reading that memory.  Marks of one engine are reached in order.
+    std::mutex mark_mutex;
+    uint64_t marks = 0;
+    uint64_t* reached = nullptr;
+
     hipEvent_t take_event();
     void give_event(hipEvent_t ev);
+    uint64_t mark();
+    bool has_reached(uint64_t m) const { return __atomic_load_n(reached, __ATOMIC_ACQUIRE) >= m; }
+    void wait_for(uint64_t m) const;
     void make_current() const;
 };
 
@@ -48,6 +57,7 @@ struct cldnn_hip_event_s {
     cldnn_hip_engine engine = nullptr;
     bool user = false;
     std::atomic<bool> user_set{false};
+    uint64_t mark = 0;           // of the engine, or 0: the end is `stop`
     hipEvent_t start = nullptr;  // only with profiling
     hipEvent_t stop = nullptr;
     // a deferred event stands for work that has not been submitted yet: it is recorded later, and whoever waits for

@@ -132,6 +132,7 @@ SIGNATURES = {
     "cldnn_hip_buffer_unlock": (C.c_int32, [C.c_void_p]),
     "cldnn_hip_buffer_map": (C.c_void_p, [C.c_void_p, C.c_void_p]),
     "cldnn_hip_buffer_unmap": (C.c_int32, [C.c_void_p]),
+    "cldnn_hip_transpose_bytes": (None, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_size_t]),
     "cldnn_hip_buffer_use": (C.c_void_p, [C.c_void_p, C.c_int32]),
     "cldnn_hip_buffer_fill": (C.c_int32, [C.c_void_p, C.c_uint8]),
     "cldnn_hip_buffer_device_ptr": (C.c_void_p, [C.c_void_p]),

@@ -178,8 +178,9 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
         if (n->side_stream) {
             where = eng->side;
             cldnn_hip_event fork = nullptr;
-            hip_check(cldnn_hip_event_record(eng->h, &fork));
+            hip_check(cldnn_hip_event_record_begin(eng->h, &fork));
             net->stream_events.push_back(fork);
+            hip_check(cldnn_hip_event_record_end(fork));
             hip_check(cldnn_hip_engine_wait_events(eng->side, &fork, 1));
         }
         // the launch at the head of a chain does the work of every member: it waits for what any of them reads
@@ -275,8 +276,9 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
         }
         if (n->side_stream) {
             cldnn_hip_event join = nullptr;
-            hip_check(cldnn_hip_event_record(eng->side, &join));
+            hip_check(cldnn_hip_event_record_begin(eng->side, &join));
             net->stream_events.push_back(join);
+            hip_check(cldnn_hip_event_record_end(join));
             joins[n] = join;
         }
         if (pev) {

@@ -620,3 +620,11 @@ def test_concatenation_in_place_needs_private_intermediate_inputs():
     prims = [cl.input_layout("i%d" % k, cl.layout(DT.i8, F.bfyx, cl.tensor(1, 16, 5, 4))) for k in range(2)]
     prims.append(cl.concatenation("cat", ["i0", "i1"], cl.concatenation_axis.along_f))
     assert by_id(cl.plan(cl.topology(*prims), cl.build_options(optimize_data=True)))["cat"]["in_place"] is False
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (16, 16), (15, 33), (1000, 128), (1001, 37), (7, 160)])
+def test_transposed_bytes(rows, cols):
+    a = np.random.default_rng(rows).integers(0, 256, (rows, cols), dtype=np.uint8)
+    out = np.empty((cols, rows), np.uint8)
+    cl.lib().cldnn_hip_transpose_bytes(a.ctypes.data, out.ctypes.data, rows, cols)
+    assert (out == a.T).all()
