@@ -931,7 +931,7 @@ cldnn_network cldnn_allocate_network(cldnn_program program, cldnn_status* status
                 continue;
             }
             if (n->chain_unkept()) continue;  // never written: the next member of the chain takes it in registers
-            if (n->writes_for) continue;  // writes its reader's buffer
+            if (n->written_by) continue;  // its buffer was taken where the convolution that writes it stands
             if (n->sibling_head) continue;  // a window into the pair's buffer, made when the pair's first node came up
             if (n->concat_in_place || n->concat_into) {
                 // an in-place concatenation owns one buffer of its own (outside the pool); its inputs, which come earlier
@@ -960,10 +960,13 @@ cldnn_network cldnn_allocate_network(cldnn_program program, cldnn_status* status
                     ++it;
                 }
             }
-            cldnn_layout want = n->out;
+            // A convolution that does its reader's work writes the reader's tensor HERE, possibly long before the reader's own
+            // place: that tensor's life begins with this launch, so it gets its buffer now, from what is idle now.
+            node* written = n->writes_for ? n->writes_for : n;
+            cldnn_layout want = written->out;
             if (n->sibling) want.size.sizes[1] += n->sibling->out.size.sizes[1];
             ref<cldnn_memory_impl> m;
-            if (pool && !n->is_output) {
+            if (pool && !written->is_output) {
                 for (auto it = idle.begin(); it != idle.end(); ++it)
                     if (same_layout((*it)->layout, want)) {
                         m = *it;
@@ -994,8 +997,8 @@ cldnn_network cldnn_allocate_network(cldnn_program program, cldnn_status* status
                 net->mem[b] = window(b->out, layout_bytes(n->out));
                 continue;
             }
-            net->mem[n] = m;
-            if (pool && !n->is_output && last_use.count(n)) in_flight.emplace_back(last_use[n], m);
+            net->mem[written] = m;
+            if (pool && !written->is_output && last_use.count(written)) in_flight.emplace_back(last_use[written], m);
         }
         net->retain();
         return net.get();

@@ -845,3 +845,59 @@ def test_paired_convolution_that_is_an_output(eng):
     np.testing.assert_array_equal(outs["shortcut"].get_memory().read(), sc)
     assert outs["reduce"].get_memory().read().min() == 0  # relu on the second convolution only
     assert sc.min() < 0
+
+
+# ------------------------------------------------------- convolutions that do their reader's work, in networks with branches
+def branched(eng, case):
+    """(topology, input, expected): a convolution finishes the pooling / the reorder behind it and so writes that tensor before
+    the primitives between the two; `case` says which of their tensors must not share its buffer"""
+    r = np.random.default_rng(41)
+    B, C, prims, ref = 2, 128, [], {}
+
+    def conv(name, src, k=3, stride=1, pad=1, relu=False):
+        w, b, q, c = rand_layer(r, C, C, k, ref[src].dtype == np.uint8)
+        prims.extend([cl.data(f"{name}_{n}", m) for n, m in zip("wbqc", [cl.make_memory(eng, w)] + [vec_mem(eng, v) for v in (b, q, c)])])
+        prims.append(cl.convolution(name, src, [name + "_w"], [name + "_b"], [name + "_q"], [name + "_c"], stride=cl.tensor(1, 1, stride, stride),
+                                    input_offset=cl.tensor(0, 0, -pad, -pad, 0), with_activation=relu, output_data_type=DT.i8))
+        ref[name] = rc.conv(ref[src], w, b, wqf=q, calib=c, stride=(stride, stride), pad=(pad, pad), out_dt="s8", act="relu" if relu else "none")
+
+    def total(a, b):
+        prims.append(cl.eltwise("out", a, b, cl.eltwise_mode.sum))
+        ref["out"] = rc.eltwise([ref[a], ref[b]], "sum")
+
+    n = 4 if case.startswith("scores") else 16
+    ref["input"] = r.integers(-128, 128, (B, C, n, n)).astype(np.int8)
+    prims.append(cl.input_layout("input", cl.layout(DT.i8, F.bfyx, cl.tensor(B, C, n, n))))
+    if case.startswith("scores"):
+        conv("x_conv", "input", 4, 1, 0)
+        prims.append(cl.reorder("x", "x_conv", F.bfyx))
+        conv("p_conv", "input", 3, 2, 0)     # (not x's window: the two would run as a pair)
+        prims.append(cl.activation("b", "x", cl.activation_func.relu))  # reads x after p has been written
+        prims.append(cl.reorder("p", "p_conv", F.bfyx))
+        ref["x"], ref["p"] = ref["x_conv"], ref["p_conv"]
+        ref["b"] = np.maximum(ref["x"], 0)
+        total("b", "p")
+    else:
+        if case == "read_in_between":
+            conv("x", "input", stride=2)     # the pooling's layout; read by b, after a has written the pooling
+            conv("a", "input", relu=True)
+            conv("b", "x")
+        else:
+            conv("a", "input", relu=True)
+            conv("x", "input", stride=2)     # is born and dies between a and the pooling
+            conv("b", "x")
+        prims.append(cl.pooling("p", "a", cl.pooling_mode.max, cl.tensor(1, 1, 2, 2), cl.tensor(1, 1, 2, 2)))
+        ref["p"] = rc.pool(ref["a"], "max", (2, 2), (2, 2))
+        conv("q", "p")
+        total("b", "q")
+    return cl.topology(*prims), ref["input"], ref["out"]
+
+
+@pytest.mark.parametrize("case", ["read_in_between", "dies_in_between", "scores_in_between"])
+def test_early_written_tensor_keeps_out_of_live_buffers(eng, case):
+    topo, x, expected = branched(eng, case)
+    net, outs = run(eng, topo, {"input": cl.make_memory(eng, x)}, True)
+    assert len(np.unique(expected)) > 32
+    for _ in range(2):
+        np.testing.assert_array_equal(outs["out"].get_memory().read(), expected)
+        outs = net.execute()
