@@ -164,6 +164,25 @@ static void record_end(cldnn_hip_event_s& ev)
     }
 }
 
+// a deferred event: block until the work it stands for has been submitted
+static void await_submission(cldnn_hip_event ev)
+{
+    if (!ev->deferred) return;
+    std::unique_lock<std::mutex> g(ev->deferred_mutex);
+    ev->deferred_cv.wait(g, [&] { return !ev->deferred_pending; });
+}
+
+// blocks until the event is complete; its handlers are left to others
+static void await_event(cldnn_hip_event ev)
+{
+    if (ev->user) {
+        while (!ev->user_set.load()) std::this_thread::sleep_for(std::chrono::microseconds(50));
+    } else {
+        await_submission(ev);
+        wait_for_end(*ev);
+    }
+}
+
 extern "C" {
 
 const char* cldnn_hip_last_error(void) { return g_last_error.c_str(); }
@@ -363,7 +382,17 @@ void* cldnn_hip_buffer_map(cldnn_hip_buffer b, cldnn_hip_event last_use)
     void* result = nullptr;
     guarded([&] {
         CHIP_REQUIRE(b, CLDNN_HIP_INVALID_ARG, "null buffer");
-        std::lock_guard<std::mutex> g(b->lock_mutex);
+        std::unique_lock<std::mutex> g(b->lock_mutex);
+        if (last_use && b->lock_count == 0 && b->newest != cldnn_hip_buffer_s::DEVICE) {
+            // kernels and uploads in flight may still use the shadow.  An event that has been waited for already costs a
+            // microsecond here, the stream 25 (it sends a marker of its own through the queue).  Waited for without the mutex,
+            // which whoever has to come first (the thread that submits a deferred event's work) or a handler of the event may
+            // need; the handlers run where they would without this call.
+            b->engine->make_current();
+            g.unlock();
+            await_event(last_use);
+            g.lock();
+        }
         if (b->lock_count == 0) {
             b->engine->make_current();
             b->need_shadow();
@@ -371,12 +400,7 @@ void* cldnn_hip_buffer_map(cldnn_hip_buffer b, cldnn_hip_event last_use)
                 CHIP_CHECK(hipMemcpyAsync(b->shadow, b->dev, b->bytes, hipMemcpyDeviceToHost, b->engine->stream));
                 CHIP_CHECK(hipStreamSynchronize(b->engine->stream));
                 b->newest = cldnn_hip_buffer_s::BOTH;
-            } else if (last_use) {
-                // kernels and uploads in flight may still use the shadow.  An event that has been waited for already costs a
-                // microsecond here, the stream 25 (it sends a marker of its own through the queue)
-                const cldnn_hip_status st = cldnn_hip_event_wait(last_use);
-                if (st != CLDNN_HIP_SUCCESS) throw error(st, cldnn_hip_last_error());
-            } else {
+            } else if (!last_use) {
                 CHIP_CHECK(hipStreamSynchronize(b->engine->stream));
             }
         }
@@ -616,14 +640,6 @@ cldnn_hip_status cldnn_hip_event_record_deferred(cldnn_hip_event ev)
     });
 }
 
-// a deferred event: block until the work it stands for has been submitted
-static void await_submission(cldnn_hip_event ev)
-{
-    if (!ev->deferred) return;
-    std::unique_lock<std::mutex> g(ev->deferred_mutex);
-    ev->deferred_cv.wait(g, [&] { return !ev->deferred_pending; });
-}
-
 cldnn_hip_status cldnn_hip_event_retain(cldnn_hip_event ev)
 {
     return guarded([&] {
@@ -665,12 +681,7 @@ cldnn_hip_status cldnn_hip_event_wait(cldnn_hip_event ev)
 {
     return guarded([&] {
         CHIP_REQUIRE(ev, CLDNN_HIP_INVALID_ARG, "null event");
-        if (ev->user) {
-            while (!ev->user_set.load()) std::this_thread::sleep_for(std::chrono::microseconds(50));
-        } else {
-            await_submission(ev);
-            wait_for_end(*ev);
-        }
+        await_event(ev);
         fire_handlers(ev);
     });
 }

@@ -1,6 +1,7 @@
 """Which copy of a mapped buffer is current (cldnn_hip_buffer_map / _unmap / _use): every order of host writes and device
 uses gives the bytes written last, also where a kernel reads or writes the host copy in place."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -66,3 +67,61 @@ def test_input_rewritten_and_reused_between_runs():
             n.set_input_data("x", mem)
             assert np.array_equal(n.execute()["y"].get_memory().read(), x.astype(np.float32))
         assert np.array_equal(mem.read(), x)
+
+
+def in_thread(f):
+    t = threading.Thread(target=f, daemon=True)
+    t.start()
+    return t
+
+
+def test_buffer_can_be_used_while_a_map_waits_for_its_event():
+    eng, L = hip.Engine(0), hip.lib()
+    buf = hip.Buffer(eng, hip.Tensor.make(hip.U8, hip.BFYX, 1, 64, 1, 1))
+    mapped(buf)[:] = 7
+    hip.check(L.cldnn_hip_buffer_unmap(buf.h))
+    gate, seen = C.c_void_p(), []
+    hip.check(L.cldnn_hip_event_create_user(eng.h, 0, C.byref(gate)))
+    waiter = in_thread(lambda: seen.append(L.cldnn_hip_buffer_map(buf.h, gate)))
+    waiter.join(0.2)
+    assert waiter.is_alive() and not seen
+    user = in_thread(lambda: L.cldnn_hip_buffer_use(buf.h, READ))  # as the run behind the gate would
+    user.join(20)
+    assert not user.is_alive()
+    hip.check(L.cldnn_hip_event_set(gate))
+    waiter.join(20)
+    assert not waiter.is_alive() and seen[0]
+    hip.check(L.cldnn_hip_buffer_unmap(buf.h))
+    hip.check(L.cldnn_hip_event_release(gate))
+    buf.close()
+    eng.close()
+
+
+def test_handler_of_an_output_event_may_lock_the_output():
+    """whichever thread sees the end of the run first: the one that locks the output or the one that calls the handler"""
+    eng = cl.engine()
+    F, DT = cl.format, cl.data_types
+    lay = cl.layout(DT.u8, F.bfyx, cl.tensor(8, 16, 64, 64))
+    net = cl.network(eng, cl.topology(cl.input_layout("x", lay), cl.reorder("y", "x", F.yxfb, DT.f32), cl.reorder("s", "y", F.bfyx, DT.u8)))
+    x = np.random.default_rng(3).integers(0, 256, (8, 16, 64, 64), dtype=np.uint8)
+    net.set_input_data("x", cl.make_memory(eng, x))
+    got, wrong = [], []
+
+    def rounds():
+        for _ in range(40):
+            out = net.execute()["s"]
+            mem, ev, done = out.get_memory(), out.get_event(), threading.Event()
+
+            def handler(_):
+                got.append(np.array_equal(mem.read(), x))
+                done.set()
+
+            cb = cl.EVENT_HANDLER(handler)
+            cl._call("cldnn_add_event_handler", ev.h, cb, None)
+            wrong.append(not np.array_equal(mem.read(), x))
+            if not done.wait(20):
+                return
+
+    t = in_thread(rounds)
+    t.join(60)
+    assert not t.is_alive() and got == [True] * 40 and not any(wrong)
