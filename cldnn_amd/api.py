@@ -413,8 +413,8 @@ class memory:  # noqa: N801
         """The logical (b, f, y, x) contents of a plain-format buffer."""
         order, full, inner, dt, nbytes = self._numpy_layout()
         with self.pointer() as p:
-            # the one copy out of the locked buffer; the bytes of [feature][batch] go 16 x 16 at a time
-            if order == "yxfb" and nbytes == inner[2].stop * inner[3].stop > inner[2].stop:
+            # the one copy out of the locked buffer; the bytes of [feature][batch] without padding go 16 x 16 at a time
+            if order == "yxfb" and nbytes == full[2] * full[3] > full[2] and all(s == slice(0, n) for s, n in zip(inner, full)):
                 out = np.empty((full[3], full[2], 1, 1), dt)
                 lib().cldnn_hip_transpose_bytes(p, out.ctypes.data, full[2], full[3])
                 return out

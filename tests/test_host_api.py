@@ -628,3 +628,20 @@ def test_transposed_bytes(rows, cols):
     out = np.empty((cols, rows), np.uint8)
     cl.lib().cldnn_hip_transpose_bytes(a.ctypes.data, out.ctypes.data, rows, cols)
     assert (out == a.T).all()
+
+
+@pytest.mark.parametrize("pad", [((0, 0), (0, 0)), ((0, 2), (0, 0)), ((0, 0), (0, 2)), ((3, 0), (0, 0)), ((0, 0), (3, 0)), ((1, 2), (3, 4))],
+                         ids=["none", "lower_f", "upper_f", "lower_b", "upper_b", "all"])
+@pytest.mark.parametrize("dtype", [np.int8, np.float32])
+@pytest.mark.parametrize("shape", [(3, 5, 1, 1), (1, 5, 1, 1), (2, 4, 3, 2)], ids=["batch", "one_image", "planes"])
+def test_read_and_write_leave_the_padding_out(shape, dtype, pad):
+    """yxfb, the layout of a batch's scores; pad: (batch, features) below and above"""
+    b, f, y, x = shape
+    lay = cl.layout(cl.DT_OF[np.dtype(dtype)], F.yxfb, cl.tensor(b, f, x, y), cl.padding(pad[0] + (0, 0), pad[1] + (0, 0)))
+    full = np.full((y, x, f + pad[0][1] + pad[1][1], b + pad[0][0] + pad[1][0]), 99, dtype)
+    m = cl.memory.attach(lay, full)
+    values = np.arange(b * f * y * x).astype(dtype).reshape(shape)
+    m.write(values)
+    got = m.read()
+    assert got.shape == shape and np.array_equal(got, values)
+    assert (full == 99).sum() == full.size - values.size
