@@ -118,14 +118,19 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
         const bool block = pl.epi[0] == EPI_KIND_CLAMPQ && (pl.epi[1] == EPI_KIND_LINEAR || pl.epi[1] == EPI_KIND_SUMLIN)
                            && (n < 3 || pl.epi[2] == EPI_KIND_CLAMPQ) && !st[1].fe->split_valid;
         const bool small = (pl.m_total + 15) / 16 <= 2ll * cus;
-        if (pl.sp[1] > 1 && !(block && small))
-            return "stage 1: a projection of more than 64 features is chained in the forms of a MobileNet block and on small planes only";
-        if (block && small && pl.ksteps0 >= 2) {
+        const int waves = pl.ksteps0 <= 8 ? std::max(4, pl.ksteps0) : std::min(8, (pl.ksteps0 + 1) / 2);
+        const int shared_lds = (waves * 4 + 1) * pl.sp[1] * 1024 + vec * 4;
+        const bool shared = block && small && pl.ksteps0 >= 2 && shared_lds <= CHAIN_MAX_LDS;
+        // (the other form has two units of 32 features of projection at most)
+        if (pl.sp[1] > 1 && !shared)
+            return "stage 1: a projection of more than 64 features is chained in the forms of a MobileNet block, on small planes and from 65 mid "
+                   "features on only, where partial sums and vectors fit into LDS";
+        if (shared) {
             pl.coop = 1, pl.nt = 1;
             pl.img_bytes = pl.sp[0] * DWCOOP_KS_BYTES + pl.units * 4096 + vec * 4;
-            pl.waves = pl.ksteps0 <= 8 ? std::max(4, pl.ksteps0) : std::min(8, (pl.ksteps0 + 1) / 2);
+            pl.waves = waves;
             pl.granules = (int)((pl.m_total + 15) / 16);
-            pl.lds_bytes = (pl.waves * 4 + 1) * pl.sp[1] * 1024 + vec * 4;
+            pl.lds_bytes = shared_lds;
             const int per_cu = std::max(1, std::min((pl.sp[1] == 1 ? 12 : 8) / pl.waves, CHAIN_MAX_LDS / pl.lds_bytes));
             pl.grid = std::min(cus * per_cu / 8 * 8, (pl.granules + 7) / 8 * 8);
             std::snprintf(pl.name, sizeof(pl.name), "conv_dwchain<%d stages,p16 shared by %d waves,mid %d,spans %d-%d>", n, pl.waves, p0.OFM, pl.sp[1],

@@ -370,3 +370,34 @@ def test_bottleneck_chain_with_weights_in_registers(eng, hw, in_dt, stages, fuse
             b.close()
             if e is not None:
                 e.close()
+
+
+@pytest.mark.parametrize("mid,proj,expand,chained", [(1792, 192, 1920, True), (1920, 192, 1920, False), (65, 96, 576, True), (64, 96, 576, False), (48, 192, 64, False)],
+                         ids=["lds_full", "lds_beyond", "two_k_steps", "one_k_step", "one_k_step_three_spans"])
+def test_wide_projections_are_chained_in_the_shared_form_only(eng, mid, proj, expand, chained):
+    """a projection of more than 64 features exists in the form whose waves share a granule alone: where that form does not
+    apply (its LDS, a single K-step) the chain is refused and the layers run one by one"""
+    r = np.random.default_rng(mid)
+    mid = -(-mid // 16) * 16
+    x = r.integers(-128, 128, (1, mid, 7, 7)).astype(np.int8)
+    xin = hip.upload(eng, x, "fs_b_yx_fsv16", (1, 1))
+    spec, ref, prev_t = [], x, xin.tensor
+    for ofm, ifm_g, fk, act, groups in [(mid, 1, 3, "relu6", mid), (proj, mid, 1, "none", 1), (expand, proj, 1, "relu6", 1)]:
+        w, bias, wqf, calib, akw = relu6_layer(r, ofm, ifm_g, fk, act)
+        d = hip.conv_desc(prev_t, w.shape, "s8", pad=(fk // 2,) * 2, groups=groups, bias_dt=hip.I32, has_wqf=True, has_calib=True, **akw)
+        spec.append((d, w, bias, wqf, calib, None))
+        ref = rc.conv(ref, w, bias, wqf=wqf, calib=calib, pad=(fk // 2,) * 2, groups=groups, out_dt="s8", **akw)
+        prev_t = hip.Tensor.make(hip.S8, hip.FS_B_YX_FSV16, 1, ofm, 7, 7)
+    if chained:
+        out = hip.Buffer(eng, spec[2][0].output)
+        ch = hip.ConvChain(eng, spec, [False, False, True])
+        assert b"shared" in ch.info().kernel_name
+        ch.enqueue(xin, [None, None, out])
+        eng.finish()
+        assert np.array_equal(hip.download(eng, out), ref) and len(np.unique(ref)) > 8
+        ch.close(), out.close()
+    else:
+        with pytest.raises(hip.HipError) as err:
+            hip.ConvChain(eng, spec, [False, False, True])
+        assert err.value.status == -6 and "projection" in str(err.value)
+    xin.close()
