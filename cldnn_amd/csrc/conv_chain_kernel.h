@@ -116,7 +116,8 @@ constexpr bool chain_reads_residual()
     return EPI == EPI_KIND_FUSED || EPI == EPI_KIND_FAST || EPI == EPI_KIND_SUMLIN;
 }
 
-// SP0 / SP1 / SP2: 64-feature spans of the three stages (chains of two run on conv_coop_kernel.h).  D: activation look-ahead of stage 0.
+// SP0 / SP1 / SP2: 64-feature spans of the three stages (SP2 == 0: two stages, whose first is no 3x3 over 64 features: that one
+// runs on conv_coop_kernel.h).  D: activation look-ahead of stage 0.
 template <int NT, int D, int SP0, int SP1, int SP2, int EPI0, int EPI1, int EPI2>
 __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
 {
@@ -185,8 +186,8 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
             };
             r.o0[nt] = ok && s0.out ? at(s0) : -1;
             r.o1[nt] = ok && s1.out ? at(s1) : -1;
-            r.o2[nt] = ok && s2.out ? at(s2) : -1;
-            r.e0[nt] = res(s0), r.e1[nt] = res(s1), r.e2[nt] = res(s2);
+            r.o2[nt] = SP2 > 0 && ok && s2.out ? at(s2) : -1;
+            r.e0[nt] = res(s0), r.e1[nt] = res(s1), r.e2[nt] = SP2 > 0 ? res(s2) : 0;
         }
     };
     auto load_b = [&](const Refs& r, const TapWalk& w, v4i (&xb)[NT]) {
@@ -289,8 +290,8 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
         }
 
         // ---------------- stage 1 span by span; every finished span is one K-step of stage 2
-        v4i acc2[SP2 * 4][NT];
-        {
+        v4i acc2[SP2 > 0 ? SP2 * 4 : 1][NT];
+        if constexpr (SP2 > 0) {
 #pragma unroll
             for (int sp = 0; sp < SP2; ++sp)
 #pragma unroll
@@ -340,7 +341,7 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
                     }
                 }
             }
-            {
+            if constexpr (SP2 > 0) {
 #pragma unroll
                 for (int sp = 0; sp < SP2; ++sp) {
                     v4i fa[4];
@@ -357,7 +358,7 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
         }
 
         // ---------------- stage 2 epilogue
-        {
+        if constexpr (SP2 > 0) {
 #pragma unroll
             for (int sp = 0; sp < SP2; ++sp) {
                 const int f0 = sp * 64 + kq * 16;

@@ -401,3 +401,34 @@ def test_wide_projections_are_chained_in_the_shared_form_only(eng, mid, proj, ex
             hip.ConvChain(eng, spec, [False, False, True])
         assert err.value.status == -6 and "projection" in str(err.value)
     xin.close()
+
+
+@pytest.mark.parametrize("fused", [True, False], ids=["fused", "plain"])
+@pytest.mark.parametrize("ifm", [192, 576, 960])
+def test_two_stage_chain_behind_a_wide_1x1(eng, ifm, fused):
+    """a reducing 1x1 (3, 9 or 15 K-steps) and the expansion behind it; the last granule of 32 pixels is not full"""
+    r = np.random.default_rng(ifm)
+    B, H, W = 3, 13, 11
+    x = r.integers(0, 256, (B, ifm, H, W)).astype(np.uint8)
+    xin = hip.upload(eng, x, "fs_b_yx_fsv16")
+    l0, l1 = layer(r, ifm, 64, 1, np.uint8), layer(r, 64, 256, 1, np.int8)
+    e, ecal = r.integers(-128, 128, (B, 256, H, W)).astype(np.int8), r.uniform(0.25, 1.0, 256).astype(np.float32)
+    ebuf = hip.upload(eng, e, "fs_b_yx_fsv16")
+    kw = dict(bias_dt=hip.I32, has_wqf=True, has_calib=True)
+    d0 = hip.conv_desc(xin.tensor, l0[0].shape, "s8", act="relu", **kw)
+    tail = dict(act="none", eltw_t=ebuf.tensor, eltw_act="relu", has_eltw_calib=True) if fused else dict(act="relu")
+    d1 = hip.conv_desc(hip.Tensor.make(hip.S8, hip.FS_B_YX_FSV16, B, 64, H, W), l1[0].shape, "s8", out_pad=(1, 1), **kw, **tail)
+    ref = [rc.conv(x, l0[0], l0[1], wqf=l0[2], calib=l0[3], out_dt="s8", act="relu")]
+    more = dict(act="none", eltw=e, eltw_act="relu", eltw_calib=ecal) if fused else dict(act="relu")
+    ref.append(rc.conv(ref[0], l1[0], l1[1], wqf=l1[2], calib=l1[3], out_dt="s8", **more))
+    out = [hip.Buffer(eng, d0.output), hip.Buffer(eng, d1.output)]
+    for keep in ([False, True], [True, True]):
+        ch = hip.ConvChain(eng, [(d0, *l0, None), (d1, *l1, ecal if fused else None)], keep)
+        assert b"2 stages,p32,d3" in ch.info().kernel_name
+        ch.enqueue(xin, [o if k else None for o, k in zip(out, keep)], [None, ebuf])
+        eng.finish()
+        assert np.array_equal(hip.download(eng, out[1]), ref[1])
+        ch.close()
+    assert np.array_equal(hip.download(eng, out[0]), ref[0])
+    for b in out + [xin, ebuf]:
+        b.close()
