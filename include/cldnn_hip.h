@@ -86,7 +86,8 @@ cldnn_hip_status cldnn_hip_buffer_unlock(cldnn_hip_buffer b);
 /* The same for a buffer whose device pointer is only taken through cldnn_hip_buffer_use, so that the library knows which
  * copy is current: map copies device -> shadow only if the device wrote since, and after the last unmap the shadow is the
  * current copy until a use needs it on the device.  Both forms may be mixed on one buffer.
- * last_use: an event recorded behind all work on the buffer, waited for instead of the stream (may be NULL). */
+ * last_use: an event recorded behind all work on the buffer, waited for instead of the stream (may be NULL).  Its handlers are
+ * not called, and the buffer may be used meanwhile. */
 void* cldnn_hip_buffer_map(cldnn_hip_buffer b, cldnn_hip_event last_use);  /* NULL on failure */
 cldnn_hip_status cldnn_hip_buffer_unmap(cldnn_hip_buffer b);
 enum {

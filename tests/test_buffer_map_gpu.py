@@ -125,3 +125,38 @@ def test_handler_of_an_output_event_may_lock_the_output():
     t = in_thread(rounds)
     t.join(60)
     assert not t.is_alive() and got == [True] * 40 and not any(wrong)
+
+
+def test_large_input_is_copied_from_the_unmap_on():
+    """beyond the in-place limit: the device has the bytes before any use asks for them, and a map that follows waits for the
+    copy whatever event it is given; a result that was only looked at is not copied back"""
+    eng, L = hip.Engine(0), hip.lib()
+    t = hip.Tensor.make(hip.U8, hip.BFYX, 1, 1 << 15, 1, 1031)
+    src, dst = hip.Buffer(eng, t), hip.Buffer(eng, t)
+    on_device = L.cldnn_hip_buffer_use(src.h, READ)  # the same pointer for the buffer's life
+    r = np.random.default_rng(2)
+    old = C.c_void_p()
+    hip.check(L.cldnn_hip_event_record(eng.h, C.byref(old)))
+    eng.finish()
+
+    def device_bytes():
+        hip.check(L.cldnn_hip_reorder(eng.h, on_device, C.byref(t), L.cldnn_hip_buffer_use(dst.h, WRITE), C.byref(t)))
+        return dst.read_raw()
+
+    for _ in range(3):
+        data = r.integers(0, 256, src.nbytes, dtype=np.uint8)
+        mapped(src)[:] = data
+        hip.check(L.cldnn_hip_buffer_unmap(src.h))
+        p = L.cldnn_hip_buffer_map(src.h, old)  # an event from before the copy
+        C.memset(p, 0x5a, src.nbytes)
+        assert np.array_equal(device_bytes(), data)
+        hip.check(L.cldnn_hip_buffer_unmap(src.h))
+        assert (device_bytes() == 0x5a).all() and (src.read_raw() == 0x5a).all()
+    L.cldnn_hip_buffer_use(src.h, WRITE)
+    mapped(src)[:] = 1
+    hip.check(L.cldnn_hip_buffer_unmap(src.h))
+    assert (device_bytes() == 0x5a).all() and (src.read_raw() == 1).all()
+    copy(eng, src, READ, dst, WRITE)
+    assert (dst.read_raw() == 1).all()
+    hip.check(L.cldnn_hip_event_release(old))
+    src.close(), dst.close(), eng.close()
