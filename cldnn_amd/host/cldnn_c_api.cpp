@@ -139,7 +139,7 @@ static int32_t use_of_output(const node* n)
 
 // Enqueue one run.  deferred_marker: the run was announced earlier (its outputs already carry that event) and is
 // submitted now that its user events are set.
-static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cldnn_event_impl* deferred_marker)
+static void enqueue_run(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cldnn_event_impl* deferred_marker)
 {
     cldnn_program_impl* prog = net->program.get();
     cldnn_engine_impl* eng = prog->engine.get();
@@ -314,6 +314,20 @@ static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cld
     if (eng->side) hip_check(cldnn_hip_engine_flush(eng->side));
     hip_check(cldnn_hip_engine_flush(eng->h));
     net->has_run = true;
+}
+
+static void submit(cldnn_network_impl* net, cldnn_event* deps, size_t ndeps, cldnn_event_impl* deferred_marker)
+{
+    try {
+        enqueue_run(net, deps, ndeps, deferred_marker);
+    } catch (...) {
+        // What was enqueued before the failure may read and write host copies of the network's memories in place, and their
+        // last use is not noted: a lock would not wait for it.
+        cldnn_engine_impl* eng = net->program->engine.get();
+        if (eng->side) (void)cldnn_hip_engine_finish(eng->side);
+        (void)cldnn_hip_engine_finish(eng->h);
+        throw;
+    }
 }
 
 static void finish_deferred_run(const std::shared_ptr<deferred_run>& run);

@@ -901,3 +901,30 @@ def test_early_written_tensor_keeps_out_of_live_buffers(eng, case):
     for _ in range(2):
         np.testing.assert_array_equal(outs["out"].get_memory().read(), expected)
         outs = net.execute()
+
+
+def test_failed_run_leaves_nothing_in_flight(eng):
+    """a run that fails midway (its second input is not set when the first one's reorder has been enqueued) is over when
+    execute returns: the memories it used may be locked"""
+    n = 64
+    lay = cl.layout(DT.i8, F.bfyx, cl.tensor(n, 64, 64, 64))
+    busy = cl.network(eng, cl.topology(cl.input_layout("x", lay), *[cl.reorder(f"r{i}", f"r{i - 1}" if i else "x", F.yxfb if i % 2 == 0 else F.bfyx)
+                                                                   for i in range(41)]))
+    busy.set_input_data("x", cl.make_memory(eng, np.zeros((n, 64, 64, 64), np.int8)))
+    busy.execute()["r40"].get_event().wait()
+    small = cl.layout(DT.i8, F.bfyx, cl.tensor(1, 16, 8, 8))
+    net = cl.network(eng, cl.topology(cl.input_layout("a", small), cl.reorder("ra", "a", F.yxfb), cl.input_layout("b", small),
+                                      cl.reorder("rb", "b", F.yxfb), cl.eltwise("sum", "ra", "rb", cl.eltwise_mode.sum)))
+    x = np.arange(1024, dtype=np.int64).astype(np.int8).reshape(1, 16, 8, 8)
+    mem = cl.make_memory(eng, x)
+    net.set_input_data("a", mem)
+    ev = busy.execute()["r40"].get_event()  # work of milliseconds in front of the failing run's
+    with pytest.raises(cl.error, match="input b"):
+        net.execute()
+    fired = []
+    cb = cl.EVENT_HANDLER(lambda p: fired.append(1))
+    cl._call("cldnn_add_event_handler", ev.h, cb, None)
+    assert fired == [1]  # at once: everything on the stream is complete
+    mem.write(x)
+    net.set_input_data("b", mem)
+    np.testing.assert_array_equal(net.execute()["sum"].get_memory().read(), rc.eltwise([x, x], "sum"))
