@@ -270,6 +270,7 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
         tap_reset(walk);  // the last D steps request the first D steps of the next granule
 #pragma unroll
         for (int d = 0; d < D; ++d) step(a.ksteps0 - D + d, d, nxt);
+        mfma_settle(acc0);
 
         // requantise stage 0: the packed results ARE the B fragments of stage 1 (K-step = span)
         v4i bf0[SP0][NT];

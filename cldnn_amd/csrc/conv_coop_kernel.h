@@ -168,22 +168,20 @@ __global__ void __launch_bounds__(512, 4) conv_coop_kernel(CoopConvArgs a)
 
     for (int g = g_begin; g < g_end; ++g) {
         // ---------------- stage 0: this wave's K-steps of all features
-        v4i acc0[N0];
+        v4i acc0[1][N0];
 #pragma unroll
-        for (int i = 0; i < N0; ++i) acc0[i] = none;
+        for (int i = 0; i < N0; ++i) acc0[0][i] = none;
 #pragma unroll
         for (int r0 = 0; r0 < R0; ++r0) {
             if (wave + r0 * W < TAPS) {
                 const v4i x = {flip(xb[r0][0], s0.xor_mask), flip(xb[r0][1], s0.xor_mask), flip(xb[r0][2], s0.xor_mask), flip(xb[r0][3], s0.xor_mask)};
 #pragma unroll
-                for (int i = 0; i < N0; ++i) acc0[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0[r0][i], x, acc0[i], 0, 0, 0);
+                for (int i = 0; i < N0; ++i) acc0[0][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0[r0][i], x, acc0[0][i], 0, 0, 0);
             }
         }
-        step_fence();
+        mfma_settle(acc0);
 #pragma unroll
-        for (int i = 0; i < N0; ++i) mfma_settle(acc0[i]);
-#pragma unroll
-        for (int i = 0; i < N0; ++i) part[(wave * N0 + i) * 64 + lane] = acc0[i];
+        for (int i = 0; i < N0; ++i) part[(wave * N0 + i) * 64 + lane] = acc0[0][i];
         const bool more = g + 1 < g_end;
         if (more) request(g + 1, nxt);
         lds_barrier();
@@ -227,9 +225,6 @@ __global__ void __launch_bounds__(512, 4) conv_coop_kernel(CoopConvArgs a)
             v4i acc2[N0];
 #pragma unroll
             for (int i = 0; i < N0; ++i) acc2[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w2[i], bf, none, 0, 0, 0);
-            step_fence();
-#pragma unroll
-            for (int i = 0; i < N0; ++i) mfma_settle(acc2[i]);
 #pragma unroll
             for (int i = 0; i < N0; ++i) part2[(wave * N0 + i) * 64 + lane] = acc2[i];
             lds_barrier();

@@ -176,9 +176,9 @@ __global__ void __launch_bounds__(512) conv_dwcoop_kernel(DwCoopArgs a)
                                                                                      + sp * 4 * a.el_pf + mt * 4));
             }
         }
-        v4i acc1[SP1 * 4];
+        v4i acc1[1][SP1 * 4];
 #pragma unroll
-        for (int i = 0; i < SP1 * 4; ++i) acc1[i] = v4i{0, 0, 0, 0};
+        for (int i = 0; i < SP1 * 4; ++i) acc1[0][i] = v4i{0, 0, 0, 0};
         const v4i none = {0, 0, 0, 0};
         for (int ks = wave; ks < a.KS; ks += W) {
             // ---------------- depthwise: 64 features of the granule's pixels
@@ -208,16 +208,14 @@ __global__ void __launch_bounds__(512) conv_dwcoop_kernel(DwCoopArgs a)
             // ---------------- its share of the projection
             const v4i bf = packed ^ v4i{(int)s1.xor_mask, (int)s1.xor_mask, (int)s1.xor_mask, (int)s1.xor_mask};
 #pragma unroll
-            for (int i = 0; i < SP1 * 4; ++i) acc1[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(u1[i], bf, acc1[i], 0, 0, 0);
+            for (int i = 0; i < SP1 * 4; ++i) acc1[0][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(u1[i], bf, acc1[0][i], 0, 0, 0);
             request(ks + W, ks + W < a.KS);
         }
         if constexpr (HAS2)
             request2(wave, wave < a.SP2);  // on its way while the waves exchange
-        step_fence();
+        mfma_settle(acc1);
 #pragma unroll
-        for (int i = 0; i < SP1 * 4; ++i) mfma_settle(acc1[i]);
-#pragma unroll
-        for (int i = 0; i < SP1 * 4; ++i) part[(wave * SP1 * 4 + i) * 64 + lane] = acc1[i];
+        for (int i = 0; i < SP1 * 4; ++i) part[(wave * SP1 * 4 + i) * 64 + lane] = acc1[0][i];
         lds_barrier();
 
         // ---------------- projection: fragment i = (span, mt) of the sum, four features of a lane

@@ -176,11 +176,7 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
             if (d < rest) mma(ra[d], rb[d]);
     }
 
-    step_fence();
-#pragma unroll
-    for (int f = 0; f < FT; ++f)
-#pragma unroll
-        for (int p = 0; p < PT; ++p) mfma_settle(acc[f][p]);
+    mfma_settle(acc);
 
     // ---- partial sums; wave w < FT * PT finishes fragment (w % FT, w / FT)
     constexpr int TILE = FT * PT * 64;

@@ -117,10 +117,21 @@ __device__ __forceinline__ void lds_barrier()
 // look-ahead queue once per loop iteration.
 __device__ __forceinline__ void step_fence() { __builtin_amdgcn_sched_barrier(0); }
 
-// Accumulators may be read from here on.  The compiler inserts the idle slots between a matrix instruction and a reader of
-// its result, but where the last one stands under a branch of its own it has been seen to count them along the longer path
-// only.
-__device__ __forceinline__ void mfma_settle(v4i& acc) { asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc)); }
+// Accumulators may be read from here on.  A v_mfma_i32_16x16x64_i8 takes eight wait states until its result may be read (the
+// 32x32x32 form twelve), which the compiler counts and fills up.  Where paths of different lengths lead from the matrix
+// instruction to the reader it counts along one of them only, and the shorter one may come out with fewer.  So: where a branch
+// may stand between the last matrix instruction and the first reader (a wave-uniform condition around it, the tap walk behind
+// it), the accumulators are settled; where the two are in straight line they need not be.  Tied to all accumulators before and
+// after, so that neither side moves across the idle slots.
+template <int N, int M>
+__device__ __forceinline__ void mfma_settle(v4i (&acc)[N][M])
+{
+#pragma unroll
+    for (int i = 0; i < N * M; ++i) asm volatile("" : "+v"(acc[i / M][i % M]));
+    asm volatile("s_nop 7");
+#pragma unroll
+    for (int i = 0; i < N * M; ++i) asm volatile("" : "+v"(acc[i / M][i % M]));
+}
 
 // Instruction order inside one K-step: after each of the M matrix instructions (16 clocks in the matrix pipe, 4 to
 // issue) the scheduler is told to place a share of the step's other work -- R LDS reads, W LDS writes, V global
@@ -1293,6 +1304,7 @@ __global__ void __launch_bounds__(256) conv_wsl_kernel(MfmaArgs a)
         tap_reset(walk);
 #pragma unroll
         for (int d = 0; d < D; ++d) step(a.ksteps - D + d, d, nxt);
+        mfma_settle(acc);
         load_residual(nxt, ev_nxt);
 
 #pragma unroll
