@@ -813,7 +813,6 @@ class network:  # noqa: N801
         self.h = _call("cldnn_build_network", eng.h, topo.h, carr, n)
         self._engine, self._topology = eng, topo
         self._outputs = None  # fixed by the build: names, encoded names, what is known of the layouts
-        self._output_layouts = {}  # so are the layouts
 
     def set_input_data(self, prim_id, mem):
         _call("cldnn_set_network_input", self.h, prim_id.encode(), mem.h)

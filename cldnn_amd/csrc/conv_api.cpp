@@ -500,11 +500,11 @@ cldnn_hip_status cldnn_hip_conv_chain_create(cldnn_hip_engine e, int32_t count, 
                                       wqf ? wqf[k] : nullptr};
             }
             chain_pack_weights(ch->in, ch->plan, cus, w8, vec, packed.data());
-            // The chain launches none of its stage objects (they never leave this file): their own operand streams (packed weights, tap table, gather
-            // scratch) would only hold every chained layer's weights on the device a second time.
+            // The chain launches none of its stage objects (they never leave this file): their own operand streams (packed weights, depthwise rows, tap
+            // table, gather scratch) would only hold every chained layer's weights on the device a second time.
             for (int k = 0; k < count; ++k) {
                 cldnn_hip_conv c = ch->stage[k];
-                for (void** buf : {&c->w_packed, &c->ktab, &c->gather}) {
+                for (void** buf : {&c->w_packed, &c->w_rows, &c->ktab, &c->gather}) {
                     if (!*buf) continue;
                     c->owned.erase(std::remove(c->owned.begin(), c->owned.end(), *buf), c->owned.end());
                     CHIP_CHECK(hipFree(*buf));

@@ -173,7 +173,6 @@ static int choose_ksplit(int64_t m, int ofm, int taps, int cb, int ksteps, bool 
 }
 
 static int choose_row(const ConvProblem& p, int cus);
-static int choose_row(const ConvProblem& p, int cus);
 static void wsl_depth(int ksteps, int* depth, int* padded);
 // Microseconds of a row on an arbitrary shape with a border: start + K-steps * time of a step + output bytes.  A step takes
 // its latency (`step`) or, with several workgroups on a CU, its throughput (`load` times the workgroups per CU), whichever

@@ -1072,8 +1072,6 @@ static void pair_siblings(cldnn_program_impl* prog)
 }
 
 // One convolution object for a pair.  false: the kernels have no short form for this pair (the pair is taken apart).
-static bool compile_siblings(cldnn_program_impl* prog, node* a);
-
 static bool compile_siblings(cldnn_program_impl* prog, node* a)
 {
     node* b = a->sibling;
