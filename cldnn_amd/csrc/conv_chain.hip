@@ -116,8 +116,8 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
         }
         pl.ksteps0 = pl.sp[0];  // K-steps the depthwise stage delivers to stage 1
         // Small planes: the waves of a workgroup share a granule.  Up to two granules per CU that beats one granule per wave with
-        // the weights in LDS (14x14, 384 mid features: 6.5 us against 14.9 at batch 16, 11.2 against 14.9 at batch 32, but 20
-        // against 17 at batch 64) and separate launches where that form does not apply, from two K-steps on (a single one
+        // the weights in LDS (14x14, 384 mid features: 6.2 us against 12.9 at batch 16, 10.3 against 13.2 at batch 32, but 16.9
+        // against 14.0 at batch 64) and separate launches where that form does not apply, from two K-steps on (a single one
         // occupies one wave of four).
         const bool block = pl.epi[0] == EPI_KIND_CLAMPQ && (pl.epi[1] == EPI_KIND_LINEAR || pl.epi[1] == EPI_KIND_SUMLIN)
                            && (n < 3 || pl.epi[2] == EPI_KIND_CLAMPQ) && !st[1].fe->split_valid;

@@ -9,9 +9,10 @@
 //   - stage 2 is split over its K again, which is where each wave's own expansion features are: they never leave its
 //     registers, only the partial sums do.
 // All weights (56 registers), the residual and the input of the next granule are requested long before they are needed, so
-// a granule costs three barriers and its instructions.  56x56, 64 mid features, batch 1: 11.0-12.5 -> 6.8-7.4 us with three
-// stages, 28x28 with two 11.4 -> 4.4.  Two stages are faster at every size (batch 128: 32.6 -> 27.4); three stages with
-// many granules are not, splitting costs more instructions per pixel: equal at 813 granules, 27 against 44 us at batch 32.
+// a granule costs three barriers and its instructions.  Kernel time, 56x56, 64 mid features, batch 1: 10.7 -> 6.2 us with three
+// stages, 28x28 with two 9.5 -> 4.0.  Inside a network, where the input comes from memory, two stages are faster at every
+// size (ResNet-50 at batch 32 12.7 -> 10.8, at batch 128 33.1 -> 29.0; repeated on warm caches 24.8 and 25.5); three stages
+// with many granules are not, splitting costs more instructions per pixel: equal at 813 granules, 26 against 43 us at batch 32.
 // 128 mid features (weights in 160 registers) gained 2 us of 12 at batch 1 and lost 8 of 28 at batch 32.
 #pragma once
 #include "conv_chain_kernel.h"

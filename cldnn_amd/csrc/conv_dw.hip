@@ -188,8 +188,8 @@ __global__ void __launch_bounds__(256) conv_dw3x3_kernel(DwArgs a)
 // against 25 and 400.  At that rate memory is the bound of large planes; a wave keeps its table in registers for `rounds`
 // sets of 64 pixels and requests the next set before it finishes the present one.  Small planes are bound by the launch and
 // the latency of one set.
-// 32 x 576 x 14x14, 3x3: 6.3 -> 5.0 us (1.4 us at the rate of a large copy and about 3 of launch); 8 x 512 x 28x28, 5x5:
-// 30.8 -> 6.0; 32 x 64 x 112x112, 5x5: 137 -> 24 (10.3 at the rate of a large copy), 3x3: 18.9 -> 17.9.
+// Kernel time, 32 x 576 x 14x14, 3x3: 6.3 -> 5.3 us (1.4 us at the rate of a large copy and about 3 of launch); 8 x 512 x 28x28,
+// 5x5: 32.4 -> 6.5; 32 x 64 x 112x112, 5x5: 143 -> 26 (10.3 at the rate of a large copy), 3x3: 22.7 -> 18.4.
 template <int FY, int NB, int EPI>
 __global__ void __launch_bounds__(256, 2) conv_dw_rows_kernel(DwArgs a)
 {

@@ -20,8 +20,8 @@
 // Work split as in the dense chain: persistent workgroups of four independent waves, granules of 16 pixels, the
 // activations of the next unit (also across granules) requested while the present one is multiplied, all weights and
 // per-feature vectors in LDS.
-// MobileNet v2 at batch 32, before (spans of 64, one tap per product) and now: 112x112 32-16-96 43.7 -> 28.6 us, 112x112
-// 96-24-144 25.0 -> 18.6, 56x56 144-24-144 30.2 -> 21.2, 28x28 192-32-192 12.9 -> 10.0.
+// MobileNet v2 at batch 32, kernel time before (spans of 64, one tap per product) and now: 112x112 32-16-96 47.1 -> 30.0 us,
+// 112x112 96-24-144 25.1 -> 18.1, 56x56 144-24-144 31.4 -> 22.1, 28x28 192-32-192 13.0 -> 9.8.
 #pragma once
 #include <type_traits>
 

@@ -2,7 +2,7 @@
 //
 // With one granule per wave a 14x14 layer of batch 32 occupies 104 of 256 CUs, and the granule's whole chain -- six K-steps
 // of nine taps, their requantisation, the projection, six spans of the expansion -- is one serial walk of one wave, behind
-// a copy of 100 KB of weights into LDS: 16 us at batch 32, 15 us at batch 1, more than three separate launches take.  What
+// a copy of 100 KB of weights into LDS: 12.4 us at batch 1, 13.2 at batch 32, about what three separate launches take.  What
 // bounds it is the number of memory round trips in a row, so here
 //   - a wave takes the K-steps wave, wave + W, ... of the depthwise stage and multiplies each result with its share of the
 //     projection's K at once; the partial sums of the projection (all there is to exchange: 4 KB per wave and 64 features)
@@ -12,8 +12,9 @@
 //     the registers the matrix instructions read; the per-feature vectors (up to 30 KB) go to LDS meanwhile;
 //   - the arguments are what the two forms of a MobileNet block need and fit into the scalar registers: the general
 //     structures took eight loads in a row, 2.4 us, before the first request went out.
-// 14x14, 384 mid features: 16.0 -> 6.6 us at batch 1, 16.4 -> 11.5 at batch 32; and it takes the blocks whose weights do not
-// fit into LDS: 14x14, 576 mid features 12.3 -> 9.6 us at batch 1 (three launches before), 7x7, 960 at batch 32 14.6 -> 12.3.
+// Kernel time, 14x14, 384 mid features: 12.4 -> 5.9 us at batch 1, 13.2 -> 10.3 at batch 32; and it takes the blocks whose weights
+// do not fit into LDS: 14x14, 576 mid features 10.8 -> 7.9 us at batch 1 (the sum of three launches before, without their
+// gaps), 7x7, 960 at batch 32 14.2 -> 10.7.
 //
 // Projection weights are requested when the taps have been multiplied and nothing is fetched for the next granule ahead of
 // time: 164 registers (64-feature projection) let a CU hold twelve waves, which is worth more than the look-ahead (221

@@ -2,7 +2,7 @@
 //
 // A network at batch 1, the late layers of any network, a fully_connected: the tile kernels give such a layer 8 to 100
 // workgroups whose four waves walk all of K one step at a time, 0.2-0.25 us a step, while most of the chip idles (7x7
-// 512 -> 512 3x3 at batch 1: 8 workgroups, 72 steps, 12.0 us; here 5.2).  What bounds the layer is the length of that
+// 512 -> 512 3x3 at batch 1: 8 workgroups, 72 steps, 10.3 us of kernel time; here 4.5).  What bounds the layer is the length of that
 // walk, so here a workgroup owns a small tile (16 .. 64 pixels x 16 .. 64 features) and its 4, 8 or 16 waves take a share
 // of the K-steps each: both operands go straight from global memory into the registers the matrix instruction reads, D
 // steps ahead, no LDS and no barrier in the loop.  With K shared out a wave has 1 to 5 steps and usually requests all its
