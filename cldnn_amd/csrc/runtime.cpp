@@ -95,7 +95,6 @@ void cldnn_hip_buffer_s::upload()
 {
     engine->make_current();
     CHIP_CHECK(hipMemcpyAsync(dev, shadow, bytes, hipMemcpyHostToDevice, engine->stream));
-    uploaded = engine->mark();
 }
 
 void cldnn_hip_engine_s::make_current() const { CHIP_CHECK(hipSetDevice(device)); }
@@ -422,10 +421,13 @@ cldnn_hip_status cldnn_hip_buffer_unmap(cldnn_hip_buffer b)
         b->newest = cldnn_hip_buffer_s::HOST, b->read_in_place = false;
         // What no kernel will read in place starts its way to the device now, beside whatever the host does before it enqueues
         // the work that needs it (19 MB of images: 0.4 ms).  Not a result: the host has only looked at it.
-        if (b->bytes > READ_IN_PLACE_BYTES && !b->is_result) {
-            b->upload();
-            b->newest = cldnn_hip_buffer_s::BOTH;
-        }
+        if (b->bytes <= READ_IN_PLACE_BYTES || b->is_result) return;
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        CHIP_CHECK(hipStreamIsCapturing(b->engine->stream, &capture));
+        if (capture != hipStreamCaptureStatusNone) return;  // a copy recorded now is not made now
+        b->upload();
+        b->uploaded = b->engine->mark();
+        b->newest = cldnn_hip_buffer_s::BOTH;
     });
 }
 

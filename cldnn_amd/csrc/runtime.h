@@ -48,10 +48,10 @@ struct cldnn_hip_buffer_s {
     copy_state newest = DEVICE;
     bool read_in_place = false;  // since the host wrote the shadow a kernel has read it where it is
     bool is_result = false;      // the last use wrote it: what the host maps it for is most likely to read it
-    uint64_t uploaded = 0;       // the engine's mark behind the last copy out of the shadow
+    uint64_t uploaded = 0;       // the engine's mark behind the last copy that an unmap started
 
     void need_shadow();
-    void upload();  // shadow -> device on the engine's stream, not waited for (`uploaded`)
+    void upload();  // shadow -> device on the engine's stream, not waited for
 };
 
 struct cldnn_hip_event_s {

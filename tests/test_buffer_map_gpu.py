@@ -160,3 +160,22 @@ def test_large_input_is_copied_from_the_unmap_on():
     assert (dst.read_raw() == 1).all()
     hip.check(L.cldnn_hip_event_release(old))
     src.close(), dst.close(), eng.close()
+
+
+def test_unmap_while_the_stream_is_captured_records_nothing():
+    eng, L = hip.Engine(0), hip.lib()
+    t = hip.Tensor.make(hip.U8, hip.BFYX, 1, 1 << 12, 1, 1031)
+    src, dst = hip.Buffer(eng, t), hip.Buffer(eng, t)
+    stream = C.c_void_p(L.cldnn_hip_engine_stream(eng.h))
+    eng.finish()
+    mapped(src)[:] = 0x33
+    graph, nodes = C.c_void_p(), C.c_size_t(99)
+    assert L.hipStreamBeginCapture(stream, 2) == 0  # relaxed
+    status = L.cldnn_hip_buffer_unmap(src.h)
+    assert L.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    hip.check(status)
+    assert L.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0 and nodes.value == 0
+    assert L.hipGraphDestroy(graph) == 0
+    copy(eng, src, READ, dst, WRITE)
+    assert (dst.read_raw() == 0x33).all()
+    src.close(), dst.close(), eng.close()
