@@ -8,7 +8,7 @@
 //     projection's K at once; the partial sums of the projection (all there is to exchange: 4 KB per wave and 64 features)
 //     meet in LDS, every wave finishes a fragment, the packed projection goes back through LDS (1 KB), and every wave
 //     computes the spans wave, wave + W, ... of the expansion;
-//   - weights are not staged: a wave needs only its own K-steps (17 KB each) and requests them with its taps, straight into
+//   - weights are not staged: a wave needs only its own K-steps (5 to 13 KB each) and requests them with its taps, straight into
 //     the registers the matrix instructions read; the per-feature vectors (up to 30 KB) go to LDS meanwhile;
 //   - the arguments are what the two forms of a MobileNet block need and fit into the scalar registers: the general
 //     structures took eight loads in a row, 2.4 us, before the first request went out.
@@ -21,7 +21,7 @@
 // registers: 20 us instead of 15 for 28x28 at batch 32).
 //
 // The depthwise weights are a dword per tap and lane here, the four features of the lane's rows of the diagonal, [K-step][lane
-// % 16][12 taps]; a byte permute moves each into its fragment.  The table of the other kernel has them spread out: 9 KB a
+// % 16][12 taps]; a byte permute moves each into its fragment.  Spread out over the lanes they would be 9 KB a
 // K-step instead of 768 bytes, and with a granule or two on the chip what one CU fetches is the time (touching the 1x1
 // weights' lines early, to have them nearer, made 7x7 blocks slower: 12.4 -> 15.4 us).
 #pragma once
