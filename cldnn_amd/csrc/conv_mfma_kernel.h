@@ -121,13 +121,13 @@ __device__ __forceinline__ void step_fence() { __builtin_amdgcn_sched_barrier(0)
 // 32x32x32 form twelve), which the compiler counts and fills up.  Where paths of different lengths lead from the matrix
 // instruction to the reader it counts along one of them only, and the shorter one may come out with fewer.  So: where a branch
 // may stand between the last matrix instruction and the first reader (a wave-uniform condition around it, the tap walk behind
-// it), the accumulators are settled; where the two are in straight line they need not be.  Tied to all accumulators before and
-// after, so that neither side moves across the idle slots.
+// it), the accumulators are settled; where the two are in straight line they need not be.  Read by empty statements before and tied
+// to others behind, so that neither side moves across the idle slots.
 template <int N, int M>
 __device__ __forceinline__ void mfma_settle(v4i (&acc)[N][M])
 {
 #pragma unroll
-    for (int i = 0; i < N * M; ++i) asm volatile("" : "+v"(acc[i / M][i % M]));
+    for (int i = 0; i < N * M; ++i) asm volatile("" ::"v"(acc[i / M][i % M]));
     asm volatile("s_nop 7");
 #pragma unroll
     for (int i = 0; i < N * M; ++i) asm volatile("" : "+v"(acc[i / M][i % M]));
