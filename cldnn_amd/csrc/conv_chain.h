@@ -32,6 +32,8 @@ struct ChainPlan {
     int unit0[3], kstride[3];  // LDS image: first 4 KB unit and units per span of every stage
     int vec0[3];               // first dword of every stage's per-feature vectors behind the weights
     int units;
+    int dwc_w1, dwc_w2, dwc_v0, dwc_v1, dwc_v2;  // shared depthwise form: parts of its image, bytes
+    int dwc_parts;             // workgroups that share the expansion of a granule
     int img_bytes;             // weights and per-feature vectors on the device
     int lds_bytes;
     int grid;

@@ -115,35 +115,45 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
             vec += 4 * pl.sp[k] * 64;
         }
         pl.ksteps0 = pl.sp[0];  // K-steps the depthwise stage delivers to stage 1
-        // Small planes: the waves of a workgroup share a granule.  Up to two granules per CU that beats one granule per wave with
-        // the weights in LDS (14x14, 384 mid features: 6.2 us against 12.9 at batch 16, 10.3 against 13.2 at batch 32, but 16.9
-        // against 14.0 at batch 64) and separate launches where that form does not apply, from two K-steps on (a single one
-        // occupies one wave of four).
+        // The waves of a workgroup share a granule where granules are few, from two K-steps on (a single one occupies one wave
+        // of four).  Against one granule per wave with the weights in LDS, and separate launches where that form does not apply:
+        // 14x14, 384-64-384 11.1 -> 6.9 us at 392 granules, 16.2 -> 14.6 at 784, but 19.2 -> 26.7 at 1568; 576-96-576 (only
+        // separate launches otherwise) 27.3 -> 19.3 us at 784 granules and 40 -> 34.6 at 1568.  Fewer K-steps: two granules a CU.
+        // Wide projections are taken up to the K-steps and spans whose partial sums and vectors would fit into LDS: beyond, a
+        // wave walks over two K-steps and more.
         const bool block = pl.epi[0] == EPI_KIND_CLAMPQ && (pl.epi[1] == EPI_KIND_LINEAR || pl.epi[1] == EPI_KIND_SUMLIN)
                            && (n < 3 || pl.epi[2] == EPI_KIND_CLAMPQ) && !st[1].fe->split_valid;
-        const bool small = (pl.m_total + 15) / 16 <= 2ll * cus;
-        const int waves = pl.ksteps0 <= 8 ? std::max(4, pl.ksteps0) : std::min(8, (pl.ksteps0 + 1) / 2);
-        const int shared_lds = (waves * 4 + 1) * pl.sp[1] * 1024 + vec * 4;
-        const bool shared = block && small && pl.ksteps0 >= 2 && shared_lds <= CHAIN_MAX_LDS;
+        const bool small = (pl.m_total + 15) / 16 <= (int64_t)cus * (pl.ksteps0 < 6 ? 2 : (pl.sp[1] == 1 ? 4 : 8));
+        const int deep = pl.ksteps0 <= 8 ? std::max(4, pl.ksteps0) : std::min(8, (pl.ksteps0 + 1) / 2);
+        const bool shared = block && small && pl.ksteps0 >= 2 && (deep * 4 + 1) * pl.sp[1] * 1024 + vec * 4 <= CHAIN_MAX_LDS;
         // (the other form has two units of 32 features of projection at most)
         if (pl.sp[1] > 1 && !shared)
             return "stage 1: a projection of more than 64 features is chained in the forms of a MobileNet block, on small planes and from 65 mid "
                    "features on only, where partial sums and vectors fit into LDS";
+        for (int k = 0; k < n; ++k) pl.u32[k] = (st[k].p->OFM + 31) / 32;
         if (shared) {
             pl.coop = 1, pl.nt = 1;
-            pl.img_bytes = pl.sp[0] * DWCOOP_KS_BYTES + pl.units * 4096 + vec * 4;
-            pl.waves = waves;
-            pl.granules = (int)((pl.m_total + 15) / 16);
-            pl.lds_bytes = shared_lds;
-            const int per_cu = std::max(1, std::min((pl.sp[1] == 1 ? 12 : 8) / pl.waves, CHAIN_MAX_LDS / pl.lds_bytes));
-            pl.grid = std::min(cus * per_cu / 8 * 8, (pl.granules + 7) / 8 * 8);
-            std::snprintf(pl.name, sizeof(pl.name), "conv_dwchain<%d stages,p16 shared by %d waves,mid %d,spans %d-%d>", n, pl.waves, p0.OFM, pl.sp[1],
-                          n > 2 ? pl.sp[2] : 0);
+            const int frags = 2 * pl.u32[1], k1 = pl.sp[1], sp2 = n > 2 ? pl.sp[2] : 0;
+            pl.dwc_w1 = 2 * pl.ksteps0 * DWCOOP_UNIT_BYTES, pl.dwc_w2 = pl.dwc_w1 + pl.ksteps0 * frags * 1024;
+            pl.dwc_v0 = pl.dwc_w2 + k1 * sp2 * 4096, pl.dwc_v1 = pl.dwc_v0 + pl.ksteps0 * DWCOOP_VEC0_BYTES;
+            pl.dwc_v2 = pl.dwc_v1 + frags * DWCOOP_VEC1_BYTES;
+            pl.img_bytes = pl.dwc_v2 + sp2 * DWCOOP_VEC0_BYTES;
+            // a wave for every K-step and every fragment of the projection
+            pl.waves = std::min((int)DWCOOP_MAX_WAVES, std::max(4, std::max(pl.ksteps0, frags)));
+            // two granules to a workgroup cost 1.3 us more than one (the weights are fetched once), which pays where the
+            // workgroups of one would not all be resident: 576-96-576 at 392 granules 12.3 -> 10.3 us, 384-64-384 6.8 -> 8.1
+            pl.nt = pl.granules > cus * (DWCOOP_MAX_WAVES / pl.waves) && pl.ksteps0 <= 9 && pl.waves <= 10 ? 2 : 1;
+            pl.granules = (int)((pl.m_total + 16 * pl.nt - 1) / (16 * pl.nt));
+            pl.lds_bytes = pl.nt * (pl.ksteps0 + k1) * 1024 + pl.waves * DWCOOP_OWN * 16;
+            // up to four (more change nothing): 576-160-960 at four granules 8.4 -> 6.7 us, 960-160-960 8.9 -> 8.4
+            pl.dwc_parts = std::max(1, std::min(std::min(sp2, 4), cus / pl.granules));
+            pl.grid = (pl.granules * pl.dwc_parts + 7) / 8 * 8;
+            std::snprintf(pl.name, sizeof(pl.name), "conv_dwchain<%d stages,p%d shared by %d waves,mid %d,spans %d-%d,parts %d>", n, 16 * pl.nt, pl.waves, p0.OFM, pl.sp[1],
+                          sp2, pl.dwc_parts);
             *out = pl;
             return std::string();
         }
         // units of 32 features (conv_dwchain_kernel.h)
-        for (int k = 0; k < n; ++k) pl.u32[k] = (st[k].p->OFM + 31) / 32;
         pl.units = pl.u32[0] + 2 * ((pl.u32[0] + 1) / 2 * pl.u32[1] + (n > 2 ? pl.u32[2] : 0));  // kilobytes of weights
         pl.lds_bytes = pl.img_bytes = pl.units * 1024 + vec * 4;
         if (pl.lds_bytes > CHAIN_MAX_LDS) return "the weights of the chain (" + std::to_string(pl.lds_bytes / 1024) + " KiB) do not fit into LDS";
@@ -247,9 +257,7 @@ static void launch_dwcoop(hipStream_t s, const ChainStageIn* st, const ChainPlan
     const ConvProblem& p1 = *st[1].p;
     DwCoopArgs a{};
     a.in = (const int8_t*)in, a.img = (const int8_t*)packed_dev, a.eltw = eltws ? (const int8_t*)eltws[1] : nullptr;
-    a.unit_bytes = pl.sp[0] * DWCOOP_KS_BYTES;
-    a.vec_bytes = a.unit_bytes + pl.units * 4096;
-    a.vec_quads = (pl.img_bytes - a.vec_bytes) / 16;
+    a.w1 = pl.dwc_w1, a.w2 = pl.dwc_w2, a.v0 = pl.dwc_v0, a.v1 = pl.dwc_v1, a.v2 = pl.dwc_v2;
     a.el_off = (int32_t)p1.eltw_p.off, a.el_pb = (int32_t)p1.eltw_p.pb, a.el_pf = (int32_t)p1.eltw_p.pf;
     a.el_py = (int32_t)p1.eltw_p.py * p1.esy, a.el_px = 16 * p1.esx;
     a.M = (uint32_t)pl.m_total;
@@ -258,9 +266,9 @@ static void launch_dwcoop(hipStream_t s, const ChainStageIn* st, const ChainPlan
     a.in_off = (int32_t)p0.in_p.off - p0.py * (int32_t)p0.in_p.py - p0.px * 16;
     a.in_pb = (int32_t)p0.in_p.pb, a.in_pf = (int32_t)p0.in_p.pf;
     a.row = p0.sy * (int32_t)p0.in_p.py, a.col = p0.sx * 16, a.tap_dy = (int32_t)p0.in_p.py;
-    a.CB = (p0.OFM + 15) / 16, a.KS = pl.sp[0], a.SP2 = pl.stages > 2 ? pl.sp[2] : 0, a.waves = pl.waves;
-    a.gpw = pl.granules / pl.grid, a.grem = pl.granules % pl.grid;
-    a.div_parts = make_fast_div((uint32_t)pl.grid);
+    a.CB = (p0.OFM + 15) / 16, a.KS = pl.ksteps0, a.F1 = 2 * pl.u32[1], a.SP2 = pl.stages > 2 ? pl.sp[2] : 0;
+    a.waves = pl.waves, a.parts = pl.dwc_parts;
+    a.div_parts = make_fast_div((uint32_t)pl.dwc_parts);
     const FastEpi &f0 = *st[0].fe, &f1 = *st[1].fe;
     const bool sum = pl.epi[1] == EPI_KIND_SUMLIN;
     CHIP_REQUIRE(!sum || a.eltw, CLDNN_HIP_INVALID_ARG, "fused stage of a chain without its second input");
@@ -274,16 +282,23 @@ static void launch_dwcoop(hipStream_t s, const ChainStageIn* st, const ChainPlan
         c.out = (int8_t*)outs[k];
         c.off = (int32_t)p.out_p.off, c.pb = (int32_t)p.out_p.pb, c.pf = (int32_t)p.out_p.pf, c.py = (int32_t)p.out_p.py;
         c.ofm = p.OFM, c.xor_mask = p.in_dt == CLDNN_HIP_U8 ? 0x80808080u : 0u;
-        c.unit0 = pl.unit0[k], c.kstride = pl.kstride[k], c.vec0 = pl.vec0[k];
     }
-#define DWCOOP_LAUNCH(SP1)                                                                    \
-    {                                                                                         \
-        if (pl.stages > 2 && sum) launch_dwcoop_instance<SP1, true, true>(s, a, pl.grid, pl.lds_bytes);   \
-        else if (pl.stages > 2) launch_dwcoop_instance<SP1, true, false>(s, a, pl.grid, pl.lds_bytes);    \
-        else if (sum) launch_dwcoop_instance<SP1, false, true>(s, a, pl.grid, pl.lds_bytes);  \
-        else launch_dwcoop_instance<SP1, false, false>(s, a, pl.grid, pl.lds_bytes);          \
+#define DWCOOP_LAUNCH(K1, KM, DEEP, NG)                                                                               \
+    {                                                                                                                 \
+        if (pl.stages > 2 && sum) launch_dwcoop_instance<K1, KM, DEEP, NG, true, true>(s, a, pl.grid, pl.lds_bytes);  \
+        else if (pl.stages > 2) launch_dwcoop_instance<K1, KM, DEEP, NG, true, false>(s, a, pl.grid, pl.lds_bytes);   \
+        else if (sum) launch_dwcoop_instance<K1, KM, DEEP, NG, false, true>(s, a, pl.grid, pl.lds_bytes);             \
+        else launch_dwcoop_instance<K1, KM, DEEP, NG, false, false>(s, a, pl.grid, pl.lds_bytes);                     \
     }
-    if (pl.sp[1] == 1) DWCOOP_LAUNCH(1) else if (pl.sp[1] == 2) DWCOOP_LAUNCH(2) else DWCOOP_LAUNCH(3)
+    // registers for the K-steps of a projection fragment: the next larger number compiled, or rounds
+    const int k1 = pl.sp[1];
+    if (pl.nt == 2) {
+        if (k1 == 1) DWCOOP_LAUNCH(1, 9, false, 2)
+        else if (k1 == 2) DWCOOP_LAUNCH(2, 9, false, 2) else DWCOOP_LAUNCH(3, 9, false, 2)
+    } else if (k1 == 1 && a.KS <= 3) DWCOOP_LAUNCH(1, 3, false, 1) else if (k1 == 1 && a.KS <= 6) DWCOOP_LAUNCH(1, 6, false, 1)
+    else if (k1 == 1 && a.KS <= 9) DWCOOP_LAUNCH(1, 9, false, 1) else if (k1 == 1) DWCOOP_LAUNCH(1, 9, true, 1) else if (k1 == 2 && a.KS <= 6) DWCOOP_LAUNCH(2, 6, false, 1)
+    else if (k1 == 2 && a.KS <= 9) DWCOOP_LAUNCH(2, 9, false, 1) else if (k1 == 2) DWCOOP_LAUNCH(2, 9, true, 1)
+    else if (a.KS <= 9) DWCOOP_LAUNCH(3, 9, false, 1) else if (a.KS <= 15) DWCOOP_LAUNCH(3, 15, false, 1) else DWCOOP_LAUNCH(3, 8, true, 1)
 #undef DWCOOP_LAUNCH
     CHIP_CHECK(hipGetLastError());
 }
@@ -377,20 +392,57 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
                         int8_t* packed)
 {
     std::memset(packed, 0, chain_packed_bytes(pl));
+    // feature of row r of fragment mt in a unit of 32, and of byte b of lane kq in (half h of) a K-step
+    auto row = [](int r, int mt) { return 16 * ((r >> 2) & 1) + 8 * (r >> 3) + 4 * mt + (r & 3); };
+    auto col = [](int kq, int b) { return 32 * (b >> 3) + 16 * (kq & 1) + 8 * (kq >> 1) + (b & 7); };
+    // fragments of a 1x1 stage behind a depthwise one: [K-step][unit][mt]
+    auto fragments = [&](int k, int ksteps, int units, int8_t* at) {
+        const int ofm = st[k].p->OFM, ifm = st[k].p->IFM;
+        for (int ks = 0; ks < ksteps; ++ks)
+            for (int u = 0; u < units; ++u)
+                for (int mt = 0; mt < 2; ++mt)
+                    for (int lane = 0; lane < 64; ++lane)
+                        for (int b = 0; b < 16; ++b, ++at) {
+                            const int f = u * 32 + row(lane & 15, mt), c = ks * 64 + col(lane >> 4, b);
+                            if (f < ofm && c < ifm) *at = w[k][(size_t)f * ifm + c];
+                        }
+        return at;
+    };
     if (pl.coop && pl.dw) {
-        // byte mt of dword (K-step, lane % 16, tap): feature 64 ks + 16 (l16 / 4) + 4 mt + l16 % 4
-        for (int ks = 0; ks < pl.sp[0]; ++ks)
-            for (int l16 = 0; l16 < 16; ++l16)
-                for (int tap = 0; tap < 9; ++tap)
-                    for (int mt = 0; mt < 4; ++mt) {
-                        const int ch = ks * 64 + 16 * (l16 >> 2) + 4 * mt + (l16 & 3);
-                        if (ch < st[0].p->OFM) packed[((ks * 16 + l16) * 12 + tap) * 4 + mt] = w[0][(size_t)ch * 9 + tap];
-                    }
-        packed += (size_t)pl.sp[0] * DWCOOP_KS_BYTES;
+        const int mid = st[0].p->OFM, sp2 = pl.stages > 2 ? pl.sp[2] : 0;
+        // byte (s / 2) * 4 + 2 (s % 2) + mt of (unit, tap half, row)
+        for (int u = 0; u < 2 * pl.ksteps0; ++u)
+            for (int half = 0; half < 2; ++half)
+                for (int r = 0; r < 16; ++r)
+                    for (int s5 = 0; s5 < DWCHAIN_STEPS; ++s5)
+                        for (int mt = 0; mt < 2; ++mt) {
+                            const int ch = u * 32 + row(r, mt), tap = 2 * s5 + half;
+                            if (ch < mid && tap < 9) packed[((size_t)(u * 2 + half) * 16 + r) * 16 + (s5 >> 1) * 4 + 2 * (s5 & 1) + mt] = w[0][(size_t)ch * 9 + tap];
+                        }
+        fragments(1, pl.ksteps0, pl.u32[1], packed + pl.dwc_w1);
+        if (sp2) fragments(2, pl.sp[1], 2 * sp2, packed + pl.dwc_w2);
+        // factors that are absent are one, or the output quantization factor
+        auto value = [&](int k, int kind, int f) {
+            const void* src[3] = {vec[k].acc_init, vec[k].calib, k == 1 ? vec[k].eltw_calib : vec[k].wqf};
+            const float fill = kind == 1 && st[k].epi->oqf_on ? st[k].epi->oqf : 1.0f;
+            int32_t bits = 0;
+            if (kind > 0) std::memcpy(&bits, &fill, 4);
+            if (src[kind] && f < st[k].p->OFM) std::memcpy(&bits, (const int32_t*)src[kind] + f, 4);
+            return bits;
+        };
+        for (int k = 0; k < pl.stages; k += 2) {
+            int32_t* v = reinterpret_cast<int32_t*>(packed + (k ? pl.dwc_v2 : pl.dwc_v0));
+            for (int sp = 0; sp < pl.sp[k]; ++sp)
+                for (int kind = 0; kind < 3; ++kind)
+                    for (int f = 0; f < 64; ++f) *v++ = value(k, kind, sp * 64 + f);
+        }
+        int32_t* v = reinterpret_cast<int32_t*>(packed + pl.dwc_v1);
+        for (int i = 0; i < 2 * pl.u32[1]; ++i)
+            for (int kind = 0; kind < 3; ++kind)
+                for (int kq = 0; kq < 4; ++kq)
+                    for (int j = 0; j < 4; ++j) *v++ = value(1, kind, (i >> 1) * 32 + row(kq * 4 + j, i & 1));
+        return;
     } else if (pl.dw) {
-        // feature of row r of fragment mt in a unit, and of byte b of lane kq in (half h of) a K-step
-        auto row = [](int r, int mt) { return 16 * ((r >> 2) & 1) + 8 * (r >> 3) + 4 * mt + (r & 3); };
-        auto col = [](int kq, int b) { return 32 * (b >> 3) + 16 * (kq & 1) + 8 * (kq >> 1) + (b & 7); };
         const int mid = st[0].p->OFM;
         for (int u = 0; u < pl.u32[0]; ++u)
             for (int lane = 0; lane < 64; ++lane)
@@ -400,19 +452,9 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
                         if (ch < mid && tap < 9) packed[((size_t)u * 64 + lane) * 16 + (s5 >> 1) * 4 + 2 * (s5 & 1) + mt] = w[0][(size_t)ch * 9 + tap];
                     }
         int8_t* at = packed + (size_t)pl.u32[0] * 1024;
-        for (int k = 1; k < pl.stages; ++k) {
-            const int ofm = st[k].p->OFM, ifm = st[k].p->IFM, ksteps = (pl.u32[k - 1] + 1) / 2;
-            for (int ks = 0; ks < ksteps; ++ks)
-                for (int u = 0; u < pl.u32[k]; ++u)
-                    for (int mt = 0; mt < 2; ++mt)
-                        for (int lane = 0; lane < 64; ++lane)
-                            for (int b = 0; b < 16; ++b, ++at) {
-                                const int f = u * 32 + row(lane & 15, mt), c = ks * 64 + col(lane >> 4, b);
-                                if (f < ofm && c < ifm) *at = w[k][(size_t)f * ifm + c];
-                            }
-        }
+        for (int k = 1; k < pl.stages; ++k) at = fragments(k, (pl.u32[k - 1] + 1) / 2, pl.u32[k], at);
     }
-    const size_t unit_bytes = (size_t)pl.units * (pl.dw && !pl.coop ? 1024 : 4096);
+    const size_t unit_bytes = (size_t)pl.units * (pl.dw ? 1024 : 4096);
     // per-feature vectors behind the weight units: per stage init, calib, eltw_calib, wqf, spans * 64 entries each
     int32_t* v = reinterpret_cast<int32_t*>(packed + unit_bytes);
     const float one = 1.0f;
@@ -430,9 +472,9 @@ void chain_pack_weights(const ChainStageIn* st, const ChainPlan& pl, int cus, co
             if (src[kind]) std::memcpy(dst, src[kind], (size_t)ofm * 4);
         }
     }
-    if (pl.dw && !pl.coop) return;
-    for (int k = pl.dw ? 1 : 0; k < pl.stages; ++k) {
-        const MfmaPlan mp = mfma_plan(*st[k].p, pl.dw ? ROW_P64_F64_FOR_DWCHAIN : ROW_WSL_P64_FOR_CHAIN, cus, true);
+    if (pl.dw) return;
+    for (int k = 0; k < pl.stages; ++k) {
+        const MfmaPlan mp = mfma_plan(*st[k].p, ROW_WSL_P64_FOR_CHAIN, cus, true);
         std::vector<int8_t> buf(mp.packed_bytes);
         std::vector<int32_t> ktab(mp.ktab_bytes / sizeof(int32_t));
         mfma_pack_weights(*st[k].p, mp, w[k], buf.data(), ktab.data());

@@ -164,7 +164,7 @@ __global__ void __launch_bounds__(512, 4) conv_coop_kernel(CoopConvArgs a)
 #pragma unroll
         for (int w = 0; w < W; ++w) sum[0] += o[w][0], sum[1] += o[w][1], sum[2] += o[w][2], sum[3] += o[w][3];
         const v4i acc4[4][1] = {{sum}, {none}, {none}, {none}};
-        return epilogue_fast16<1, RELU>(e, acc4, 0, cal, cal, cal, none, 16)[0];
+        return epilogue_fast16<1, RELU, 4>(e, acc4, 0, cal, cal, cal, none, 16)[0];
     };
 
     for (int g = g_begin; g < g_end; ++g) {
@@ -213,7 +213,7 @@ __global__ void __launch_bounds__(512, 4) conv_coop_kernel(CoopConvArgs a)
 #pragma unroll
             for (int d = 0; d < F1; ++d) ev4[d] = ev[d];
         }
-        const v4i packed1 = epilogue_fast16<1, EPI1>(e1, acc1, 0, cal, cal, ecal, ev4, 16);
+        const v4i packed1 = epilogue_fast16<1, EPI1, 8>(e1, acc1, 0, cal, cal, ecal, ev4, 16);
         if (s1.out && cur.ok)
             *reinterpret_cast<int2*>(s1.out + at(s1, cur, span1 * 4 + kq) + half * 8) = make_int2(packed1[0], packed1[1]);
         if (more) residual(nxt);

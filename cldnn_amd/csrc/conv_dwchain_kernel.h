@@ -157,7 +157,7 @@ __global__ void __launch_bounds__(256, EPI0 == EPI_KIND_FAST ? 2 : (P1 == 1 ? 4 
         if constexpr (EPI == EPI_KIND_FUSED || EPI == EPI_KIND_SUMLIN || EPI == EPI_KIND_FAST) vec8(st.vec0 + 2 * n + f0, ecal);
         if constexpr (EPI == EPI_KIND_CLAMPQ || EPI == EPI_KIND_FAST) vec8(st.vec0 + 3 * n + f0, wq);
         const v4i none = {0, 0, 0, 0}, acc4[4][1] = {{acc[0]}, {acc[1]}, {none}, {none}}, ev4 = {ev.x, ev.y, 0, 0};
-        const v4i p = epilogue_fast16<1, EPI>(st, acc4, 0, wq, cal, ecal, ev4, valid);
+        const v4i p = epilogue_fast16<1, EPI, EPI == EPI_KIND_CLAMPQ ? 8 : 16>(st, acc4, 0, wq, cal, ecal, ev4, valid);
         return make_int2(p[0], p[1]);
     };
     const std::integral_constant<int, EPI0> kind0{};

@@ -258,7 +258,7 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
             for (int i = 0; i < valid; ++i) dst[i] = v[i];
     } else {
         v4i acc4[4][1] = {{sum}, {v4i{0, 0, 0, 0}}, {v4i{0, 0, 0, 0}}, {v4i{0, 0, 0, 0}}};
-        const v4i packed = epilogue_fast16<1, EPI == EPI_KIND_POOL ? EPI_KIND_RELU : EPI>(a, acc4, 0, sc.wq, sc.cal, sc.ecal, ev4, valid);
+        const v4i packed = epilogue_fast16<1, EPI == EPI_KIND_POOL ? EPI_KIND_RELU : EPI, 4>(a, acc4, 0, sc.wq, sc.cal, sc.ecal, ev4, valid);
         int8_t* dst = (int8_t*)a.out + obase;
         if (a.out_f == 1) *reinterpret_cast<int*>(dst) = packed[0];
         else  // images innermost: the lanes next to this one write the bytes beside these

@@ -213,7 +213,7 @@ __device__ __forceinline__ float relu1(float x) { return __builtin_amdgcn_fmed3f
 // but the NaNs were compared on the device).  Only the conversions run in that mode: the first asm takes every value as
 // an input, so the arithmetic that made them (rounded to nearest even, as the reference's) is complete before the mode
 // changes, and it hands out the zero that every dword starts from, so no conversion can start before it; the second asm
-// takes the four dwords.  The scheduling fences keep unrelated float arithmetic of the surrounding code out of the window.
+// takes the four dwords.  (pack_nonneg8, pack_nonneg4: the same for fewer.)  The scheduling fences keep unrelated float arithmetic of the surrounding code out of the window.
 __device__ __forceinline__ void pack_nonneg16(const float (&v)[16], v4i& packed)
 {
     unsigned w0, w1, w2, w3;
@@ -233,6 +233,47 @@ __device__ __forceinline__ void pack_nonneg16(const float (&v)[16], v4i& packed)
     asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0" : "+v"(w0), "+v"(w1), "+v"(w2), "+v"(w3));
     __builtin_amdgcn_sched_barrier(0);
     packed[0] = (int)w0, packed[1] = (int)w1, packed[2] = (int)w2, packed[3] = (int)w3;
+}
+__device__ __forceinline__ int pack_nonneg4(const float* v)
+{
+    unsigned w;
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 3\n\tv_mov_b32 %0, 0" : "=v"(w) : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w = __builtin_amdgcn_cvt_pk_u8_f32(v[i], i, w);
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0" : "+v"(w));
+    __builtin_amdgcn_sched_barrier(0);
+    return (int)w;
+}
+__device__ __forceinline__ int2 pack_nonneg8(const float* v)
+{
+    unsigned w0, w1;
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 3\n\tv_mov_b32 %0, 0"
+                 : "=v"(w0)
+                 : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]));
+    w1 = w0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        w0 = __builtin_amdgcn_cvt_pk_u8_f32(v[i], i, w0);
+        w1 = __builtin_amdgcn_cvt_pk_u8_f32(v[4 + i], i, w1);
+    }
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0" : "+v"(w0), "+v"(w1));
+    __builtin_amdgcn_sched_barrier(0);
+    return make_int2((int)w0, (int)w1);
+}
+// the first N values of a lane (4, 8 or 16); the other dwords are zero
+template <int N>
+__device__ __forceinline__ void pack_nonneg(const float (&v)[16], v4i& packed)
+{
+    if constexpr (N == 16) {
+        pack_nonneg16(v, packed);
+    } else if constexpr (N == 8) {
+        const int2 q = pack_nonneg8(v);
+        packed = v4i{q.x, q.y, 0, 0};
+    } else {
+        packed = v4i{pack_nonneg4(v), 0, 0, 0};
+    }
 }
 // four values inside [-128, 255] -> one dword of bytes
 __device__ __forceinline__ int pack_signed(const float* v)
@@ -271,7 +312,9 @@ __device__ __forceinline__ void zero_padding_features(v4i& packed, int valid)
 // (the bounds are integers), round-half-away is trunc(x + copysign(0.49999997f, x)), and
 // max(0, x) * s becomes clamp(x * s, 0, hi) when s >= 0.  The truncating float->int conversion
 // completes the rounding.
-template <int NT, int EPI, class Args>
+// N: values a lane has: 16, or 8 or 4 at the front (a conversion into bytes is kept whether its value is a real one or not, so a
+// lane with few values says so)
+template <int NT, int EPI, int N = 16, class Args>
 __device__ __forceinline__ v4i epilogue_fast16(const Args& a, const v4i (&acc)[4][NT], int nt, const float (&wq)[16],
                                                const float (&cal)[16], const float (&ecal)[16], const v4i& ev4,
                                                int valid)
@@ -325,8 +368,8 @@ __device__ __forceinline__ v4i epilogue_fast16(const Args& a, const v4i (&acc)[4
         // has checked to be inside the output range (the clamp_folded case of the run-time form below)
         v4i packed;
 #pragma unroll
-        for (int c = 0; c < 16; ++c) v[c] = med3(v[c] * wq[c], F.act_m, F.act_n) * cal[c] + 0.49999997f;
-        pack_nonneg16(v, packed);
+        for (int c = 0; c < N; ++c) v[c] = med3(v[c] * wq[c], F.act_m, F.act_n) * cal[c] + 0.49999997f;
+        pack_nonneg<N>(v, packed);
         zero_padding_features(packed, valid);
         return packed;
     }
@@ -334,23 +377,23 @@ __device__ __forceinline__ v4i epilogue_fast16(const Args& a, const v4i (&acc)[4
         v4i packed;
         if constexpr (EPI == EPI_KIND_RELU) {
 #pragma unroll
-            for (int c = 0; c < 16; ++c) v[c] = med3(v[c] * cal[c], 0.0f, F.hi) + 0.49999997f;
+            for (int c = 0; c < N; ++c) v[c] = med3(v[c] * cal[c], 0.0f, F.hi) + 0.49999997f;
         } else {
             if (F.eltw_u8) {
                 keep_branch();
 #pragma unroll
-                for (int c = 0; c < 16; ++c)
+                for (int c = 0; c < N; ++c)
                     v[c] = rha(v[c] * cal[c]) + (float)(((unsigned)ev4[c >> 2] >> (8 * (c & 3))) & 255u);
             } else {
                 keep_branch();
 #pragma unroll
-                for (int c = 0; c < 16; ++c)
+                for (int c = 0; c < N; ++c)
                     v[c] = rha(v[c] * cal[c]) + (float)(int)(int8_t)((unsigned)ev4[c >> 2] >> (8 * (c & 3)));
             }
 #pragma unroll
-            for (int c = 0; c < 16; ++c) v[c] = med3(v[c] * ecal[c], 0.0f, F.hi) + 0.49999997f;
+            for (int c = 0; c < N; ++c) v[c] = med3(v[c] * ecal[c], 0.0f, F.hi) + 0.49999997f;
         }
-        pack_nonneg16(v, packed);
+        pack_nonneg<N>(v, packed);
         zero_padding_features(packed, valid);
         return packed;
     }
@@ -648,7 +691,7 @@ __device__ __forceinline__ void finish_pool(const MfmaArgs& a, const v4i (&acc)[
             else v = max_dpp<0xb1>(max(acc[d][nt][i], acc[d][nt + 1][i]));
             acc4[d % OWN][0][i] = d < OWN || sub == d / OWN ? v : acc4[d % OWN][0][i];
         }
-    const v4i packed = epilogue_fast16<1, EPI_KIND_RELU>(a, acc4, 0, sc.wq, sc.cal, sc.ecal, none, 16);
+    const v4i packed = epilogue_fast16<1, EPI_KIND_RELU, OWN * 4>(a, acc4, 0, sc.wq, sc.cal, sc.ecal, none, 16);
     int8_t* dst = (int8_t*)a.out + obase + sub * OWN * 4;
     unsigned keep[OWN];  // features past the end of the tensor stay zero
 #pragma unroll

@@ -305,10 +305,16 @@ def test_depthwise_chain_on_small_planes(eng, mid, proj, stride, stages, hw, in_
     """waves that share a granule: one to three spans of projection, more K-steps and spans than waves, a last granule that
     is not full; and large planes with a granule per wave: odd numbers of slices and of 32-feature units; with and without
     the block's sum, against the oracle's separate convolutions"""
+    run_depthwise_chain(eng, mid, proj, stride, stages, hw, in_dt, saturate)
+
+
+def run_depthwise_chain(eng, mid, proj, stride, stages, hw, in_dt, saturate, shared=None):
     r = np.random.default_rng(mid + proj)
     H, W = hw
     B = 3 if H * W < 4000 else 1
     OH, OW = (H + 2 - 3) // stride + 1, (W + 2 - 3) // stride + 1
+    if shared is None:
+        shared = B * OH * OW <= 8192
     lo, hi = (0, 256) if in_dt == np.uint8 else (-128, 128)
     x = r.integers(lo, hi, (B, mid, H, W)).astype(in_dt)
     xin = hip.upload(eng, x, "fs_b_yx_fsv16", (1, 1))
@@ -337,7 +343,7 @@ def test_depthwise_chain_on_small_planes(eng, mid, proj, stride, stages, hw, in_
         ref_in, prev_t = refs[-1], hip.Tensor.make(hip.S8, hip.FS_B_YX_FSV16, B, ofm, OH, OW)
     for keep in ([False] * (stages - 1) + [True], None):
         ch = hip.ConvChain(eng, spec, keep)
-        assert b"conv_dwchain" in ch.info().kernel_name and (b"shared" in ch.info().kernel_name) == (B * OH * OW <= 8192)
+        assert b"conv_dwchain" in ch.info().kernel_name and (b"shared" in ch.info().kernel_name) == shared
         ch.enqueue(xin, [b if keep is None or keep[k] else None for k, b in enumerate(bufs)], [None, ebuf, None])
         eng.finish()
         for k in range(stages):
@@ -347,6 +353,16 @@ def test_depthwise_chain_on_small_planes(eng, mid, proj, stride, stages, hw, in_
         ch.close()
     for b in bufs + [xin, ebuf]:
         b.close()
+
+
+@pytest.mark.parametrize("mid,proj,stride,hw", [(576, 96, 1, (35, 39)), (576, 24, 1, (37, 37)), (576, 96, 1, (37, 37)), (528, 160, 1, (37, 37)),
+                                                (448, 64, 1, (9, 7)), (1152, 64, 1, (5, 5)), (704, 96, 2, (9, 9)), (1040, 160, 1, (5, 5)), (384, 64, 1, (53, 53))],
+                         ids=["256_granules", "two_a_group_narrow", "two_a_group", "two_a_group_wide", "seven_k_steps", "more_k_steps_than_waves",
+                              "rounds_two_spans", "rounds_three_spans", "more_than_two_granules_a_cu"])
+def test_shared_granules_at_the_edges_of_their_forms(eng, mid, proj, stride, hw):
+    """one and two granules to a workgroup (the last of 257 granules stands alone, and is not full), K-steps that fill the
+    registers of a wave and K-steps that take several rounds, more granules than the device holds"""
+    run_depthwise_chain(eng, mid, proj, stride, 3, hw, np.uint8, 0, shared=True)
 
 
 @pytest.mark.parametrize("hw", [(1, 1), (17, 15), (46, 41)], ids=["one_pixel", "ragged", "several_granules"])
