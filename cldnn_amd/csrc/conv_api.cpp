@@ -406,7 +406,7 @@ static void run(cldnn_hip_conv c, const void* in, void* out, const void* eltw, i
         CHIP_REQUIRE(eltw, CLDNN_HIP_INVALID_ARG, "fused convolution without its second input");
     }
     c->engine->make_current();
-    hipStream_t s = c->engine->stream;
+    hipStream_t s = c->engine->launch_stream();
     switch (c->impl) {
     case CLDNN_HIP_IMPL_REF:
         launch_conv_ref(s, p, c->epi, in, c->w_raw, eltw, out, raw);
@@ -570,7 +570,7 @@ cldnn_hip_status cldnn_hip_conv_chain_enqueue(cldnn_hip_conv_chain ch, const voi
             }
         }
         ch->engine->make_current();
-        launch_conv_chain(ch->engine->stream, ch->in, ch->plan, ch->packed, input_dev, outs, el);
+        launch_conv_chain(ch->engine->launch_stream(), ch->in, ch->plan, ch->packed, input_dev, outs, el);
     });
 }
 
@@ -748,7 +748,7 @@ cldnn_hip_status cldnn_hip_reorder(cldnn_hip_engine e, const void* src_dev, cons
     return guarded([&] {
         CHIP_REQUIRE(e && src_dev && src && dst_dev && dst, CLDNN_HIP_INVALID_ARG, "null argument");
         e->make_current();
-        launch_reorder(e->stream, *src, src_dev, *dst, dst_dev);
+        launch_reorder(e->launch_stream(), *src, src_dev, *dst, dst_dev);
     });
 }
 
@@ -758,7 +758,7 @@ cldnn_hip_status cldnn_hip_copy_region(cldnn_hip_engine e, const void* src_dev, 
     return guarded([&] {
         CHIP_REQUIRE(e && src_dev && src && dst_dev && dst, CLDNN_HIP_INVALID_ARG, "null argument");
         e->make_current();
-        launch_copy_region(e->stream, *src, src_dev, *dst, dst_dev, offset_b, offset_f, offset_y, offset_x);
+        launch_copy_region(e->launch_stream(), *src, src_dev, *dst, dst_dev, offset_b, offset_f, offset_y, offset_x);
     });
 }
 
@@ -768,7 +768,7 @@ cldnn_hip_status cldnn_hip_activation(cldnn_hip_engine e, const void* src_dev, c
     return guarded([&] {
         CHIP_REQUIRE(e && src_dev && src && dst_dev && dst, CLDNN_HIP_INVALID_ARG, "null argument");
         e->make_current();
-        launch_pointwise(e->stream, *src, src_dev, nullptr, nullptr, *dst, dst_dev, 0, nullptr, 1.0f, activation, m, n);
+        launch_pointwise(e->launch_stream(), *src, src_dev, nullptr, nullptr, *dst, dst_dev, 0, nullptr, 1.0f, activation, m, n);
     });
 }
 
@@ -780,7 +780,7 @@ cldnn_hip_status cldnn_hip_eltwise_sum(cldnn_hip_engine e, const void* a_dev, co
     return guarded([&] {
         CHIP_REQUIRE(e && a_dev && a && b_dev && b && dst_dev && dst, CLDNN_HIP_INVALID_ARG, "null argument");
         e->make_current();
-        launch_pointwise(e->stream, *a, a_dev, b, b_dev, *dst, dst_dev, quantized, calib_dev, output_quantization_factor,
+        launch_pointwise(e->launch_stream(), *a, a_dev, b, b_dev, *dst, dst_dev, quantized, calib_dev, output_quantization_factor,
                          activation, m, n);
     });
 }
@@ -791,7 +791,7 @@ cldnn_hip_status cldnn_hip_eltwise(cldnn_hip_engine e, const cldnn_hip_eltwise_d
     return guarded([&] {
         CHIP_REQUIRE(e && desc && inputs_dev && output_dev, CLDNN_HIP_INVALID_ARG, "null argument");
         e->make_current();
-        launch_eltwise(e->stream, *desc, inputs_dev, calib_dev, output_dev);
+        launch_eltwise(e->launch_stream(), *desc, inputs_dev, calib_dev, output_dev);
     });
 }
 
@@ -800,7 +800,7 @@ cldnn_hip_status cldnn_hip_pooling(cldnn_hip_engine e, const cldnn_hip_pooling_d
     return guarded([&] {
         CHIP_REQUIRE(e && desc && input_dev && output_dev, CLDNN_HIP_INVALID_ARG, "null argument");
         e->make_current();
-        launch_pooling(e->stream, *desc, input_dev, output_dev);
+        launch_pooling(e->launch_stream(), *desc, input_dev, output_dev);
     });
 }
 

@@ -97,6 +97,15 @@ void cldnn_hip_buffer_s::upload()
     CHIP_CHECK(hipMemcpyAsync(dev, shadow, bytes, hipMemcpyHostToDevice, engine->stream));
 }
 
+// one recording to a thread: its engine, and the stream that collects the launches
+struct thread_recording {
+    cldnn_hip_engine engine = nullptr;
+    hipStream_t stream = nullptr;
+};
+static thread_local thread_recording g_recording;
+
+hipStream_t cldnn_hip_engine_s::launch_stream() const { return g_recording.engine == this ? g_recording.stream : stream; }
+
 void cldnn_hip_engine_s::make_current() const { CHIP_CHECK(hipSetDevice(device)); }
 
 hipEvent_t cldnn_hip_engine_s::take_event()
@@ -285,6 +294,77 @@ cldnn_hip_status cldnn_hip_engine_finish(cldnn_hip_engine e)
         CHIP_REQUIRE(e, CLDNN_HIP_INVALID_ARG, "null engine");
         e->make_current();
         e->wait_for(e->mark());
+    });
+}
+
+cldnn_hip_status cldnn_hip_engine_record_begin(cldnn_hip_engine e)
+{
+    return guarded([&] {
+        CHIP_REQUIRE(e, CLDNN_HIP_INVALID_ARG, "null engine");
+        CHIP_REQUIRE(!g_recording.engine, CLDNN_HIP_ERROR, "this thread is recording already");
+        e->make_current();
+        hipStream_t s = nullptr;
+        CHIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+        // of this thread only: other threads go on allocating and waiting
+        const hipError_t r = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
+        if (r != hipSuccess) {
+            (void)hipStreamDestroy(s);
+            CHIP_CHECK(r);
+        }
+        g_recording = {e, s};
+        e->refs.fetch_add(1);
+    });
+}
+
+cldnn_hip_status cldnn_hip_engine_record_end(cldnn_hip_engine e, cldnn_hip_recording* out)
+{
+    if (out) *out = nullptr;
+    return guarded([&] {
+        CHIP_REQUIRE(e && g_recording.engine == e, CLDNN_HIP_INVALID_ARG, "this thread is not recording on that engine");
+        const hipStream_t s = g_recording.stream;
+        g_recording = {};
+        hipGraph_t graph = nullptr;
+        hipGraphExec_t exec = nullptr;
+        hipError_t r = hipStreamEndCapture(s, &graph);
+        if (r == hipSuccess && out) r = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+        if (r == hipSuccess && exec) r = hipGraphUpload(exec, e->stream);  // the first run pays for nothing
+        if (graph) (void)hipGraphDestroy(graph);
+        (void)hipStreamDestroy(s);
+        if (r != hipSuccess || !out) {
+            if (exec) (void)hipGraphExecDestroy(exec);
+            cldnn_hip_engine_release(e);
+            CHIP_CHECK(r);
+            return;
+        }
+        auto* rec = new cldnn_hip_recording_s();
+        rec->engine = e, rec->exec = exec;
+        *out = rec;
+    });
+}
+
+cldnn_hip_status cldnn_hip_recording_enqueue(cldnn_hip_recording r)
+{
+    return guarded([&] {
+        CHIP_REQUIRE(r, CLDNN_HIP_INVALID_ARG, "null recording");
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        CHIP_CHECK(hipStreamIsCapturing(r->engine->stream, &capture));
+        CHIP_REQUIRE(capture == hipStreamCaptureStatusNone && r->engine->launch_stream() == r->engine->stream, CLDNN_HIP_ERROR,
+                     "a recording is not enqueued into a capture");
+        r->engine->make_current();
+        CHIP_CHECK(hipGraphLaunch(r->exec, r->engine->stream));
+    });
+}
+
+cldnn_hip_status cldnn_hip_recording_release(cldnn_hip_recording r)
+{
+    return guarded([&] {
+        CHIP_REQUIRE(r, CLDNN_HIP_INVALID_ARG, "null recording");
+        cldnn_hip_engine e = r->engine;
+        (void)hipSetDevice(e->device);
+        (void)hipStreamSynchronize(e->stream);
+        (void)hipGraphExecDestroy(r->exec);
+        delete r;
+        cldnn_hip_engine_release(e);
     });
 }
 

@@ -33,6 +33,14 @@ struct cldnn_hip_engine_s {
     bool has_reached(uint64_t m) const { return __atomic_load_n(reached, __ATOMIC_ACQUIRE) >= m; }
     void wait_for(uint64_t m) const;
     void make_current() const;
+    // where a launch of this thread goes: the stream, or what the thread is recording (cldnn_hip_engine_record_begin)
+    hipStream_t launch_stream() const;
+};
+
+// The launches of a recording as an instantiated graph.
+struct cldnn_hip_recording_s {
+    cldnn_hip_engine engine = nullptr;
+    hipGraphExec_t exec = nullptr;
 };
 
 struct cldnn_hip_buffer_s {

@@ -122,6 +122,10 @@ SIGNATURES = {
     "cldnn_hip_engine_get_info": (C.c_int32, [C.c_void_p, C.POINTER(EngineInfo)]),
     "cldnn_hip_engine_stream": (C.c_void_p, [C.c_void_p]),
     "cldnn_hip_engine_flush": (C.c_int32, [C.c_void_p]),
+    "cldnn_hip_engine_record_begin": (C.c_int32, [C.c_void_p]),
+    "cldnn_hip_engine_record_end": (C.c_int32, [C.c_void_p, C.POINTER(C.c_void_p)]),
+    "cldnn_hip_recording_enqueue": (C.c_int32, [C.c_void_p]),
+    "cldnn_hip_recording_release": (C.c_int32, [C.c_void_p]),
     "cldnn_hip_engine_finish": (C.c_int32, [C.c_void_p]),
     "cldnn_hip_engine_used_memory": (C.c_int64, [C.c_void_p]),
     "cldnn_hip_engine_max_used_memory": (C.c_int64, [C.c_void_p]),

@@ -266,6 +266,12 @@ struct cldnn_network_impl : host::refcounted {
     host::ref<cldnn_event_impl> run_end;  // behind everything the last submitted run enqueued
     bool has_run = false;
     size_t allocated_bytes = 0;  // device bytes of the buffers the network allocated for its primitives' outputs
+    // Launches that are the same in every run: nodes [begin, end) of the program, in whose place `launches` is enqueued.
+    struct recorded_part {
+        size_t begin, end;
+        cldnn_hip_recording launches;
+    };
+    std::vector<recorded_part> recorded;
     size_t pooled_tensors = 0;   // outputs that reuse the buffer of an earlier, finished tensor
     ~cldnn_network_impl() override;
 };

@@ -69,6 +69,16 @@ void* cldnn_hip_engine_stream(cldnn_hip_engine e);
 /* replaces gpu_toolkit::flush / finish (reference src/gpu/ocl_toolkit.cpp:291-300) */
 cldnn_hip_status cldnn_hip_engine_flush(cldnn_hip_engine e);
 cldnn_hip_status cldnn_hip_engine_finish(cldnn_hip_engine e);
+/* A recording: between record_begin and record_end the launches that the CALLING THREAD makes on this engine are collected
+ * instead of enqueued (a HIP graph); nothing but launches may be made meanwhile.  recording_enqueue puts all of them on the
+ * engine's stream with one call, as often as wanted; the pointers they were made with must stay valid until the recording
+ * is released.  A stream that is being captured by the application takes no recording (CLDNN_HIP_ERROR, nothing enqueued):
+ * the launches are made one by one there. */
+typedef struct cldnn_hip_recording_s* cldnn_hip_recording;
+cldnn_hip_status cldnn_hip_engine_record_begin(cldnn_hip_engine e);
+cldnn_hip_status cldnn_hip_engine_record_end(cldnn_hip_engine e, cldnn_hip_recording* out); /* out == NULL: thrown away */
+cldnn_hip_status cldnn_hip_recording_enqueue(cldnn_hip_recording r);
+cldnn_hip_status cldnn_hip_recording_release(cldnn_hip_recording r);
 /* bytes currently / at most allocated through this engine (reference src/include/engine_impl.h:123-124) */
 int64_t cldnn_hip_engine_used_memory(cldnn_hip_engine e);
 int64_t cldnn_hip_engine_max_used_memory(cldnn_hip_engine e);

@@ -928,3 +928,78 @@ def test_failed_run_leaves_nothing_in_flight(eng):
     mem.write(x)
     net.set_input_data("b", mem)
     np.testing.assert_array_equal(net.execute()["sum"].get_memory().read(), rc.eltwise([x, x], "sum"))
+
+
+# ------------------------------------------------------- launches that are the same in every run go out as one recording
+def small_layers(eng, batch, side, output_in_the_middle):
+    """(topology, reference): fourteen 3x3 layers of 32 features, a residual sum over the last two"""
+    r = np.random.default_rng(97)
+    C, L = 32, 14
+    prims, layers = [cl.input_layout("input", cl.layout(DT.i8, F.bfyx, cl.tensor(batch, C, side, side)))], []
+    for k in range(L):
+        w, b, q, c = rand_layer(r, C, C, 3, False)
+        layers.append((w, b, q, c))
+        n = f"c{k}"
+        prims += [cl.data(f"{n}_{x}", m) for x, m in zip("wbqc", [cl.make_memory(eng, w)] + [vec_mem(eng, v) for v in (b, q, c)])]
+        prims.append(cl.convolution(n, f"c{k - 1}" if k else "input", [n + "_w"], [n + "_b"], [n + "_q"], [n + "_c"],
+                                    input_offset=cl.tensor(0, 0, -1, -1, 0), with_activation=k % 2 == 0, output_data_type=DT.i8))
+    prims.append(cl.eltwise("out", f"c{L - 3}", f"c{L - 1}", cl.eltwise_mode.sum))
+
+    def reference(x):
+        t = [x]
+        for k, (w, b, q, c) in enumerate(layers):
+            t.append(rc.conv(t[-1], w, b, wqf=q, calib=c, pad=(1, 1), out_dt="s8", act="relu" if k % 2 == 0 else "none"))
+        return t[7], rc.eltwise([t[L - 2], t[L]], "sum")
+    outputs = ["out"] + (["c6"] if output_in_the_middle else [])
+    return cl.topology(*prims), outputs, reference
+
+
+@pytest.mark.parametrize("output_in_the_middle", [False, True], ids=["one_output", "output_in_the_middle"])
+@pytest.mark.parametrize("pool", [True, False], ids=["pool", "no_pool"])
+def test_recorded_launches_over_many_runs(pool, output_in_the_middle):
+    """every run against the oracle: inputs rewritten in place and replaced by another memory, results locked and overwritten by
+    the application, work of another network on the stream in between, two networks of one program taking turns"""
+    e = cl.engine(enable_memory_pool=pool)
+    topo, outputs, reference = small_layers(e, 2, 11, output_in_the_middle)
+    opts = cl.build_options(optimize_data=True, outputs=outputs)
+    nets = [cl.network(e, topo, opts) for _ in range(2)]
+    for n in nets:  # an output in the middle: two recordings, the reorder to it between them
+        assert n.get_primitive_info("c2").get("recorded") and n.get_primitive_info("c9").get("recorded")
+        assert "recorded" not in n.get_primitive_info("out") and (not output_in_the_middle or "recorded" not in n.get_primitive_info("c6"))
+    other_topo, _, other_reference = small_layers(e, 1, 40, False)
+    other = cl.network(e, other_topo, cl.build_options(optimize_data=False))
+    r = np.random.default_rng(5)
+    mems = [cl.make_memory(e, np.zeros((2, 32, 11, 11), np.int8)) for _ in range(2)]
+    y = r.integers(-128, 128, (1, 32, 40, 40)).astype(np.int8)
+    other.set_input_data("input", cl.make_memory(e, y))
+    for i in range(6):
+        x = r.integers(-128, 128, (2, 32, 11, 11)).astype(np.int8)
+        m, net = mems[(i // 2) % 2], nets[i % 2]
+        m.write(x)
+        net.set_input_data("input", m)
+        outs = net.execute()
+        if i == 2:
+            last = other.execute()
+            np.testing.assert_array_equal(last["out"].get_memory().read(), other_reference(y)[1])
+        mid, expected = reference(x)
+        np.testing.assert_array_equal(outs["out"].get_memory().read(), expected)
+        if output_in_the_middle:
+            np.testing.assert_array_equal(outs["c6"].get_memory().read(), mid)
+        outs["out"].get_memory().write(np.full(expected.shape, 77, expected.dtype))
+        outs = net.execute()  # again, queued twice
+        outs = net.execute()
+        np.testing.assert_array_equal(outs["out"].get_memory().read(), expected)
+
+
+def test_large_launches_and_profiling_engines_record_nothing():
+    """9.7 Gop to a launch: one by one; an engine with profiling has an event behind every launch"""
+    e = cl.engine()
+    topo, outputs, _ = small_layers(e, 32, 128, False)
+    big = cl.network(e, topo, cl.build_options(optimize_data=True))
+    assert "recorded" not in big.get_primitive_info("c2")
+    p = cl.engine(enable_profiling=True)
+    topo, outputs, reference = small_layers(p, 2, 11, False)
+    x = np.random.default_rng(6).integers(-128, 128, (2, 32, 11, 11)).astype(np.int8)
+    net, outs = run(p, topo, {"input": cl.make_memory(p, x)}, True)
+    assert "recorded" not in net.get_primitive_info("c2")
+    np.testing.assert_array_equal(outs["out"].get_memory().read(), reference(x)[1])
