@@ -22,6 +22,7 @@ struct cldnn_hip_conv_s {
     FastEpi fe{};
     MfmaPlan mplan{};
     DwPlan dplan{};
+    StemPlan splan{};     // a first layer that reads its bfyx image itself
     // device allocations
     void* w_raw = nullptr;    // dense weights (reference kernel)
     void* w_packed = nullptr; // MFMA / depthwise operand stream
@@ -201,13 +202,25 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
     // Layers whose dense weights would be more than 64 MiB stay on the one-thread-per-output kernel.
     const bool grouped = d.groups > 1 && !depthwise;
     const bool grouped_dense = grouped && blocked && (size_t)d.ofm * d.ifm * d.fy * d.fx <= ((size_t)64 << 20);
+    // a plain image of at most four features: the first-layer kernel reads it where it lies (its epilogue decides below)
+    const bool planar = d.impl == CLDNN_HIP_IMPL_AUTO && d.tile_override == 0 && int_path && d.groups == 1 && !d.fused && !e.fc && !d.sibling_split
+                        && d.input.format == CLDNN_HIP_FMT_BFYX && d.output.format == CLDNN_HIP_FMT_FS_B_YX_FSV16 && d.ifm <= 4;
+    if (planar) {
+        Epilogue probe = e;
+        probe.bias = bias && d.bias_dtype == CLDNN_HIP_F32 ? (const void*)weights : nullptr;
+        probe.calib = calib_on ? calib : nullptr;
+        if (mfma_fast_epilogue(p, probe, calib_on ? calib : nullptr, eltw_calib, wqf, &c->fe))
+            c->splan = stem_plan(p, c->fe, probe, c->engine->props.multiProcessorCount);
+    }
     int impl = d.impl;
-    if (impl == CLDNN_HIP_IMPL_AUTO) {
+    if (c->splan.ok) {
+        impl = CLDNN_HIP_IMPL_MFMA;
+    } else if (impl == CLDNN_HIP_IMPL_AUTO) {
         if ((blocked || stem) && int_path && (d.groups == 1 || grouped_dense)) impl = CLDNN_HIP_IMPL_MFMA;
         else if (blocked && int_path && depthwise) impl = CLDNN_HIP_IMPL_DEPTHWISE;
         else impl = CLDNN_HIP_IMPL_REF;
     }
-    if (impl == CLDNN_HIP_IMPL_MFMA)
+    if (impl == CLDNN_HIP_IMPL_MFMA && !c->splan.ok)
         CHIP_REQUIRE((blocked || stem) && int_path && (d.groups == 1 || grouped_dense), CLDNN_HIP_UNSUPPORTED_FORMAT,
                      "the MFMA kernel needs int8 data in fs_b_yx_fsv16 (first layers: bordered b_fs_yx_fsv4 input), "
                      "quantisation, and groups == 1 or a block-diagonal weight matrix of at most 64 MiB");
@@ -281,6 +294,15 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
         e.bias_dt = CLDNN_HIP_NO_TYPE;
     }
 
+    if (c->splan.ok) {
+        std::vector<int8_t> packed(c->splan.packed_bytes);
+        stem_pack_weights(p, c->splan, w8, packed.data());
+        c->w_packed = upload(c, packed.data(), packed.size());
+        c->w_raw = upload(c, weights, wcount);  // for the accumulators alone
+        inf.tile_pixels = 64, inf.tile_ofm = 64, inf.grid = c->splan.grid, inf.block = 256, inf.lds_bytes = c->splan.lds_bytes;
+        std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_stem_plain<%d k-steps,%d fragments,fast>", c->splan.ksteps, c->splan.frags_f);
+        return;
+    }
     std::vector<int8_t> dense;
     if (impl == CLDNN_HIP_IMPL_MFMA && grouped) {
         // [ofm][ifm / groups][fy][fx] -> [ofm][features its span of 64 reads][fy][fx].  The groups of a span read a run of
@@ -412,6 +434,11 @@ static void run(cldnn_hip_conv c, const void* in, void* out, const void* eltw, i
         launch_conv_ref(s, p, c->epi, in, c->w_raw, eltw, out, raw);
         break;
     case CLDNN_HIP_IMPL_MFMA: {
+        if (c->splan.ok) {
+            if (raw) launch_conv_ref(s, p, c->epi, in, c->w_raw, nullptr, nullptr, raw);
+            else launch_conv_stem(s, p, c->splan, c->w_packed, (const int32_t*)c->acc_init, c->epi, c->fe, in, out);
+            break;
+        }
         MfmaBuffers wb{(const int8_t*)c->w_packed, (const int32_t*)c->ktab, c->gather, (const int32_t*)c->origin};
         if (static_scratch) {
             // the gather scratch comes from the array inside the code object instead of the object's own allocation
@@ -726,6 +753,22 @@ cldnn_hip_status cldnn_hip_conv_pool_output(cldnn_hip_conv c, const cldnn_hip_po
                      CLDNN_HIP_DIMENSION_MISMATCH, "the pooling does not read this convolution's result");
         const bool halves = d->mode == CLDNN_HIP_POOL_MAX && d->size_y == 2 && d->size_x == 2 && d->stride_y == 2 && d->stride_x == 2 && d->pad_y == 0
                             && d->pad_x == 0 && o.y * 2 == p.OH && o.x * 2 == p.OW && o.format == CLDNN_HIP_FMT_FS_B_YX_FSV16;
+        // a first layer also takes the 3x3 window at stride 2, the last one cut off at the edge or not
+        if (c->splan.ok) {
+            auto ends = [](int from, int to) { return from >= 3 && to == (from - 3 + 1) / 2 + 1; };
+            const bool thirds = d->mode == CLDNN_HIP_POOL_MAX && d->size_y == 3 && d->size_x == 3 && d->stride_y == 2 && d->stride_x == 2 && d->pad_y == 0
+                                && d->pad_x == 0 && o.format == CLDNN_HIP_FMT_FS_B_YX_FSV16 && ends(p.OH, o.y) && ends(p.OW, o.x);
+            CHIP_REQUIRE(thirds && !p.pooled && tensor_elems(o) < (1ull << 31), CLDNN_HIP_UNSUPPORTED_FORMAT, "this convolution cannot pool its own result");
+            ConvProblem q = p;
+            q.pooled = 1, q.out_t = o, q.out_p = make_pitch(o);
+            const StemPlan s = stem_plan(q, c->fe, c->epi, c->engine->props.multiProcessorCount);
+            CHIP_REQUIRE(s.ok, CLDNN_HIP_UNSUPPORTED_FORMAT, "this convolution cannot pool its own result");
+            p = q, c->splan = s;
+            c->info.grid = s.grid, c->info.lds_bytes = s.lds_bytes;
+            c->info.bytes -= (int64_t)p.B * p.OFM * ((int64_t)p.OH * p.OW - (int64_t)o.y * o.x);
+            std::snprintf(c->info.kernel_name, sizeof(c->info.kernel_name), "conv_stem_plain<%d k-steps,%d fragments,pooled,fast>", s.ksteps, s.frags_f);
+            return;
+        }
         CHIP_REQUIRE(halves && !p.pooled && c->impl == CLDNN_HIP_IMPL_MFMA && c->fast && mfma_can_pool(p, c->mplan, c->fe, c->epi)
                          && tensor_elems(o) < (1ull << 31),
                      CLDNN_HIP_UNSUPPORTED_FORMAT, "this convolution cannot pool its own result");

@@ -512,7 +512,7 @@ struct LaneScales {
 template <int EPI, class Args>
 __device__ __forceinline__ void load_scales4(const Args& a, int f0, LaneScales& sc, int d = 0)
 {
-    const Epilogue& e = a.epi;
+    const auto& e = a.epi;
     if constexpr (EPI == EPI_KIND_RELU || EPI == EPI_KIND_FUSED || EPI == EPI_KIND_LINEAR) {
         // these kinds are only chosen when the vectors they read exist
         const float4 c4 = *reinterpret_cast<const float4*>(e.calib + f0);

@@ -11,7 +11,7 @@ struct ConvProblem {
     int in_dt, w_dt, out_dt, eltw_dt;
     cldnn_hip_tensor in_t, out_t, eltw_t;
     Pitch in_p, out_p, eltw_p;
-    int pooled;     // the output tensor holds the maxima over 2x2 windows of the OH x OW result
+    int pooled;     // the output tensor holds the maxima over 2x2 windows (first layers: 3x3 at stride 2) of the OH x OW result
     int plain_out;  // one output pixel per image, written as bfyx or yxfb; split-K kernel
     int by_span;  // grouped: IFM counts the features that a span of 64 outputs reads, from an origin of its own
 };
@@ -133,6 +133,20 @@ void launch_conv_mfma(hipStream_t s, const ConvProblem& p, const MfmaPlan& plan,
 
 // can the plan's kernel pool its result (2x2 windows) as it writes it?
 bool mfma_can_pool(const ConvProblem& p, const MfmaPlan& pl, const FastEpi& fast, const Epilogue& epi);
+
+// ---- first layers straight from a bfyx image (conv_stem.hip)
+struct StemPlan {
+    int ok;              // the kernel takes this layer
+    int epi, frags_f, ksteps, nch;  // epilogue kind, fragments of 16 features, K-steps, chunks of four taps to a filter row
+    int tiles, tile_cols, wave_rows;  // pooling: column strips of a workgroup, their width, rows of a wave
+    int wg_rows, wg_cols, frags, row_groups, col_groups, total, grid;
+    int lds_rows, pitch, lds_bytes;
+    size_t packed_bytes;
+};
+StemPlan stem_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e, int cus);
+void stem_pack_weights(const ConvProblem& p, const StemPlan& s, const int8_t* w, int8_t* packed);
+void launch_conv_stem(hipStream_t st, const ConvProblem& p, const StemPlan& s, const void* packed, const int32_t* acc_init, const Epilogue& epi,
+                      const FastEpi& fe, const void* in, void* out);
 
 // ---- depthwise bandwidth kernel on fs_b_yx_fsv16 (conv_dw.hip)
 struct DwPlan {

@@ -149,16 +149,18 @@ static void launch_node(cldnn_network_impl* net, node* n)
         return it->second.get();
     };
     auto out_of = [&](node* d) { return mem_of(d)->use(use_of_output(d)); };
+    // what a reorder reads: an image that it alone reads need not be copied to the device first
+    auto image_of = [&](node* r) {
+        node* src = r->deps[0];
+        const bool once = src->p->type == prim_type::input_layout && src->users.size() == 1;
+        return mem_of(src)->use(once ? CLDNN_HIP_USE_READ_ONCE : CLDNN_HIP_USE_READ);
+    };
     const cldnn_hip_tensor ot = to_hip(n->out);
     switch (p.type) {
     case prim_type::reorder: {
-        if (n->written_by) break;
-        node* src = n->deps[0];
-        // an image that only this reorder reads need not be copied to the device first
-        const bool once = src->p->type == prim_type::input_layout && src->users.size() == 1;
-        const void* in = mem_of(src)->use(once ? CLDNN_HIP_USE_READ_ONCE : CLDNN_HIP_USE_READ);
-        const cldnn_hip_tensor it = to_hip(src->out);
-        hip_check(cldnn_hip_reorder(eng->h, in, &it, out_of(n), &ot));
+        if (n->written_by || n->read_by) break;
+        const cldnn_hip_tensor it = to_hip(n->deps[0]->out);
+        hip_check(cldnn_hip_reorder(eng->h, image_of(n), &it, out_of(n), &ot));
         break;
     }
     case prim_type::concatenation: {
@@ -214,7 +216,7 @@ static void launch_node(cldnn_network_impl* net, node* n)
     case prim_type::fused_conv_eltwise: {
         if (n->chain_head) break;  // written by the launch of its chain's head
         if (n->sibling_head) break;  // written by the launch of the convolution it is paired with
-        const void* in = mem_of(n->deps[0])->read_ptr();
+        const void* in = n->reads_for ? image_of(n->reads_for) : mem_of(n->deps[0])->read_ptr();
         if (n->chain) {
             void* outs[3] = {nullptr, nullptr, nullptr};
             const void* eltws[3] = {nullptr, nullptr, nullptr};
@@ -259,7 +261,7 @@ static void record_launches(cldnn_network_impl* net)
     for (auto& u : prog->nodes)
         if (u->constant || u->is_output) visible.insert(memory(u.get()));
     auto hidden = [&](node* d) { return d->p->type != prim_type::input_layout && !d->constant && memory(d) && !visible.count(memory(d)); };
-    auto launches = [](const node* n) { return !n->written_by && !n->concat_in_place && !n->chain_head && !n->sibling_head; };
+    auto launches = [](const node* n) { return !n->written_by && !n->read_by && !n->concat_in_place && !n->chain_head && !n->sibling_head; };
     auto same_every_run = [&](node* n) {
         if (!launches(n)) return true;
         const bool conv = n->p->type == prim_type::convolution || n->p->type == prim_type::fused_conv_eltwise;
@@ -270,7 +272,7 @@ static void record_launches(cldnn_network_impl* net)
             // the weights and factors of a convolution were packed when it was created
             const size_t reads = conv ? (fused ? 2 : 1) : m->deps.size();
             for (size_t i = k ? 1 : 0; i < reads; ++i)
-                if (!hidden(m->deps[i])) return false;
+                if (!hidden(m->reads_for && i == 0 ? m->reads_for->deps[0] : m->deps[i])) return false;
             if (n->chain && !n->chain_keep[k]) continue;
             if (!hidden(m->writes_for ? m->writes_for : m)) return false;
             if (m->sibling && !hidden(m->sibling)) return false;
@@ -1000,6 +1002,9 @@ cldnn_network cldnn_allocate_network(cldnn_program program, cldnn_status* status
         }
         for (auto& u : program->nodes)
             for (node* d : u->deps) last_use[d] = std::max(last_use[d], index[u.get()]);
+        // a first layer reads the image at its own place, not at the reorder's
+        for (auto& u : program->nodes)
+            if (u->reads_for) last_use[u->reads_for->deps[0]] = std::max(last_use[u->reads_for->deps[0]], index[u.get()]);
         // a primitive on the second stream may still read its inputs while the first stream moves on: they stay
         // reserved until the primitive that waits for it
         for (auto& u : program->nodes)
@@ -1034,6 +1039,7 @@ cldnn_network cldnn_allocate_network(cldnn_program program, cldnn_status* status
                 continue;
             }
             if (n->chain_unkept()) continue;  // never written: the next member of the chain takes it in registers
+            if (n->read_by) continue;     // its result is never written: the convolution reads what it would have read
             if (n->written_by) continue;  // its buffer was taken where the convolution that writes it stands
             if (n->sibling_head) continue;  // a window into the pair's buffer, made when the pair's first node came up
             if (n->concat_in_place || n->concat_into) {

@@ -212,6 +212,10 @@ struct node {
     // convolution.  The convolution has no buffer.
     node* writes_for = nullptr;
     node* written_by = nullptr;
+    // a first layer that reads the plain image itself: `reads_for` (on the convolution) is the reorder into its layout, whose
+    // input it reads; `read_by` (on the reorder) is the convolution.  The reorder has no buffer and launches nothing.
+    node* reads_for = nullptr;
+    node* read_by = nullptr;
     cldnn_padding unpaired_padding{};  // the output padding this node had before it took the wider border of its pair
     // member of a chain whose result stays in registers: it has no buffer and nobody but the next member reads it
     bool chain_unkept() const

@@ -983,6 +983,16 @@ static node* plain_reader(const cldnn_program_impl* prog, const node* n)
     return n->out.size.sizes[2] == 1 && n->out.size.sizes[3] == 1 ? r : nullptr;
 }
 
+// The reorder of a plain int8 image into the layout of a first layer that is its only reader, or nullptr: a kernel reads such an
+// image itself, and the image's own place in the order is the convolution's then.
+static node* image_reorder(const cldnn_program_impl* prog, const node* n)
+{
+    if (!prog->optimize_data || prog->tuning.mode != cldnn_tuning_disabled || !n->first_layer || n->side_stream || n->p->type != prim_type::convolution) return nullptr;
+    node* r = n->deps[0];
+    if (r->p->type != prim_type::reorder || r->is_output || r->users.size() != 1 || r->concat_into || r->written_by || r->out.data_type != r->deps[0]->out.data_type) return nullptr;
+    return r->deps[0]->out.format == cldnn_format_bfyx && !r->deps[0]->constant ? r : nullptr;
+}
+
 static bool only_pooled(const node* n)
 {
     return n->p->type == prim_type::convolution && !n->is_output && !n->side_stream && !n->concat_into && n->users.size() == 1
@@ -1013,9 +1023,27 @@ static void compile_conv(cldnn_program_impl* prog, node* n)
         }
         d.output = own;
     }
-    apply_tuning(prog, d, wv.data(), bias_ptr, wqf_ptr, calib_ptr, (const float*)eltw_calib);
-    hip_check(cldnn_hip_conv_create(n->side_stream ? prog->engine->side : prog->engine->h, &d, wv.data(), bias_ptr, wqf_ptr, calib_ptr,
-                                    (const float*)eltw_calib, &n->conv));
+    node* r = image_reorder(prog, n);
+    const cldnn_hip_tensor own = d.input;
+    // (a positive input offset describes the data as a smaller tensor: left to the reorder)
+    if (r && own.y == r->out.size.sizes[3] && own.x == r->out.size.sizes[2]) {
+        d.input = to_hip(r->deps[0]->out);
+        if (cldnn_hip_conv_create(prog->engine->h, &d, wv.data(), bias_ptr, wqf_ptr, calib_ptr, (const float*)eltw_calib, &n->conv) == CLDNN_HIP_SUCCESS) {
+            hip_check(cldnn_hip_conv_get_info(n->conv, &n->conv_info));
+            if (n->conv_info.impl == CLDNN_HIP_IMPL_MFMA) {
+                n->reads_for = r, r->read_by = n;
+            } else {
+                cldnn_hip_conv_release(n->conv);
+                n->conv = nullptr;
+            }
+        }
+        d.input = own;
+    }
+    if (!n->conv) {
+        apply_tuning(prog, d, wv.data(), bias_ptr, wqf_ptr, calib_ptr, (const float*)eltw_calib);
+        hip_check(cldnn_hip_conv_create(n->side_stream ? prog->engine->side : prog->engine->h, &d, wv.data(), bias_ptr, wqf_ptr, calib_ptr,
+                                        (const float*)eltw_calib, &n->conv));
+    }
     // a max pooling behind it that nobody else reads past
     if (prog->optimize_data && only_pooled(n)) {
         const cldnn_hip_pooling_desc pd = pooling_descriptor(n->users[0]);
@@ -1408,6 +1436,8 @@ std::string describe_node(const node* n)
             s += "]";
         }
     }
+    if (n->reads_for) s += ",\"reads\":\"" + n->reads_for->deps[0]->p->id + "\"";
+    if (n->read_by) s += ",\"left_to\":\"" + n->read_by->p->id + "\"";
     if (n->sibling) s += ",\"launches_also\":\"" + n->sibling->p->id + "\"";
     if (n->sibling_head) s += ",\"launched_by\":\"" + n->sibling_head->p->id + "\"";
     if (n->conv || n->chain || n->chain_head)

@@ -1,6 +1,8 @@
 """Parity of the HIP convolution (through the C-ABI) with the CPU oracle and with the
 reference's known-answer tables.  Integer results must be bit-exact; float outputs are
 compared at 1e-5 relative (they are the same sequence of float operations)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -983,3 +985,83 @@ def test_scores_written_in_plain_layouts(eng, shape, form, out_fmt):
     c.enqueue(xin, out)
     eng.finish()
     assert_same(ref, hip.download(eng, out))
+
+
+# ------------------------------------------------------- first layers that read a plain image themselves
+STEMS = [  # batch, features in / out, filter, stride, padding, plane
+    (2, 3, 64, (7, 7), (2, 2), (3, 3), (41, 67)),     # ResNet's, odd plane
+    (1, 3, 64, (7, 7), (2, 2), (3, 3), (224, 224)),   # four strips of pooled columns
+    (3, 3, 32, (3, 3), (2, 2), (1, 1), (33, 30)),     # MobileNet's: two fragments
+    (2, 3, 64, (3, 3), (1, 1), (1, 1), (19, 300)),    # VGG's, two groups of columns
+    (1, 4, 48, (5, 5), (1, 1), (2, 2), (9, 17)),      # four features, a feature count that fills three slices
+    (2, 1, 17, (3, 5), (2, 1), (0, 2), (12, 23)),     # one feature in, a last slice of one feature, unequal strides
+    (1, 2, 8, (1, 1), (1, 1), (0, 0), (3, 4)),        # the smallest row
+    (40, 3, 16, (3, 3), (2, 2), (1, 1), (5, 4)),      # one strip of one or two pooled columns, four row groups
+    (1, 3, 33, (4, 4), (4, 4), (0, 0), (21, 80)),     # filter rows that fill a chunk, stride 4
+]
+
+
+def stem_layer(r, ifm, ofm, k, in_dt, act):
+    x_rms = 147.4 if in_dt == np.uint8 else 73.9
+    w = r.integers(-127, 128, (ofm, ifm, *k)).astype(np.int8)
+    bias = r.integers(-1000, 1001, ofm).astype(np.int32)
+    f = (r.uniform(0.5, 2.0, ofm) / (np.sqrt(ifm * k[0] * k[1]) * x_rms * 73.3)).astype(np.float32)
+    if act == "clamp":
+        return w, bias, np.float32(3.0) * f, np.full(ofm, 127.0 / 6.0, np.float32), dict(act="clamp", act_m=0.0, act_n=6.0)
+    return w, bias, np.ones(ofm, np.float32), np.float32(40.0) * f, dict(act=act)
+
+
+@pytest.mark.parametrize("in_dt,act", [(np.uint8, "relu"), (np.int8, "none"), (np.uint8, "clamp")], ids=["u8_relu", "s8_linear", "u8_relu6"])
+@pytest.mark.parametrize("case", STEMS, ids=lambda c: "%dx%d-%d_%dx%d_%dx%d" % (c[0], c[1], c[2], *c[3], *c[6]))
+def test_first_layer_reads_a_plain_image(eng, case, in_dt, act):
+    B, ifm, ofm, k, stride, pad, (H, W) = case
+    r = np.random.default_rng(B + ofm)
+    lo, hi = (0, 256) if in_dt == np.uint8 else (-128, 128)
+    x = r.integers(lo, hi, (B, ifm, H, W)).astype(in_dt)
+    w, bias, wqf, calib, kw = stem_layer(r, ifm, ofm, k, in_dt, act)
+    ref, ref_acc = rc.conv(x, w, bias, wqf=wqf, calib=calib, stride=stride, pad=pad, out_dt="s8", want_acc=True, **kw)
+    for in_pad in ((0, 0), (1, 2)):
+        src = hip.upload(eng, x, "bfyx", in_pad)
+        d = hip.conv_desc(src.tensor, w.shape, "s8", stride=stride, pad=pad, out_fmt=hip.FS_B_YX_FSV16, out_pad=(1, 1), bias_dt=hip.I32, has_wqf=True,
+                          has_calib=True, **kw)
+        c = hip.Conv(eng, d, w, bias, wqf, calib)
+        assert b"conv_stem" in c.info().kernel_name and c.info().impl == hip.IMPL_MFMA
+        dst = hip.Buffer(eng, d.output)
+        c.enqueue(src, dst)
+        eng.finish()
+        bad = np.argwhere(hip.download(eng, dst) != ref)
+        assert bad.size == 0, "%d differ, first at %s" % (len(bad), bad[0])
+        np.testing.assert_array_equal(c.accumulators(src), ref_acc)
+        raw = np.frombuffer(dst.read_raw(), np.int8)  # the border and the features that fill up a slice stay zero
+        assert np.count_nonzero(raw) == np.count_nonzero(ref)
+        for b in (c, src, dst):
+            b.close()
+
+
+@pytest.mark.parametrize("in_dt", [np.uint8, np.int8], ids=["u8", "s8"])
+@pytest.mark.parametrize("case", [c for c in STEMS if c[6][0] > 10], ids=lambda c: "%dx%d-%d_%dx%d_%dx%d" % (c[0], c[1], c[2], *c[3], *c[6]))
+def test_first_layer_finishes_the_3x3_pooling_behind_it(eng, case, in_dt):
+    """windows that end at the edge of the plane and windows that are cut off there, in both directions"""
+    B, ifm, ofm, k, stride, pad, (H, W) = case
+    for H, W in ((H, W), (H + stride[0], W + stride[1])):
+        r = np.random.default_rng(B + ofm + H)
+        lo, hi = (0, 256) if in_dt == np.uint8 else (-128, 128)
+        x = r.integers(lo, hi, (B, ifm, H, W)).astype(in_dt)
+        w, bias, wqf, calib, kw = stem_layer(r, ifm, ofm, k, in_dt, "relu")
+        ref = rc.pool(rc.conv(x, w, bias, wqf=wqf, calib=calib, stride=stride, pad=pad, out_dt="s8", **kw), "max", (3, 3), (2, 2))
+        src = hip.upload(eng, x, "bfyx")
+        d = hip.conv_desc(src.tensor, w.shape, "s8", stride=stride, pad=pad, out_fmt=hip.FS_B_YX_FSV16, bias_dt=hip.I32, has_wqf=True, has_calib=True, **kw)
+        c = hip.Conv(eng, d, w, bias, wqf, calib)
+        pd = hip.PoolingDesc()
+        pd.input, pd.output = d.output, hip.Tensor.make(hip.S8, hip.FS_B_YX_FSV16, B, ofm, ref.shape[2], ref.shape[3], 1, 1)
+        pd.mode, pd.size_y, pd.size_x, pd.stride_y, pd.stride_x = hip.POOL_MAX, 3, 3, 2, 2
+        assert hip.lib().cldnn_hip_conv_pool_output(c.h, C.byref(pd)) == 0
+        assert hip.lib().cldnn_hip_conv_pool_output(c.h, C.byref(pd)) == -6  # once
+        dst = hip.Buffer(eng, pd.output)
+        c.enqueue(src, dst)
+        eng.finish()
+        bad = np.argwhere(hip.download(eng, dst) != ref)
+        assert bad.size == 0, "%d differ, first at %s" % (len(bad), bad[0])
+        assert np.count_nonzero(np.frombuffer(dst.read_raw(), np.int8)) == np.count_nonzero(ref)
+        for b in (c, src, dst):
+            b.close()
