@@ -23,6 +23,7 @@ struct cldnn_hip_conv_s {
     MfmaPlan mplan{};
     DwPlan dplan{};
     StemPlan splan{};     // a first layer that reads its bfyx image itself
+    PlanePlan pplan{};
     // device allocations
     void* w_raw = nullptr;    // dense weights (reference kernel)
     void* w_packed = nullptr; // MFMA / depthwise operand stream
@@ -79,6 +80,15 @@ void* upload(cldnn_hip_conv c, const void* host, size_t bytes, size_t padded_byt
     if (host && bytes) CHIP_CHECK(hipMemcpyAsync(d, host, bytes, hipMemcpyHostToDevice, c->engine->stream));
     CHIP_CHECK(hipStreamSynchronize(c->engine->stream));
     return d;
+}
+
+void describe_plane(cldnn_hip_conv c)
+{
+    const PlanePlan& s = c->pplan;
+    cldnn_hip_conv_info& inf = c->info;
+    inf.tile_pixels = s.np * 32, inf.tile_ofm = 32, inf.grid = s.grid, inf.block = 256, inf.lds_bytes = s.lds_bytes;
+    std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_plane<%d groups of %dx%d,%d blocks%s,fast>", 32 >> s.shift, s.np, s.cols, s.jobs,
+                  c->p.pooled ? ",pooled" : "");
 }
 
 void build(cldnn_hip_conv c, const void* weights, const void* bias, const float* wqf, const float* calib,
@@ -227,6 +237,9 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE)
         CHIP_REQUIRE(blocked && int_path && depthwise, CLDNN_HIP_UNSUPPORTED_FORMAT,
                      "the depthwise kernel needs int8 data in fs_b_yx_fsv16, quantisation and groups == features");
+    if (impl == CLDNN_HIP_IMPL_PLANE)
+        CHIP_REQUIRE(blocked && int_path && d.groups == 1 && !d.fused && !e.fc && !d.sibling_split && !p.plain_out, CLDNN_HIP_UNSUPPORTED_FORMAT,
+                     "the patch kernel needs int8 data in fs_b_yx_fsv16, quantisation and one group");
     c->impl = impl;
 
     const int ifm_g = p.IFM / p.groups;
@@ -269,17 +282,25 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
         probe.bias = bias && (d.bias_dtype == CLDNN_HIP_F32 || e.fc) ? (const void*)weights : nullptr;
         c->fast = mfma_fast_epilogue(p, probe, calib_on ? calib : nullptr, eltw_calib, wqf, &c->fe);
     }
+    if (impl == CLDNN_HIP_IMPL_PLANE) {
+        Epilogue probe = e;
+        probe.bias = bias && d.bias_dtype == CLDNN_HIP_F32 ? (const void*)weights : nullptr;
+        if (c->fast) c->pplan = plane_plan(p, c->fe, probe, c->engine->props.multiProcessorCount);
+        CHIP_REQUIRE(c->pplan.ok && (d.tile_override == 1 || plane_pays(p, c->pplan, c->engine->props.multiProcessorCount)), CLDNN_HIP_UNSUPPORTED_FORMAT,
+                     "the patch kernel does not take this convolution");
+    }
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE && e.fc) c->fast = false;  // the depthwise kernels have no short fully_connected form
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE && c->fe.f32) c->fast = false;  // nor a float one
     const bool dw_fast = impl == CLDNN_HIP_IMPL_DEPTHWISE && p.FY == 3 && p.FX == 3 && dw_fast_applies(p, c->fast);
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE) c->dplan = dw_plan(p, c->fast, c->engine->props.multiProcessorCount);
-    const bool xor_u8 = (impl == CLDNN_HIP_IMPL_MFMA || dw_fast || c->dplan.rows) && p.in_dt == CLDNN_HIP_U8;
+    const bool matrix = impl == CLDNN_HIP_IMPL_MFMA || impl == CLDNN_HIP_IMPL_PLANE;
+    const bool xor_u8 = (matrix || dw_fast || c->dplan.rows) && p.in_dt == CLDNN_HIP_U8;
     for (int f = 0; f < p.OFM; ++f) {
         int64_t s = 0;
         if (xor_u8)
             for (size_t i = 0; i < (size_t)ifm_g * p.FY * p.FX; ++i) s += w8[(size_t)f * ifm_g * p.FY * p.FX + i];
         uint32_t v = (uint32_t)(int32_t)(128 * s);
-        init_raw[f] = impl == CLDNN_HIP_IMPL_MFMA ? (int32_t)v : 0;  // the accumulator probe of the depthwise path never flips signs
+        init_raw[f] = matrix ? (int32_t)v : 0;  // the accumulator probe of the depthwise path never flips signs
         // (the fully_connected form adds its bias as a float after the dequantisation, whatever its type)
         if (bias && d.bias_dtype == CLDNN_HIP_I32 && !e.bias_after && !e.fc) v += (uint32_t)((const int32_t*)bias)[f];
         init[f] = (int32_t)v;
@@ -301,6 +322,13 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
         c->w_raw = upload(c, weights, wcount);  // for the accumulators alone
         inf.tile_pixels = 64, inf.tile_ofm = 64, inf.grid = c->splan.grid, inf.block = 256, inf.lds_bytes = c->splan.lds_bytes;
         std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_stem_plain<%d k-steps,%d fragments,fast>", c->splan.ksteps, c->splan.frags_f);
+        return;
+    }
+    if (impl == CLDNN_HIP_IMPL_PLANE) {
+        std::vector<int8_t> packed(c->pplan.packed_bytes);
+        plane_pack_weights(p, c->pplan, w8, packed.data());
+        c->w_packed = upload(c, packed.data(), packed.size());
+        describe_plane(c);
         return;
     }
     std::vector<int8_t> dense;
@@ -455,6 +483,9 @@ static void run(cldnn_hip_conv c, const void* in, void* out, const void* eltw, i
                              out, nullptr);
         break;
     }
+    case CLDNN_HIP_IMPL_PLANE:
+        launch_conv_plane(s, p, c->pplan, c->w_packed, (const int32_t*)(raw ? c->acc_init_raw : c->acc_init), c->epi, c->fe, in, out, raw);
+        break;
     case CLDNN_HIP_IMPL_DEPTHWISE:
         launch_conv_dw(s, p, c->dplan, (const int8_t*)c->w_packed, (const int32_t*)c->w_masked, (const int32_t*)c->w_rows,
                        (const int32_t*)(raw ? c->acc_init_raw : c->acc_init), c->epi, c->fast ? &c->fe : nullptr, in, eltw, out,
@@ -767,6 +798,18 @@ cldnn_hip_status cldnn_hip_conv_pool_output(cldnn_hip_conv c, const cldnn_hip_po
             c->info.grid = s.grid, c->info.lds_bytes = s.lds_bytes;
             c->info.bytes -= (int64_t)p.B * p.OFM * ((int64_t)p.OH * p.OW - (int64_t)o.y * o.x);
             std::snprintf(c->info.kernel_name, sizeof(c->info.kernel_name), "conv_stem_plain<%d k-steps,%d fragments,pooled,fast>", s.ksteps, s.frags_f);
+            return;
+        }
+        if (c->impl == CLDNN_HIP_IMPL_PLANE) {
+            CHIP_REQUIRE(halves && !p.pooled && tensor_elems(o) < (1ull << 31), CLDNN_HIP_UNSUPPORTED_FORMAT, "this convolution cannot pool its own result");
+            ConvProblem q = p;
+            q.pooled = 1, q.out_t = o, q.out_p = make_pitch(o);
+            const PlanePlan s = plane_plan(q, c->fe, c->epi, c->engine->props.multiProcessorCount);
+            CHIP_REQUIRE(s.ok && (c->desc.tile_override == 1 || plane_pays(q, s, c->engine->props.multiProcessorCount)), CLDNN_HIP_UNSUPPORTED_FORMAT,
+                         "this convolution cannot pool its own result");
+            p = q, c->pplan = s;
+            c->info.bytes -= (int64_t)p.B * p.OFM * ((int64_t)p.OH * p.OW - (int64_t)o.y * o.x);
+            describe_plane(c);
             return;
         }
         CHIP_REQUIRE(halves && !p.pooled && c->impl == CLDNN_HIP_IMPL_MFMA && c->fast && mfma_can_pool(p, c->mplan, c->fe, c->epi)

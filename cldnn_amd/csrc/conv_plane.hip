@@ -1,0 +1,131 @@
+// Host side of the kernel whose waves split K over a patch in LDS: which layers it takes, the tile of pixels, weights, launch.
+#include <algorithm>
+
+#include "conv_plane_kernel.h"
+
+namespace chip {
+
+namespace {
+
+int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+struct Form {
+    int np, nl;  // fragments (rows of a group), loads of 64 positions
+};
+constexpr Form FORMS[] = {{4, 4}, {7, 5}, {7, 6}};
+
+}  // namespace
+
+PlanePlan plane_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e, int cus)
+{
+    PlanePlan best{};
+    if (p.FY != 3 || p.FX != 3 || p.sy != 1 || p.sx != 1 || p.dy != 1 || p.dx != 1 || p.groups != 1 || p.by_span || p.plain_out) return best;
+    if (p.in_t.format != CLDNN_HIP_FMT_FS_B_YX_FSV16 || p.out_t.format != CLDNN_HIP_FMT_FS_B_YX_FSV16) return best;
+    if (!conv_border_covers(p)) return best;
+    if (f.f32 || f.fc || f.fused || f.split_valid || f.has_wqf || !e.calib) return best;
+    if (!f.relu_folded && f.act != CLDNN_HIP_ACT_NONE) return best;
+    if (p.pooled && (!f.relu_folded || p.OH % 2 || p.OW % 2)) return best;
+    if (tensor_elems(p.in_t) >= (1ull << 31) || tensor_elems(p.out_t) >= (1ull << 31)) return best;
+    if (p.in_p.py >= (1 << 24) || p.out_p.py >= (1 << 24)) return best;  // 24-bit products
+    const int jobs = p.IFM / 128, ftiles = ceil_div(p.OFM, PLANE_FEATURES);
+    if (p.IFM % 128 || (jobs != 1 && jobs % 2)) return best;
+    double least = 0;
+    for (const Form& form : FORMS) {
+        if (p.pooled && form.np % 2) continue;
+        PlanePlan s{};
+        s.strips = ceil_div(p.OW, 32), s.cols = ceil_div(p.OW, s.strips);
+        if (p.pooled) s.cols += s.cols % 2;
+        s.strips = ceil_div(p.OW, s.cols);
+        s.shift = s.cols <= 8 ? 3 : s.cols <= 16 ? 4 : 5;
+        const int groups = 32 >> s.shift;
+        s.pitch = s.cols + 2, s.positions = groups * (form.np + 2) * s.pitch;
+        if (s.positions > form.nl * 64) continue;
+        s.image_units = ceil_div(p.OH, form.np) * s.strips;
+        if ((int64_t)p.B * s.image_units * ftiles >= (1 << 30)) continue;
+        s.units = p.B * s.image_units;
+        s.total = ceil_div(s.units, groups) * ftiles;
+        // (512 bytes: what idle lanes read past the end)
+        s.lds_bytes = std::max((jobs == 1 ? 1 : 2) * 4 * 2 * s.positions * 16 + 512, PLANE_MEET * 4 * 4096);
+        // clocks: what a workgroup's matrix instructions take, and what it waits for at its start and its end
+        const int resident = s.lds_bytes <= 80 * 1024 ? 2 : 1;
+        const int64_t full = s.total / (cus * resident), left = s.total % (cus * resident);
+        const double work = form.np * 9 * jobs * 32.0, idle = 5000.0;
+        const double cost = full * (resident * work + idle) + (left > cus ? 2 * work + idle : left ? work + idle : 0);
+        if (best.ok && cost >= least) continue;
+        least = cost;
+        s.ok = 1, s.np = form.np, s.nl = form.nl, s.jobs = jobs, s.ftiles = ftiles;
+        s.grid = ceil_div(s.total, 8) * 8;
+        s.kind = f.relu_folded ? EPI_KIND_RELU : EPI_KIND_LINEAR;
+        s.packed_bytes = (size_t)ftiles * 4 * jobs * 9 * 1024;
+        best = s;
+    }
+    return best;
+}
+
+// Up to a workgroup per CU the launch is one prologue, one loop and one meeting of the sums, and more than half of the CUs have to be
+// in it: below that the split-K row is as fast (us by workgroups, row of the table / this kernel: 64 4.2 / 4.9, 128 4.9 / 4.9, 192
+// 7.1 / 5.0 for 256 features at 14x14; 64 5.2 / 6.5, 128 6.5 / 6.6, 256 10.5 / 6.8 for 512 at 7x7).  Beyond that workgroups take turns, and
+// what they compute for lanes and rows that do not exist counts: 28, 14 and 7 columns leave an eighth to a quarter idle (512 workgroups
+// 12.0 / 11.1, 768 18.4 / 15.1, 1024 19.6 / 19.1, 2048 31.2 / 34.3 for 256 features; 1024 34.1 / 31.5, 2048 54.4 / 60.2 for 512), 17
+// and 20 columns a half (384 8.8 / 10.0, 768 11.5 / 14.1).  One block of 32 features to a wave is the least work beside the same fixed
+// cost: 768 workgroups 12.8 / 11.0, 1024 12.9 / 13.1.
+bool plane_pays(const ConvProblem& p, const PlanePlan& s, int cus)
+{
+    const double used = (double)p.B * p.OH * p.OW * s.ftiles / ((double)s.total * s.np * 32);
+    if (s.total <= cus) return s.total * 2 > cus && used > 0.4;
+    return used > 0.75 && s.total <= (s.jobs == 1 ? 3 : 4) * cus;
+}
+
+void plane_pack_weights(const ConvProblem& p, const PlanePlan& s, const int8_t* w, int8_t* packed)
+{
+    for (int ft = 0; ft < s.ftiles; ++ft)
+        for (int wave = 0; wave < 4; ++wave)
+            for (int j = 0; j < s.jobs; ++j)
+                for (int tap = 0; tap < 9; ++tap)
+                    for (int lane = 0; lane < 64; ++lane)
+                        for (int k = 0; k < 16; ++k, ++packed) {
+                            // the order of the rows gives a lane 16 consecutive features
+                            const int r = lane & 31, o = ft * PLANE_FEATURES + 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
+                            const int c = (wave + 4 * j) * 32 + (lane >> 5) * 16 + k;
+                            *packed = o < p.OFM ? w[((size_t)o * p.IFM + c) * 9 + tap] : 0;
+                        }
+}
+
+void launch_conv_plane(hipStream_t st, const ConvProblem& p, const PlanePlan& s, const void* packed, const int32_t* acc_init, const Epilogue& epi,
+                       const FastEpi& fe, const void* in, void* out, int32_t* raw)
+{
+    PlaneArgs a{};
+    a.in = (const int8_t*)in, a.wpk = (const v4i*)packed, a.acc_init = acc_init, a.calib = epi.calib, a.out = (int8_t*)out, a.raw = raw;
+    a.hi = fe.hi, a.lo = fe.lo;
+    a.in_pb = (int32_t)p.in_p.pb, a.in_pf = (int32_t)p.in_p.pf, a.in_py = (int32_t)p.in_p.py;
+    a.in_off = (int32_t)p.in_p.off - p.py * a.in_py - p.px * 16;
+    a.out_off = (int32_t)p.out_p.off, a.out_pb = (int32_t)p.out_p.pb, a.out_pf = (int32_t)p.out_p.pf, a.out_py = (int32_t)p.out_p.py;
+    a.OFM = p.OFM, a.OH = p.OH, a.OW = p.OW, a.B = p.B;
+    a.ftiles = s.ftiles, a.total = s.total, a.div_ftiles = make_fast_div((uint32_t)s.ftiles);
+    a.units = s.units, a.image_units = s.image_units, a.strips = s.strips, a.cols = s.cols, a.shift = s.shift;
+    a.div_image = make_fast_div((uint32_t)s.image_units), a.div_strips = make_fast_div((uint32_t)s.strips);
+    a.pitch = s.pitch, a.positions = s.positions;
+    a.div_patch = make_small_div((s.np + 2) * s.pitch), a.div_pitch = make_small_div(s.pitch);
+    a.jobs = s.jobs, a.kind = s.kind;
+    a.xor_mask = p.in_dt == CLDNN_HIP_U8 ? 0x80808080u : 0u;
+#define PLANE_LAUNCH(NP, NL, JOBS, POOL)                                                                                             \
+    {                                                                                                                                \
+        if (a.xor_mask) hipLaunchKernelGGL((conv_plane_kernel<NP, NL, JOBS, POOL, true>), dim3(s.grid), dim3(256), s.lds_bytes, st, a); \
+        else hipLaunchKernelGGL((conv_plane_kernel<NP, NL, JOBS, POOL, false>), dim3(s.grid), dim3(256), s.lds_bytes, st, a);          \
+    }
+#define PLANE_FORM(NP, NL, POOL)                            \
+    {                                                       \
+        if (s.jobs == 1) PLANE_LAUNCH(NP, NL, 1, POOL)      \
+        else if (s.jobs == 2) PLANE_LAUNCH(NP, NL, 2, POOL) \
+        else PLANE_LAUNCH(NP, NL, 0, POOL)                  \
+    }
+    if (p.pooled && !raw) PLANE_FORM(4, 4, true)
+    else if (s.np == 4) PLANE_FORM(4, 4, false)
+    else if (s.nl == 5) PLANE_FORM(7, 5, false)
+    else PLANE_FORM(7, 6, false)
+#undef PLANE_FORM
+#undef PLANE_LAUNCH
+    CHIP_CHECK(hipGetLastError());
+}
+
+}  // namespace chip

@@ -148,6 +148,21 @@ void stem_pack_weights(const ConvProblem& p, const StemPlan& s, const int8_t* w,
 void launch_conv_stem(hipStream_t st, const ConvProblem& p, const StemPlan& s, const void* packed, const int32_t* acc_init, const Epilogue& epi,
                       const FastEpi& fe, const void* in, void* out);
 
+// ---- nine taps at stride 1, the waves of a workgroup split K over a patch in LDS (conv_plane.hip)
+struct PlanePlan {
+    int ok;              // the kernel takes this layer
+    int kind;            // epilogue
+    int np, nl, jobs;    // fragments of 32 pixels, loads of 64 positions to a slice of the patch, blocks of 32 features to a wave
+    int strips, cols, shift, pitch, positions, image_units, units;  // conv_plane_kernel.h
+    int ftiles, total, grid, lds_bytes;
+    size_t packed_bytes;
+};
+PlanePlan plane_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e, int cus);
+bool plane_pays(const ConvProblem& p, const PlanePlan& s, int cus);  // against the table's row
+void plane_pack_weights(const ConvProblem& p, const PlanePlan& s, const int8_t* w, int8_t* packed);
+void launch_conv_plane(hipStream_t st, const ConvProblem& p, const PlanePlan& s, const void* packed, const int32_t* acc_init, const Epilogue& epi,
+                       const FastEpi& fe, const void* in, void* out, int32_t* raw);
+
 // ---- depthwise bandwidth kernel on fs_b_yx_fsv16 (conv_dw.hip)
 struct DwPlan {
     int grid, block;

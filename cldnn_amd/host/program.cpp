@@ -1039,15 +1039,34 @@ static void compile_conv(cldnn_program_impl* prog, node* n)
         }
         d.input = own;
     }
+    // a max pooling behind it that nobody else reads past
+    const bool pooled = prog->optimize_data && only_pooled(n);
+    cldnn_hip_pooling_desc pd{};
+    if (pooled) pd = pooling_descriptor(n->users[0]);
+    auto pools = [&] {
+        if (!pooled || cldnn_hip_conv_pool_output(n->conv, &pd) != CLDNN_HIP_SUCCESS) return false;
+        n->writes_for = n->users[0], n->users[0]->written_by = n;
+        return true;
+    };
+    // the kernel whose waves split K over a patch in LDS, where it is faster than the table's row; not in place of a row that pools
+    cldnn_hip_conv plane = nullptr;
+    if (!n->conv && prog->optimize_data && prog->tuning.mode == cldnn_tuning_disabled && !n->side_stream && d.impl == CLDNN_HIP_IMPL_AUTO) {
+        d.impl = CLDNN_HIP_IMPL_PLANE;
+        if (cldnn_hip_conv_create(prog->engine->h, &d, wv.data(), bias_ptr, wqf_ptr, calib_ptr, (const float*)eltw_calib, &n->conv) == CLDNN_HIP_SUCCESS
+            && pooled && !pools())
+            std::swap(plane, n->conv);
+        d.impl = CLDNN_HIP_IMPL_AUTO;
+    }
     if (!n->conv) {
         apply_tuning(prog, d, wv.data(), bias_ptr, wqf_ptr, calib_ptr, (const float*)eltw_calib);
-        hip_check(cldnn_hip_conv_create(n->side_stream ? prog->engine->side : prog->engine->h, &d, wv.data(), bias_ptr, wqf_ptr, calib_ptr,
-                                        (const float*)eltw_calib, &n->conv));
+        const cldnn_hip_status st = cldnn_hip_conv_create(n->side_stream ? prog->engine->side : prog->engine->h, &d, wv.data(), bias_ptr, wqf_ptr,
+                                                          calib_ptr, (const float*)eltw_calib, &n->conv);
+        if (!plane) hip_check(st);
     }
-    // a max pooling behind it that nobody else reads past
-    if (prog->optimize_data && only_pooled(n)) {
-        const cldnn_hip_pooling_desc pd = pooling_descriptor(n->users[0]);
-        if (cldnn_hip_conv_pool_output(n->conv, &pd) == CLDNN_HIP_SUCCESS) n->writes_for = n->users[0], n->users[0]->written_by = n;
+    if (!n->writes_for) {
+        const bool done = n->conv && pools();
+        if (plane && !done) std::swap(plane, n->conv);
+        if (plane) cldnn_hip_conv_release(plane);
     }
     hip_check(cldnn_hip_conv_get_info(n->conv, &n->conv_info));
 }

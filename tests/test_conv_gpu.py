@@ -987,6 +987,63 @@ def test_scores_written_in_plain_layouts(eng, shape, form, out_fmt):
     assert_same(ref, hip.download(eng, out))
 
 
+# ------------------------------------------------------- nine taps, the waves of a workgroup split K over a patch in LDS
+PLANES = [  # batch, features in / out, plane
+    (5, 256, 256, (14, 14)),   # two groups of columns, two blocks to a wave
+    (3, 512, 96, (7, 7)),      # four groups, the last tile half empty; four blocks to a wave
+    (2, 128, 128, (28, 28)),   # one group, one block
+    (1, 768, 17, (9, 13)),     # six blocks, a last slice of one feature
+    (2, 256, 33, (17, 35)),    # two strips of columns, rows that do not divide the plane
+    (1, 128, 64, (6, 301)),    # strips that do not either
+    (40, 256, 48, (1, 1)),
+    (11, 128, 32, (3, 6)),     # planes smaller than a group
+    (1, 1024, 32, (16, 16)),   # groups as wide as they can be
+    (1, 256, 40, (32, 32)),
+    (2, 256, 32, (8, 8)),
+]
+
+
+@pytest.mark.parametrize("in_dt,out_dt,act", [(np.int8, "s8", "relu"), (np.uint8, "u8", "relu"), (np.uint8, "s8", "none")], ids=["s8_relu", "u8_relu", "u8_linear"])
+@pytest.mark.parametrize("pooled", [False, True], ids=["plain", "pooled"])
+@pytest.mark.parametrize("case", PLANES, ids=lambda c: "%dx%d-%d_%dx%d" % (c[0], c[1], c[2], *c[3]))
+def test_waves_that_split_k_over_a_patch(eng, case, pooled, in_dt, out_dt, act):
+    B, ifm, ofm, (H, W) = case
+    if pooled and act != "relu":
+        pytest.skip("maxima are taken before a requantisation that never falls")
+    if pooled:
+        H, W = H + H % 2, W + W % 2
+    r = np.random.default_rng(ifm + ofm + H)
+    lo, hi = (0, 256) if in_dt == np.uint8 else (-128, 128)
+    x = r.integers(lo, hi, (B, ifm, H, W)).astype(in_dt)
+    w = r.integers(-127, 128, (ofm, ifm, 3, 3)).astype(np.int8)
+    bias = r.integers(-1000, 1001, ofm).astype(np.int32)
+    calib = (r.uniform(0.5, 2.0, ofm) * 40.0 / (np.sqrt(ifm * 9) * (147.4 if in_dt == np.uint8 else 73.9) * 73.3)).astype(np.float32)
+    ref, ref_acc = rc.conv(x, w, bias, wqf=np.ones(ofm, np.float32), calib=calib, pad=(1, 1), out_dt=out_dt, act=act, want_acc=True)
+    src = hip.upload(eng, x, "fs_b_yx_fsv16", (2, 1))
+    d = hip.conv_desc(src.tensor, w.shape, out_dt, pad=(1, 1), out_fmt=hip.FS_B_YX_FSV16, out_pad=(1, 2), bias_dt=hip.I32, has_wqf=True, has_calib=True, act=act,
+                      impl=hip.IMPL_PLANE, tile=1)
+    c = hip.Conv(eng, d, w, bias, np.ones(ofm, np.float32), calib)
+    out = d.output
+    if pooled:
+        pd = hip.PoolingDesc()
+        pd.input, pd.output = d.output, hip.Tensor.make(d.output.dtype, hip.FS_B_YX_FSV16, B, ofm, H // 2, W // 2, 1, 2)
+        pd.mode, pd.size_y, pd.size_x, pd.stride_y, pd.stride_x = hip.POOL_MAX, 2, 2, 2, 2
+        assert hip.lib().cldnn_hip_conv_pool_output(c.h, C.byref(pd)) == 0
+        out = pd.output
+        ref = ref.reshape(B, ofm, H // 2, 2, W // 2, 2).max(axis=(3, 5))
+    assert c.info().kernel_name.startswith(b"conv_plane<"), c.info().kernel_name
+    dst = hip.Buffer(eng, out)
+    for _ in range(2):
+        c.enqueue(src, dst)
+    eng.finish()
+    bad = np.argwhere(hip.download(eng, dst) != ref)
+    assert bad.size == 0, "%d differ, first at %s" % (len(bad), bad[0])
+    np.testing.assert_array_equal(c.accumulators(src), ref_acc)
+    assert np.count_nonzero(np.frombuffer(dst.read_raw(), np.int8)) == np.count_nonzero(ref)  # the border stays zero
+    for b in (c, src, dst):
+        b.close()
+
+
 # ------------------------------------------------------- first layers that read a plain image themselves
 STEMS = [  # batch, features in / out, filter, stride, padding, plane
     (2, 3, 64, (7, 7), (2, 2), (3, 3), (41, 67)),     # ResNet's, odd plane

@@ -991,6 +991,32 @@ def test_recorded_launches_over_many_runs(pool, output_in_the_middle):
         np.testing.assert_array_equal(outs["out"].get_memory().read(), expected)
 
 
+@pytest.mark.parametrize("case", [(12, 256, 256, 14, False, True), (16, 256, 256, 14, True, True), (96, 128, 64, 28, True, False)],
+                         ids=["plain", "pooled", "left_to_a_row_that_pools"])
+def test_split_k_over_a_patch_through_network(eng, case):
+    """where it is the faster kernel, with the pooling behind it or, if that would make it the slower one, in neither"""
+    B, C, M, side, pooled, plane = case
+    r = np.random.default_rng(3)
+    x = r.integers(-128, 128, (B, C, side, side)).astype(np.int8)
+    w, b, q, c = rand_layer(r, M, C, 3, False)
+    prims = [cl.input_layout("input", cl.layout(DT.i8, F.bfyx, cl.tensor(B, C, side, side)))]
+    prims += [cl.data(n, m) for n, m in zip("wbqc", [cl.make_memory(eng, w)] + [vec_mem(eng, v) for v in (b, q, c)])]
+    prims.append(cl.convolution("conv", "input", ["w"], ["b"], ["q"], ["c"], input_offset=cl.tensor(0, 0, -1, -1, 0), with_activation=True, output_data_type=DT.i8))
+    if pooled:
+        prims.append(cl.pooling("pool", "conv", cl.pooling_mode.max, size=cl.tensor(1, 1, 2, 2), stride=cl.tensor(1, 1, 2, 2)))
+    last = "pool" if pooled else "conv"
+    prims.append(cl.reorder("out", last, cl.layout(DT.i8, F.bfyx, cl.tensor(B, M, side // (1 + pooled), side // (1 + pooled)))))
+    net = cl.network(eng, cl.topology(*prims), cl.build_options(optimize_data=True, outputs=["out"]))
+    kernel = str(net.get_primitive_info("conv"))
+    assert ("conv_plane<" in kernel) == plane, kernel
+    assert ("pooled" in kernel) == (pooled and plane), kernel
+    net.set_input_data("input", cl.make_memory(eng, x))
+    got = net.execute()["out"].get_memory().read()
+    some = [0, B - 1]
+    ref = rc.conv(x[some], w, b, wqf=q, calib=c, pad=(1, 1), out_dt="s8", act="relu")
+    np.testing.assert_array_equal(got[some], rc.pool(ref, "max", (2, 2), (2, 2)) if pooled else ref)
+
+
 def test_large_launches_and_profiling_engines_record_nothing():
     """9.7 Gop to a launch: one by one; an engine with profiling has an event behind every launch"""
     e = cl.engine()
