@@ -86,8 +86,8 @@ void describe_plane(cldnn_hip_conv c)
 {
     const PlanePlan& s = c->pplan;
     cldnn_hip_conv_info& inf = c->info;
-    inf.tile_pixels = s.np * 32, inf.tile_ofm = 32, inf.grid = s.grid, inf.block = 256, inf.lds_bytes = s.lds_bytes;
-    std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_plane<%d groups of %dx%d,%d blocks%s,fast>", 32 >> s.shift, s.np, s.cols, s.jobs,
+    inf.tile_pixels = s.np * 32, inf.tile_ofm = s.wide ? 128 : 32, inf.grid = s.grid, inf.block = 256, inf.lds_bytes = s.lds_bytes;
+    std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_plane%s<%d groups of %dx%d,%d blocks%s,fast>", s.wide ? "_wide" : "", 32 >> s.shift, s.np, s.cols, s.jobs,
                   c->p.pooled ? ",pooled" : "");
 }
 
@@ -285,8 +285,8 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
     if (impl == CLDNN_HIP_IMPL_PLANE) {
         Epilogue probe = e;
         probe.bias = bias && d.bias_dtype == CLDNN_HIP_F32 ? (const void*)weights : nullptr;
-        if (c->fast) c->pplan = plane_plan(p, c->fe, probe, c->engine->props.multiProcessorCount);
-        CHIP_REQUIRE(c->pplan.ok && (d.tile_override == 1 || plane_pays(p, c->pplan, c->engine->props.multiProcessorCount)), CLDNN_HIP_UNSUPPORTED_FORMAT,
+        if (c->fast) c->pplan = plane_plan(p, c->fe, probe, c->engine->props.multiProcessorCount, d.tile_override - 1);
+        CHIP_REQUIRE(c->pplan.ok && (d.tile_override > 0 || plane_pays(p, c->pplan, c->engine->props.multiProcessorCount)), CLDNN_HIP_UNSUPPORTED_FORMAT,
                      "the patch kernel does not take this convolution");
     }
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE && e.fc) c->fast = false;  // the depthwise kernels have no short fully_connected form
@@ -804,8 +804,8 @@ cldnn_hip_status cldnn_hip_conv_pool_output(cldnn_hip_conv c, const cldnn_hip_po
             CHIP_REQUIRE(halves && !p.pooled && tensor_elems(o) < (1ull << 31), CLDNN_HIP_UNSUPPORTED_FORMAT, "this convolution cannot pool its own result");
             ConvProblem q = p;
             q.pooled = 1, q.out_t = o, q.out_p = make_pitch(o);
-            const PlanePlan s = plane_plan(q, c->fe, c->epi, c->engine->props.multiProcessorCount);
-            CHIP_REQUIRE(s.ok && (c->desc.tile_override == 1 || plane_pays(q, s, c->engine->props.multiProcessorCount)), CLDNN_HIP_UNSUPPORTED_FORMAT,
+            const PlanePlan s = plane_plan(q, c->fe, c->epi, c->engine->props.multiProcessorCount, c->desc.tile_override - 1);
+            CHIP_REQUIRE(s.ok && (c->desc.tile_override > 0 || plane_pays(q, s, c->engine->props.multiProcessorCount)), CLDNN_HIP_UNSUPPORTED_FORMAT,
                          "this convolution cannot pool its own result");
             p = q, c->pplan = s;
             c->info.bytes -= (int64_t)p.B * p.OFM * ((int64_t)p.OH * p.OW - (int64_t)o.y * o.x);

@@ -10,13 +10,13 @@ namespace {
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 struct Form {
-    int np, nl;  // fragments (rows of a group), loads of 64 positions
+    int wide, np, nl;  // 128 features and all of K to a wave; fragments (rows of a group), loads of 64 positions
 };
-constexpr Form FORMS[] = {{4, 4}, {7, 5}, {7, 6}};
+constexpr Form FORMS[] = {{0, 4, 4}, {0, 7, 5}, {0, 7, 6}, {1, 7, 5}, {1, 7, 6}, {1, 8, 6}};
 
 }  // namespace
 
-PlanePlan plane_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e, int cus)
+static PlanePlan form_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e, int cus, int wide)
 {
     PlanePlan best{};
     if (p.FY != 3 || p.FX != 3 || p.sy != 1 || p.sx != 1 || p.dy != 1 || p.dx != 1 || p.groups != 1 || p.by_span || p.plain_out) return best;
@@ -27,12 +27,14 @@ PlanePlan plane_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e, 
     if (p.pooled && (!f.relu_folded || p.OH % 2 || p.OW % 2)) return best;
     if (tensor_elems(p.in_t) >= (1ull << 31) || tensor_elems(p.out_t) >= (1ull << 31)) return best;
     if (p.in_p.py >= (1 << 24) || p.out_p.py >= (1 << 24)) return best;  // 24-bit products
-    const int jobs = p.IFM / 128, ftiles = ceil_div(p.OFM, PLANE_FEATURES);
-    if (p.IFM % 128 || (jobs != 1 && jobs % 2)) return best;
+    const int spans = ceil_div(p.OFM, PLANE_FEATURES);
+    if (p.IFM % 64) return best;
     double least = 0;
     for (const Form& form : FORMS) {
-        if (p.pooled && form.np % 2) continue;
+        if (form.wide != wide || (form.np == 8 ? !p.pooled : p.pooled && form.np % 2)) continue;
         PlanePlan s{};
+        s.wide = form.wide, s.jobs = p.IFM / (form.wide ? 32 : 128), s.ftiles = form.wide ? ceil_div(spans, 4) : spans;
+        if (!form.wide && (p.IFM % 128 || (s.jobs != 1 && s.jobs % 2))) continue;
         s.strips = ceil_div(p.OW, 32), s.cols = ceil_div(p.OW, s.strips);
         if (p.pooled) s.cols += s.cols % 2;
         s.strips = ceil_div(p.OW, s.cols);
@@ -41,54 +43,68 @@ PlanePlan plane_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e, 
         s.pitch = s.cols + 2, s.positions = groups * (form.np + 2) * s.pitch;
         if (s.positions > form.nl * 64) continue;
         s.image_units = ceil_div(p.OH, form.np) * s.strips;
-        if ((int64_t)p.B * s.image_units * ftiles >= (1 << 30)) continue;
+        if ((int64_t)p.B * s.image_units * spans >= (1 << 30)) continue;
         s.units = p.B * s.image_units;
-        s.total = ceil_div(s.units, groups) * ftiles;
+        s.total = ceil_div(s.units, groups) * s.ftiles;
         // (512 bytes: what idle lanes read past the end)
-        s.lds_bytes = std::max((jobs == 1 ? 1 : 2) * 4 * 2 * s.positions * 16 + 512, PLANE_MEET * 4 * 4096);
+        s.lds_bytes = form.wide ? 3 * 2 * s.positions * 16 + 512 : std::max((s.jobs == 1 ? 1 : 2) * 4 * 2 * s.positions * 16 + 512, PLANE_MEET * 4 * 4096);
         // clocks: what a workgroup's matrix instructions take, and what it waits for at its start and its end
         const int resident = s.lds_bytes <= 80 * 1024 ? 2 : 1;
         const int64_t full = s.total / (cus * resident), left = s.total % (cus * resident);
-        const double work = form.np * 9 * jobs * 32.0, idle = 5000.0;
+        const double work = form.np * 9 * s.jobs * 32.0, idle = 5000.0;
         const double cost = full * (resident * work + idle) + (left > cus ? 2 * work + idle : left ? work + idle : 0);
         if (best.ok && cost >= least) continue;
         least = cost;
-        s.ok = 1, s.np = form.np, s.nl = form.nl, s.jobs = jobs, s.ftiles = ftiles;
+        s.ok = 1, s.np = form.np, s.nl = form.nl, s.spans = spans;
         s.grid = ceil_div(s.total, 8) * 8;
         s.kind = f.relu_folded ? EPI_KIND_RELU : EPI_KIND_LINEAR;
-        s.packed_bytes = (size_t)ftiles * 4 * jobs * 9 * 1024;
+        s.packed_bytes = (size_t)spans * (p.IFM / 32) * 9 * 1024;
         best = s;
     }
     return best;
 }
 
-// Up to a workgroup per CU the launch is one prologue, one loop and one meeting of the sums, and more than half of the CUs have to be
-// in it: below that the split-K row is as fast (us by workgroups, row of the table / this kernel: 64 4.2 / 4.9, 128 4.9 / 4.9, 192
-// 7.1 / 5.0 for 256 features at 14x14; 64 5.2 / 6.5, 128 6.5 / 6.6, 256 10.5 / 6.8 for 512 at 7x7).  Beyond that workgroups take turns, and
-// what they compute for lanes and rows that do not exist counts: 28, 14 and 7 columns leave an eighth to a quarter idle (512 workgroups
-// 12.0 / 11.1, 768 18.4 / 15.1, 1024 19.6 / 19.1, 2048 31.2 / 34.3 for 256 features; 1024 34.1 / 31.5, 2048 54.4 / 60.2 for 512), 17
-// and 20 columns a half (384 8.8 / 10.0, 768 11.5 / 14.1).  One block of 32 features to a wave is the least work beside the same fixed
-// cost: 768 workgroups 12.8 / 11.0, 1024 12.9 / 13.1.
+// Narrow form.  Up to a workgroup per CU the launch is one prologue, one loop and one meeting of the sums, and more than half of the CUs
+// have to be in it: below that the split-K row is as fast (us by workgroups, row of the table / this kernel: 64 4.2 / 4.9, 128 4.9 /
+// 4.9, 192 7.1 / 4.9 for 256 features at 14x14; 64 5.2 / 6.5, 128 6.5 / 6.6, 256 10.5 / 6.6 for 512 at 7x7).  Beyond that workgroups
+// take turns: 512 11.8 / 10.1, 768 18.0 / 14.0, 1024 18.9 / 17.4, 2048 30.7 / 32.7 for 256 features, 1024 34.3 / 30.5, 2048 55.3 / 59.5
+// for 512.  One block of 32 features to a wave is the least work beside the same fixed cost: 768 12.3 / 10.6, 1024 12.7 / 12.5.
+// Wide form, for which more than five eighths of the CUs have to have a workgroup: 128 features at 28x28, 128 workgroups 8.4 / 8.8,
+// 192 12.3 / 9.0, 256 12.7 / 9.4, 384 18.5 / 14.6, 512 18.7 / 16.3; 512 at 28x28, 256 34.3 / 26.6, 512 55.3 / 51.1, 1024 110 / 99.4.  Where
+// both would do it is the faster one (192 workgroups: 9.0 against 10.6, 13.4 against 14.0, 22.6 against 23.0).
+// Both compute for lanes, rows and features that do not exist: 28, 14 and 7 columns leave an eighth or a quarter idle, 20 or 17 columns
+// a half (256 features at 20x20, 16 images 11.8 / 13.1, 64 31.0 / 39.4), 64 output features half of the wide form's 128 (14.0 / 18.4).
+static double used(const ConvProblem& p, const PlanePlan& s)
+{
+    return (double)p.B * p.OH * p.OW * p.OFM / ((double)s.total * s.np * 32 * PLANE_FEATURES * (s.wide ? 4 : 1));
+}
+
 bool plane_pays(const ConvProblem& p, const PlanePlan& s, int cus)
 {
-    const double used = (double)p.B * p.OH * p.OW * s.ftiles / ((double)s.total * s.np * 32);
-    if (s.total <= cus) return s.total * 2 > cus && used > 0.4;
-    return used > 0.75 && s.total <= (s.jobs == 1 ? 3 : 4) * cus;
+    if (s.wide) return s.total * 8 > 5 * cus && used(p, s) > 0.76;
+    if (s.total <= cus) return s.total * 2 > cus && used(p, s) > 0.7;
+    return s.total <= (s.jobs == 1 ? 3 : 4) * cus && used(p, s) > 0.76;
+}
+
+PlanePlan plane_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e, int cus, int only)
+{
+    if (only >= 0) return form_plan(p, f, e, cus, only);
+    const PlanePlan wide = form_plan(p, f, e, cus, 1);
+    return wide.ok && plane_pays(p, wide, cus) ? wide : form_plan(p, f, e, cus, 0);
 }
 
 void plane_pack_weights(const ConvProblem& p, const PlanePlan& s, const int8_t* w, int8_t* packed)
 {
-    for (int ft = 0; ft < s.ftiles; ++ft)
-        for (int wave = 0; wave < 4; ++wave)
-            for (int j = 0; j < s.jobs; ++j)
-                for (int tap = 0; tap < 9; ++tap)
-                    for (int lane = 0; lane < 64; ++lane)
-                        for (int k = 0; k < 16; ++k, ++packed) {
-                            // the order of the rows gives a lane 16 consecutive features
-                            const int r = lane & 31, o = ft * PLANE_FEATURES + 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
-                            const int c = (wave + 4 * j) * 32 + (lane >> 5) * 16 + k;
-                            *packed = o < p.OFM ? w[((size_t)o * p.IFM + c) * 9 + tap] : 0;
-                        }
+    for (int span = 0; span < s.spans; ++span)
+        for (int block = 0; block < p.IFM / 32; ++block)
+            for (int tap = 0; tap < 9; ++tap)
+                for (int lane = 0; lane < 64; ++lane)
+                    for (int k = 0; k < 16; ++k, ++packed) {
+                        // the order of the rows gives a lane 16 consecutive features
+                        const int r = lane & 31, o = span * PLANE_FEATURES + 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
+                        const int c = block * 32 + (lane >> 5) * 16 + k;
+                        *packed = o < p.OFM ? w[((size_t)o * p.IFM + c) * 9 + tap] : 0;
+                    }
 }
 
 void launch_conv_plane(hipStream_t st, const ConvProblem& p, const PlanePlan& s, const void* packed, const int32_t* acc_init, const Epilogue& epi,
@@ -101,7 +117,7 @@ void launch_conv_plane(hipStream_t st, const ConvProblem& p, const PlanePlan& s,
     a.in_off = (int32_t)p.in_p.off - p.py * a.in_py - p.px * 16;
     a.out_off = (int32_t)p.out_p.off, a.out_pb = (int32_t)p.out_p.pb, a.out_pf = (int32_t)p.out_p.pf, a.out_py = (int32_t)p.out_p.py;
     a.OFM = p.OFM, a.OH = p.OH, a.OW = p.OW, a.B = p.B;
-    a.ftiles = s.ftiles, a.total = s.total, a.div_ftiles = make_fast_div((uint32_t)s.ftiles);
+    a.spans = s.spans, a.ftiles = s.ftiles, a.total = s.total, a.div_ftiles = make_fast_div((uint32_t)s.ftiles);
     a.units = s.units, a.image_units = s.image_units, a.strips = s.strips, a.cols = s.cols, a.shift = s.shift;
     a.div_image = make_fast_div((uint32_t)s.image_units), a.div_strips = make_fast_div((uint32_t)s.strips);
     a.pitch = s.pitch, a.positions = s.positions;
@@ -119,10 +135,20 @@ void launch_conv_plane(hipStream_t st, const ConvProblem& p, const PlanePlan& s,
         else if (s.jobs == 2) PLANE_LAUNCH(NP, NL, 2, POOL) \
         else PLANE_LAUNCH(NP, NL, 0, POOL)                  \
     }
-    if (p.pooled && !raw) PLANE_FORM(4, 4, true)
+#define PLANE_WIDE(NP, NL, POOL)                                                                                                        \
+    {                                                                                                                                \
+        if (a.xor_mask) hipLaunchKernelGGL((conv_plane_wide_kernel<NP, NL, POOL, true>), dim3(s.grid), dim3(256), s.lds_bytes, st, a);  \
+        else hipLaunchKernelGGL((conv_plane_wide_kernel<NP, NL, POOL, false>), dim3(s.grid), dim3(256), s.lds_bytes, st, a);            \
+    }
+    if (s.wide && p.pooled && !raw) PLANE_WIDE(8, 6, true)
+    else if (s.wide && s.np == 8) PLANE_WIDE(8, 6, false)
+    else if (s.wide && s.nl == 5) PLANE_WIDE(7, 5, false)
+    else if (s.wide) PLANE_WIDE(7, 6, false)
+    else if (p.pooled && !raw) PLANE_FORM(4, 4, true)
     else if (s.np == 4) PLANE_FORM(4, 4, false)
     else if (s.nl == 5) PLANE_FORM(7, 5, false)
     else PLANE_FORM(7, 6, false)
+#undef PLANE_WIDE
 #undef PLANE_FORM
 #undef PLANE_LAUNCH
     CHIP_CHECK(hipGetLastError());

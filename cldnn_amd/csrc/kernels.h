@@ -152,12 +152,14 @@ void launch_conv_stem(hipStream_t st, const ConvProblem& p, const StemPlan& s, c
 struct PlanePlan {
     int ok;              // the kernel takes this layer
     int kind;            // epilogue
+    int wide;            // 128 features to a workgroup, all of K to a wave
     int np, nl, jobs;    // fragments of 32 pixels, loads of 64 positions to a slice of the patch, blocks of 32 features to a wave
     int strips, cols, shift, pitch, positions, image_units, units;  // conv_plane_kernel.h
-    int ftiles, total, grid, lds_bytes;
+    int spans, ftiles, total, grid, lds_bytes;
     size_t packed_bytes;
 };
-PlanePlan plane_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e, int cus);
+// only: 0 or 1 for the narrow or the wide form, below for the faster one
+PlanePlan plane_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e, int cus, int only = -1);
 bool plane_pays(const ConvProblem& p, const PlanePlan& s, int cus);  // against the table's row
 void plane_pack_weights(const ConvProblem& p, const PlanePlan& s, const int8_t* w, int8_t* packed);
 void launch_conv_plane(hipStream_t st, const ConvProblem& p, const PlanePlan& s, const void* packed, const int32_t* acc_init, const Epilogue& epi,

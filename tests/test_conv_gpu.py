@@ -987,7 +987,7 @@ def test_scores_written_in_plain_layouts(eng, shape, form, out_fmt):
     assert_same(ref, hip.download(eng, out))
 
 
-# ------------------------------------------------------- nine taps, the waves of a workgroup split K over a patch in LDS
+# ------------------------------------------------------- nine taps over a patch in LDS
 PLANES = [  # batch, features in / out, plane
     (5, 256, 256, (14, 14)),   # two groups of columns, two blocks to a wave
     (3, 512, 96, (7, 7)),      # four groups, the last tile half empty; four blocks to a wave
@@ -1000,18 +1000,25 @@ PLANES = [  # batch, features in / out, plane
     (1, 1024, 32, (16, 16)),   # groups as wide as they can be
     (1, 256, 40, (32, 32)),
     (2, 256, 32, (8, 8)),
+    (2, 384, 200, (13, 24)),   # twelve blocks; features that end inside a tile of 128
+    (3, 64, 130, (20, 30)),    # two blocks, a span of two features
 ]
 
 
 @pytest.mark.parametrize("in_dt,out_dt,act", [(np.int8, "s8", "relu"), (np.uint8, "u8", "relu"), (np.uint8, "s8", "none")], ids=["s8_relu", "u8_relu", "u8_linear"])
 @pytest.mark.parametrize("pooled", [False, True], ids=["plain", "pooled"])
+@pytest.mark.parametrize("wide", [False, True], ids=["split_k", "wide"])
 @pytest.mark.parametrize("case", PLANES, ids=lambda c: "%dx%d-%d_%dx%d" % (c[0], c[1], c[2], *c[3]))
-def test_waves_that_split_k_over_a_patch(eng, case, pooled, in_dt, out_dt, act):
+def test_nine_taps_over_a_patch(eng, case, wide, pooled, in_dt, out_dt, act):
     B, ifm, ofm, (H, W) = case
     if pooled and act != "relu":
         pytest.skip("maxima are taken before a requantisation that never falls")
     if pooled:
         H, W = H + H % 2, W + W % 2
+    if not wide and ifm != 128 and ifm % 256:
+        pytest.skip("four waves to share the blocks, an even number each")
+    if wide and pooled and W == 8:
+        pytest.skip("the patch of four groups of eight rows and columns is too large")
     r = np.random.default_rng(ifm + ofm + H)
     lo, hi = (0, 256) if in_dt == np.uint8 else (-128, 128)
     x = r.integers(lo, hi, (B, ifm, H, W)).astype(in_dt)
@@ -1021,7 +1028,7 @@ def test_waves_that_split_k_over_a_patch(eng, case, pooled, in_dt, out_dt, act):
     ref, ref_acc = rc.conv(x, w, bias, wqf=np.ones(ofm, np.float32), calib=calib, pad=(1, 1), out_dt=out_dt, act=act, want_acc=True)
     src = hip.upload(eng, x, "fs_b_yx_fsv16", (2, 1))
     d = hip.conv_desc(src.tensor, w.shape, out_dt, pad=(1, 1), out_fmt=hip.FS_B_YX_FSV16, out_pad=(1, 2), bias_dt=hip.I32, has_wqf=True, has_calib=True, act=act,
-                      impl=hip.IMPL_PLANE, tile=1)
+                      impl=hip.IMPL_PLANE, tile=2 if wide else 1)
     c = hip.Conv(eng, d, w, bias, np.ones(ofm, np.float32), calib)
     out = d.output
     if pooled:
@@ -1031,7 +1038,7 @@ def test_waves_that_split_k_over_a_patch(eng, case, pooled, in_dt, out_dt, act):
         assert hip.lib().cldnn_hip_conv_pool_output(c.h, C.byref(pd)) == 0
         out = pd.output
         ref = ref.reshape(B, ofm, H // 2, 2, W // 2, 2).max(axis=(3, 5))
-    assert c.info().kernel_name.startswith(b"conv_plane<"), c.info().kernel_name
+    assert c.info().kernel_name.startswith(b"conv_plane_wide<" if wide else b"conv_plane<"), c.info().kernel_name
     dst = hip.Buffer(eng, out)
     for _ in range(2):
         c.enqueue(src, dst)

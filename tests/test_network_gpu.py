@@ -991,9 +991,10 @@ def test_recorded_launches_over_many_runs(pool, output_in_the_middle):
         np.testing.assert_array_equal(outs["out"].get_memory().read(), expected)
 
 
-@pytest.mark.parametrize("case", [(12, 256, 256, 14, False, True), (16, 256, 256, 14, True, True), (96, 128, 64, 28, True, False)],
-                         ids=["plain", "pooled", "left_to_a_row_that_pools"])
-def test_split_k_over_a_patch_through_network(eng, case):
+@pytest.mark.parametrize("case", [(12, 256, 256, 14, False, "conv_plane<"), (16, 256, 256, 14, True, "conv_plane<"), (96, 128, 64, 28, True, None),
+                                  (48, 64, 128, 28, False, "conv_plane_wide<"), (13, 64, 128, 56, True, "conv_plane_wide<")],
+                         ids=["plain", "pooled", "left_to_a_row_that_pools", "wide", "wide_pooled"])
+def test_nine_taps_over_a_patch_through_network(eng, case):
     """where it is the faster kernel, with the pooling behind it or, if that would make it the slower one, in neither"""
     B, C, M, side, pooled, plane = case
     r = np.random.default_rng(3)
@@ -1008,8 +1009,8 @@ def test_split_k_over_a_patch_through_network(eng, case):
     prims.append(cl.reorder("out", last, cl.layout(DT.i8, F.bfyx, cl.tensor(B, M, side // (1 + pooled), side // (1 + pooled)))))
     net = cl.network(eng, cl.topology(*prims), cl.build_options(optimize_data=True, outputs=["out"]))
     kernel = str(net.get_primitive_info("conv"))
-    assert ("conv_plane<" in kernel) == plane, kernel
-    assert ("pooled" in kernel) == (pooled and plane), kernel
+    assert plane in kernel if plane else "conv_plane" not in kernel, kernel
+    assert ("pooled" in kernel) == (pooled and plane is not None), kernel
     net.set_input_data("input", cl.make_memory(eng, x))
     got = net.execute()["out"].get_memory().read()
     some = [0, B - 1]
