@@ -24,6 +24,7 @@ struct cldnn_hip_conv_s {
     DwPlan dplan{};
     StemPlan splan{};     // a first layer that reads its bfyx image itself
     PlanePlan pplan{};
+    PointPlan tplan{};
     // device allocations
     void* w_raw = nullptr;    // dense weights (reference kernel)
     void* w_packed = nullptr; // MFMA / depthwise operand stream
@@ -240,6 +241,9 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
     if (impl == CLDNN_HIP_IMPL_PLANE)
         CHIP_REQUIRE(blocked && int_path && d.groups == 1 && !d.fused && !e.fc && !d.sibling_split && !p.plain_out, CLDNN_HIP_UNSUPPORTED_FORMAT,
                      "the patch kernel needs int8 data in fs_b_yx_fsv16, quantisation and one group");
+    if (impl == CLDNN_HIP_IMPL_POINT)
+        CHIP_REQUIRE(blocked && int_path && d.groups == 1 && !e.fc && !p.plain_out, CLDNN_HIP_UNSUPPORTED_FORMAT,
+                     "the wide 1x1 kernel needs int8 data in fs_b_yx_fsv16, quantisation and one group");
     c->impl = impl;
 
     const int ifm_g = p.IFM / p.groups;
@@ -289,11 +293,15 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
         CHIP_REQUIRE(c->pplan.ok && (d.tile_override > 0 || plane_pays(p, c->pplan, c->engine->props.multiProcessorCount)), CLDNN_HIP_UNSUPPORTED_FORMAT,
                      "the patch kernel does not take this convolution");
     }
+    if (impl == CLDNN_HIP_IMPL_POINT) {
+        if (c->fast) c->tplan = point_plan(p, c->fe, e);
+        CHIP_REQUIRE(c->tplan.ok && (d.tile_override == 1 || point_pays(p, c->tplan, c->engine->props.multiProcessorCount)), CLDNN_HIP_UNSUPPORTED_FORMAT, "the wide 1x1 kernel does not take this convolution");
+    }
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE && e.fc) c->fast = false;  // the depthwise kernels have no short fully_connected form
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE && c->fe.f32) c->fast = false;  // nor a float one
     const bool dw_fast = impl == CLDNN_HIP_IMPL_DEPTHWISE && p.FY == 3 && p.FX == 3 && dw_fast_applies(p, c->fast);
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE) c->dplan = dw_plan(p, c->fast, c->engine->props.multiProcessorCount);
-    const bool matrix = impl == CLDNN_HIP_IMPL_MFMA || impl == CLDNN_HIP_IMPL_PLANE;
+    const bool matrix = impl == CLDNN_HIP_IMPL_MFMA || impl == CLDNN_HIP_IMPL_PLANE || impl == CLDNN_HIP_IMPL_POINT;
     const bool xor_u8 = (matrix || dw_fast || c->dplan.rows) && p.in_dt == CLDNN_HIP_U8;
     for (int f = 0; f < p.OFM; ++f) {
         int64_t s = 0;
@@ -329,6 +337,15 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
         plane_pack_weights(p, c->pplan, w8, packed.data());
         c->w_packed = upload(c, packed.data(), packed.size());
         describe_plane(c);
+        return;
+    }
+    if (impl == CLDNN_HIP_IMPL_POINT) {
+        const PointPlan& t = c->tplan;
+        std::vector<int8_t> packed(t.packed_bytes);
+        point_pack_weights(p, t, w8, packed.data());
+        c->w_packed = upload(c, packed.data(), packed.size());
+        inf.tile_pixels = 64, inf.tile_ofm = 256, inf.grid = t.grid, inf.block = 256, inf.lds_bytes = t.lds_bytes;
+        std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_point<%d blocks,%s,fast>", t.jobs, d.fused ? "sum" : d.sibling_split ? "pair" : "plain");
         return;
     }
     std::vector<int8_t> dense;
@@ -485,6 +502,9 @@ static void run(cldnn_hip_conv c, const void* in, void* out, const void* eltw, i
     }
     case CLDNN_HIP_IMPL_PLANE:
         launch_conv_plane(s, p, c->pplan, c->w_packed, (const int32_t*)(raw ? c->acc_init_raw : c->acc_init), c->epi, c->fe, in, out, raw);
+        break;
+    case CLDNN_HIP_IMPL_POINT:
+        launch_conv_point(s, p, c->tplan, c->w_packed, (const int32_t*)(raw ? c->acc_init_raw : c->acc_init), c->epi, c->fe, in, eltw, out, raw);
         break;
     case CLDNN_HIP_IMPL_DEPTHWISE:
         launch_conv_dw(s, p, c->dplan, (const int8_t*)c->w_packed, (const int32_t*)c->w_masked, (const int32_t*)c->w_rows,

@@ -165,6 +165,20 @@ void plane_pack_weights(const ConvProblem& p, const PlanePlan& s, const int8_t* 
 void launch_conv_plane(hipStream_t st, const ConvProblem& p, const PlanePlan& s, const void* packed, const int32_t* acc_init, const Epilogue& epi,
                        const FastEpi& fe, const void* in, void* out, int32_t* raw);
 
+// ---- 1x1 layers, 256 output features to a workgroup (conv_point.hip)
+struct PointPlan {
+    int ok;              // the kernel takes this layer
+    int kind;            // epilogue
+    int jobs;            // blocks of 128 input features
+    int spans, ftiles, total, grid, lds_bytes;
+    size_t packed_bytes;
+};
+PointPlan point_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e);
+bool point_pays(const ConvProblem& p, const PointPlan& s, int cus);  // against the table's row
+void point_pack_weights(const ConvProblem& p, const PointPlan& s, const int8_t* w, int8_t* packed);
+void launch_conv_point(hipStream_t st, const ConvProblem& p, const PointPlan& s, const void* packed, const int32_t* acc_init, const Epilogue& epi,
+                       const FastEpi& fe, const void* in, const void* eltw, void* out, int32_t* raw);
+
 // ---- depthwise bandwidth kernel on fs_b_yx_fsv16 (conv_dw.hip)
 struct DwPlan {
     int grid, block;

@@ -15,7 +15,7 @@ LIB_PATH = os.path.join(_HERE, "libcldnn_hip.so")
 S8, U8, I32, F32, NO_TYPE = 0, 1, 2, 3, -1
 BFYX, YXFB, BYXF, FS_B_YX_FSV16, B_FS_YX_FSV4 = 0, 1, 2, 3, 4
 ACT_NONE, ACT_RELU, ACT_RELU_SLOPE, ACT_CLAMP = 0, 1, 2, 3
-IMPL_AUTO, IMPL_REF, IMPL_MFMA, IMPL_DEPTHWISE, IMPL_PLANE = 0, 1, 2, 3, 4
+IMPL_AUTO, IMPL_REF, IMPL_MFMA, IMPL_DEPTHWISE, IMPL_PLANE, IMPL_POINT = 0, 1, 2, 3, 4, 5
 
 NP_OF = {S8: np.int8, U8: np.uint8, I32: np.int32, F32: np.float32}
 DT_OF = {np.dtype(np.int8): S8, np.dtype(np.uint8): U8, np.dtype(np.int32): I32, np.dtype(np.float32): F32}

@@ -999,6 +999,11 @@ static bool only_pooled(const node* n)
            && n->users[0]->p->type == prim_type::pooling && !n->users[0]->concat_into;
 }
 
+static bool beside_the_table(const cldnn_program_impl* prog, const cldnn_hip_conv_desc& d)
+{
+    return prog->optimize_data && prog->tuning.mode == cldnn_tuning_disabled && d.impl == CLDNN_HIP_IMPL_AUTO && d.tile_override == 0;
+}
+
 static void compile_conv(cldnn_program_impl* prog, node* n)
 {
     conv_build cb;
@@ -1048,10 +1053,10 @@ static void compile_conv(cldnn_program_impl* prog, node* n)
         n->writes_for = n->users[0], n->users[0]->written_by = n;
         return true;
     };
-    // the kernel whose waves split K over a patch in LDS, where it is faster than the table's row; not in place of a row that pools
+    // the kernels for 3x3 and 1x1 layers beside the tile table, where they are the faster; not in place of a row that pools
     cldnn_hip_conv plane = nullptr;
-    if (!n->conv && prog->optimize_data && prog->tuning.mode == cldnn_tuning_disabled && !n->side_stream && d.impl == CLDNN_HIP_IMPL_AUTO) {
-        d.impl = CLDNN_HIP_IMPL_PLANE;
+    if (!n->conv && !n->side_stream && beside_the_table(prog, d)) {
+        d.impl = d.fx == 1 ? CLDNN_HIP_IMPL_POINT : CLDNN_HIP_IMPL_PLANE;
         if (cldnn_hip_conv_create(prog->engine->h, &d, wv.data(), bias_ptr, wqf_ptr, calib_ptr, (const float*)eltw_calib, &n->conv) == CLDNN_HIP_SUCCESS
             && pooled && !pools())
             std::swap(plane, n->conv);
@@ -1136,6 +1141,15 @@ static bool compile_siblings(cldnn_program_impl* prog, node* a)
         auto join = [](std::vector<uint8_t>& x, const std::vector<uint8_t>& y) { x.insert(x.end(), y.begin(), y.end()); };
         join(ca.wv, cb.wv), join(ca.bv, cb.bv), join(ca.qv, cb.qv), join(ca.cv, cb.cv);
         cldnn_hip_conv c = nullptr;
+        if (d.fx == 1 && beside_the_table(prog, d)) {
+            d.impl = CLDNN_HIP_IMPL_POINT;
+            if (cldnn_hip_conv_create(prog->engine->h, &d, ca.weights(), ca.bias(), ca.wqf(), ca.calib(), nullptr, &c) == CLDNN_HIP_SUCCESS) {
+                a->conv = c;
+                hip_check(cldnn_hip_conv_get_info(c, &a->conv_info));
+                return true;
+            }
+            d.impl = CLDNN_HIP_IMPL_AUTO;
+        }
         apply_tuning(prog, d, ca.weights(), ca.bias(), ca.wqf(), ca.calib(), nullptr);
         const cldnn_hip_status st = cldnn_hip_conv_create(prog->engine->h, &d, ca.weights(), ca.bias(), ca.wqf(), ca.calib(), nullptr, &c);
         if (st == CLDNN_HIP_SUCCESS) {

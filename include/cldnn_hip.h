@@ -291,7 +291,11 @@ enum {
      * for 128, the waves split the output features (any multiple of 64 input features).  One group, calibrated int8 output
      * with or without a plain relu; refused otherwise, and where the tile table's row is the faster unless tile_override names
      * a form (1 or 2). */
-    CLDNN_HIP_IMPL_PLANE = 4
+    CLDNN_HIP_IMPL_PLANE = 4,
+    /* 1x1 without padding on int8 MFMA, fs_b_yx_fsv16, 256 output features to a workgroup: a multiple of 256 input features, one group,
+     * calibrated int8 output with or without a plain relu, two convolutions in one launch, or a residual sum with a relu behind
+     * it; refused otherwise, and where the tile table's row is the faster unless tile_override is 1. */
+    CLDNN_HIP_IMPL_POINT = 5
 };
 
 typedef struct {

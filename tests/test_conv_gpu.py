@@ -1051,6 +1051,51 @@ def test_nine_taps_over_a_patch(eng, case, wide, pooled, in_dt, out_dt, act):
         b.close()
 
 
+# ------------------------------------------------------- 1x1, 256 output features to a workgroup
+POINTS = [  # batch, features in / out, plane, stride
+    (2, 256, 256, (14, 14), (1, 1)),
+    (3, 512, 320, (7, 7), (1, 1)),      # a tile of features that is a quarter full
+    (1, 1024, 33, (9, 13), (2, 2)),     # a last slice of one feature, every second pixel
+    (1, 512, 1040, (5, 3), (1, 2)),     # fewer pixels than a fragment has
+    (5, 2048, 512, (4, 4), (1, 1)),
+    (1, 256, 64, (1, 129), (1, 1)),     # one pixel past a tile
+]
+
+
+@pytest.mark.parametrize("form", ["s8_relu", "u8_linear", "u8_pair", "s8_sum", "u8_sum_in_place"])
+@pytest.mark.parametrize("case", POINTS, ids=lambda c: "%dx%d-%d_%dx%d" % (c[0], c[1], c[2], *c[3]))
+def test_wide_1x1(eng, case, form):
+    B, ifm, ofm, (H, W), stride = case
+    r = np.random.default_rng(ifm + ofm + H)
+    unsigned = form.startswith("u8")
+    x = r.integers(*((0, 256) if unsigned else (-128, 128)), (B, ifm, H, W)).astype(np.uint8 if unsigned else np.int8)
+    w = r.integers(-127, 128, (ofm, ifm, 1, 1)).astype(np.int8)
+    bias = r.integers(-1000, 1001, ofm).astype(np.int32)
+    calib = (r.uniform(0.5, 2.0, ofm) * 40.0 / (np.sqrt(ifm) * (147.4 if unsigned else 73.9) * 73.3)).astype(np.float32)
+    ones = np.ones(ofm, np.float32)
+    kw = dict(stride=stride, out_dt="u8" if form == "u8_sum_in_place" else "s8", act="relu" if form == "s8_relu" else "none")
+    dev = {}
+    OH, OW = (H - 1) // stride[0] + 1, (W - 1) // stride[1] + 1
+    if "sum" in form:
+        e = r.integers(*((0, 256) if unsigned else (-128, 128)), (B, ofm, OH, OW)).astype(np.uint8 if unsigned else np.int8)
+        kw.update(eltw=e, eltw_act="relu", eltw_calib=r.uniform(0.5, 1.0, ofm).astype(np.float32))
+        dev.update(in_place="in_place" in form)
+    if form == "u8_pair":
+        if ofm <= 48:
+            pytest.skip("nothing to divide")
+        dev.update(sibling_split=48, sibling_act="relu")
+    got, acc, info = hip.conv_forward(eng, x, w, bias, ones, calib, fmt="fs_b_yx_fsv16", out_pad=(1, 2), impl=hip.IMPL_POINT, tile=1, want_acc=True, want_info=True, **kw, **dev)
+    assert info.kernel_name.startswith(b"conv_point<"), info.kernel_name
+    if form == "u8_pair":
+        sides = [rc.conv(x, w[k], bias[k], wqf=ones[k], calib=calib[k], stride=stride, out_dt="s8", act=a) for k, a in ((slice(0, 48), "none"), (slice(48, None), "relu"))]
+        ref, ref_acc = np.concatenate(sides, axis=1), rc.conv(x, w, bias, wqf=ones, calib=calib, stride=stride, out_dt="s8", want_acc=True)[1]
+    else:
+        ref, ref_acc = rc.conv(x, w, bias, wqf=ones, calib=calib, want_acc=True, **kw)
+    bad = np.argwhere(got != ref)
+    assert bad.size == 0, "%d differ, first at %s" % (len(bad), bad[0])
+    np.testing.assert_array_equal(acc, ref_acc)
+
+
 # ------------------------------------------------------- first layers that read a plain image themselves
 STEMS = [  # batch, features in / out, filter, stride, padding, plane
     (2, 3, 64, (7, 7), (2, 2), (3, 3), (41, 67)),     # ResNet's, odd plane

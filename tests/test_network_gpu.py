@@ -613,7 +613,7 @@ def test_events_and_profiling():
     prof = ev.get_profiling_info()
     assert set(prof) == {"submission", "starting", "executing"}
     assert 0 < prof["executing"] < 50_000_000
-    np.testing.assert_array_equal(outs["out"].get_memory().read(), oracle())
+    np.testing.assert_array_equal(outs["out"].get_memory().read(), oracle()[1])
     fired = []
     cb = cl.EVENT_HANDLER(lambda p: fired.append(1))
     cl._call("cldnn_add_event_handler", ev.h, cb, None)
@@ -641,7 +641,7 @@ def test_execute_behind_a_user_event_that_is_set_afterwards(profiling):
     assert fired == []                           # one gate is still closed
     gate_b.set()                                 # submits the run from this thread
     ev.wait()
-    np.testing.assert_array_equal(outs["out"].get_memory().read(), oracle())
+    np.testing.assert_array_equal(outs["out"].get_memory().read(), oracle()[1])
     import time
     for _ in range(200):                         # the handler of a stream event is called from a helper thread
         if fired:
@@ -662,7 +662,7 @@ def test_execute_behind_a_user_event_that_is_set_afterwards(profiling):
     outs = net.execute([gate_c])
     threading.Timer(0.05, gate_c.set).start()
     net.set_input_data("input", cl.make_memory(eng, x2))   # blocks until the timer opens the gate and the run is over
-    np.testing.assert_array_equal(outs["out"].get_memory().read(), oracle())
+    np.testing.assert_array_equal(outs["out"].get_memory().read(), oracle()[1])
 
 
 def test_unsupported_requests_fail_loudly(eng):
@@ -1016,6 +1016,17 @@ def test_nine_taps_over_a_patch_through_network(eng, case):
     some = [0, B - 1]
     ref = rc.conv(x[some], w, b, wqf=q, calib=c, pad=(1, 1), out_dt="s8", act="relu")
     np.testing.assert_array_equal(got[some], rc.pool(ref, "max", (2, 2), (2, 2)) if pooled else ref)
+
+
+@pytest.mark.parametrize("batch,wide", [(40, True), (8, False)])
+def test_wide_1x1_through_network(eng, batch, wide):
+    """two convolutions in one launch and one with a sum behind it: on the wide kernel where pixels are many"""
+    topo, x, oracle = projection_block(eng, 8, B=batch, C=256, M=256, H=16, W=16)
+    net = cl.network(eng, topo, cl.build_options(optimize_data=True, outputs=["out"]))
+    kernels = [net.get_primitive_info(n)["kernel"] for n in ("shortcut", "expand_fused_sum")]
+    assert all(k.startswith("conv_point<") == wide for k in kernels), kernels
+    net.set_input_data("input", cl.make_memory(eng, x))
+    np.testing.assert_array_equal(net.execute()["out"].get_memory().read(), oracle()[1])
 
 
 def test_large_launches_and_profiling_engines_record_nothing():
