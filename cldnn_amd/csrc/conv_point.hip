@@ -7,15 +7,16 @@ namespace chip {
 
 static int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
-// From a workgroup for every second CU on, and with nine tenths of the features of the tiles in use.  Us by workgroups, row of the table
-// / this kernel: 256 -> 1024 with a sum at 14x14 104 4.8 / 5.5, 200 6.0 / 5.7, 392 8.0 / 7.3; 512 -> 256 + 1024 from 28x28 128 6.5 / 5.4,
-// 248 8.5 / 6.1; 1024 -> 256 at 14x14 104 6.3 / 6.7, 200 8.6 / 6.9; 2048 -> 512 at 7x7 104 8.8 / 9.8, 200 13.7 / 12.2; 512 -> 256 at 28x28 56
-// 4.0 / 5.1, 152 6.8 / 5.3, 1232 20.6 / 17.2.  640 output features, five sixths in use: 13.2 / 12.7, 39.0 / 39.2; 128, a half: 15.9 / 21.1.
+// From a workgroup for every second CU on, with sums for every CU, and with nine tenths of the features of the tiles in use.  Us by
+// workgroups, row of the table / this kernel: 512 -> 256 + 1024 from 28x28 128 6.5 / 5.4, 248 8.5 / 6.1; 1024 -> 256 at 14x14 104 6.3 / 6.7,
+// 200 8.6 / 6.9; 512 -> 256 at 28x28 56 4.0 / 5.1, 152 6.8 / 5.3, 1232 20.6 / 17.2; with a sum 256 -> 1024 at 14x14 104 4.8 / 5.5, 200 6.0 /
+// 5.7, 392 8.0 / 7.3, and 512 -> 2048 at 7x7 200 7.2 / 6.5 alone, but 8.5 / 9.0 between other layers.  640 output features, five sixths in
+// use: 13.2 / 12.7, 39.0 / 39.2; 128, a half: 15.9 / 21.1.
 // Up to 1024 input features: a block's successor is requested 600 clocks ahead, enough where the weights lie in L2, and a workgroup reads
 // all of its 256 features' (2048 -> 512 at batch 128 alone 13.7 / 12.2, between other layers, its weights in memory, 14.3 / 18.4).
 bool point_pays(const ConvProblem& p, const PointPlan& s, int cus)
 {
-    return p.IFM <= 1024 && s.total * 2 > cus && p.OFM * 10 >= s.ftiles * POINT_FEATURES * 9;
+    return p.IFM <= 1024 && s.total * (s.kind == EPI_KIND_FUSED ? 1 : 2) > cus && p.OFM * 10 >= s.ftiles * POINT_FEATURES * 9;
 }
 
 PointPlan point_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e)

@@ -1018,7 +1018,7 @@ def test_nine_taps_over_a_patch_through_network(eng, case):
     np.testing.assert_array_equal(got[some], rc.pool(ref, "max", (2, 2), (2, 2)) if pooled else ref)
 
 
-@pytest.mark.parametrize("batch,wide", [(40, True), (8, False)])
+@pytest.mark.parametrize("batch,wide", [(66, True), (8, False)])
 def test_wide_1x1_through_network(eng, batch, wide):
     """two convolutions in one launch and one with a sum behind it: on the wide kernel where pixels are many"""
     topo, x, oracle = projection_block(eng, 8, B=batch, C=256, M=256, H=16, W=16)
