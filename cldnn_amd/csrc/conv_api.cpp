@@ -244,6 +244,21 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
     if (impl == CLDNN_HIP_IMPL_POINT)
         CHIP_REQUIRE(blocked && int_path && d.groups == 1 && !e.fc && !p.plain_out, CLDNN_HIP_UNSUPPORTED_FORMAT,
                      "the wide 1x1 kernel needs int8 data in fs_b_yx_fsv16, quantisation and one group");
+    if (impl == CLDNN_HIP_IMPL_PLANE || impl == CLDNN_HIP_IMPL_POINT) {  // before anything is uploaded: a caller may only be asking
+        const int cus = c->engine->props.multiProcessorCount;
+        Epilogue probe = e;
+        probe.bias = bias && d.bias_dtype == CLDNN_HIP_F32 ? (const void*)weights : nullptr;
+        probe.calib = calib_on ? calib : nullptr, probe.eltw_calib = eltw_calib;
+        bool takes = mfma_fast_epilogue(p, probe, calib_on ? calib : nullptr, eltw_calib, wqf, &c->fe);
+        if (takes && impl == CLDNN_HIP_IMPL_PLANE) {
+            c->pplan = plane_plan(p, c->fe, probe, cus, d.tile_override - 1);
+            takes = c->pplan.ok && (d.tile_override > 0 || plane_pays(p, c->pplan, cus));
+        } else if (takes) {
+            c->tplan = point_plan(p, c->fe, probe);
+            takes = c->tplan.ok && (d.tile_override > 0 || point_pays(p, c->tplan, cus));
+        }
+        CHIP_REQUIRE(takes, CLDNN_HIP_UNSUPPORTED_FORMAT, "this kernel does not take the convolution");
+    }
     c->impl = impl;
 
     const int ifm_g = p.IFM / p.groups;
@@ -285,17 +300,6 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
         Epilogue probe = e;
         probe.bias = bias && (d.bias_dtype == CLDNN_HIP_F32 || e.fc) ? (const void*)weights : nullptr;
         c->fast = mfma_fast_epilogue(p, probe, calib_on ? calib : nullptr, eltw_calib, wqf, &c->fe);
-    }
-    if (impl == CLDNN_HIP_IMPL_PLANE) {
-        Epilogue probe = e;
-        probe.bias = bias && d.bias_dtype == CLDNN_HIP_F32 ? (const void*)weights : nullptr;
-        if (c->fast) c->pplan = plane_plan(p, c->fe, probe, c->engine->props.multiProcessorCount, d.tile_override - 1);
-        CHIP_REQUIRE(c->pplan.ok && (d.tile_override > 0 || plane_pays(p, c->pplan, c->engine->props.multiProcessorCount)), CLDNN_HIP_UNSUPPORTED_FORMAT,
-                     "the patch kernel does not take this convolution");
-    }
-    if (impl == CLDNN_HIP_IMPL_POINT) {
-        if (c->fast) c->tplan = point_plan(p, c->fe, e);
-        CHIP_REQUIRE(c->tplan.ok && (d.tile_override == 1 || point_pays(p, c->tplan, c->engine->props.multiProcessorCount)), CLDNN_HIP_UNSUPPORTED_FORMAT, "the wide 1x1 kernel does not take this convolution");
     }
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE && e.fc) c->fast = false;  // the depthwise kernels have no short fully_connected form
     if (impl == CLDNN_HIP_IMPL_DEPTHWISE && c->fe.f32) c->fast = false;  // nor a float one
