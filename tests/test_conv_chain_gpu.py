@@ -388,6 +388,18 @@ def test_bottleneck_chain_with_weights_in_registers(eng, hw, in_dt, stages, fuse
                 e.close()
 
 
+@pytest.mark.parametrize("fused", [True, False], ids=["fused", "plain"])
+def test_three_stages_with_weights_in_registers_over_more_granules_than_workgroups(eng, fused):
+    xin, spec, bufs, refs = bottleneck_tail(eng, 22, 3, 73, 74, 64, 3, fused, np.uint8, out_pad=(1, 1))  # 1013 granules
+    ch = hip.ConvChain(eng, spec, [False, True, True])
+    assert b"shared by 8 waves" in ch.info().kernel_name
+    ch.enqueue(xin, [b if k else None for k, (b, _) in enumerate(bufs)], [e for _, e in bufs])
+    eng.finish()
+    for k in (1, 2):
+        np.testing.assert_array_equal(hip.download(eng, bufs[k][0]), refs[k])
+    ch.close()
+
+
 @pytest.mark.parametrize("mid,proj,expand,chained", [(1792, 192, 1920, True), (1920, 192, 1920, False), (65, 96, 576, True), (64, 96, 576, False), (48, 192, 64, False)],
                          ids=["lds_full", "lds_beyond", "two_k_steps", "one_k_step", "one_k_step_three_spans"])
 def test_wide_projections_are_chained_in_the_shared_form_only(eng, mid, proj, expand, chained):
