@@ -1,5 +1,6 @@
 // Host side of the kernel whose waves split K over a patch in LDS: which layers it takes, the tile of pixels, weights, launch.
 #include <algorithm>
+#include <mutex>
 
 #include "conv_plane_kernel.h"
 
@@ -107,6 +108,20 @@ void plane_pack_weights(const ConvProblem& p, const PlanePlan& s, const int8_t* 
                     }
 }
 
+using PlaneKernel = void (*)(PlaneArgs);
+template <PlaneKernel K>
+struct Instance {
+    static constexpr PlaneKernel kernel = K;
+};
+
+template <PlaneKernel K>
+static void launch_instance(hipStream_t st, const PlaneArgs& a, const PlanePlan& s)
+{
+    static std::once_flag once;  // more than 64 KB of LDS has to be allowed
+    std::call_once(once, [] { CHIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(K), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)); });
+    hipLaunchKernelGGL(K, dim3(s.grid), dim3(256), s.lds_bytes, st, a);
+}
+
 void launch_conv_plane(hipStream_t st, const ConvProblem& p, const PlanePlan& s, const void* packed, const int32_t* acc_init, const Epilogue& epi,
                        const FastEpi& fe, const void* in, void* out, int32_t* raw)
 {
@@ -124,21 +139,17 @@ void launch_conv_plane(hipStream_t st, const ConvProblem& p, const PlanePlan& s,
     a.div_patch = make_small_div((s.np + 2) * s.pitch), a.div_pitch = make_small_div(s.pitch);
     a.jobs = s.jobs, a.kind = s.kind;
     a.xor_mask = p.in_dt == CLDNN_HIP_U8 ? 0x80808080u : 0u;
-#define PLANE_LAUNCH(NP, NL, JOBS, POOL)                                                                                             \
-    {                                                                                                                                \
-        if (a.xor_mask) hipLaunchKernelGGL((conv_plane_kernel<NP, NL, JOBS, POOL, true>), dim3(s.grid), dim3(256), s.lds_bytes, st, a); \
-        else hipLaunchKernelGGL((conv_plane_kernel<NP, NL, JOBS, POOL, false>), dim3(s.grid), dim3(256), s.lds_bytes, st, a);          \
-    }
-#define PLANE_FORM(NP, NL, POOL)                            \
-    {                                                       \
-        if (s.jobs == 1) PLANE_LAUNCH(NP, NL, 1, POOL)      \
-        else if (s.jobs == 2) PLANE_LAUNCH(NP, NL, 2, POOL) \
-        else PLANE_LAUNCH(NP, NL, 0, POOL)                  \
-    }
-#define PLANE_WIDE(NP, NL, POOL)                                                                                                        \
-    {                                                                                                                                \
-        if (a.xor_mask) hipLaunchKernelGGL((conv_plane_wide_kernel<NP, NL, POOL, true>), dim3(s.grid), dim3(256), s.lds_bytes, st, a);  \
-        else hipLaunchKernelGGL((conv_plane_wide_kernel<NP, NL, POOL, false>), dim3(s.grid), dim3(256), s.lds_bytes, st, a);            \
+    auto go = [&](auto flipped, auto plain) {
+        if (a.xor_mask) launch_instance<decltype(flipped)::kernel>(st, a, s);
+        else launch_instance<decltype(plain)::kernel>(st, a, s);
+    };
+#define PLANE_NARROW(NP, NL, JOBS, POOL) go(Instance<&conv_plane_kernel<NP, NL, JOBS, POOL, true>>{}, Instance<&conv_plane_kernel<NP, NL, JOBS, POOL, false>>{})
+#define PLANE_WIDE(NP, NL, POOL) go(Instance<&conv_plane_wide_kernel<NP, NL, POOL, true>>{}, Instance<&conv_plane_wide_kernel<NP, NL, POOL, false>>{});
+#define PLANE_FORM(NP, NL, POOL)                          \
+    {                                                     \
+        if (s.jobs == 1) PLANE_NARROW(NP, NL, 1, POOL);   \
+        else if (s.jobs == 2) PLANE_NARROW(NP, NL, 2, POOL); \
+        else PLANE_NARROW(NP, NL, 0, POOL);               \
     }
     if (s.wide && p.pooled && !raw) PLANE_WIDE(8, 6, true)
     else if (s.wide && s.np == 8) PLANE_WIDE(8, 6, false)
@@ -150,7 +161,7 @@ void launch_conv_plane(hipStream_t st, const ConvProblem& p, const PlanePlan& s,
     else PLANE_FORM(7, 6, false)
 #undef PLANE_WIDE
 #undef PLANE_FORM
-#undef PLANE_LAUNCH
+#undef PLANE_NARROW
     CHIP_CHECK(hipGetLastError());
 }
 
