@@ -87,7 +87,7 @@ void describe_plane(cldnn_hip_conv c)
 {
     const PlanePlan& s = c->pplan;
     cldnn_hip_conv_info& inf = c->info;
-    inf.tile_pixels = s.np * 32, inf.tile_ofm = s.wide ? 128 : 32, inf.grid = s.grid, inf.block = 256, inf.lds_bytes = s.lds_bytes;
+    inf.tile_pixels = s.np * 32 * (s.wide == 2 ? 2 : 1), inf.tile_ofm = s.wide == 2 ? 64 : s.wide ? 128 : 32, inf.grid = s.grid, inf.block = 256, inf.lds_bytes = s.lds_bytes;
     std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_plane%s<%d groups of %dx%d,%d blocks%s,fast>", s.wide ? "_wide" : "", 32 >> s.shift, s.np, s.cols, s.jobs,
                   c->p.pooled ? ",pooled" : "");
 }

@@ -11,9 +11,9 @@ namespace {
 int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 struct Form {
-    int wide, np, nl;  // 128 features and all of K to a wave; fragments (rows of a group), loads of 64 positions
+    int wide, np, nl;  // 1: 128 features, 2: 64 features and two tiles of pixels, all of K to a wave; fragments (rows of a group), loads of 64 positions
 };
-constexpr Form FORMS[] = {{0, 4, 4}, {0, 7, 5}, {0, 7, 6}, {1, 7, 5}, {1, 7, 6}, {1, 8, 6}};
+constexpr Form FORMS[] = {{0, 4, 4}, {0, 7, 5}, {0, 7, 6}, {1, 7, 5}, {1, 7, 6}, {1, 8, 6}, {2, 7, 6}, {2, 8, 6}};
 
 }  // namespace
 
@@ -34,7 +34,7 @@ static PlanePlan form_plan(const ConvProblem& p, const FastEpi& f, const Epilogu
     for (const Form& form : FORMS) {
         if (form.wide != wide || (form.np == 8 ? !p.pooled : p.pooled && form.np % 2)) continue;
         PlanePlan s{};
-        s.wide = form.wide, s.jobs = p.IFM / (form.wide ? 32 : 128), s.ftiles = form.wide ? ceil_div(spans, 4) : spans;
+        s.wide = form.wide, s.jobs = p.IFM / (form.wide ? 32 : 128), s.ftiles = form.wide ? ceil_div(spans, 4 / form.wide) : spans;
         if (!form.wide && (p.IFM % 128 || (s.jobs != 1 && s.jobs % 2))) continue;
         s.strips = ceil_div(p.OW, 32), s.cols = ceil_div(p.OW, s.strips);
         if (p.pooled) s.cols += s.cols % 2;
@@ -46,9 +46,9 @@ static PlanePlan form_plan(const ConvProblem& p, const FastEpi& f, const Epilogu
         s.image_units = ceil_div(p.OH, form.np) * s.strips;
         if ((int64_t)p.B * s.image_units * spans >= (1 << 30)) continue;
         s.units = p.B * s.image_units;
-        s.total = ceil_div(s.units, groups) * s.ftiles;
+        s.total = ceil_div(ceil_div(s.units, groups), form.wide == 2 ? 2 : 1) * s.ftiles;
         // (512 bytes: what idle lanes read past the end)
-        s.lds_bytes = form.wide ? 3 * 2 * s.positions * 16 + 512 : std::max((s.jobs == 1 ? 1 : 2) * 4 * 2 * s.positions * 16 + 512, PLANE_MEET * 4 * 4096);
+        s.lds_bytes = form.wide ? form.wide * 3 * 2 * s.positions * 16 + 512 : std::max((s.jobs == 1 ? 1 : 2) * 4 * 2 * s.positions * 16 + 512, PLANE_MEET * 4 * 4096);
         // clocks: what a workgroup's matrix instructions take, and what it waits for at its start and its end
         const int resident = s.lds_bytes <= 80 * 1024 ? 2 : 1;
         const int64_t full = s.total / (cus * resident), left = s.total % (cus * resident);
@@ -70,11 +70,13 @@ static PlanePlan form_plan(const ConvProblem& p, const FastEpi& f, const Epilogu
 // 4.9, 192 7.1 / 4.9 for 256 features at 14x14; 64 5.2 / 6.5, 128 6.5 / 6.6, 256 10.5 / 6.6 for 512 at 7x7).  Beyond that workgroups
 // take turns: 512 11.8 / 10.1, 768 18.0 / 14.0, 1024 18.9 / 17.4, 2048 30.7 / 32.7 for 256 features, 1024 34.3 / 30.5, 2048 55.3 / 59.5
 // for 512.  One block of 32 features to a wave is the least work beside the same fixed cost: 768 12.3 / 10.6, 1024 12.7 / 12.5.
-// Wide form, for which more than five eighths of the CUs have to have a workgroup: 128 features at 28x28, 128 workgroups 8.4 / 8.8,
-// 192 12.3 / 9.0, 256 12.7 / 9.4, 384 18.5 / 14.6, 512 18.7 / 16.3; 512 at 28x28, 256 34.3 / 26.6, 512 55.3 / 51.1, 1024 110 / 99.4.  Where
-// both would do it is the faster one (192 workgroups: 9.0 against 10.6, 13.4 against 14.0, 22.6 against 23.0).
-// Both compute for lanes, rows and features that do not exist: 28, 14 and 7 columns leave an eighth or a quarter idle, 20 or 17 columns
-// a half (256 features at 20x20, 16 images 11.8 / 13.1, 64 31.0 / 39.4), 64 output features half of the wide form's 128 (14.0 / 18.4).
+// Wide forms, for which more than five eighths of the CUs have to have a workgroup: 128 features at 28x28, 128 workgroups 8.4 / 8.8,
+// 192 12.3 / 9.0, 256 12.7 / 9.4, 384 18.5 / 14.6, 512 18.7 / 16.3; 512 at 28x28, 256 34.3 / 26.6, 512 55.3 / 51.1, 1024 110 / 99.4.
+// 64 features at 56x56 128 6.5 / 6.8, 256 9.0 / 7.6, 512 14.1 / 12.0, 1024 21.6 / 21.5, pooled 224 8.0 / 6.3, 448 12.2 / 10.0, 896 19.3 / 17.6;
+// at 224x224, pooled, 1568 34.3 / 30.2.  Where a narrow and a wide form would do, the wide one is the faster (192 workgroups: 9.0 against
+// 10.6, 13.4 against 14.0, 22.6 against 23.0).
+// All compute for lanes, rows and features that do not exist: 28, 14 and 7 columns leave an eighth or a quarter idle, 20 or 17 columns
+// a half (256 features at 20x20, 16 images 11.8 / 13.1, 64 31.0 / 39.4), 64 output features half of a form for 128 (14.0 / 20.1 at 56x56, 64 images).
 static double used(const ConvProblem& p, const PlanePlan& s)
 {
     return (double)p.B * p.OH * p.OW * p.OFM / ((double)s.total * s.np * 32 * PLANE_FEATURES * (s.wide ? 4 : 1));
@@ -90,7 +92,7 @@ bool plane_pays(const ConvProblem& p, const PlanePlan& s, int cus)
 PlanePlan plane_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e, int cus, int only)
 {
     if (only >= 0) return form_plan(p, f, e, cus, only);
-    const PlanePlan wide = form_plan(p, f, e, cus, 1);
+    const PlanePlan wide = form_plan(p, f, e, cus, p.OFM <= 64 ? 2 : 1);
     return wide.ok && plane_pays(p, wide, cus) ? wide : form_plan(p, f, e, cus, 0);
 }
 
@@ -144,17 +146,20 @@ void launch_conv_plane(hipStream_t st, const ConvProblem& p, const PlanePlan& s,
         else launch_instance<decltype(plain)::kernel>(st, a, s);
     };
 #define PLANE_NARROW(NP, NL, JOBS, POOL) go(Instance<&conv_plane_kernel<NP, NL, JOBS, POOL, true>>{}, Instance<&conv_plane_kernel<NP, NL, JOBS, POOL, false>>{})
-#define PLANE_WIDE(NP, NL, POOL) go(Instance<&conv_plane_wide_kernel<NP, NL, POOL, true>>{}, Instance<&conv_plane_wide_kernel<NP, NL, POOL, false>>{});
+#define PLANE_WIDE(NP, NL, SPANS, POOL) go(Instance<&conv_plane_wide_kernel<NP, NL, SPANS, POOL, true>>{}, Instance<&conv_plane_wide_kernel<NP, NL, SPANS, POOL, false>>{});
 #define PLANE_FORM(NP, NL, POOL)                          \
     {                                                     \
         if (s.jobs == 1) PLANE_NARROW(NP, NL, 1, POOL);   \
         else if (s.jobs == 2) PLANE_NARROW(NP, NL, 2, POOL); \
         else PLANE_NARROW(NP, NL, 0, POOL);               \
     }
-    if (s.wide && p.pooled && !raw) PLANE_WIDE(8, 6, true)
-    else if (s.wide && s.np == 8) PLANE_WIDE(8, 6, false)
-    else if (s.wide && s.nl == 5) PLANE_WIDE(7, 5, false)
-    else if (s.wide) PLANE_WIDE(7, 6, false)
+    if (s.wide == 2 && p.pooled && !raw) PLANE_WIDE(8, 6, 2, true)
+    else if (s.wide == 2 && s.np == 8) PLANE_WIDE(8, 6, 2, false)
+    else if (s.wide == 2) PLANE_WIDE(7, 6, 2, false)
+    else if (s.wide && p.pooled && !raw) PLANE_WIDE(8, 6, 4, true)
+    else if (s.wide && s.np == 8) PLANE_WIDE(8, 6, 4, false)
+    else if (s.wide && s.nl == 5) PLANE_WIDE(7, 5, 4, false)
+    else if (s.wide) PLANE_WIDE(7, 6, 4, false)
     else if (p.pooled && !raw) PLANE_FORM(4, 4, true)
     else if (s.np == 4) PLANE_FORM(4, 4, false)
     else if (s.nl == 5) PLANE_FORM(7, 5, false)

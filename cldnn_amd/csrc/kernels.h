@@ -152,13 +152,13 @@ void launch_conv_stem(hipStream_t st, const ConvProblem& p, const StemPlan& s, c
 struct PlanePlan {
     int ok;              // the kernel takes this layer
     int kind;            // epilogue
-    int wide;            // 128 features to a workgroup, all of K to a wave
+    int wide;            // all of K to a wave; 1: 128 features to a workgroup, 2: 64 and two tiles of pixels
     int np, nl, jobs;    // fragments of 32 pixels, loads of 64 positions to a slice of the patch, blocks of 32 features to a wave
     int strips, cols, shift, pitch, positions, image_units, units;  // conv_plane_kernel.h
     int spans, ftiles, total, grid, lds_bytes;
     size_t packed_bytes;
 };
-// only: 0 or 1 for the narrow or the wide form, below for the faster one
+// only: 0, 1 or 2 for a form (PlanePlan::wide), below for the fastest
 PlanePlan plane_plan(const ConvProblem& p, const FastEpi& f, const Epilogue& e, int cus, int only = -1);
 bool plane_pays(const ConvProblem& p, const PlanePlan& s, int cus);  // against the table's row
 void plane_pack_weights(const ConvProblem& p, const PlanePlan& s, const int8_t* w, int8_t* packed);

@@ -287,10 +287,10 @@ enum {
     CLDNN_HIP_IMPL_MFMA = 2,      /* implicit GEMM on int8 MFMA, fs_b_yx_fsv16 */
     CLDNN_HIP_IMPL_DEPTHWISE = 3, /* bandwidth kernel, fs_b_yx_fsv16, groups == features */
     /* 3x3 at stride 1 and dilation 1 on int8 MFMA, fs_b_yx_fsv16, over a patch of the input in LDS, whose reads serve three taps.
-     * Two forms: for 32 output features, the waves of a workgroup split the input features (128 or a multiple of 256 of them);
-     * for 128, the waves split the output features (any multiple of 64 input features).  One group, calibrated int8 output
-     * with or without a plain relu; refused otherwise, and where the tile table's row is the faster unless tile_override names
-     * a form (1 or 2). */
+     * Three forms: for 32 output features, the waves of a workgroup split the input features (128 or a multiple of 256 of them);
+     * for 128, or 64 of two tiles of pixels, the waves split the output features (any multiple of 64 input features).  One group,
+     * calibrated int8 output with or without a plain relu; refused otherwise, and where the tile table's row is the faster
+     * unless tile_override names a form (1, 2 or 3). */
     CLDNN_HIP_IMPL_PLANE = 4,
     /* 1x1 without padding on int8 MFMA, fs_b_yx_fsv16, 256 output features to a workgroup: a multiple of 256 input features, one group,
      * calibrated int8 output with or without a plain relu, two convolutions in one launch, or a residual sum with a relu behind

@@ -1007,7 +1007,7 @@ PLANES = [  # batch, features in / out, plane
 
 @pytest.mark.parametrize("in_dt,out_dt,act", [(np.int8, "s8", "relu"), (np.uint8, "u8", "relu"), (np.uint8, "s8", "none")], ids=["s8_relu", "u8_relu", "u8_linear"])
 @pytest.mark.parametrize("pooled", [False, True], ids=["plain", "pooled"])
-@pytest.mark.parametrize("wide", [False, True], ids=["split_k", "wide"])
+@pytest.mark.parametrize("wide", [0, 1, 2], ids=["split_k", "wide", "wide_64"])
 @pytest.mark.parametrize("case", PLANES, ids=lambda c: "%dx%d-%d_%dx%d" % (c[0], c[1], c[2], *c[3]))
 def test_nine_taps_over_a_patch(eng, case, wide, pooled, in_dt, out_dt, act):
     B, ifm, ofm, (H, W) = case
@@ -1028,7 +1028,7 @@ def test_nine_taps_over_a_patch(eng, case, wide, pooled, in_dt, out_dt, act):
     ref, ref_acc = rc.conv(x, w, bias, wqf=np.ones(ofm, np.float32), calib=calib, pad=(1, 1), out_dt=out_dt, act=act, want_acc=True)
     src = hip.upload(eng, x, "fs_b_yx_fsv16", (2, 1))
     d = hip.conv_desc(src.tensor, w.shape, out_dt, pad=(1, 1), out_fmt=hip.FS_B_YX_FSV16, out_pad=(1, 2), bias_dt=hip.I32, has_wqf=True, has_calib=True, act=act,
-                      impl=hip.IMPL_PLANE, tile=2 if wide else 1)
+                      impl=hip.IMPL_PLANE, tile=1 + wide)
     c = hip.Conv(eng, d, w, bias, np.ones(ofm, np.float32), calib)
     out = d.output
     if pooled:

@@ -991,9 +991,9 @@ def test_recorded_launches_over_many_runs(pool, output_in_the_middle):
         np.testing.assert_array_equal(outs["out"].get_memory().read(), expected)
 
 
-@pytest.mark.parametrize("case", [(12, 256, 256, 14, False, "conv_plane<"), (16, 256, 256, 14, True, "conv_plane<"), (96, 128, 64, 28, True, None),
-                                  (48, 64, 128, 28, False, "conv_plane_wide<"), (13, 64, 128, 56, True, "conv_plane_wide<")],
-                         ids=["plain", "pooled", "left_to_a_row_that_pools", "wide", "wide_pooled"])
+@pytest.mark.parametrize("case", [(12, 256, 256, 14, False, "conv_plane<"), (16, 256, 256, 14, True, "conv_plane<"), (64, 128, 96, 28, True, None),
+                                  (48, 64, 128, 28, False, "conv_plane_wide<"), (13, 64, 128, 56, True, "conv_plane_wide<"), (26, 64, 64, 56, True, "conv_plane_wide<")],
+                         ids=["plain", "pooled", "left_to_a_row_that_pools", "wide", "wide_pooled", "wide_64_pooled"])
 def test_nine_taps_over_a_patch_through_network(eng, case):
     """where it is the faster kernel, with the pooling behind it or, if that would make it the slower one, in neither"""
     B, C, M, side, pooled, plane = case
