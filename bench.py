@@ -59,7 +59,21 @@ def chain_groups(layers, fuse_residual):
     return out
 
 
-def build_stack(eng, layers, batch, fuse_residual, seed=1337, tile=0, in_dt=np.uint8, chains=True, siblings=None, calibration="benchmark"):
+def beside_the_table(eng, desc, *arrays):
+    """the convolution on the kernel for 3x3 or 1x1 layers beside the tile table, as a network's layers ask for it, or None
+    where that kernel refuses it"""
+    d = hip.ConvDesc.from_buffer_copy(desc)
+    d.impl = hip.IMPL_POINT if d.fx == 1 else hip.IMPL_PLANE
+    try:
+        return hip.Conv(eng, d, *arrays)
+    except hip.HipError as e:
+        if e.status != -6:
+            raise
+        return None
+
+
+def build_stack(eng, layers, batch, fuse_residual, seed=1337, tile=0, in_dt=np.uint8, chains=True, siblings=None, calibration="benchmark",
+                beside=False):
     """Create device tensors and convolution objects for every layer (seeded synthetic data).
 
     chains: neighbouring layers that feed each other in the network (follows_prev) run as ONE launch of the
@@ -139,7 +153,8 @@ def build_stack(eng, layers, batch, fuse_residual, seed=1337, tile=0, in_dt=np.u
             kw["out_fmt"] = hip.FS_B_YX_FSV16
         L.desc = hip.conv_desc(in_tensor, L.w.shape, "s8", tile=0 if first else tile, **kw)
         try:
-            L.conv = hip.Conv(eng, L.desc, L.w, L.bias, L.wqf, L.calib, L.ecal)
+            L.conv = (beside and not tile and beside_the_table(eng, L.desc, L.w, L.bias, L.wqf, L.calib, L.ecal)) \
+                or hip.Conv(eng, L.desc, L.w, L.bias, L.wqf, L.calib, L.ecal)
         except hip.HipError:
             if not tile:
                 raise
@@ -193,8 +208,9 @@ def build_stack(eng, layers, batch, fuse_residual, seed=1337, tile=0, in_dt=np.u
         kw = dict(H.kw, sibling_split=H.spec["ofm"], sibling_act=M.kw["act"], sibling_act_m=M.kw.get("act_m", 0.0),
                   sibling_act_n=M.kw.get("act_n", 0.0))
         desc = hip.conv_desc(H.xin.tensor, w.shape, "s8", **kw)
+        args = (w, cat(H.bias, M.bias), cat(H.wqf, M.wqf), cat(H.calib, M.calib), None)
         try:
-            both = hip.Conv(eng, desc, w, cat(H.bias, M.bias), cat(H.wqf, M.wqf), cat(H.calib, M.calib), None)
+            both = (beside and beside_the_table(eng, desc, *args)) or hip.Conv(eng, desc, *args)
         except hip.HipError as e:
             if e.status != -6:
                 raise
@@ -606,7 +622,7 @@ def measure_stack(args, wl, steps, warmup, in_flight_n, cpu_seconds, extras):
             sys.exit(2)
     eng = hip.Engine(0, profiling=True)
     t0 = time.perf_counter()
-    stack = build_stack(eng, layers, batch, fuse, tile=args.tile, chains=not args.no_chains)
+    stack = build_stack(eng, layers, batch, fuse, tile=args.tile, chains=not args.no_chains, beside=not args.tuning_cache and not args.tune)
     seq = launches(stack)
     heads = [L for L in stack if not L.follows]
     eng.finish()
@@ -637,7 +653,7 @@ def measure_stack(args, wl, steps, warmup, in_flight_n, cpu_seconds, extras):
         # device and fill what one request's kernels leave idle.
         import threading
         engines = [eng] + [hip.Engine(0, profiling=False) for _ in range(in_flight_n - 1)]
-        stacks = [stack] + [build_stack(e, layers, batch, fuse, seed=1337 + 1000 * (k + 1), tile=args.tile, chains=not args.no_chains)
+        stacks = [stack] + [build_stack(e, layers, batch, fuse, seed=1337 + 1000 * (k + 1), tile=args.tile, chains=not args.no_chains, beside=True)
                             for k, e in enumerate(engines[1:])]
         seqs = [seq] + [launches(st) for st in stacks[1:]]
 

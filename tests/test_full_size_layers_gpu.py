@@ -109,6 +109,21 @@ def test_layer_at_its_real_batch_matches_the_oracle(eng, wl, group):
 
 
 @pytest.mark.parametrize("wl,group", cases())
+def test_layer_at_its_real_batch_on_the_kernel_beside_the_table(eng, wl, group):
+    """as the benchmark and a network run it: on the 3x3 or 1x1 kernel where that takes the layer"""
+    _, batch, fuse, images = CONFIGS[wl]
+    stack = bench.build_stack(eng, group, batch, fuse, calibration="spread", beside=True)
+    if not any(k in (L.info.kernel_name if L.info else b"") for L in stack for k in (b"conv_plane", b"conv_point")):
+        bench.release_stack(stack)
+        pytest.skip("on the table's row")
+    bench.run_step(bench.launches(stack))
+    eng.finish()
+    _, _, checked, mismatches = bench.cpu_pass(eng, stack, 1, verify=True)
+    assert checked > 0 and mismatches == 0, "%d of %d outputs differ from the oracle" % (mismatches, checked)
+    bench.release_stack(stack)
+
+
+@pytest.mark.parametrize("wl,group", cases())
 def test_layer_at_its_real_batch_with_spread_outputs_and_accumulators(eng, wl, group):
     from oracle import refconv as rc
     _, batch, fuse, images = CONFIGS[wl]
