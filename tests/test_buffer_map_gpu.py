@@ -179,3 +179,29 @@ def test_unmap_while_the_stream_is_captured_records_nothing():
     copy(eng, src, READ, dst, WRITE)
     assert (dst.read_raw() == 0x33).all()
     src.close(), dst.close(), eng.close()
+
+
+def test_a_failure_of_the_runtime_is_reported_once():
+    """by the entry it happened in, not again by the launch behind it: an allocation beyond the device's memory, and a recording that is
+    broken off by an allocation, whose launches then go out one by one"""
+    eng, L = hip.Engine(0), hip.lib()
+    src, dst = (hip.Buffer(eng, hip.Tensor.make(hip.U8, hip.BFYX, 1, 3, 5, 7)) for _ in range(2))
+    best, us = C.c_int32(), C.c_float()
+    huge = hip.Tensor.make(hip.S8, hip.FS_B_YX_FSV16, 1 << 22, 64, 256, 256)  # 16 TiB
+    w = np.ones((64, 64, 1, 1), np.int8)
+    desc = hip.conv_desc(huge, w.shape, "s8")
+    assert L.cldnn_hip_conv_tune(eng.h, C.byref(desc), w.ctypes.data_as(C.c_void_p), None, None, None, None, 1, C.byref(best), C.byref(us), None, None) != 0
+    assert b"hipMalloc" in L.cldnn_hip_last_error()
+    hip.check(L.cldnn_hip_buffer_fill(src.h, 1))
+    copy(eng, src, READ, dst, WRITE)
+    assert (dst.read_raw() == 1).all()
+
+    recording, refused = C.c_void_p(), C.c_void_p()
+    hip.check(L.cldnn_hip_engine_record_begin(eng.h))
+    copy(eng, src, READ, dst, WRITE)
+    assert L.cldnn_hip_buffer_alloc(eng.h, 64, C.byref(refused)) != 0
+    assert L.cldnn_hip_engine_record_end(eng.h, C.byref(recording)) != 0 and not recording.value
+    hip.check(L.cldnn_hip_buffer_fill(src.h, 2))
+    copy(eng, src, READ, dst, WRITE)
+    assert (dst.read_raw() == 2).all()
+    src.close(), dst.close(), eng.close()
