@@ -622,7 +622,8 @@ def measure_stack(args, wl, steps, warmup, in_flight_n, cpu_seconds, extras):
             sys.exit(2)
     eng = hip.Engine(0, profiling=True)
     t0 = time.perf_counter()
-    stack = build_stack(eng, layers, batch, fuse, tile=args.tile, chains=not args.no_chains, beside=not args.tuning_cache and not args.tune)
+    options = dict(tile=args.tile, chains=not args.no_chains, beside=not args.tuning_cache and not args.tune)
+    stack = build_stack(eng, layers, batch, fuse, **options)
     seq = launches(stack)
     heads = [L for L in stack if not L.follows]
     eng.finish()
@@ -653,8 +654,7 @@ def measure_stack(args, wl, steps, warmup, in_flight_n, cpu_seconds, extras):
         # device and fill what one request's kernels leave idle.
         import threading
         engines = [eng] + [hip.Engine(0, profiling=False) for _ in range(in_flight_n - 1)]
-        stacks = [stack] + [build_stack(e, layers, batch, fuse, seed=1337 + 1000 * (k + 1), tile=args.tile, chains=not args.no_chains, beside=True)
-                            for k, e in enumerate(engines[1:])]
+        stacks = [stack] + [build_stack(e, layers, batch, fuse, seed=1337 + 1000 * (k + 1), **options) for k, e in enumerate(engines[1:])]
         seqs = [seq] + [launches(st) for st in stacks[1:]]
 
         def request_loop(k, count):

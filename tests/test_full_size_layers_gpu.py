@@ -9,6 +9,8 @@ profiles name as dominant are asserted by name.
 The benchmark's calibration factors saturate most outputs (about half are ReLU zeros, most of the rest 127), so a second
 test runs every signature with factors that spread the outputs over the int8 range, and compares the raw int32
 accumulators of the first image as well."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 
@@ -173,3 +175,20 @@ def test_staged_patch_rows_at_full_size(eng, name, row):
     _, _, checked, mismatches = bench.cpu_pass(eng, stack, 1, verify=True)
     assert checked > 0 and mismatches == 0, "%d of %d outputs differ from the oracle (%s)" % (mismatches, checked, kernel)
     bench.release_stack(stack)
+
+
+@pytest.mark.parametrize("options,kernel", [({}, b"conv_plane<"), (dict(tuning_cache="rows.json"), b"conv_bdir<")], ids=["default", "rows_of_the_table"])
+def test_every_request_in_flight_runs_the_kernels_of_the_first(monkeypatch, options, kernel):
+    args = SimpleNamespace(tile=0, no_chains=False, tuning_cache="", tune=False, only="", clock_warmup=0.0, host_io=False, per_layer=False)
+    args.__dict__.update(options)
+    layer = next(l for l in workloads.resnet50() if l["name"] == "res4b_branch2b")
+    build, kernels = bench.build_stack, []
+
+    def build_and_note(*a, **k):
+        stack = build(*a, **k)
+        kernels.append([L.info.kernel_name for L in stack])
+        return stack
+    monkeypatch.setattr(bench, "build_stack", build_and_note)
+    monkeypatch.setattr(bench, "stack_of", lambda wl: ([dict(layer)], 32, False))
+    bench.measure_stack(args, "resnet50_b32", 2, 1, 2, 0.0, True)
+    assert len(kernels) == 2 and kernels[0] == kernels[1] and kernels[0][0].startswith(kernel), kernels
