@@ -34,6 +34,7 @@ struct ChainPlan {
     int units;
     int dwc_w1, dwc_w2, dwc_v0, dwc_v1, dwc_v2;  // shared depthwise form: parts of its image, bytes
     int dwc_parts;             // workgroups that share the expansion of a granule
+    int dwc_rounds;            // 1: more K-steps of the projection than a wave has registers for
     int img_bytes;             // weights and per-feature vectors on the device
     int lds_bytes;
     int grid;

@@ -148,8 +148,9 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
             // up to four (more change nothing): 576-160-960 at four granules 8.4 -> 6.7 us, 960-160-960 8.9 -> 8.4
             pl.dwc_parts = std::max(1, std::min(std::min(sp2, 4), cus / pl.granules));
             pl.grid = (pl.granules * pl.dwc_parts + 7) / 8 * 8;
-            std::snprintf(pl.name, sizeof(pl.name), "conv_dwchain<%d stages,p%d shared by %d waves,mid %d,spans %d-%d,parts %d>", n, 16 * pl.nt, pl.waves, p0.OFM, pl.sp[1],
-                          sp2, pl.dwc_parts);
+            pl.dwc_rounds = pl.ksteps0 > (k1 < 3 ? 9 : 15);
+            std::snprintf(pl.name, sizeof(pl.name), "conv_dwchain<%d stages,p%d shared by %d waves,mid %d%s,spans %d-%d,parts %d>", n, 16 * pl.nt, pl.waves, p0.OFM,
+                          pl.dwc_rounds ? " in rounds" : "", pl.sp[1], sp2, pl.dwc_parts);
             *out = pl;
             return std::string();
         }
@@ -296,10 +297,12 @@ static void launch_dwcoop(hipStream_t s, const ChainStageIn* st, const ChainPlan
     if (pl.nt == 2) {
         if (k1 == 1) DWCOOP_LAUNCH(1, 9, false, 2)
         else if (k1 == 2) DWCOOP_LAUNCH(2, 9, false, 2) else DWCOOP_LAUNCH(3, 9, false, 2)
+    } else if (pl.dwc_rounds) {
+        if (k1 == 1) DWCOOP_LAUNCH(1, 9, true, 1)
+        else if (k1 == 2) DWCOOP_LAUNCH(2, 9, true, 1) else DWCOOP_LAUNCH(3, 8, true, 1)
     } else if (k1 == 1 && a.KS <= 3) DWCOOP_LAUNCH(1, 3, false, 1) else if (k1 == 1 && a.KS <= 6) DWCOOP_LAUNCH(1, 6, false, 1)
-    else if (k1 == 1 && a.KS <= 9) DWCOOP_LAUNCH(1, 9, false, 1) else if (k1 == 1) DWCOOP_LAUNCH(1, 9, true, 1) else if (k1 == 2 && a.KS <= 6) DWCOOP_LAUNCH(2, 6, false, 1)
-    else if (k1 == 2 && a.KS <= 9) DWCOOP_LAUNCH(2, 9, false, 1) else if (k1 == 2) DWCOOP_LAUNCH(2, 9, true, 1)
-    else if (a.KS <= 9) DWCOOP_LAUNCH(3, 9, false, 1) else if (a.KS <= 15) DWCOOP_LAUNCH(3, 15, false, 1) else DWCOOP_LAUNCH(3, 8, true, 1)
+    else if (k1 == 1) DWCOOP_LAUNCH(1, 9, false, 1) else if (k1 == 2 && a.KS <= 6) DWCOOP_LAUNCH(2, 6, false, 1) else if (k1 == 2) DWCOOP_LAUNCH(2, 9, false, 1)
+    else if (a.KS <= 9) DWCOOP_LAUNCH(3, 9, false, 1) else DWCOOP_LAUNCH(3, 15, false, 1)
 #undef DWCOOP_LAUNCH
     CHIP_CHECK(hipGetLastError());
 }

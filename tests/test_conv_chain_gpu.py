@@ -308,7 +308,7 @@ def test_depthwise_chain_on_small_planes(eng, mid, proj, stride, stages, hw, in_
     run_depthwise_chain(eng, mid, proj, stride, stages, hw, in_dt, saturate)
 
 
-def run_depthwise_chain(eng, mid, proj, stride, stages, hw, in_dt, saturate, shared=None):
+def run_depthwise_chain(eng, mid, proj, stride, stages, hw, in_dt, saturate, shared=None, form=()):
     r = np.random.default_rng(mid + proj)
     H, W = hw
     B = 3 if H * W < 4000 else 1
@@ -344,6 +344,7 @@ def run_depthwise_chain(eng, mid, proj, stride, stages, hw, in_dt, saturate, sha
     for keep in ([False] * (stages - 1) + [True], None):
         ch = hip.ConvChain(eng, spec, keep)
         assert b"conv_dwchain" in ch.info().kernel_name and (b"shared" in ch.info().kernel_name) == shared
+        assert all(part in ch.info().kernel_name for part in form), ch.info().kernel_name
         ch.enqueue(xin, [b if keep is None or keep[k] else None for k, b in enumerate(bufs)], [None, ebuf, None])
         eng.finish()
         for k in range(stages):
@@ -355,14 +356,17 @@ def run_depthwise_chain(eng, mid, proj, stride, stages, hw, in_dt, saturate, sha
         b.close()
 
 
-@pytest.mark.parametrize("mid,proj,stride,hw", [(576, 96, 1, (35, 39)), (576, 24, 1, (37, 37)), (576, 96, 1, (37, 37)), (528, 160, 1, (37, 37)),
-                                                (448, 64, 1, (9, 7)), (1152, 64, 1, (5, 5)), (704, 96, 2, (9, 9)), (1040, 160, 1, (5, 5)), (384, 64, 1, (53, 53))],
+@pytest.mark.parametrize("mid,proj,stride,hw,granules,rounds",
+                         [(576, 96, 1, (35, 39), 1, False), (576, 24, 1, (37, 37), 2, False), (576, 96, 1, (37, 37), 2, False), (528, 160, 1, (37, 37), 2, False),
+                          (448, 64, 1, (9, 7), 1, False), (1152, 64, 1, (5, 5), 1, True), (704, 96, 2, (9, 9), 1, True), (960, 160, 1, (5, 5), 1, False),
+                          (1040, 160, 1, (5, 5), 1, True), (384, 64, 1, (53, 53), 2, False)],
                          ids=["256_granules", "two_a_group_narrow", "two_a_group", "two_a_group_wide", "seven_k_steps", "more_k_steps_than_waves",
-                              "rounds_two_spans", "rounds_three_spans", "more_than_two_granules_a_cu"])
-def test_shared_granules_at_the_edges_of_their_forms(eng, mid, proj, stride, hw):
+                              "rounds_two_spans", "fifteen_k_steps", "rounds_three_spans", "more_than_two_granules_a_cu"])
+def test_shared_granules_at_the_edges_of_their_forms(eng, mid, proj, stride, hw, granules, rounds):
     """one and two granules to a workgroup (the last of 257 granules stands alone, and is not full), K-steps that fill the
     registers of a wave and K-steps that take several rounds, more granules than the device holds"""
-    run_depthwise_chain(eng, mid, proj, stride, 3, hw, np.uint8, 0, shared=True)
+    run_depthwise_chain(eng, mid, proj, stride, 3, hw, np.uint8, 0, shared=True,
+                        form=(b"p%d shared" % (16 * granules), b"mid %d%s," % (mid, b" in rounds" if rounds else b"")))
 
 
 @pytest.mark.parametrize("hw", [(1, 1), (17, 15), (46, 41)], ids=["one_pixel", "ragged", "several_granules"])
