@@ -1005,20 +1005,29 @@ PLANES = [  # batch, features in / out, plane
 ]
 
 
-@pytest.mark.parametrize("in_dt,out_dt,act", [(np.int8, "s8", "relu"), (np.uint8, "u8", "relu"), (np.uint8, "s8", "none")], ids=["s8_relu", "u8_relu", "u8_linear"])
-@pytest.mark.parametrize("pooled", [False, True], ids=["plain", "pooled"])
-@pytest.mark.parametrize("wide", [0, 1, 2], ids=["split_k", "wide", "wide_64"])
-@pytest.mark.parametrize("case", PLANES, ids=lambda c: "%dx%d-%d_%dx%d" % (c[0], c[1], c[2], *c[3]))
+def plane_forms():
+    """every form that takes a case: the narrow one has four waves to share the blocks of 32 features, an even number each; of the
+    wide ones a pooled patch of four groups of eight rows and columns is too large; maxima are taken in front of a requantisation
+    that never falls, so only with a ReLU"""
+    out = []
+    for case in PLANES:
+        _, ifm, _, (_, W) = case
+        name = "%dx%d-%d_%dx%d" % (case[0], case[1], case[2], *case[3])
+        for wide, form in enumerate(("split_k", "wide", "wide_64")):
+            for pooled in (False, True):
+                if not wide and ifm != 128 and ifm % 256 or wide and pooled and W + W % 2 == 8:
+                    continue
+                for in_dt, out_dt, act in ((np.int8, "s8", "relu"), (np.uint8, "u8", "relu")) + (() if pooled else ((np.uint8, "s8", "none"),)):
+                    ids = (name, form, "pooled" if pooled else "plain", ("s8_" if in_dt == np.int8 else "u8_") + ("relu" if act == "relu" else "linear"))
+                    out.append(pytest.param(case, wide, pooled, in_dt, out_dt, act, id="-".join(ids)))
+    return out
+
+
+@pytest.mark.parametrize("case,wide,pooled,in_dt,out_dt,act", plane_forms())
 def test_nine_taps_over_a_patch(eng, case, wide, pooled, in_dt, out_dt, act):
     B, ifm, ofm, (H, W) = case
-    if pooled and act != "relu":
-        pytest.skip("maxima are taken before a requantisation that never falls")
     if pooled:
         H, W = H + H % 2, W + W % 2
-    if not wide and ifm != 128 and ifm % 256:
-        pytest.skip("four waves to share the blocks, an even number each")
-    if wide and pooled and W == 8:
-        pytest.skip("the patch of four groups of eight rows and columns is too large")
     r = np.random.default_rng(ifm + ofm + H)
     lo, hi = (0, 256) if in_dt == np.uint8 else (-128, 128)
     x = r.integers(lo, hi, (B, ifm, H, W)).astype(in_dt)
@@ -1062,8 +1071,11 @@ POINTS = [  # batch, features in / out, plane, stride
 ]
 
 
-@pytest.mark.parametrize("form", ["s8_relu", "u8_linear", "u8_pair", "s8_sum", "u8_sum_in_place"])
-@pytest.mark.parametrize("case", POINTS, ids=lambda c: "%dx%d-%d_%dx%d" % (c[0], c[1], c[2], *c[3]))
+POINT_FORMS = [pytest.param(c, form, id="%dx%d-%d_%dx%d-%s" % (c[0], c[1], c[2], *c[3], form)) for c in POINTS
+               for form in ("s8_relu", "u8_linear", "u8_pair", "s8_sum", "u8_sum_in_place") if form != "u8_pair" or c[2] > 48]
+
+
+@pytest.mark.parametrize("case,form", POINT_FORMS)
 def test_wide_1x1(eng, case, form):
     B, ifm, ofm, (H, W), stride = case
     r = np.random.default_rng(ifm + ofm + H)
@@ -1081,8 +1093,6 @@ def test_wide_1x1(eng, case, form):
         kw.update(eltw=e, eltw_act="relu", eltw_calib=r.uniform(0.5, 1.0, ofm).astype(np.float32))
         dev.update(in_place="in_place" in form)
     if form == "u8_pair":
-        if ofm <= 48:
-            pytest.skip("nothing to divide")
         dev.update(sibling_split=48, sibling_act="relu")
     got, acc, info = hip.conv_forward(eng, x, w, bias, ones, calib, fmt="fs_b_yx_fsv16", out_pad=(1, 2), impl=hip.IMPL_POINT, tile=1, want_acc=True, want_info=True, **kw, **dev)
     assert info.kernel_name.startswith(b"conv_point<"), info.kernel_name
