@@ -333,7 +333,7 @@ void build(cldnn_hip_conv c, const void* weights, const void* bias, const float*
         c->w_packed = upload(c, packed.data(), packed.size());
         c->w_raw = upload(c, weights, wcount);  // for the accumulators alone
         inf.tile_pixels = 64, inf.tile_ofm = 64, inf.grid = c->splan.grid, inf.block = 256, inf.lds_bytes = c->splan.lds_bytes;
-        std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_stem_plain<%d k-steps,%d fragments,fast>", c->splan.ksteps, c->splan.frags_f);
+        std::snprintf(inf.kernel_name, sizeof(inf.kernel_name), "conv_stem_plain<%d k-steps,%d fragments,%d rows,fast>", c->splan.ksteps, c->splan.frags_f, c->splan.wg_rows);
         return;
     }
     if (impl == CLDNN_HIP_IMPL_PLANE) {
@@ -821,7 +821,7 @@ cldnn_hip_status cldnn_hip_conv_pool_output(cldnn_hip_conv c, const cldnn_hip_po
             p = q, c->splan = s;
             c->info.grid = s.grid, c->info.lds_bytes = s.lds_bytes;
             c->info.bytes -= (int64_t)p.B * p.OFM * ((int64_t)p.OH * p.OW - (int64_t)o.y * o.x);
-            std::snprintf(c->info.kernel_name, sizeof(c->info.kernel_name), "conv_stem_plain<%d k-steps,%d fragments,pooled,fast>", s.ksteps, s.frags_f);
+            std::snprintf(c->info.kernel_name, sizeof(c->info.kernel_name), "conv_stem_plain<%d k-steps,%d fragments,%d rows pooled,fast>", s.ksteps, s.frags_f, s.wave_rows);
             return;
         }
         if (c->impl == CLDNN_HIP_IMPL_PLANE) {

@@ -1117,7 +1117,11 @@ STEMS = [  # batch, features in / out, filter, stride, padding, plane
     (1, 2, 8, (1, 1), (1, 1), (0, 0), (3, 4)),        # the smallest row
     (40, 3, 16, (3, 3), (2, 2), (1, 1), (5, 4)),      # one strip of one or two pooled columns, four row groups
     (1, 3, 33, (4, 4), (4, 4), (0, 0), (21, 80)),     # filter rows that fill a chunk, stride 4
+    (20, 3, 16, (3, 3), (2, 2), (1, 1), (75, 9)),     # workgroups for every CU at two rows each
+    (70, 3, 16, (3, 3), (2, 2), (1, 1), (75, 9)),     # at four; pooled, at two rows a wave
+    (130, 3, 16, (3, 3), (2, 2), (1, 1), (75, 9)),    # pooled, at four
 ]
+STEM_ROWS = {20: (b"2 rows,", b"1 rows pooled"), 70: (b"4 rows,", b"2 rows pooled"), 130: (b"4 rows,", b"4 rows pooled")}  # by batch: plain, pooled
 
 
 def stem_layer(r, ifm, ofm, k, in_dt, act):
@@ -1145,6 +1149,7 @@ def test_first_layer_reads_a_plain_image(eng, case, in_dt, act):
                           has_calib=True, **kw)
         c = hip.Conv(eng, d, w, bias, wqf, calib)
         assert b"conv_stem" in c.info().kernel_name and c.info().impl == hip.IMPL_MFMA
+        assert STEM_ROWS.get(B, [b"rows,"])[0] in c.info().kernel_name, c.info().kernel_name
         dst = hip.Buffer(eng, d.output)
         c.enqueue(src, dst)
         eng.finish()
@@ -1176,6 +1181,7 @@ def test_first_layer_finishes_the_3x3_pooling_behind_it(eng, case, in_dt):
         pd.mode, pd.size_y, pd.size_x, pd.stride_y, pd.stride_x = hip.POOL_MAX, 3, 3, 2, 2
         assert hip.lib().cldnn_hip_conv_pool_output(c.h, C.byref(pd)) == 0
         assert hip.lib().cldnn_hip_conv_pool_output(c.h, C.byref(pd)) == -6  # once
+        assert STEM_ROWS.get(B, [b"pooled"])[-1] in c.info().kernel_name, c.info().kernel_name
         dst = hip.Buffer(eng, pd.output)
         c.enqueue(src, dst)
         eng.finish()
