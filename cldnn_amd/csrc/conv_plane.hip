@@ -75,8 +75,16 @@ static PlanePlan form_plan(const ConvProblem& p, const FastEpi& f, const Epilogu
 // 64 features at 56x56 128 6.5 / 6.8, 256 9.0 / 7.6, 512 14.1 / 12.0, 1024 21.6 / 21.5, pooled 224 8.0 / 6.3, 448 12.2 / 10.0, 896 19.3 / 17.6;
 // at 224x224, pooled, 1568 34.3 / 30.2.  Where a narrow and a wide form would do, the wide one is the faster (192 workgroups: 9.0 against
 // 10.6, 13.4 against 14.0, 22.6 against 23.0).
-// All compute for lanes, rows and features that do not exist: 28, 14 and 7 columns leave an eighth or a quarter idle, 20 or 17 columns
-// a half (256 features at 20x20, 16 images 11.8 / 13.1, 64 31.0 / 39.4), 64 output features half of a form for 128 (14.0 / 20.1 at 56x56, 64 images).
+// All compute for lanes, rows and features that do not exist.  Row of the table / this kernel by the share in use, planes of other images
+// than those of 224 pixels among them:
+//   narrow, more than a workgroup per CU: 0.75 (26 and 13 columns) 8.3 / 7.5, 11.6 / 10.9, 18.7 / 17.5; 0.70 (25) 8.2 / 7.5; 0.64 (24, 12 and 6)
+//     8.2 / 7.4, 11.5 / 10.7, 18.3 / 16.9; 0.60 (20) 6.5 / 7.1, 9.0 / 10.3, 12.0 / 14.9; 0.48 (18) 8.9 / 10.2; 0.45 (10 and 5) 9.0 / 10.5, 13.3 / 16.3
+//   narrow, up to one: 0.75 (26, 13 and 12) 6.4 / 5.4, 13.8 / 10.0, 7.1 / 4.9; 0.70 6.4 / 5.4; 0.64 to 0.66 6.4 / 5.4, 7.1 / 4.9, 8.8 / 6.7, 13.6 / 9.8; 0.60
+//     5.0 / 5.4, 7.1 / 6.4; 0.56 (6) 10.4 / 6.7; 0.52 (10) 4.9 / 4.9; 0.45 7.2 / 6.6, 10.5 / 9.6; 0.39 (5) 6.6 / 6.6; 0.36 (9) 7.2 / 6.5, 10.5 / 9.6
+//   wide: 0.75 12.9 / 9.7, 18.7 / 15.0, 33.0 / 26.4; 64 features, 52 columns 8.9 / 7.2; 0.70 12.7 / 9.5, 8.9 / 7.2; 0.64 12.7 / 9.7, 18.2 / 14.7; 0.60
+//     8.5 / 8.9, 19.6 / 25.3; 0.45 20.0 / 25.0; 64 output features on the form for 128 14.0 / 20.1 at 56x56, 64 images.
+// The lines at 0.76 and 0.70 keep to one side of that: whatever passes them is faster here, and what lies between 0.64 and them would be too.
+// Planes of images of 224 pixels have 0.766 and more.
 static double used(const ConvProblem& p, const PlanePlan& s)
 {
     return (double)p.B * p.OH * p.OW * p.OFM / ((double)s.total * s.np * 32 * PLANE_FEATURES * (s.wide ? 4 : 1));

@@ -30,7 +30,7 @@ namespace chip {
 
 enum { PLANE_FEATURES = 32, PLANE_MEET = 4 };
 
-// q / d for q < 512, d < 2048: full-rate 24-bit products instead of quarter-rate ones
+// q / d for q < 512, d < 2048: a 24-bit product and a shift instead of the high half of a 32-bit product
 struct SmallDiv {
     uint32_t mul;
     __device__ uint32_t div(uint32_t q) const { return __umul24(q, mul) >> 20; }

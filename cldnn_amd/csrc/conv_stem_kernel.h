@@ -15,8 +15,8 @@
 // factors that are not negative the ReLU requantisation is monotonic, and a pooled value costs one requantisation
 // instead of four.  The even column past the edge starts from a number no sum reaches.
 //
-// Bound by the vector ALU (unpacking, maxima, requantisation; 56 % of the cycles) and the matrix cores (38 %) together; the image,
-// the weights and the output at a copy's rate are a sixth of the time at batch 128.  Kernel time, three or two launches before and
+// Bound by the vector ALU (unpacking, maxima, requantisation; 56 % of the cycles) and the matrix cores (38 %) together; the image
+// and the output at a copy's rate (5.16 TB/s) are 8.7 of the 36.7 us at batch 128, a quarter.  Kernel time, three or two launches before and
 // now: ResNet-50 (7x7, pooled) batch 1 15.6 -> 10.4 us, 32 34 -> 15.1, 128 94 -> 36.7; MobileNet-v2 (3x3, 32 features) batch 1
 // 10.7 -> 8.1, 32 21 -> 10.9; VGG-16 (3x3, 64 features) batch 1 10.8 -> 9.1, 16 23.8 -> 17.6.  (At batch 1 the image is read over the
 // host link.)

@@ -422,7 +422,7 @@ cldnn_hip_status cldnn_hip_conv_chain_get_info(cldnn_hip_conv_chain chain, cldnn
 int32_t cldnn_hip_conv_out_extent(int32_t in, int32_t pad, int32_t filt, int32_t dil, int32_t stride);
 
 /* Kernel runner for tuning: times the table's own choice and every row of the tile-config table that accepts this
- * convolution, on scratch tensors of the descriptor's shapes filled with pseudo-random bytes, and reports the fastest.
+ * convolution (not CLDNN_HIP_IMPL_PLANE or _POINT), on scratch tensors of the descriptor's shapes filled with pseudo-random bytes, and reports the fastest.
  * Replaces the reference's kernel_runner (src/gpu/kernel_runner.cpp:106-190, used by tuning_mode tune_and_cache through
  * kernel_selector/core/kernel_selector.cpp GetAutoTuneBestKernel): the device is kept busy for 150 ms first (the
  * clocks of an idle device rise over tens of milliseconds, and the candidates timed first would lose to the later ones),
