@@ -18,15 +18,15 @@ struct error : std::runtime_error {
 
 void set_last_error(const std::string& m);
 
-// A failure is reported here and taken back from the runtime, which would hand it to the next caller of hipGetLastError: a launch
-// that is made after this one has been answered with something else (a smaller request, launches one by one) asks for its own.
-#define CHIP_CHECK(expr)                                                                                    \
-    do {                                                                                                    \
-        const hipError_t e_ = (expr);                                                                       \
-        if (e_ != hipSuccess) {                                                                             \
-            (void)hipGetLastError();                                                                        \
-            throw ::chip::error(CLDNN_HIP_DEVICE_ERROR, std::string(#expr) + ": " + hipGetErrorString(e_)); \
-        }                                                                                                   \
+// Throws what a call of the runtime failed with.  The error is taken back from the runtime, which would hand it to the next caller of
+// hipGetLastError: a launch that is made after the failure has been answered with something else (a smaller request, launches one
+// by one) asks for its own.
+[[noreturn]] void runtime_failed(hipError_t e, const char* call);
+
+#define CHIP_CHECK(expr)                                         \
+    do {                                                         \
+        const hipError_t e_ = (expr);                            \
+        if (e_ != hipSuccess) ::chip::runtime_failed(e_, #expr); \
     } while (0)
 
 #define CHIP_REQUIRE(cond, status, msg)                      \

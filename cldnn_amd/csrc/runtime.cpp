@@ -13,6 +13,12 @@ namespace chip {
 static thread_local std::string g_last_error;
 void set_last_error(const std::string& m) { g_last_error = m; }
 
+void runtime_failed(hipError_t e, const char* call)
+{
+    (void)hipGetLastError();
+    throw error(CLDNN_HIP_DEVICE_ERROR, std::string(call) + ": " + hipGetErrorString(e));
+}
+
 size_t dtype_size(int dt)
 {
     switch (dt) {
