@@ -31,12 +31,37 @@ __global__ void __launch_bounds__(256) gemv_gather_kernel(MfmaArgs a)
     const_cast<v4i*>(a.bpk)[((size_t)ptile * (a.ksteps + GEMV_SLACK) + ks) * 64 + lane] = v ^ xm;
 }
 
-void launch_ksplit_lanes(hipStream_t s, const MfmaArgs& a, int ft, int pt, int grid, int epi);
+void launch_ksplit_lanes(hipStream_t s, const KsplitArgs& a, int ft, int pt, int grid, int epi);
 
-void launch_ksplit(hipStream_t s, const MfmaArgs& a, int ft, int pt, int grid, bool lanes, int epi)
+static KsplitArgs ksplit_args(const MfmaArgs& m)
 {
-    if (a.bpk) {
-        hipLaunchKernelGGL(gemv_gather_kernel, dim3((a.ksteps + 3) / 4, a.mtiles * pt), dim3(256), 0, s, a);
+    KsplitArgs a{};
+    a.in = m.in + (m.in_off - m.py * m.in_py - m.px * 16);
+    a.inside = (uint32_t)(m.py * m.in_py + m.px * 16);
+    a.wpk = m.wpk, a.bpk = m.bpk, a.acc_init = m.acc_init, a.out = m.out, a.eltw = (const int8_t*)m.eltw, a.raw = m.raw, a.origin = m.origin;
+    a.mtiles = m.mtiles, a.ftiles = m.ofm_tiles;
+    a.features_outer = m.by_features != 0, a.die_bits = m.by_features == 2 ? 0 : 3;
+    a.inner = a.features_outer ? a.mtiles : a.ftiles;
+    a.div_inner = make_even_div((uint32_t)a.inner);
+    a.M = m.M, a.OFM = m.OFM, a.OHW = m.OHW, a.OW = m.OW, a.OH = m.OH, a.IH = m.IH, a.IW = m.IW;
+    a.div_ohw = make_even_div((uint32_t)m.OHW), a.div_ow = make_even_div((uint32_t)m.OW);
+    a.ksteps = m.ksteps, a.kper = m.kper, a.kwaves = m.kwaves;
+    a.in_pb = m.in_pb, a.in_row = m.sy * m.in_py, a.in_col = m.sx * 16, a.in_pf = m.in_pf;
+    a.taps = m.FX * m.FY, a.FX = m.FX, a.tap_dy = m.tap_dy, a.tap_dx = m.tap_dx, a.last_group = m.CB - 4;
+    a.div_taps = make_even_div((uint32_t)a.taps), a.div_fx = make_even_div((uint32_t)m.FX), a.div_cb = make_even_div((uint32_t)m.CB);
+    a.out_off = m.out_off, a.out_pb = m.out_pb, a.out_pf = m.out_pf, a.out_py = m.out_py, a.out_f = m.out_f;
+    a.el_off = m.el_off, a.el_pb = m.el_pb, a.el_pf = m.el_pf, a.el_row = m.esy * m.el_py, a.el_col = m.esx * 16;
+    a.xor_mask = m.xor_mask;
+    a.CB = m.CB, a.kchunks = m.kchunks, a.checked = m.checked, a.sy = m.sy, a.sx = m.sx, a.py = m.py, a.px = m.px, a.dil_y = m.dil_y, a.dil_x = m.dil_x;
+    a.fe = m.fe, a.epi = m.epi;
+    return a;
+}
+
+void launch_ksplit(hipStream_t s, const MfmaArgs& m, int ft, int pt, int grid, bool lanes, int epi)
+{
+    const KsplitArgs a = ksplit_args(m);
+    if (m.bpk) {
+        hipLaunchKernelGGL(gemv_gather_kernel, dim3((m.ksteps + 3) / 4, m.mtiles * pt), dim3(256), 0, s, m);
         if (pt == 1) launch_ksplit_instance<1, 1, ADDR_GATHERED>(s, a, grid, epi);
         else launch_ksplit_instance<1, 2, ADDR_GATHERED>(s, a, grid, epi);
     } else if (lanes) {

@@ -3,7 +3,7 @@
 
 namespace chip {
 
-void launch_ksplit_lanes(hipStream_t s, const MfmaArgs& a, int ft, int pt, int grid, int epi)
+void launch_ksplit_lanes(hipStream_t s, const KsplitArgs& a, int ft, int pt, int grid, int epi)
 {
     launch_ksplit_tile<ADDR_LANES>(s, a, ft, pt, grid, epi);
 }

@@ -763,7 +763,6 @@ void launch_conv_mfma(hipStream_t s, const ConvProblem& p, const MfmaPlan& pl, c
         a.ofm_tiles = pl.ofm_tiles * (4 / pl.ks_ft);
         a.div_ofm_tiles = make_div((uint32_t)a.ofm_tiles);
         a.kwaves = pl.ks_waves, a.kper = pl.ks_per, a.checked = pl.checked, a.dil_y = p.dy, a.dil_x = p.dx;
-        a.div_taps = make_div((uint32_t)(p.FY * p.FX));
         launch_ksplit(s, a, pl.ks_ft, pl.ks_pt, pl.grid, pl.ks_lanes != 0, kind);
     }
     else if (pl.stream) launch_stream(s, a, tc.wave_pixels / 16, pl.grid, kind);

@@ -77,7 +77,6 @@ struct MfmaArgs {
     const v4i* bpk;     // split-K kernel: scratch for the activations in fragment order (nullptr: read them in place)
     // split-K kernel: waves per workgroup, K-steps per wave, bounds checks (input without a border)
     int32_t kwaves, kper, checked, dil_y, dil_x;
-    FastDiv div_taps;
     int32_t out_f;          // split-K kernel: bytes between neighbouring features of the output
     const int32_t* origin;  // grouped: byte offset of the first input slice that each span of 64 output features reads
     FastEpi fe;
@@ -627,7 +626,8 @@ __device__ __forceinline__ void fetch_arguments(const MfmaArgs& a)
                  "s"(a.epi.calib), "s"(a.epi.eltw_calib), "s"(a.epi.wqf), "s"(a.fe.hi), "s"(a.fe.lo), "s"(a.origin));
 }
 
-__device__ __forceinline__ PixelPos pixel_pos(const MfmaArgs& a, uint32_t m)
+template <class Args>
+__device__ __forceinline__ PixelPos pixel_pos(const Args& a, uint32_t m)
 {
     PixelPos p;
     p.b = a.div_ohw.div(m);
@@ -640,8 +640,8 @@ __device__ __forceinline__ PixelPos pixel_pos(const MfmaArgs& a, uint32_t m)
 // whole 2x2 windows.  With two or more fragments, fragments 2k and 2k + 1 are the same sixteen columns of two rows, so that a
 // load instruction still covers sixteen neighbours (OHW and OW then count columns of row pairs); a single fragment is four
 // windows of four adjacent lanes (OHW and OW count windows).
-template <int EPI, int NT>
-__device__ __forceinline__ PixelPos pixel_at(const MfmaArgs& a, uint32_t m0, int nt, int l16, bool& ok)
+template <int EPI, int NT, class Args>
+__device__ __forceinline__ PixelPos pixel_at(const Args& a, uint32_t m0, int nt, int l16, bool& ok)
 {
     if constexpr (EPI != EPI_KIND_POOL) {
         const uint32_t m = m0 + nt * 16 + l16;

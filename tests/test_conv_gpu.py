@@ -887,6 +887,17 @@ def test_split_k_rows(eng, row, shape):
         assert_same(ro, go)
 
 
+@pytest.mark.parametrize("row", ["ksplit_p16_f16", "ksplit_p32_f16", "ksplit_p64_f16", "ksplit_p32_f32", "ksplit_p32_f64"])
+def test_split_k_shares_of_more_steps_than_lanes(eng, row):
+    """1035 K-steps: a wave's share (65, or 130 with eight waves) is more than the 64 whose offsets its lanes hold at once"""
+    x, w, bias, wqf, calib = problem(93, 1, 7312, 2, 2, 18, 3, 3)
+    kw = dict(pad=(1, 1), act="relu")
+    (ro, ra), (go, ga, info) = both(eng, x, w, bias, wqf, calib, fmt="fs_b_yx_fsv16", tile=tile_names().index(row) + 1, in_pad=(1, 1), **kw)
+    assert b"conv_ksplit<" + row.encode() in info.kernel_name
+    np.testing.assert_array_equal(ga, ra)
+    assert_same(ro, go)
+
+
 @pytest.mark.parametrize("OFM", [1, 16, 35, 126])
 def test_float_output_of_every_row(eng, OFM):
     """float results leave through the short float epilogue: partly filled slices and groups of four, factors present and absent"""
