@@ -3,7 +3,8 @@
 //
 // conv_chain_kernel.h gives every wave granules of its own and keeps the weights in LDS, which takes a copy of 70 KB first;
 // on a small plane (ResNet-50 at batch 1: 196 granules at 56x56) that is one long walk of dependent steps on a few CUs.  Here
-//   - stage 0 is split over its K-steps: wave w takes the taps w and w + 8 of all features, and the partial sums meet in LDS;
+//   - stage 0 is split over its K-steps: wave w takes tap w of all features, waves 0 to 3 a fragment of the ninth tap each, and the
+//     partial sums meet in LDS;
 //   - the rounded result (1 KB) goes back through LDS and every wave computes an eighth of the expansion's features, adds its
 //     part of the residual and stores it;
 //   - stage 2 is split over its K again, which is where each wave's own expansion features are: they never leave its
@@ -13,6 +14,8 @@
 // stages, 28x28 with two 9.5 -> 4.0.  Inside a network, where the input comes from memory, two stages are faster at every
 // size (ResNet-50 at batch 32 12.7 -> 10.8, at batch 128 33.1 -> 29.0; repeated on warm caches 24.8 and 25.5); three stages
 // with many granules are not, splitting costs more instructions per pixel: 13.1 -> 11.7 us at 1016 granules, 26 against 43 us at batch 32.
+// (The ninth tap's weights in the registers of one wave were four more fragments for every wave: with three stages 128 registers were not
+// enough, and a request waited for one that was spilled behind it.)
 // 128 mid features (weights in 160 registers) gained 2 us of 12 at batch 1 and lost 8 of 28 at batch 32.
 #pragma once
 #include "conv_chain_kernel.h"
@@ -47,14 +50,28 @@ struct CoopConvEpi {
     FastEpi fe;
 };
 
+// all arguments behind one wait
+__device__ __forceinline__ void fetch_arguments(const CoopConvArgs& a)
+{
+    asm volatile("" ::"s"(a.in), "s"(a.img), "s"(a.eltw), "s"(a.vec_bytes), "s"(a.vec_quads), "s"(a.el_off), "s"(a.el_pb), "s"(a.el_pf), "s"(a.el_py), "s"(a.el_px), "s"(a.M), "s"(a.OHW),
+                 "s"(a.OW), "s"(a.div_ohw.mul), "s"(a.div_ohw.shift), "s"(a.div_ow.mul), "s"(a.div_ow.shift), "s"(a.in_off), "s"(a.in_pb), "s"(a.in_pf), "s"(a.row), "s"(a.col),
+                 "s"(a.tap_dy), "s"(a.gpw), "s"(a.grem), "s"(a.div_parts.mul), "s"(a.div_parts.shift), "s"(gridDim.x));
+#pragma unroll
+    for (int k = 0; k < CHAIN_MAX_STAGES; ++k)
+        asm volatile("" ::"s"(a.st[k].out), "s"(a.st[k].off), "s"(a.st[k].pb), "s"(a.st[k].pf), "s"(a.st[k].py), "s"(a.st[k].xor_mask), "s"(a.st[k].unit0), "s"(a.st[k].kstride),
+                     "s"(a.st[k].vec0), "s"(a.st[k].hi));
+    asm volatile("" ::"s"(a.st[1].eltw_u8));
+}
+
 // 64 features in the first stage and the reduction, 256 in the expansion
 template <bool HAS2, bool SUM>
 __global__ void __launch_bounds__(512, 4) conv_coop_kernel(CoopConvArgs a)
 {
-    constexpr int W = 8, TAPS = 9, R0 = 2;
+    constexpr int W = 8, LAST_TAP = 8;
     constexpr int N0 = 4;  // fragments of stages 0 and 2
     constexpr int F1 = 2;  // fragments of the expansion per wave: half a span
     constexpr int RELU = EPI_KIND_RELU, EPI1 = SUM ? EPI_KIND_FUSED : EPI_KIND_RELU;
+    fetch_arguments(a);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kq = lane >> 4;
@@ -84,7 +101,7 @@ __global__ void __launch_bounds__(512, 4) conv_coop_kernel(CoopConvArgs a)
         uint32_t b, oy, ox;
         bool ok;
     };
-    v4i xb[R0];
+    v4i xb, xb8;  // the wave's tap, the ninth
     int ev[F1];
     Pos cur, nxt;
     auto request = [&](int g, Pos& p) {
@@ -96,15 +113,13 @@ __global__ void __launch_bounds__(512, 4) conv_coop_kernel(CoopConvArgs a)
         p.oy = a.div_ow.div(r);
         p.ox = r - p.oy * a.OW;
         const uint32_t off = (uint32_t)(a.in_off + (int)p.b * a.in_pb + (int)p.oy * a.row + (int)p.ox * a.col + kq * a.in_pf);
-#pragma unroll
-        for (int r0 = 0; r0 < R0; ++r0) {
-            const int tap = wave + r0 * W;
-            if (tap < TAPS) {
-                xb[r0] = *reinterpret_cast<const v4i*>(a.in + ((tap / 3) * a.tap_dy + (tap % 3) * 16) + off);
-            } else {
-                asm volatile("" : "=v"(xb[r0]));
-            }
-        }
+        auto of_tap = [&](int tap) {
+            const int ty = (tap * 11) >> 5;
+            return *reinterpret_cast<const v4i*>(a.in + (off + (uint32_t)(ty * a.tap_dy + (tap - ty * 3) * 16)));
+        };
+        xb = of_tap(wave);
+        if (wave < N0) xb8 = of_tap(LAST_TAP);
+        else asm volatile("" : "=v"(xb8));
     };
     auto residual = [&](const Pos& p) {
         if constexpr (SUM) {
@@ -116,7 +131,7 @@ __global__ void __launch_bounds__(512, 4) conv_coop_kernel(CoopConvArgs a)
     auto at = [&](const CoopConvStage& st, const Pos& p, int slice) { return (uint32_t)(st.off + (int)p.b * st.pb + slice * st.pf + (int)p.oy * st.py + (int)p.ox * 16); };
 
     // ---------------- everything that is needed first, in the order of its use
-    v4i w0[R0][N0], w1[F1], w2[HAS2 ? N0 : 1];
+    v4i w0[N0], w8, w1[F1], w2[HAS2 ? N0 : 1];  // w8: the wave's fragment of the ninth tap
     {
         v4i r[2];
 #pragma unroll
@@ -124,14 +139,9 @@ __global__ void __launch_bounds__(512, 4) conv_coop_kernel(CoopConvArgs a)
         step_fence();
         request(g_begin, cur);
 #pragma unroll
-        for (int r0 = 0; r0 < R0; ++r0)
-            if (wave + r0 * W < TAPS) {
-#pragma unroll
-                for (int i = 0; i < N0; ++i) w0[r0][i] = unit(s0.unit0 + wave + r0 * W, i);
-            } else {
-#pragma unroll
-                for (int i = 0; i < N0; ++i) asm volatile("" : "=v"(w0[r0][i]));
-            }
+        for (int i = 0; i < N0; ++i) w0[i] = unit(s0.unit0 + wave, i);
+        if (wave < N0) w8 = unit(s0.unit0 + LAST_TAP, wave);
+        else asm volatile("" : "=v"(w8));
         step_fence();
         residual(cur);
 #pragma unroll
@@ -168,17 +178,17 @@ __global__ void __launch_bounds__(512, 4) conv_coop_kernel(CoopConvArgs a)
     };
 
     for (int g = g_begin; g < g_end; ++g) {
-        // ---------------- stage 0: this wave's K-steps of all features
+        // ---------------- stage 0: this wave's tap of all features
         v4i acc0[1][N0];
+        const v4i xm = {(int)s0.xor_mask, (int)s0.xor_mask, (int)s0.xor_mask, (int)s0.xor_mask};
+        const v4i x = xb ^ xm;
 #pragma unroll
-        for (int i = 0; i < N0; ++i) acc0[0][i] = none;
+        for (int i = 0; i < N0; ++i) acc0[0][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0[i], x, none, 0, 0, 0);
+        if (wave < N0) {
+            const v4i x8 = xb8 ^ xm;
 #pragma unroll
-        for (int r0 = 0; r0 < R0; ++r0) {
-            if (wave + r0 * W < TAPS) {
-                const v4i x = {flip(xb[r0][0], s0.xor_mask), flip(xb[r0][1], s0.xor_mask), flip(xb[r0][2], s0.xor_mask), flip(xb[r0][3], s0.xor_mask)};
-#pragma unroll
-                for (int i = 0; i < N0; ++i) acc0[0][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w0[r0][i], x, acc0[0][i], 0, 0, 0);
-            }
+            for (int i = 0; i < N0; ++i)
+                if (i == wave) acc0[0][i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w8, x8, acc0[0][i], 0, 0, 0);
         }
         mfma_settle(acc0);
 #pragma unroll

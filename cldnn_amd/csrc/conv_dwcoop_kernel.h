@@ -19,6 +19,10 @@
 // Kernel time in a network, before (a wave walked over two K-steps of 64 with one tap a product, partial sums of the projection
 // went through LDS) and now: 14x14, 384-64-384 6.5 -> 5.6 us at batch 1, 11.1 -> 6.9 at batch 32; 576-96-576 9.2 -> 6.4 and 15.5 ->
 // 10.6; 7x7, 960-160-960 11.8 -> 8.4 and 11.8 -> 8.6.
+// A wave is alone on its SIMD at batch 1, and an instruction of its is 3 to 4 ns: of 3.9 us (384-64-384) 0.2 are the arguments, 0.5 the
+// way to the last request, 0.4 the taps on their way, 0.4 the depthwise products, 0.55 their requantisation, 0.5 projection and barriers,
+// 0.9 its requantisation and the expansion.  Words of the later weights asked for ahead, so that they come from L2, cost as much
+// of L1's time as the weights themselves (960-160-960 7.7 -> 9.4).
 #pragma once
 #include "conv_dwchain_kernel.h"
 
@@ -59,12 +63,28 @@ struct CoopEpi {
     FastEpi fe;
 };
 
+// All arguments behind one wait: fetched where they are first used they were four trips to memory in a row.
+__device__ __forceinline__ void fetch_arguments(const DwCoopArgs& a)
+{
+    asm volatile("" ::"s"(a.in), "s"(a.img), "s"(a.eltw), "s"(a.w1), "s"(a.w2), "s"(a.v0), "s"(a.v1), "s"(a.v2), "s"(a.el_off), "s"(a.el_pb), "s"(a.el_pf), "s"(a.el_py), "s"(a.el_px),
+                 "s"(a.M), "s"(a.OHW), "s"(a.OW), "s"(a.div_ohw.mul), "s"(a.div_ohw.shift), "s"(a.div_ow.mul), "s"(a.div_ow.shift), "s"(a.in_off), "s"(a.in_pb), "s"(a.in_pf), "s"(a.row),
+                 "s"(a.col), "s"(a.tap_dy));
+    asm volatile("" ::"s"(a.CB), "s"(a.KS), "s"(a.F1), "s"(a.SP2), "s"(a.waves), "s"(a.parts), "s"(a.div_parts.mul), "s"(a.div_parts.shift), "s"(a.clamp_m0), "s"(a.clamp_n0),
+                 "s"(a.clamp_m2), "s"(a.clamp_n2), "s"(a.lo1), "s"(a.hi1), "s"(a.conv_lo), "s"(a.conv_hi), "s"(a.eltw_u8), "s"(gridDim.x));
+#pragma unroll
+    for (int k = 0; k < CHAIN_MAX_STAGES; ++k)
+        asm volatile("" ::"s"(a.st[k].out), "s"(a.st[k].off), "s"(a.st[k].pb), "s"(a.st[k].pf), "s"(a.st[k].py), "s"(a.st[k].ofm), "s"(a.st[k].xor_mask));
+}
+
 // K1: K-steps of the expansion.  KM: K-steps of the projection that a wave has registers for.  DEEP: there are more of them, or more
 // than waves: both are walked in rounds.  NG: granules of a workgroup (at most ten waves with two).
 template <int K1, int KM, bool DEEP, int NG, bool HAS2, bool SUM>
 __global__ void __launch_bounds__(NG > 1 ? 640 : 64 * DWCOOP_MAX_WAVES, NG > 1 ? 3 : 4) conv_dwcoop_kernel(DwCoopArgs a)
 {
     constexpr int CQ = EPI_KIND_CLAMPQ, EPI1 = SUM ? EPI_KIND_SUMLIN : EPI_KIND_LINEAR, S = DWCHAIN_STEPS;
+    // the expansion's weights fit into the registers of the taps beside the projection's: both are requested together
+    constexpr bool BOTH = HAS2 && !DEEP && NG == 1 && KM + 4 * K1 <= 17;
+    fetch_arguments(a);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int W = a.waves;
@@ -208,6 +228,9 @@ __global__ void __launch_bounds__(NG > 1 ? 640 : 64 * DWCOOP_MAX_WAVES, NG > 1 ?
             }
     v4i acc0[NG * 4][1];
     auto depthwise = [&] {
+        // (the last word of a unit's weights is not read below: were it free to be overwritten, whatever does so would wait for
+        // the weights, in front of the requests for the taps)
+        asm volatile("" ::"v"(dw[0]), "v"(dw[1]));
 #pragma unroll
         for (int n = 0; n < NG; ++n)
 #pragma unroll
@@ -263,8 +286,14 @@ __global__ void __launch_bounds__(NG > 1 ? 640 : 64 * DWCOOP_MAX_WAVES, NG > 1 ?
     } else {
         if (works0) depthwise();
         else forget(reinterpret_cast<v4i(&)[NG * 4]>(acc0));
+        if constexpr (BOTH)
+            if (lane < 48) own[60 + lane] = vec;
         if (works1) request1(0, wave);  // the registers of the taps are free
         else forget(u1);
+        if constexpr (BOTH) {
+            if (sp_first < a.SP2) request2(sp_first);
+            else forget(u2);
+        }
         step_fence();
         if (works0) finish0(wave);
     }
@@ -291,7 +320,7 @@ __global__ void __launch_bounds__(NG > 1 ? 640 : 64 * DWCOOP_MAX_WAVES, NG > 1 ?
         }
         mfma_settle(acc1);
     }
-    if constexpr (HAS2) {
+    if constexpr (HAS2 && !BOTH) {
         if (sp_first < a.SP2) request2(sp_first);
         else forget(u2);
         if (lane < 48) own[60 + lane] = vec;

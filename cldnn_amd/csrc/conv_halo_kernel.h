@@ -110,9 +110,9 @@ __global__ void __launch_bounds__(WP * WF * 64) conv_halo_kernel(HaloArgs h)
     // Everything the prologue and the loop read from the argument block is requested here, behind ONE wait: left to
     // itself the compiler fetches arguments where they are first used, four dependent round trips to memory (about
     // 0.4 us each) before the first operand request goes out.
-    asm volatile("" ::"s"(a.in), "s"(a.wpk), "s"(a.acc_init), "s"(a.ofm_tiles), "s"(a.div_ofm_tiles.mul), "s"(a.div_ofm_tiles.shift), "s"(a.div_ofm_tiles.one), "s"(a.ksteps), "s"(a.in_pf), "s"(a.xor_mask),
+    asm volatile("" ::"s"(a.in), "s"(a.wpk), "s"(a.acc_init), "s"(a.ofm_tiles), "s"(a.div_ofm_tiles.mul), "s"(a.div_ofm_tiles.shift), "s"(a.ksteps), "s"(a.in_pf), "s"(a.xor_mask),
                  "s"(h.pos_total), "s"(h.halo_lo), "s"(h.patch_len), "s"(h.cps), "s"(h.div_cps.mul), "s"(h.div_cps.shift),
-                 "s"(h.div_cps.one), "s"(h.blocks), "s"(h.ptiles), "s"(h.parts), "s"(h.tap[0]), "s"(h.tap[1]), "s"(h.tap[2]),
+                 "s"(h.blocks), "s"(h.ptiles), "s"(h.parts), "s"(h.tap[0]), "s"(h.tap[1]), "s"(h.tap[2]),
                  "s"(h.tap[3]), "s"(h.tap[4]), "s"(h.tap[5]), "s"(h.tap[6]), "s"(h.tap[7]), "s"(h.tap[8]));
 
     // Workgroup ids are dealt round-robin to the eight dies.  A die takes a contiguous eighth of the partitions with

@@ -42,13 +42,13 @@ static KsplitArgs ksplit_args(const MfmaArgs& m)
     a.mtiles = m.mtiles, a.ftiles = m.ofm_tiles;
     a.features_outer = m.by_features != 0, a.die_bits = m.by_features == 2 ? 0 : 3;
     a.inner = a.features_outer ? a.mtiles : a.ftiles;
-    a.div_inner = make_even_div((uint32_t)a.inner);
+    a.div_inner = make_fast_div((uint32_t)a.inner);
     a.M = m.M, a.OFM = m.OFM, a.OHW = m.OHW, a.OW = m.OW, a.OH = m.OH, a.IH = m.IH, a.IW = m.IW;
-    a.div_ohw = make_even_div((uint32_t)m.OHW), a.div_ow = make_even_div((uint32_t)m.OW);
+    a.div_ohw = make_fast_div((uint32_t)m.OHW), a.div_ow = make_fast_div((uint32_t)m.OW);
     a.ksteps = m.ksteps, a.kper = m.kper, a.kwaves = m.kwaves;
     a.in_pb = m.in_pb, a.in_row = m.sy * m.in_py, a.in_col = m.sx * 16, a.in_pf = m.in_pf;
     a.taps = m.FX * m.FY, a.FX = m.FX, a.tap_dy = m.tap_dy, a.tap_dx = m.tap_dx, a.last_group = m.CB - 4;
-    a.div_taps = make_even_div((uint32_t)a.taps), a.div_fx = make_even_div((uint32_t)m.FX), a.div_cb = make_even_div((uint32_t)m.CB);
+    a.div_taps = make_fast_div((uint32_t)a.taps), a.div_fx = make_fast_div((uint32_t)m.FX), a.div_cb = make_fast_div((uint32_t)m.CB);
     a.out_off = m.out_off, a.out_pb = m.out_pb, a.out_pf = m.out_pf, a.out_py = m.out_py, a.out_f = m.out_f;
     a.el_off = m.el_off, a.el_pb = m.el_pb, a.el_pf = m.el_pf, a.el_row = m.esy * m.el_py, a.el_col = m.esx * 16;
     a.xor_mask = m.xor_mask;

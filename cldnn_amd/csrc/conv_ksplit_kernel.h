@@ -38,18 +38,6 @@ namespace chip {
 enum { ADDR_UNIFORM = 0, ADDR_LANES = 1, ADDR_GATHERED = 2 };
 enum { GEMV_SLACK = 32 };  // K-steps of slack behind every gathered pixel fragment
 
-// q = n / d for n < 2^31: FastDiv's constants with the numerator doubled, which leaves no case apart for d == 1
-struct EvenDiv {
-    uint32_t mul, shift;
-    __device__ __forceinline__ uint32_t div(uint32_t n) const { return __umulhi(n << 1, mul) >> shift; }
-};
-inline EvenDiv make_even_div(uint32_t d)
-{
-    uint32_t s = 0;
-    while ((1ull << s) < d) ++s;
-    return {(uint32_t)(((1ull << (31 + s)) + d - 1) / d), s};
-}
-
 struct KsplitArgs {
     const int8_t* in;                    // of tap (0, 0) of output pixel (0, 0)
     const v4i *wpk, *bpk;                // weights; activations in fragment order (GATHERED)
@@ -57,7 +45,7 @@ struct KsplitArgs {
     void* out;
     const int8_t* eltw;
     const int32_t* origin;
-    EvenDiv div_inner, div_ohw, div_ow, div_taps, div_fx;
+    FastDiv div_inner, div_ohw, div_ow, div_taps, div_fx;
     // workgroup id -> (outer tile, inner tile): dies take every eighth outer one (die_bits 3) or tiles are counted off (0)
     int32_t inner, die_bits, features_outer, mtiles, ftiles;
     uint32_t M;
@@ -69,7 +57,7 @@ struct KsplitArgs {
     int32_t el_off, el_pb, el_pf, el_row, el_col;
     uint32_t xor_mask;
     // LANES, and the accumulators alone
-    EvenDiv div_cb;
+    FastDiv div_cb;
     int32_t CB, kchunks, checked, sy, sx, py, px, dil_y, dil_x, IH, IW, OH;
     uint32_t inside;                     // of a byte that exists, behind `in`
     int32_t* raw;

@@ -88,17 +88,10 @@ FastDiv make_fast_div(uint32_t d);
 static FastDiv make_div(uint32_t d) { return make_fast_div(d); }
 FastDiv make_fast_div(uint32_t d)
 {
-    FastDiv f{};
-    if (d <= 1) {
-        f.one = 1;
-        return f;
-    }
+    if (!d) d = 1;  // (of an extent that a form does not use)
     uint32_t s = 0;
-    while ((1ull << s) < d) ++s;              // s = ceil(log2 d) >= 1
-    const unsigned p = 31 + s;
-    f.mul = (uint32_t)(((1ull << p) + d - 1) / d);  // ceil(2^p / d) < 2^32
-    f.shift = p - 32;
-    return f;
+    while ((1ull << s) < d) ++s;  // ceil(log2 d)
+    return {(uint32_t)(((1ull << (31 + s)) + d - 1) / d), s};
 }
 
 // does the input buffer carry a zero border that covers every tap of every output pixel?

@@ -36,10 +36,11 @@ namespace chip {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-// q = n / d for 0 <= n < 2^31 by multiply-high and shift
+// q = n / d for 0 <= n < 2^31 by multiply-high and shift.  The numerator is doubled, so that the multiplier of d == 1 fits too and
+// there is no case apart (which was a branch, or two selects, in front of the first request).
 struct FastDiv {
-    uint32_t mul, shift, one;
-    __device__ __forceinline__ uint32_t div(uint32_t n) const { return one ? n : (__umulhi(n, mul) >> shift); }
+    uint32_t mul, shift;
+    __device__ __forceinline__ uint32_t div(uint32_t n) const { return __umulhi(n << 1, mul) >> shift; }
 };
 
 FastDiv make_fast_div(uint32_t d);  // host
@@ -615,14 +616,14 @@ __device__ __forceinline__ void fetch_arguments(const MfmaArgs& a)
 {
     asm volatile("" ::"s"(a.in), "s"(a.wpk), "s"(a.ktab), "s"(a.acc_init), "s"(a.out), "s"(a.eltw), "s"(a.M), "s"(a.OFM),
                  "s"(a.ofm_tiles), "s"(a.mtiles), "s"(a.OHW), "s"(a.OW), "s"(a.div_ohw.mul), "s"(a.div_ohw.shift),
-                 "s"(a.div_ohw.one), "s"(a.div_ow.mul), "s"(a.div_ow.shift), "s"(a.div_ow.one), "s"(a.sy), "s"(a.sx), "s"(a.py),
+                 "s"(a.div_ow.mul), "s"(a.div_ow.shift), "s"(a.sy), "s"(a.sx), "s"(a.py),
                  "s"(a.px), "s"(a.esy), "s"(a.esx));
     asm volatile("" ::"s"(a.in_off), "s"(a.in_pb), "s"(a.in_pf), "s"(a.in_py), "s"(a.out_off), "s"(a.out_pb), "s"(a.out_pf),
                  "s"(a.out_py), "s"(a.el_off), "s"(a.el_pb), "s"(a.el_pf), "s"(a.el_py), "s"(a.ksteps), "s"(a.CB), "s"(a.FX),
                  "s"(a.kchunks), "s"(a.tap_dy), "s"(a.tap_dx), "s"(a.linear), "s"(a.px_bytes), "s"(a.by_features));
-    asm volatile("" ::"s"(a.div_cb.mul), "s"(a.div_cb.shift), "s"(a.div_cb.one), "s"(a.div_fx.mul), "s"(a.div_fx.shift),
-                 "s"(a.div_fx.one), "s"(a.div_mtiles.mul), "s"(a.div_mtiles.shift), "s"(a.div_mtiles.one), "s"(a.div_ofm_tiles.mul),
-                 "s"(a.div_ofm_tiles.shift), "s"(a.div_ofm_tiles.one), "s"(a.xor_mask), "s"(a.wsl_parts), "s"(a.wsl_tpp), "s"(a.FY),
+    asm volatile("" ::"s"(a.div_cb.mul), "s"(a.div_cb.shift), "s"(a.div_fx.mul), "s"(a.div_fx.shift),
+                 "s"(a.div_mtiles.mul), "s"(a.div_mtiles.shift), "s"(a.div_ofm_tiles.mul),
+                 "s"(a.div_ofm_tiles.shift), "s"(a.xor_mask), "s"(a.wsl_parts), "s"(a.wsl_tpp), "s"(a.FY),
                  "s"(a.epi.calib), "s"(a.epi.eltw_calib), "s"(a.epi.wqf), "s"(a.fe.hi), "s"(a.fe.lo), "s"(a.origin));
 }
 
