@@ -18,12 +18,16 @@ struct ChainStageIn {
     const int32_t* dw_wmask = nullptr;
 };
 
+// waves of a workgroup whose waves take one granule of 16 * nt pixels each
+constexpr int chain_waves(int nt) { return nt == 1 ? 8 : 4; }
+
 struct ChainPlan {
     int stages;
     int dw;                    // 1: the first stage is a depthwise 3x3
     int coop;                  // 1: its form for small planes, a workgroup's waves share a granule (conv_dwcoop_kernel.h)
     int waves;                 // waves per workgroup
     int nt;                    // 16-pixel fragments per wave and granule
+    int eltw_u8;               // the residual of stage 1 is unsigned
     int depth;                 // activation look-ahead of stage 0 in K-steps
     int ksteps0;               // K-steps of stage 0 (padded to a multiple of depth)
     int sp[3];                 // 64-feature spans per stage

@@ -33,26 +33,29 @@ int epilogue_kind(const ChainStageIn& s)
 
 struct Instance {
     int nt, d, sp0, sp1, sp2, e0, e1, e2;
+    bool u8;  // of the residual
     void (*launch)(hipStream_t, const ChainArgs&, int, int);
 };
-#define CHAIN_INSTANCE(NT, D, SP0, SP1, SP2, E0, E1, E2) \
-    {NT, D, SP0, SP1, SP2, E0, E1, E2, &launch_chain_instance<NT, D, SP0, SP1, SP2, E0, E1, E2>}
+#define CHAIN_INSTANCE(NT, D, SP0, SP1, SP2, E0, E1, E2, U8) \
+    {NT, D, SP0, SP1, SP2, E0, E1, E2, U8, &launch_chain_instance<NT, D, SP0, SP1, SP2, E0, E1, E2, U8>}
 // What is compiled: the tails of ResNet bottlenecks with 64 mid features (3x3 -> expansion [+ residual] -> next
 // reduction), residual fused or not; and pairs of an expansion to 256 features and a first stage with 3 or 9 K-steps, such as
 // a 1x1 from 192 or 576 features (the 3x3 over 64, also 9, runs on conv_coop_kernel.h): 56x56 at batch 32 13.7 and 18.2 us
 // against 18.9 and 23.8 in two launches, equal at batch 1.
 const Instance g_instances[] = {
-    CHAIN_INSTANCE(2, 3, 1, 4, 1, EPI_KIND_RELU, EPI_KIND_FUSED, EPI_KIND_RELU),
-    CHAIN_INSTANCE(2, 3, 1, 4, 0, EPI_KIND_RELU, EPI_KIND_FUSED, EPI_KIND_RELU),
-    CHAIN_INSTANCE(2, 3, 1, 4, 1, EPI_KIND_RELU, EPI_KIND_RELU, EPI_KIND_RELU),
-    CHAIN_INSTANCE(2, 3, 1, 4, 0, EPI_KIND_RELU, EPI_KIND_RELU, EPI_KIND_RELU),
+    CHAIN_INSTANCE(1, 3, 1, 4, 1, EPI_KIND_RELU, EPI_KIND_FUSED, EPI_KIND_RELU, true),
+    CHAIN_INSTANCE(2, 3, 1, 4, 0, EPI_KIND_RELU, EPI_KIND_FUSED, EPI_KIND_RELU, true),
+    CHAIN_INSTANCE(1, 3, 1, 4, 1, EPI_KIND_RELU, EPI_KIND_FUSED, EPI_KIND_RELU, false),
+    CHAIN_INSTANCE(2, 3, 1, 4, 0, EPI_KIND_RELU, EPI_KIND_FUSED, EPI_KIND_RELU, false),
+    CHAIN_INSTANCE(1, 3, 1, 4, 1, EPI_KIND_RELU, EPI_KIND_RELU, EPI_KIND_RELU, false),
+    CHAIN_INSTANCE(2, 3, 1, 4, 0, EPI_KIND_RELU, EPI_KIND_RELU, EPI_KIND_RELU, false),
 };
 
 const Instance* find_instance(const ChainPlan& pl)
 {
     for (const Instance& i : g_instances)
         if (i.nt == pl.nt && i.d == pl.depth && i.sp0 == pl.sp[0] && i.sp1 == pl.sp[1] && i.sp2 == pl.sp[2] && i.e0 == pl.epi[0]
-            && i.e1 == pl.epi[1] && (pl.stages < 3 || i.e2 == pl.epi[2]))
+            && i.e1 == pl.epi[1] && (pl.stages < 3 || i.e2 == pl.epi[2]) && i.u8 == (pl.eltw_u8 != 0))
             return &i;
     return nullptr;
 }
@@ -170,7 +173,7 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
         *out = pl;
         return std::string();
     }
-    pl.nt = 2, pl.waves = 4;
+    pl.nt = n > 2 ? 1 : 2, pl.waves = chain_waves(pl.nt);
     pl.granules = (int)((pl.m_total + 16 * pl.nt - 1) / (16 * pl.nt));
     // K-steps of every stage as the weights-stationary row packs them
     MfmaPlan mp[3]{};
@@ -198,7 +201,7 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
         }
         // The weights in the registers of eight waves that share a granule: chains of two stages, and of three up to four
         // granules per CU (with more, one granule per wave needs fewer instructions a pixel; conv_coop_kernel.h).  Inside ResNet-50,
-        // one granule per wave / shared: 588 granules 13.1 / 11.1 us, 784 13.2 / 12.3, 938 13.7 / 12.1, 1016 13.1 / 11.7.
+        // one granule per wave / shared: 588 granules 9.6 / 7.9 us, 784 9.9 / 9.0, 980 10.2 / 9.4, 1568 11.6 / 14.1, 1960 12.4 / 14.6.
         const bool block = p0.FY == 3 && p0.FX == 3 && pl.sp[0] == 1 && p0.IFM == 64 && pl.sp[1] == 4 && (n < 3 || pl.sp[2] == 1)
                            && pl.epi[0] == EPI_KIND_RELU && (pl.epi[1] == EPI_KIND_RELU || pl.epi[1] == EPI_KIND_FUSED)
                            && (n < 3 || pl.epi[2] == EPI_KIND_RELU);
@@ -215,11 +218,12 @@ std::string chain_plan(const ChainStageIn* st, int n, int cus, ChainPlan* out)
             return std::string();
         }
         pl.depth = mp[0].wsl_depth, pl.ksteps0 = mp[0].ksteps;
+        pl.eltw_u8 = pl.epi[1] == EPI_KIND_FUSED && st[1].fe->eltw_u8;
         pl.lds_bytes = pl.img_bytes = pl.units * 4096 + vec * 4;
         if (mp[0].wsl_depth > 0 && pl.lds_bytes <= CHAIN_MAX_LDS && find_instance(pl)) {
             const int per_cu = pl.lds_bytes * 2 <= CHAIN_MAX_LDS ? 2 : 1;
             int grid = cus * per_cu / 8 * 8;
-            const int wanted = ((pl.granules + 3) / 4 + 7) / 8 * 8;  // at least one granule per wave
+            const int wanted = ((pl.granules + pl.waves - 1) / pl.waves + 7) / 8 * 8;  // at least one granule per wave
             if (grid > wanted) grid = wanted;
             if (grid < 8) grid = 8;
             pl.grid = grid;
@@ -499,8 +503,8 @@ void launch_conv_chain(hipStream_t s, const ChainStageIn* st, const ChainPlan& p
     a.units = pl.units;
     a.vec_quads = (pl.lds_bytes - pl.units * 4096) / 16;
     a.granules = pl.granules;
-    a.gpw = pl.granules / (pl.grid * 4), a.grem = pl.granules % (pl.grid * 4);
-    a.div_waves = make_fast_div((uint32_t)pl.grid * 4u);
+    a.gpw = pl.granules / (pl.grid * pl.waves), a.grem = pl.granules % (pl.grid * pl.waves);
+    a.div_waves = make_fast_div((uint32_t)pl.grid * (uint32_t)pl.waves);
     a.M = (uint32_t)pl.m_total;
     a.OHW = p0.OH * p0.OW, a.OW = p0.OW;
     a.div_ohw = make_fast_div((uint32_t)a.OHW), a.div_ow = make_fast_div((uint32_t)a.OW);

@@ -9,10 +9,20 @@
 // stage for its 16*NT pixels therefore feeds the next stage straight from its registers: the intermediate tensor
 // is never written (unless somebody else reads it) and never read back.
 //
-// Work split: persistent workgroups of four INDEPENDENT waves.  All weights of all stages (a few tens of KB) and
+// Work split: persistent workgroups of INDEPENDENT waves.  All weights of all stages (a few tens of KB) and
 // the per-feature vectors are copied into LDS once per workgroup; after that a wave walks over its own range of
 // 16*NT-pixel granules without any barrier.  Feature counts are multiples of 64.  Stage 0 reads its activations straight from global memory, D K-steps
 // ahead of their use, and the look-ahead runs across granule boundaries (as in the weights-stationary kernel).
+// The residual of stage 1 is asked for a whole granule ahead, each span's as soon as the previous granule has used its registers:
+// requests of a wave return in order, so one that goes to memory at the start of a granule also holds up every activation
+// requested behind it.
+//
+// What bounds it: nothing alone.  Without the requantisation the chain of three stages below takes 63 us instead of 73, without its
+// stores 64, with a residual that lies in L1 60; the waves wait for memory a third of the time.  So three stages go 16 pixels at a
+// time (NT == 1) in 128 registers: eight waves to a workgroup, four to a SIMD, where 32 pixels at a time leave two.  The weights are
+// read from LDS twice as often for it, a third of what LDS delivers.  64 -> 64 -> 256 + sum -> 64 at 56x56, batch 128: 77.9 us with
+// 32 pixels, 73.2 with 16, 68.4 with the residual ahead as well (32 pixels and the residual ahead: 70.5); batch 32: 25.6, 24.1, 22.9
+// (24.6).
 // Every stage has its own epilogue kind, per-feature vectors, output tensor and (optional) residual tensor.
 #pragma once
 #include <mutex>
@@ -117,12 +127,12 @@ constexpr bool chain_reads_residual()
 }
 
 // SP0 / SP1 / SP2: 64-feature spans of the three stages (SP2 == 0: two stages, whose first is no 3x3 over 64 features: that one
-// runs on conv_coop_kernel.h).  D: activation look-ahead of stage 0.
-template <int NT, int D, int SP0, int SP1, int SP2, int EPI0, int EPI1, int EPI2>
-__global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
+// runs on conv_coop_kernel.h).  D: activation look-ahead of stage 0.  U8: the residual of stage 1 is unsigned.
+template <int NT, int D, int SP0, int SP1, int SP2, int EPI0, int EPI1, int EPI2, bool U8>
+__global__ void __launch_bounds__(64 * chain_waves(NT), NT == 1 ? 4 : 1) conv_chain_kernel(ChainArgs a)
 {
+    static_assert(EPI0 == EPI_KIND_RELU && EPI1 != EPI_KIND_FAST && EPI2 != EPI_KIND_FAST, "a kind that adds has something to add");
     constexpr int WP = NT * 16;
-    constexpr int EVD = SP1 < 4 ? SP1 : 4;  // residual look-ahead of stage 1, in spans
     const int t = threadIdx.x;
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -139,14 +149,14 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
         // one bulk copy: the image holds the weight units and, behind them, the per-feature vectors of all stages
         // (absent vectors filled with their neutral values by the host); all requests of a thread are in flight at once
         const int total = a.units * 256 + a.vec_quads;
-        constexpr int BATCH = 20;
-        for (int i = t; i < total; i += BATCH * 256) {
+        constexpr int THREADS = 64 * chain_waves(NT), BATCH = 5120 / THREADS;  // 80 KB at a time
+        for (int i = t; i < total; i += BATCH * THREADS) {
             v4i r[BATCH];
 #pragma unroll
-            for (int u = 0; u < BATCH; ++u) r[u] = a.wpk[min(i + u * 256, total - 1)];
+            for (int u = 0; u < BATCH; ++u) r[u] = a.wpk[min(i + u * THREADS, total - 1)];
 #pragma unroll
             for (int u = 0; u < BATCH; ++u)
-                if (i + u * 256 < total) ldsW[i + u * 256] = r[u];
+                if (i + u * THREADS < total) ldsW[i + u * THREADS] = r[u];
         }
     }
 
@@ -157,7 +167,7 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
     const int per_xcd = gridDim.x >> 3;  // the grid is a multiple of 8
     const uint32_t vb = (blockIdx.x & 7u) * (uint32_t)per_xcd + (blockIdx.x >> 3);
     // (a 64-bit division of two run-time values here costs every wave a few hundred instructions before its first request)
-    const uint32_t gw = vb * 4u + (uint32_t)wave;
+    const uint32_t gw = vb * (uint32_t)chain_waves(NT) + (uint32_t)wave;
     const int g_begin = (int)(gw * (uint32_t)a.gpw + a.div_waves.div(gw * (uint32_t)a.grem));
     const int g1 = (int)((gw + 1) * (uint32_t)a.gpw + a.div_waves.div((gw + 1) * (uint32_t)a.grem));
 
@@ -165,6 +175,11 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
     const v4i xm1 = {(int)s1.xor_mask, (int)s1.xor_mask, (int)s1.xor_mask, (int)s1.xor_mask};
     const v4i xm2 = {(int)s2.xor_mask, (int)s2.xor_mask, (int)s2.xor_mask, (int)s2.xor_mask};
     const int cb4 = a.CB >> 2;
+    // (a constant, so that both forms of the sum are not compiled into every span: they cost 30 registers)
+    struct {
+        FastEpi fe;
+    } e1{s1.fe};
+    e1.fe.eltw_u8 = U8;
 
     struct Refs {
         uint32_t boff[NT];
@@ -197,9 +212,7 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
     };
     auto unit = [&](const ChainStage& st, int span, int ks) { return ldsW + (size_t)(st.unit0 + span * st.kstride + ks) * 256; };
     auto residual = [&](const ChainStage& st, int ebase, int span) {
-        v4i v = {0, 0, 0, 0};
-        if (st.fe.fused) v = *reinterpret_cast<const v4i*>((const int8_t*)st.eltw + ebase + span * 4 * st.el_pf);
-        return v;
+        return *reinterpret_cast<const v4i*>((const int8_t*)st.eltw + span * 4 * st.el_pf + (uint32_t)ebase);
     };
 
     if (g_begin >= g1) {
@@ -216,19 +229,18 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
         load_b(cur, walk, rb[d]);
         chain_tap_advance(a, walk, cb4);
     }
+    // residual of stage 1: a span's is requested where the previous granule has used its registers, a granule ahead
+    v4i ev1[SP1][NT];
+    if constexpr (chain_reads_residual<EPI1>()) {
+#pragma unroll
+        for (int s = 0; s < SP1; ++s)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) ev1[s][nt] = residual(s1, cur.e1[nt], s);
+    }
     __syncthreads();  // weights and vectors are in LDS; no barrier after this point
 
     for (int g = g_begin; g < g1; ++g) {
         setup(g + 1, nxt);
-        // residual of stage 1 for the first spans: requested now, used after the whole of stage 0
-        v4i ev1[EVD][NT];
-        if constexpr (chain_reads_residual<EPI1>()) {
-#pragma unroll
-            for (int s = 0; s < EVD; ++s)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) ev1[s][nt] = residual(s1, cur.e1[nt], s);
-        }
-
         // ---------------- stage 0: the spatial convolution, all SP0 spans at once
         v4i acc0[SP0 * 4][NT];
 #pragma unroll
@@ -247,7 +259,8 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
                 for (int mt = 0; mt < 4; ++mt) fa[sp * 4 + mt] = unit(s0, sp, ks)[kq * 64 + mt * 16 + l16];
         };
         auto step = [&](int ks, int d, const Refs& refill_from) {
-            load_a0(ks + 1 < a.ksteps0 ? ks + 1 : 0, fa_nxt);
+            if constexpr (NT == 1) load_a0(ks, fa_cur);
+            else load_a0(ks + 1 < a.ksteps0 ? ks + 1 : 0, fa_nxt);
             v4i fb[NT];
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) fb[nt] = rb[d][nt] ^ xm0;
@@ -258,11 +271,13 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
                     acc0[m][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa_cur[m], fb[nt], acc0[m][nt], 0, 0, 0);
             load_b(refill_from, walk, rb[d]);
             chain_tap_advance(a, walk, cb4);
+            if constexpr (NT > 1) {
 #pragma unroll
-            for (int m = 0; m < SP0 * 4; ++m) fa_cur[m] = fa_nxt[m];
+                for (int m = 0; m < SP0 * 4; ++m) fa_cur[m] = fa_nxt[m];
+            }
             step_fence();
         };
-        load_a0(0, fa_cur);
+        if constexpr (NT > 1) load_a0(0, fa_cur);
         for (int ks0 = 0; ks0 + D < a.ksteps0; ks0 += D) {
 #pragma unroll
             for (int d = 0; d < D; ++d) step(ks0 + d, d, cur);
@@ -285,7 +300,7 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
                 v4i ev = {0, 0, 0, 0};
                 if constexpr (chain_reads_residual<EPI0>()) ev = residual(s0, cur.e0[nt], sp);
                 const v4i packed = epilogue_fast16<NT, EPI0>(s0, acc_sp, nt, sc.wq, sc.cal, sc.ecal, ev, 16);
-                if (cur.o0[nt] >= 0) *reinterpret_cast<v4i*>((int8_t*)s0.out + cur.o0[nt] + sp * 4 * s0.out_pf) = packed;
+                if (cur.o0[nt] >= 0) *reinterpret_cast<v4i*>((int8_t*)s0.out + sp * 4 * s0.out_pf + (uint32_t)cur.o0[nt]) = packed;
                 bf0[sp][nt] = packed ^ xm1;
             }
         }
@@ -323,25 +338,23 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
                     for (int nt = 0; nt < NT; ++nt)
                         acc1[mt][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[mt], bf0[ks][nt], acc1[mt][nt], 0, 0, 0);
             }
+            if constexpr (NT == 1) step_fence();
             LaneScales sc;
             chain_scales<EPI1>(s1, ldsV, SP1, f0, sc);
             v4i bf1[NT];
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 v4i ev = {0, 0, 0, 0};
-                if constexpr (chain_reads_residual<EPI1>()) ev = ev1[s % EVD][nt];
-                const v4i packed = epilogue_fast16<NT, EPI1>(s1, acc1, nt, sc.wq, sc.cal, sc.ecal, ev, 16);
-                if (cur.o1[nt] >= 0) *reinterpret_cast<v4i*>((int8_t*)s1.out + cur.o1[nt] + s * 4 * s1.out_pf) = packed;
+                if constexpr (chain_reads_residual<EPI1>()) ev = ev1[s][nt];
+                const v4i packed = epilogue_fast16<NT, EPI1>(e1, acc1, nt, sc.wq, sc.cal, sc.ecal, ev, 16);
+                if (cur.o1[nt] >= 0) *reinterpret_cast<v4i*>((int8_t*)s1.out + s * 4 * s1.out_pf + (uint32_t)cur.o1[nt]) = packed;
                 bf1[nt] = packed ^ xm2;
             }
             if constexpr (chain_reads_residual<EPI1>()) {
-                if constexpr (SP1 > EVD) {
-                    if (s + EVD < SP1) {
 #pragma unroll
-                        for (int nt = 0; nt < NT; ++nt) ev1[s % EVD][nt] = residual(s1, cur.e1[nt], s + EVD);
-                    }
-                }
+                for (int nt = 0; nt < NT; ++nt) ev1[s][nt] = residual(s1, nxt.e1[nt], s);
             }
+            if constexpr (NT == 1) step_fence();
             if constexpr (SP2 > 0) {
 #pragma unroll
                 for (int sp = 0; sp < SP2; ++sp) {
@@ -372,7 +385,7 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
                     v4i ev = {0, 0, 0, 0};
                     if constexpr (chain_reads_residual<EPI2>()) ev = residual(s2, cur.e2[nt], sp);
                     const v4i packed = epilogue_fast16<NT, EPI2>(s2, acc_sp, nt, sc.wq, sc.cal, sc.ecal, ev, 16);
-                    *reinterpret_cast<v4i*>((int8_t*)s2.out + cur.o2[nt] + sp * 4 * s2.out_pf) = packed;
+                    *reinterpret_cast<v4i*>((int8_t*)s2.out + sp * 4 * s2.out_pf + (uint32_t)cur.o2[nt]) = packed;
                 }
             }
         }
@@ -380,16 +393,16 @@ __global__ void __launch_bounds__(256) conv_chain_kernel(ChainArgs a)
     }
 }
 
-template <int NT, int D, int SP0, int SP1, int SP2, int EPI0, int EPI1, int EPI2>
+template <int NT, int D, int SP0, int SP1, int SP2, int EPI0, int EPI1, int EPI2, bool U8>
 void launch_chain_instance(hipStream_t s, const ChainArgs& a, int grid, int lds)
 {
     // more than 64 KiB of dynamic LDS has to be allowed per kernel, once
     static std::once_flag allowed;
     std::call_once(allowed, [] {
-        CHIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_chain_kernel<NT, D, SP0, SP1, SP2, EPI0, EPI1, EPI2>),
+        CHIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_chain_kernel<NT, D, SP0, SP1, SP2, EPI0, EPI1, EPI2, U8>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     });
-    hipLaunchKernelGGL((conv_chain_kernel<NT, D, SP0, SP1, SP2, EPI0, EPI1, EPI2>), dim3(grid), dim3(256), lds, s, a);
+    hipLaunchKernelGGL((conv_chain_kernel<NT, D, SP0, SP1, SP2, EPI0, EPI1, EPI2, U8>), dim3(grid), dim3(64 * chain_waves(NT)), lds, s, a);
 }
 
 }  // namespace chip

@@ -13,7 +13,7 @@
 // a granule costs three barriers and its instructions.  Kernel time, 56x56, 64 mid features, batch 1: 10.7 -> 6.2 us with three
 // stages, 28x28 with two 9.5 -> 4.0.  Inside a network, where the input comes from memory, two stages are faster at every
 // size (ResNet-50 at batch 32 12.7 -> 10.8, at batch 128 33.1 -> 29.0; repeated on warm caches 24.8 and 25.5); three stages
-// with many granules are not, splitting costs more instructions per pixel: 13.1 -> 11.7 us at 1016 granules, 26 against 43 us at batch 32.
+// with many granules are not, splitting costs more instructions per pixel: 10.2 -> 9.4 us at 980 granules, 11.6 -> 14.1 at 1568.
 // (The ninth tap's weights in the registers of one wave were four more fragments for every wave: with three stages 128 registers were not
 // enough, and a request waited for one that was spilled behind it.)
 // 128 mid features (weights in 160 registers) gained 2 us of 12 at batch 1 and lost 8 of 28 at batch 32.

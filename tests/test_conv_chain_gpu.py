@@ -464,3 +464,40 @@ def test_two_stage_chain_behind_a_wide_1x1(eng, ifm, fused):
     assert np.array_equal(hip.download(eng, out[0]), ref[0])
     for b in out + [xin, ebuf]:
         b.close()
+
+
+@pytest.mark.parametrize("B,H,W", [(5, 57, 59), (3, 150, 149)], ids=["waves_without_work", "one_granule_or_two"])
+@pytest.mark.parametrize("eltw_dt", [np.int8, np.uint8, None], ids=["sum_s8", "sum_u8", "plain"])
+def test_three_stage_chain_of_one_granule_per_wave(eng, B, H, W, eltw_dt):
+    """1051 granules over 1088 waves, 4191 over 4096; the last granule of 16 pixels is not full.  Integers: the same bits."""
+    r = np.random.default_rng(23)
+    x = r.integers(0, 256, (B, 64, H, W)).astype(np.uint8)
+    xin = hip.upload(eng, x, "fs_b_yx_fsv16", (1, 1))
+    l = [layer(r, 64, 64, 3, np.uint8), layer(r, 64, 256, 1, np.int8), layer(r, 256, 64, 1, np.int8)]
+    kw = dict(bias_dt=hip.I32, has_wqf=True, has_calib=True)
+    between = [hip.Tensor.make(hip.S8, hip.FS_B_YX_FSV16, B, f, H, W) for f in (64, 256)]
+    tail, more, ecal, ebuf = dict(act="relu"), dict(act="relu"), None, None
+    if eltw_dt is not None:
+        lo = 0 if eltw_dt == np.uint8 else -128
+        e, ecal = r.integers(lo, lo + 256, (B, 256, H, W)).astype(eltw_dt), r.uniform(0.25, 1.0, 256).astype(np.float32)
+        ebuf = hip.upload(eng, e, "fs_b_yx_fsv16")
+        tail = dict(act="none", eltw_t=ebuf.tensor, eltw_act="relu", has_eltw_calib=True)
+        more = dict(act="none", eltw=e, eltw_act="relu", eltw_calib=ecal)
+    d = [hip.conv_desc(xin.tensor, l[0][0].shape, "s8", pad=(1, 1), act="relu", **kw),
+         hip.conv_desc(between[0], l[1][0].shape, "s8", out_pad=(1, 1), **kw, **tail),
+         hip.conv_desc(between[1], l[2][0].shape, "s8", act="relu", **kw)]
+    ref = [rc.conv(x, l[0][0], l[0][1], wqf=l[0][2], calib=l[0][3], pad=(1, 1), out_dt="s8", act="relu")]
+    ref.append(rc.conv(ref[0], l[1][0], l[1][1], wqf=l[1][2], calib=l[1][3], out_dt="s8", **more))
+    ref.append(rc.conv(ref[1], l[2][0], l[2][1], wqf=l[2][2], calib=l[2][3], out_dt="s8", act="relu"))
+    out = [None] + [hip.Buffer(eng, q.output) for q in d[1:]]
+    ch = hip.ConvChain(eng, [(d[0], *l[0], None), (d[1], *l[1], ecal), (d[2], *l[2], None)], [False, True, True])
+    assert b"3 stages,p16,d3" in ch.info().kernel_name
+    ch.enqueue(xin, out, [None, ebuf, None])
+    eng.finish()
+    for k in (1, 2):
+        bad = np.argwhere(hip.download(eng, out[k]) != ref[k])
+        assert bad.size == 0, "stage %d: %d differ, first at %s" % (k, len(bad), bad[0])
+    assert len(np.unique(ref[2])) > 8
+    ch.close(), xin.close(), out[1].close(), out[2].close()
+    if ebuf is not None:
+        ebuf.close()
