@@ -59,6 +59,23 @@ __device__ __forceinline__ void static_for(F&& f)
 
 typedef const __attribute__((address_space(1))) void* halo_gptr;
 typedef __attribute__((address_space(3))) void* halo_lptr;
+// Pointers into global memory that say so.  One that has been through an asm statement is otherwise a pointer into any address
+// space: its loads are flat ones, which may come out of LDS and so count as LDS reads too, in no order: every wait for an LDS
+// read then waits for the weights that have just been requested.  (In conv_point_kernel.h and conv_plane_kernel.h, where pointers were
+// of that kind: 1024 -> 256 at 14x14, batch 128, 12.8 -> 12.5 us, 2048 -> 512 + 2048 25.0 -> 24.5; 3x3 at 28x28, batch 32, 8.4 -> 8.1.)
+template <class T>
+using global = __attribute__((address_space(1))) T;
+typedef const global<int8_t>* global_bytes;
+template <class T>
+__device__ __forceinline__ const global<T>* in_global(const T* p)
+{
+    return (const global<T>*)p;
+}
+template <class T>
+__device__ __forceinline__ global<T>* in_global(T* p)
+{
+    return (global<T>*)p;
+}
 
 typedef int v16i __attribute__((ext_vector_type(16)));
 

@@ -35,6 +35,8 @@
 namespace chip {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 // q = n / d for 0 <= n < 2^31 by multiply-high and shift.  The numerator is doubled, so that the multiplier of d == 1 fits too and
 // there is no case apart (which was a branch, or two selects, in front of the first request).

@@ -126,12 +126,12 @@ __global__ void __launch_bounds__(256, 2) conv_plane_kernel(PlaneArgs a)
     asm volatile("" ::"s"(a.in), "s"(a.wpk), "s"(a.in_off), "s"(a.in_pb), "s"(a.in_pf), "s"(a.in_py), "s"(a.total), "s"(a.units), "s"(a.strips), "s"(a.cols), "s"(a.shift),
                  "s"(a.pitch), "s"(a.positions), "s"(a.jobs), "s"(a.xor_mask), "s"(a.acc_init), "s"(a.calib), "s"(a.OH), "s"(a.OW), "s"(a.div_patch.mul), "s"(a.div_pitch.mul));
     // (values of their own, or the compiler fetches the arguments again where they are used)
-    const int32_t* first = a.acc_init;
-    const float* factors = a.calib;
-    const int8_t* in = a.in + a.in_off;
+    const global<int32_t>* first = in_global(a.acc_init);
+    const global<float>* factors = in_global(a.calib);
+    global_bytes in = in_global(a.in + a.in_off);
     int in_pf = a.in_pf, row_bytes = a.pitch * 16;
-    int8_t* out = a.out;
-    int32_t* raw = a.raw;
+    global<int8_t>* out = in_global(a.out);
+    global<int32_t>* raw = in_global(a.raw);
     int out_off = a.out_off, out_pb = a.out_pb, out_pf = a.out_pf, out_py = a.out_py, kind = a.kind, OFM = a.OFM, OH = a.OH, units = a.units;
     float hi = a.hi, lo = a.lo;
     asm volatile("" : "+s"(first), "+s"(factors), "+s"(in), "+s"(in_pf), "+s"(row_bytes), "+s"(out), "+s"(raw), "+s"(out_off), "+s"(out_pb), "+s"(out_pf), "+s"(out_py),
@@ -151,7 +151,7 @@ __global__ void __launch_bounds__(256, 2) conv_plane_kernel(PlaneArgs a)
 #pragma unroll
     for (int i = 0; i < NL; ++i) src[i] = tile.source(a, (uint32_t)(min(i * 64, a.positions - 64) + lane));  // the last load ends where the patch does
     const int buffer_units = 2 * a.positions, wave_units = wave * BUFFERS * buffer_units;  // of 16 bytes
-    const int8_t* weights = (const int8_t*)(a.wpk + (size_t)(ftile * 4 + (uint32_t)wave) * a.jobs * 9 * 64);
+    global_bytes weights = (global_bytes)(a.wpk + (size_t)(ftile * 4 + (uint32_t)wave) * a.jobs * 9 * 64);
     asm volatile("" : "+s"(weights));
     const uint32_t lane_bytes = (uint32_t)lane * 16u;
     v4i w[BUFFERS][9];
@@ -161,10 +161,10 @@ __global__ void __launch_bounds__(256, 2) conv_plane_kernel(PlaneArgs a)
         constexpr int P = decltype(buffer)::value, R = decltype(rc)::value;
         if constexpr (R < 2 * NL) {
             constexpr int S = R / NL, I = R % NL;
-            const int8_t* base = in + (int64_t)((wave * a.jobs + j) * 2 + S) * in_pf;
+            global_bytes base = in + (int64_t)((wave * a.jobs + j) * 2 + S) * in_pf;
             __builtin_amdgcn_global_load_lds((halo_gptr)(base + src[I]), (halo_lptr)(lds + wave_units + P * buffer_units + S * a.positions + min(I * 64, a.positions - 64)), 16, 0, 0);
         } else if constexpr (R < REQUESTS) {
-            w[P][R - 2 * NL] = *reinterpret_cast<const v4i*>(weights + (uint32_t)(j * 9 + R - 2 * NL) * 1024u + lane_bytes);
+            w[P][R - 2 * NL] = *(const global<v4i>*)(weights + (uint32_t)(j * 9 + R - 2 * NL) * 1024u + lane_bytes);
         }
     };
     using B0 = std::integral_constant<int, 0>;
@@ -222,8 +222,8 @@ __global__ void __launch_bounds__(256, 2) conv_plane_kernel(PlaneArgs a)
             if constexpr (LAST && R == Read::count / 2) {  // for the end
 #pragma unroll
                 for (int d = 0; d < N / 4; ++d) {
-                    init[d] = *reinterpret_cast<const v4i*>(first + fl + d * 4);
-                    const float4 c = *reinterpret_cast<const float4*>(factors + fl + d * 4);
+                    init[d] = *(const global<v4i>*)(first + fl + d * 4);
+                    const v4f c = *(const global<v4f>*)(factors + fl + d * 4);
                     cal[d * 4] = c.x, cal[d * 4 + 1] = c.y, cal[d * 4 + 2] = c.z, cal[d * 4 + 3] = c.w;
                 }
             }
@@ -282,7 +282,7 @@ __global__ void __launch_bounds__(256, 2) conv_plane_kernel(PlaneArgs a)
             const v4i q = epilogue_fast16<1, EPI_KIND_RELU, 8>(e, best, 0, wq, cal, cal, none, OFM - fl);
             const int y = yl + 2 * k;
             if (mine && y < OH && !(lane & 1))
-                *reinterpret_cast<int2*>(out + ((uint32_t)(out_off + b * out_pb + slice * out_pf + (x >> 1) * 16 + d0 * 4) + __umul24(y >> 1, out_py))) = make_int2(q[0], q[1]);
+                *(global<v2i>*)(out + ((uint32_t)(out_off + b * out_pb + slice * out_pf + (x >> 1) * 16 + d0 * 4) + __umul24(y >> 1, out_py))) = v2i{q[0], q[1]};
         } else {
             if (r0 + wave >= NP) continue;
             v4i sum[4][1], others[4][3];
@@ -317,7 +317,7 @@ __global__ void __launch_bounds__(256, 2) conv_plane_kernel(PlaneArgs a)
                 keep_branch();
                 q = epilogue_fast16<1, EPI_KIND_LINEAR>(e, sum, 0, wq, cal, cal, none, OFM - f0);
             }
-            if (ok) *reinterpret_cast<v4i*>(out + ((uint32_t)(out_off + b * out_pb + slice * out_pf + x * 16) + __umul24(y, out_py))) = q;
+            if (ok) *(global<v4i>*)(out + ((uint32_t)(out_off + b * out_pb + slice * out_pf + x * 16) + __umul24(y, out_py))) = q;
         }
     }
 }
@@ -345,12 +345,12 @@ __global__ void __launch_bounds__(256, 2) conv_plane_wide_kernel(PlaneArgs a)
     asm volatile("" ::"s"(a.in), "s"(a.wpk), "s"(a.in_off), "s"(a.in_pb), "s"(a.in_pf), "s"(a.in_py), "s"(a.total), "s"(a.units), "s"(a.strips), "s"(a.cols), "s"(a.shift),
                  "s"(a.pitch), "s"(a.positions), "s"(a.jobs), "s"(a.spans), "s"(a.xor_mask), "s"(a.acc_init), "s"(a.calib), "s"(a.OH), "s"(a.OW), "s"(a.div_patch.mul),
                  "s"(a.div_pitch.mul));
-    const int32_t* first = a.acc_init;
-    const float* factors = a.calib;
-    const int8_t* in = a.in + a.in_off;
+    const global<int32_t>* first = in_global(a.acc_init);
+    const global<float>* factors = in_global(a.calib);
+    global_bytes in = in_global(a.in + a.in_off);
     int in_pf = a.in_pf, row_bytes = a.pitch * 16;
-    int8_t* out = a.out;
-    int32_t* raw = a.raw;
+    global<int8_t>* out = in_global(a.out);
+    global<int32_t>* raw = in_global(a.raw);
     int out_off = a.out_off, out_pb = a.out_pb, out_pf = a.out_pf, out_py = a.out_py, kind = a.kind, OFM = a.OFM, OH = a.OH, units = a.units;
     float hi = a.hi, lo = a.lo;
     asm volatile("" : "+s"(first), "+s"(factors), "+s"(in), "+s"(in_pf), "+s"(row_bytes), "+s"(out), "+s"(raw), "+s"(out_off), "+s"(out_pb), "+s"(out_pf), "+s"(out_py),
@@ -373,7 +373,7 @@ __global__ void __launch_bounds__(256, 2) conv_plane_wide_kernel(PlaneArgs a)
         src[i] = tile.source(a, (uint32_t)(q + lane)) + (uint32_t)(s * in_pf), dst[i] = pair_units + s * a.positions + q;
     }
     const int span = (int)ftile * SPANS + member;  // (spans past the last one: its weights, nothing is stored)
-    const int8_t* weights = (const int8_t*)(a.wpk + (size_t)min(span, a.spans - 1) * a.jobs * 9 * 64);
+    global_bytes weights = (global_bytes)(a.wpk + (size_t)min(span, a.spans - 1) * a.jobs * 9 * 64);
     asm volatile("" : "+s"(weights));
     const uint32_t lane_bytes = (uint32_t)lane * 16u;
     v4i w[2][9];
@@ -382,7 +382,7 @@ __global__ void __launch_bounds__(256, 2) conv_plane_wide_kernel(PlaneArgs a)
         if constexpr (R < LOADS)
             __builtin_amdgcn_global_load_lds((halo_gptr)(in + (int64_t)(2 * j) * in_pf + src[R]), (halo_lptr)(lds + buffer + dst[R]), 16, 0, 0);
         else if constexpr (R < REQUESTS)
-            w[P][R - LOADS] = *reinterpret_cast<const v4i*>(weights + (uint32_t)(j * 9 + R - LOADS) * 1024u + lane_bytes);
+            w[P][R - LOADS] = *(const global<v4i>*)(weights + (uint32_t)(j * 9 + R - LOADS) * 1024u + lane_bytes);
     };
     using B0 = std::integral_constant<int, 0>;
     using B1 = std::integral_constant<int, 1>;
@@ -437,8 +437,8 @@ __global__ void __launch_bounds__(256, 2) conv_plane_wide_kernel(PlaneArgs a)
             if constexpr (LAST && R == Read::count / 2) {
 #pragma unroll
                 for (int d = 0; d < N / 4; ++d) {
-                    init[d] = *reinterpret_cast<const v4i*>(first + fl + d * 4);
-                    const float4 c = *reinterpret_cast<const float4*>(factors + fl + d * 4);
+                    init[d] = *(const global<v4i>*)(first + fl + d * 4);
+                    const v4f c = *(const global<v4f>*)(factors + fl + d * 4);
                     cal[d * 4] = c.x, cal[d * 4 + 1] = c.y, cal[d * 4 + 2] = c.z, cal[d * 4 + 3] = c.w;
                 }
             }
@@ -486,7 +486,7 @@ __global__ void __launch_bounds__(256, 2) conv_plane_wide_kernel(PlaneArgs a)
                 }
             best[0][0] += init[0], best[1][0] += init[1];
             const v4i q = epilogue_fast16<1, EPI_KIND_RELU, 8>(e, best, 0, wq, cal, cal, none, OFM - f0 - (lane & 1) * 8);
-            if (mine && yl + 2 * k < OH) *reinterpret_cast<int2*>(out + at) = make_int2(q[0], q[1]);
+            if (mine && yl + 2 * k < OH) *(global<v2i>*)(out + at) = v2i{q[0], q[1]};
             at += (uint32_t)out_py;
         }
     } else {
@@ -512,14 +512,14 @@ __global__ void __launch_bounds__(256, 2) conv_plane_wide_kernel(PlaneArgs a)
             keep_branch();
             each([&](int i, const v4i (&sum)[4][1]) {
                 const v4i q = epilogue_fast16<1, EPI_KIND_RELU>(e, sum, 0, wq, cal, cal, none, OFM - f0);
-                if (mine && yl + i < OH) *reinterpret_cast<v4i*>(out + at) = q;
+                if (mine && yl + i < OH) *(global<v4i>*)(out + at) = q;
                 at += (uint32_t)out_py;
             });
         } else {
             keep_branch();
             each([&](int i, const v4i (&sum)[4][1]) {
                 const v4i q = epilogue_fast16<1, EPI_KIND_LINEAR>(e, sum, 0, wq, cal, cal, none, OFM - f0);
-                if (mine && yl + i < OH) *reinterpret_cast<v4i*>(out + at) = q;
+                if (mine && yl + i < OH) *(global<v4i>*)(out + at) = q;
                 at += (uint32_t)out_py;
             });
         }

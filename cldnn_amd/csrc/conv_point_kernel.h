@@ -55,8 +55,8 @@ __global__ void __launch_bounds__(256, 2) conv_point_kernel(PointArgs a)
     asm volatile("" ::"s"(a.in), "s"(a.wpk), "s"(a.acc_init), "s"(a.calib), "s"(a.in_off), "s"(a.in_pb), "s"(a.in_pf), "s"(a.in_row), "s"(a.in_col), "s"(a.M), "s"(a.OHW), "s"(a.OW),
                  "s"(a.total), "s"(a.ftiles), "s"(a.spans), "s"(a.jobs), "s"(a.xor_mask), "s"(a.div_ohw.mul), "s"(a.div_ow.mul), "s"(a.div_ftiles.mul));
     // (values of their own, or the compiler fetches the arguments again where they are used)
-    const int8_t *in = a.in + a.in_off, *eltw = a.eltw;
-    int8_t* out = a.out;
+    global_bytes in = in_global(a.in + a.in_off), eltw = in_global(a.eltw);
+    global<int8_t>* out = in_global(a.out);
     int in_pf = a.in_pf, out_off = a.out_off, out_pb = a.out_pb, out_pf = a.out_pf, out_py = a.out_py, OFM = a.OFM;
     int el_off = a.el_off, el_pb = a.el_pb, el_pf = a.el_pf, el_row = a.el_row, el_col = a.el_col;
     asm volatile("" : "+s"(in), "+s"(eltw), "+s"(out), "+s"(in_pf), "+s"(out_off), "+s"(out_pb), "+s"(out_pf), "+s"(out_py), "+s"(OFM), "+s"(el_off), "+s"(el_pb), "+s"(el_pf),
@@ -90,10 +90,10 @@ __global__ void __launch_bounds__(256, 2) conv_point_kernel(PointArgs a)
         src = b * (uint32_t)a.in_pb + oy * (uint32_t)a.in_row + ox * (uint32_t)a.in_col;
     }
     const int span0 = (int)ftile * 8 + wave * 2;
-    const int8_t* weights[2];
+    global_bytes weights[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-        weights[s] = (const int8_t*)(a.wpk + (size_t)min(span0 + s, a.spans - 1) * a.jobs * 4 * 64);  // past the last span: not stored
+        weights[s] = (global_bytes)(a.wpk + (size_t)min(span0 + s, a.spans - 1) * a.jobs * 4 * 64);  // past the last span: not stored
         asm volatile("" : "+s"(weights[s]));
     }
     const uint32_t lane_bytes = (uint32_t)lane * 16u;
@@ -104,7 +104,7 @@ __global__ void __launch_bounds__(256, 2) conv_point_kernel(PointArgs a)
             __builtin_amdgcn_global_load_lds((halo_gptr)(in + (int64_t)(j * 8 + wave * 2 + R) * in_pf + src), (halo_lptr)(lds + buffer + (wave * 2 + R) * SLICE), 16, 0, 0);
         } else if constexpr (R < REQUESTS) {
             constexpr int T = R - LOADS;
-            w[P][T] = *reinterpret_cast<const v4i*>(weights[T / 4] + (uint32_t)(j * 4 + T % 4) * 1024u + lane_bytes);
+            w[P][T] = *(const global<v4i>*)(weights[T / 4] + (uint32_t)(j * 4 + T % 4) * 1024u + lane_bytes);
         }
     };
     using B0 = std::integral_constant<int, 0>;
@@ -159,7 +159,7 @@ __global__ void __launch_bounds__(256, 2) conv_point_kernel(PointArgs a)
 #pragma unroll
                     for (int s = 0; s < 2; ++s) {
                         const int slice = min((span0 + s) * 2 + half, (OFM - 1) >> 4);
-                        if (!a.raw) residual[s][R] = *reinterpret_cast<const v4i*>(eltw + (eb + (uint32_t)slice * (uint32_t)el_pf));
+                        if (!a.raw) residual[s][R] = *(const global<v4i>*)(eltw + (eb + (uint32_t)slice * (uint32_t)el_pf));
                     }
                 }
             }
@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(256, 2) conv_point_kernel(PointArgs a)
                 continue;
             }
             const v4i q = epilogue_fast16<1, EPI>(a, sum, 0, wq, cal, ecal, residual[s][i], OFM - f0);
-            if (ok) *reinterpret_cast<v4i*>(out + (ob[i] + (uint32_t)slice * (uint32_t)out_pf)) = q;
+            if (ok) *(global<v4i>*)(out + (ob[i] + (uint32_t)slice * (uint32_t)out_pf)) = q;
         }
     }
 }
