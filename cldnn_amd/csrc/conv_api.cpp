@@ -524,6 +524,14 @@ cldnn_hip_status cldnn_hip_conv_enqueue(cldnn_hip_conv c, const void* input_dev,
     return guarded([&] { run(c, input_dev, output_dev, eltw_dev, nullptr); });
 }
 
+cldnn_hip_status cldnn_hip_conv_enqueue_buffers(cldnn_hip_conv c, cldnn_hip_buffer input, cldnn_hip_buffer output, cldnn_hip_buffer eltw)
+{
+    const void* in = cldnn_hip_buffer_device_ptr(input);
+    void* out = cldnn_hip_buffer_device_ptr(output);
+    const void* added = eltw ? cldnn_hip_buffer_device_ptr(eltw) : nullptr;
+    return cldnn_hip_conv_enqueue(c, in, out, added);
+}
+
 cldnn_hip_status cldnn_hip_conv_enqueue_static_scratch(cldnn_hip_conv c, const void* input_dev, void* output_dev,
                                                        const void* eltw_dev)
 {

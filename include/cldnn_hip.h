@@ -365,6 +365,9 @@ cldnn_hip_status cldnn_hip_conv_release(cldnn_hip_conv c);
 /* asynchronous on the engine stream; device pointers */
 cldnn_hip_status cldnn_hip_conv_enqueue(cldnn_hip_conv c, const void* input_dev, void* output_dev,
                                         const void* eltw_dev);
+/* The same for whole buffers: cldnn_hip_conv_enqueue of their cldnn_hip_buffer_device_ptr, in one call (for callers to whom
+ * a call across a language boundary costs a fifth of a microsecond).  eltw: NULL without a second input. */
+cldnn_hip_status cldnn_hip_conv_enqueue_buffers(cldnn_hip_conv c, cldnn_hip_buffer input, cldnn_hip_buffer output, cldnn_hip_buffer eltw);
 /* cldnn_hip_conv_enqueue for callers that must not allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  Same arguments and
  * results as cldnn_hip_conv_enqueue; the one kernel family with a scratch buffer -- the small-batch kernel, which

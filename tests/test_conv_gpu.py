@@ -1201,3 +1201,28 @@ def test_first_layer_finishes_the_3x3_pooling_behind_it(eng, case, in_dt):
         assert np.count_nonzero(np.frombuffer(dst.read_raw(), np.int8)) == np.count_nonzero(ref)
         for b in (c, src, dst):
             b.close()
+
+
+@pytest.mark.parametrize("fused", [False, True], ids=["plain", "fused"])
+def test_enqueue_of_whole_buffers_equals_enqueue_of_addresses(eng, fused):
+    """integers: the same bits; a missing buffer is refused with the same status by both"""
+    r = np.random.default_rng(71)
+    x, w, bias, wqf, calib = problem(71, 2, 48, 9, 7, 40, 1, 1, np.int8)
+    src = hip.upload(eng, x, "fs_b_yx_fsv16")
+    e = hip.upload(eng, r.integers(-128, 128, (2, 40, 9, 7)).astype(np.int8), "fs_b_yx_fsv16") if fused else None
+    more = dict(act="none", eltw_t=e.tensor, eltw_act="relu", has_eltw_calib=True) if fused else dict(act="relu")
+    d = hip.conv_desc(src.tensor, w.shape, "s8", bias_dt=hip.I32, has_wqf=True, has_calib=True, **more)
+    conv = hip.Conv(eng, d, w, bias, wqf, calib, r.uniform(0.5, 1, 40).astype(np.float32) if fused else None)
+    out = [hip.Buffer(eng, d.output) for _ in range(2)]
+    conv.enqueue(src, out[0], e)
+    assert hip.lib().cldnn_hip_conv_enqueue(conv.h, src.ptr, out[1].ptr, e.ptr if fused else None) == 0
+    eng.finish()
+    a, b = (hip.download(eng, o) for o in out)
+    assert np.array_equal(a, b) and len(np.unique(a)) > 8
+    refused = hip.lib().cldnn_hip_conv_enqueue(conv.h, None, out[1].ptr, e.ptr if fused else None)
+    assert refused != 0 and hip.lib().cldnn_hip_conv_enqueue_buffers(conv.h, None, out[1].h, e.h if fused else None) == refused
+    if fused:
+        refused = hip.lib().cldnn_hip_conv_enqueue(conv.h, src.ptr, out[1].ptr, None)
+        assert refused != 0 and hip.lib().cldnn_hip_conv_enqueue_buffers(conv.h, src.h, out[1].h, None) == refused
+    for o in out + [src, conv] + ([e] if fused else []):
+        o.close()
