@@ -20,6 +20,9 @@
 // 18.6 -> 17.1; 512 at 7x7, batch 32 10.5 -> 6.4; 512 at 14x14, batch 16 13.1 -> 9.2; 512 at 28x28, batch 16 33.6 -> 29.8.  At batch 32
 // of the first, 12200 clocks: 2100 until all requests are out, 600 until they have arrived, 5200 in the loop (126 matrix
 // instructions: 4030), 4200 in the two meetings of partial sums.
+// Since then the arguments come behind one wait (three: the size of the grid and a divisor came in turns of their own) and the first
+// job's weights are requested before the addresses of its patch are computed: 256 at 14x14, batch 32, 7.7 -> 7.2 us inside ResNet-50;
+// 512 at 28x28, batch 1, 5.2 -> 4.7; the wide form, 256 at 14x14, batch 128, 15.6 -> 15.0.
 //
 // LDS reads are issued by hand and waited for by count (conv_halo_kernel.h).  A fetch through the scalar unit between them
 // only makes a wait longer.
@@ -124,7 +127,7 @@ __global__ void __launch_bounds__(256, 2) conv_plane_kernel(PlaneArgs a)
     const int l32 = lane & 31;
     // everything the loop needs, behind one wait
     asm volatile("" ::"s"(a.in), "s"(a.wpk), "s"(a.in_off), "s"(a.in_pb), "s"(a.in_pf), "s"(a.in_py), "s"(a.total), "s"(a.units), "s"(a.strips), "s"(a.cols), "s"(a.shift),
-                 "s"(a.pitch), "s"(a.positions), "s"(a.jobs), "s"(a.xor_mask), "s"(a.acc_init), "s"(a.calib), "s"(a.OH), "s"(a.OW), "s"(a.div_patch.mul), "s"(a.div_pitch.mul));
+                 "s"(a.pitch), "s"(a.positions), "s"(a.jobs), "s"(a.xor_mask), "s"(a.acc_init), "s"(a.calib), "s"(a.OH), "s"(a.OW), "s"(a.div_patch.mul), "s"(a.div_pitch.mul), "s"(a.ftiles), "s"(a.div_ftiles.mul), "s"(a.div_ftiles.shift), "s"(gridDim.x));
     // (values of their own, or the compiler fetches the arguments again where they are used)
     const global<int32_t>* first = in_global(a.acc_init);
     const global<float>* factors = in_global(a.calib);
@@ -146,16 +149,13 @@ __global__ void __launch_bounds__(256, 2) conv_plane_kernel(PlaneArgs a)
     extern __shared__ __align__(16) unsigned char smem[];
     v4i* lds = reinterpret_cast<v4i*>(smem);
 
-    // ---------------- the wave's patch of job j into LDS
-    uint32_t src[NL];
-#pragma unroll
-    for (int i = 0; i < NL; ++i) src[i] = tile.source(a, (uint32_t)(min(i * 64, a.positions - 64) + lane));  // the last load ends where the patch does
     const int buffer_units = 2 * a.positions, wave_units = wave * BUFFERS * buffer_units;  // of 16 bytes
     global_bytes weights = (global_bytes)(a.wpk + (size_t)(ftile * 4 + (uint32_t)wave) * a.jobs * 9 * 64);
     asm volatile("" : "+s"(weights));
     const uint32_t lane_bytes = (uint32_t)lane * 16u;
+    uint32_t src[NL];
     v4i w[BUFFERS][9];
-    // request R of a job: its patch, then its weights
+    // request R of a job: the wave's patch, into LDS, then its weights
     constexpr int REQUESTS = 2 * NL + 9;
     auto request = [&](int j, auto buffer, auto rc) {
         constexpr int P = decltype(buffer)::value, R = decltype(rc)::value;
@@ -169,7 +169,15 @@ __global__ void __launch_bounds__(256, 2) conv_plane_kernel(PlaneArgs a)
     };
     using B0 = std::integral_constant<int, 0>;
     using B1 = std::integral_constant<int, BUFFERS - 1>;
-    static_for<0, REQUESTS>([&](auto rc) {
+    // of the first job the weights go out first (in front of the patch, so its arrival is everybody's): the addresses of the patch
+    // take a hundred and fifty instructions
+    static_for<2 * NL, REQUESTS>([&](auto rc) {
+        request(0, B0{}, rc);
+        step_fence();
+    });
+#pragma unroll
+    for (int i = 0; i < NL; ++i) src[i] = tile.source(a, (uint32_t)(min(i * 64, a.positions - 64) + lane));  // the last load ends where the patch does
+    static_for<0, 2 * NL>([&](auto rc) {
         request(0, B0{}, rc);
         step_fence();
     });
@@ -230,7 +238,7 @@ __global__ void __launch_bounds__(256, 2) conv_plane_kernel(PlaneArgs a)
             step_fence();
         });
     };
-    patch_arrived();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     static_for<0, RG - 1>([&](auto ic) { read(B0{}, ic); });
     if constexpr (JOBS == 0)
         for (int j = 0; j + 2 < a.jobs; j += 2) {
@@ -344,7 +352,7 @@ __global__ void __launch_bounds__(256, 2) conv_plane_wide_kernel(PlaneArgs a)
     const int member = wave % SPANS, pair = wave / SPANS;  // of the waves of a tile; which tile
     asm volatile("" ::"s"(a.in), "s"(a.wpk), "s"(a.in_off), "s"(a.in_pb), "s"(a.in_pf), "s"(a.in_py), "s"(a.total), "s"(a.units), "s"(a.strips), "s"(a.cols), "s"(a.shift),
                  "s"(a.pitch), "s"(a.positions), "s"(a.jobs), "s"(a.spans), "s"(a.xor_mask), "s"(a.acc_init), "s"(a.calib), "s"(a.OH), "s"(a.OW), "s"(a.div_patch.mul),
-                 "s"(a.div_pitch.mul));
+                 "s"(a.div_pitch.mul), "s"(a.ftiles), "s"(a.div_ftiles.mul), "s"(a.div_ftiles.shift), "s"(gridDim.x));
     const global<int32_t>* first = in_global(a.acc_init);
     const global<float>* factors = in_global(a.calib);
     global_bytes in = in_global(a.in + a.in_off);
@@ -363,19 +371,12 @@ __global__ void __launch_bounds__(256, 2) conv_plane_wide_kernel(PlaneArgs a)
 
     extern __shared__ __align__(16) unsigned char smem[];
     v4i* lds = reinterpret_cast<v4i*>(smem);
-    const int buffer_units = 2 * a.positions, pair_units = pair * 3 * buffer_units;
-    // the wave's loads of a patch; those that are left over repeat the last one
-    uint32_t src[LOADS];
-    int dst[LOADS];
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-        const int c = min(i * SPANS + member, 2 * NL - 1), s = c >= NL ? 1 : 0, q = min((c - s * NL) * 64, a.positions - 64);
-        src[i] = tile.source(a, (uint32_t)(q + lane)) + (uint32_t)(s * in_pf), dst[i] = pair_units + s * a.positions + q;
-    }
     const int span = (int)ftile * SPANS + member;  // (spans past the last one: its weights, nothing is stored)
     global_bytes weights = (global_bytes)(a.wpk + (size_t)min(span, a.spans - 1) * a.jobs * 9 * 64);
     asm volatile("" : "+s"(weights));
     const uint32_t lane_bytes = (uint32_t)lane * 16u;
+    uint32_t src[LOADS];
+    int dst[LOADS];
     v4i w[2][9];
     auto request = [&](int j, int buffer, auto pc, auto rc) {
         constexpr int P = decltype(pc)::value, R = decltype(rc)::value;
@@ -386,7 +387,18 @@ __global__ void __launch_bounds__(256, 2) conv_plane_wide_kernel(PlaneArgs a)
     };
     using B0 = std::integral_constant<int, 0>;
     using B1 = std::integral_constant<int, 1>;
-    static_for<0, REQUESTS>([&](auto rc) {
+    static_for<LOADS, REQUESTS>([&](auto rc) {
+        request(0, 0, B0{}, rc);
+        step_fence();
+    });
+    const int buffer_units = 2 * a.positions, pair_units = pair * 3 * buffer_units;
+    // the wave's loads of a patch; those that are left over repeat the last one
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int c = min(i * SPANS + member, 2 * NL - 1), s = c >= NL ? 1 : 0, q = min((c - s * NL) * 64, a.positions - 64);
+        src[i] = tile.source(a, (uint32_t)(q + lane)) + (uint32_t)(s * in_pf), dst[i] = pair_units + s * a.positions + q;
+    }
+    static_for<0, LOADS>([&](auto rc) {
         request(0, 0, B0{}, rc);
         step_fence();
     });
@@ -446,7 +458,7 @@ __global__ void __launch_bounds__(256, 2) conv_plane_wide_kernel(PlaneArgs a)
         });
         buffer = next;
     };
-    patch_arrived();
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     static_for<0, RG - 1>([&](auto ic) { read(0, ic); });
     for (int j = 0; j + 2 < a.jobs; j += 2) {
         job(j, B0{}, std::false_type{});

@@ -53,7 +53,8 @@ __global__ void __launch_bounds__(256, 2) conv_point_kernel(PointArgs a)
     const int half = lane >> 5;
     const int l32 = lane & 31;
     asm volatile("" ::"s"(a.in), "s"(a.wpk), "s"(a.acc_init), "s"(a.calib), "s"(a.in_off), "s"(a.in_pb), "s"(a.in_pf), "s"(a.in_row), "s"(a.in_col), "s"(a.M), "s"(a.OHW), "s"(a.OW),
-                 "s"(a.total), "s"(a.ftiles), "s"(a.spans), "s"(a.jobs), "s"(a.xor_mask), "s"(a.div_ohw.mul), "s"(a.div_ow.mul), "s"(a.div_ftiles.mul));
+                 "s"(a.total), "s"(a.ftiles), "s"(a.spans), "s"(a.jobs), "s"(a.xor_mask), "s"(a.div_ohw.mul), "s"(a.div_ow.mul), "s"(a.div_ftiles.mul), "s"(a.div_ftiles.shift),
+                 "s"(gridDim.x));
     // (values of their own, or the compiler fetches the arguments again where they are used)
     global_bytes in = in_global(a.in + a.in_off), eltw = in_global(a.eltw);
     global<int8_t>* out = in_global(a.out);
