@@ -1399,22 +1399,37 @@ __global__ void __launch_bounds__(256) conv_stream_kernel(MfmaArgs a)
     const bool live = f0 < a.OFM;
     const int valid = a.OFM - f0;
 
+    // ---- requests: the weights first, whose addresses are there; the activations' take a while to compute
+    v4i fb[KS][NT], ev[NT], fa[KS][4], init[4];
+    const v4i* wsrc = a.wpk + (size_t)span * KS * 256 + kq * 64 + l16;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) fa[ks][mt] = wsrc[ks * 256 + mt * 16];
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) init[mt] = *reinterpret_cast<const v4i*>(a.acc_init + f0 + mt * 4);
+    step_fence();
+
     // tap offsets of this lane's K-chunks, computed instead of looked up (a table load would put a second
     // memory round trip in front of the activation loads)
     int koff[KS];
+    if (a.kchunks == a.CB) {  // one tap: no divisions (their lanes' branches were half of the way to the first request)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        const uint32_t kc = ks * 4 + kq;
-        const uint32_t tap = a.div_cb.div(kc);
-        const uint32_t cb = kc - tap * a.CB;
-        const uint32_t fy = a.div_fx.div(tap);
-        const uint32_t fx = tap - fy * a.FX;
-        koff[ks] = kc < (uint32_t)a.kchunks ? (int)(cb * a.in_pf + fy * a.tap_dy + fx * a.tap_dx) : 0;
+        for (int ks = 0; ks < KS; ++ks) koff[ks] = ks * 4 + kq < a.kchunks ? (ks * 4 + kq) * a.in_pf : 0;
+    } else {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const uint32_t kc = ks * 4 + kq;
+            const uint32_t tap = a.div_cb.div(kc);
+            const uint32_t cb = kc - tap * a.CB;
+            const uint32_t fy = a.div_fx.div(tap);
+            const uint32_t fx = tap - fy * a.FX;
+            koff[ks] = kc < (uint32_t)a.kchunks ? (int)(cb * a.in_pf + fy * a.tap_dy + fx * a.tap_dx) : 0;
+        }
     }
 
-    // ---- requests
     const int origin = a.in_off + span_origin(a, span);
-    v4i fb[KS][NT], ev[NT], fa[KS][4], init[4];
+    const int es = min(fs, (a.OFM - 1) >> 4);  // (a span's slices past the last one are not finished)
     int ob[NT], eb[NT];
     PixelPos pos[NT];
 #pragma unroll
@@ -1425,14 +1440,14 @@ __global__ void __launch_bounds__(256) conv_stream_kernel(MfmaArgs a)
         if (a.linear) {  // dense tensors, 1x1 / stride 1: pixel m sits at m * 16, no division needed
             pix = origin + (int)mm * 16;
             o = a.out_off + fs * a.out_pf + (int)mm * 16;
-            e = a.el_off + fs * a.el_pf + (int)mm * 16;
+            e = a.el_off + es * a.el_pf + (int)mm * 16;
             pos[nt] = PixelPos{0, 0, 0};
         } else {
             const PixelPos pp = pixel_pos(a, mm);
             pos[nt] = pp;
             pix = origin + (int)pp.b * a.in_pb + ((int)pp.oy * a.sy - a.py) * a.in_py + ((int)pp.ox * a.sx - a.px) * a.px_bytes;
             o = a.out_off + (int)pp.b * a.out_pb + fs * a.out_pf + (int)pp.oy * a.out_py + (int)pp.ox * 16;
-            e = a.el_off + (int)pp.b * a.el_pb + fs * a.el_pf + (int)(pp.oy * a.esy) * a.el_py + (int)(pp.ox * a.esx) * 16;
+            e = a.el_off + (int)pp.b * a.el_pb + es * a.el_pf + (int)(pp.oy * a.esy) * a.el_py + (int)(pp.ox * a.esx) * 16;
         }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) fb[ks][nt] = *reinterpret_cast<const v4i*>(a.in + (pix + koff[ks]));
@@ -1440,18 +1455,11 @@ __global__ void __launch_bounds__(256) conv_stream_kernel(MfmaArgs a)
         eb[nt] = e;
         ev[nt] = v4i{0, 0, 0, 0};
         if constexpr (EPI == EPI_KIND_FUSED) {
-            if (live) ev[nt] = *reinterpret_cast<const v4i*>((const int8_t*)a.eltw + e);
+            ev[nt] = *reinterpret_cast<const v4i*>((const int8_t*)a.eltw + e);
         } else if constexpr (EPI == EPI_KIND_FAST) {
-            if (a.fe.fused && live) ev[nt] = *reinterpret_cast<const v4i*>((const int8_t*)a.eltw + e);
+            if (a.fe.fused) ev[nt] = *reinterpret_cast<const v4i*>((const int8_t*)a.eltw + e);
         }
     }
-    const v4i* wsrc = a.wpk + (size_t)span * KS * 256 + kq * 64 + l16;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt) fa[ks][mt] = wsrc[ks * 256 + mt * 16];
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) init[mt] = *reinterpret_cast<const v4i*>(a.acc_init + f0 + mt * 4);
     LaneScales sc;
     if (live) load_scales<EPI>(a, f0, sc);
 
