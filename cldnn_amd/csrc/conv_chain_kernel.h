@@ -22,7 +22,7 @@
 // time (NT == 1) in 128 registers: eight waves to a workgroup, four to a SIMD, where 32 pixels at a time leave two.  The weights are
 // read from LDS twice as often for it, a third of what LDS delivers.  64 -> 64 -> 256 + sum -> 64 at 56x56, batch 128: 77.9 us with
 // 32 pixels, 73.2 with 16, 68.4 with the residual ahead as well (32 pixels and the residual ahead: 70.5); batch 32: 25.6, 24.1, 22.9
-// (24.6).
+// (24.6), and 22.1 with the first granule's requests out while the weights are on their way to LDS.
 // Every stage has its own epilogue kind, per-feature vectors, output tensor and (optional) residual tensor.
 #pragma once
 #include <mutex>
@@ -145,20 +145,28 @@ __global__ void __launch_bounds__(64 * chain_waves(NT), NT == 1 ? 4 : 1) conv_ch
     extern __shared__ __align__(16) unsigned char smem[];
     v4i* ldsW = reinterpret_cast<v4i*>(smem);                              // [units][4][64]
     int32_t* ldsV = reinterpret_cast<int32_t*>(smem + (size_t)a.units * 4096);  // per-feature vectors
-    {
-        // one bulk copy: the image holds the weight units and, behind them, the per-feature vectors of all stages
-        // (absent vectors filled with their neutral values by the host); all requests of a thread are in flight at once
-        const int total = a.units * 256 + a.vec_quads;
-        constexpr int THREADS = 64 * chain_waves(NT), BATCH = 5120 / THREADS;  // 80 KB at a time
-        for (int i = t; i < total; i += BATCH * THREADS) {
-            v4i r[BATCH];
+    // one bulk copy: the image holds the weight units and, behind them, the per-feature vectors of all stages
+    // (absent vectors filled with their neutral values by the host); all requests of a thread are in flight at once, and wait in
+    // registers until the first granule's have gone out too
+    constexpr int THREADS = 64 * chain_waves(NT), BATCH = 5120 / THREADS;  // 80 KB at a time
+    const int total = a.units * 256 + a.vec_quads;
+    v4i copy[BATCH];
+    auto request_image = [&](int i) {
 #pragma unroll
-            for (int u = 0; u < BATCH; ++u) r[u] = a.wpk[min(i + u * THREADS, total - 1)];
+        for (int u = 0; u < BATCH; ++u) copy[u] = a.wpk[min(i + u * THREADS, total - 1)];
+    };
+    auto store_image = [&](int i) {
 #pragma unroll
-            for (int u = 0; u < BATCH; ++u)
-                if (i + u * THREADS < total) ldsW[i + u * THREADS] = r[u];
-        }
+        for (int u = 0; u < BATCH; ++u)
+            if (i + u * THREADS < total) ldsW[i + u * THREADS] = copy[u];
+    };
+    int copied = t;
+    for (; copied + BATCH * THREADS < total; copied += BATCH * THREADS) {
+        request_image(copied);
+        store_image(copied);
     }
+    request_image(copied);
+    step_fence();
 
     // Every die gets one contiguous run of workgroups, every wave one contiguous range of granules: rows that
     // share filter taps stay inside one die's L2.  (A shared counter that hands out granules one by one was tried:
@@ -216,6 +224,7 @@ __global__ void __launch_bounds__(64 * chain_waves(NT), NT == 1 ? 4 : 1) conv_ch
     };
 
     if (g_begin >= g1) {
+        store_image(copied);
         __syncthreads();
         return;
     }
@@ -237,6 +246,8 @@ __global__ void __launch_bounds__(64 * chain_waves(NT), NT == 1 ? 4 : 1) conv_ch
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) ev1[s][nt] = residual(s1, cur.e1[nt], s);
     }
+    step_fence();
+    store_image(copied);
     __syncthreads();  // weights and vectors are in LDS; no barrier after this point
 
     for (int g = g_begin; g < g1; ++g) {

@@ -66,17 +66,25 @@ __global__ void __launch_bounds__(256, EPI0 == EPI_KIND_FAST ? 2 : (P1 == 1 ? 4 
     extern __shared__ __align__(16) unsigned char smem[];
     v4i* lds = reinterpret_cast<v4i*>(smem);
     const int32_t* V = reinterpret_cast<const int32_t*>(lds + a.vec);
-    {
-        constexpr int BATCH = 8;
-        for (int i = t; i < a.quads; i += BATCH * 256) {
-            v4i r[BATCH];
+    // the image's way into LDS; the last pieces wait in registers until the first granule's requests have gone out
+    constexpr int BATCH = 8;
+    v4i copy[BATCH];
+    auto request_image = [&](int i) {
 #pragma unroll
-            for (int u = 0; u < BATCH; ++u) r[u] = a.img[min(i + u * 256, a.quads - 1)];
+        for (int u = 0; u < BATCH; ++u) copy[u] = a.img[min(i + u * 256, a.quads - 1)];
+    };
+    auto store_image = [&](int i) {
 #pragma unroll
-            for (int u = 0; u < BATCH; ++u)
-                if (i + u * 256 < a.quads) lds[i + u * 256] = r[u];
-        }
+        for (int u = 0; u < BATCH; ++u)
+            if (i + u * 256 < a.quads) lds[i + u * 256] = copy[u];
+    };
+    int copied = t;
+    for (; copied + BATCH * 256 < a.quads; copied += BATCH * 256) {
+        request_image(copied);
+        store_image(copied);
     }
+    request_image(copied);
+    step_fence();
 
     const int per_xcd = gridDim.x >> 3;  // the grid is a multiple of 8
     const uint32_t vb = (blockIdx.x & 7u) * (uint32_t)per_xcd + (blockIdx.x >> 3);
@@ -84,6 +92,7 @@ __global__ void __launch_bounds__(256, EPI0 == EPI_KIND_FAST ? 2 : (P1 == 1 ? 4 
     const int g_begin = (int)(gw * (uint32_t)a.gpw + a.div_waves.div(gw * (uint32_t)a.grem));
     const int g_end = (int)((gw + 1) * (uint32_t)a.gpw + a.div_waves.div((gw + 1) * (uint32_t)a.grem));
     if (g_begin >= g_end) {
+        store_image(copied);
         __syncthreads();
         return;
     }
@@ -175,6 +184,8 @@ __global__ void __launch_bounds__(256, EPI0 == EPI_KIND_FAST ? 2 : (P1 == 1 ? 4 
 #pragma unroll
         for (int s = 0; s < S; ++s) load_step(cur, so, s);
     }
+    step_fence();
+    store_image(copied);
     __syncthreads();  // weights and vectors are in LDS; no barrier after this point
 
     for (int g = g_begin; g < g_end; ++g) {
