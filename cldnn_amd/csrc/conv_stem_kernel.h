@@ -64,6 +64,11 @@ __global__ void __launch_bounds__(256, POOL && F * KS > 8 ? 3 : 4) conv_stem_ker
     extern __shared__ __align__(16) unsigned char smem[];
     uint32_t* tile = reinterpret_cast<uint32_t*>(smem);
 
+    // what the weights and the image rows need, behind one wait (three otherwise; 3x3 with 32 features, batch 32, 10.4 -> 10.0 us, batch 1
+    // 8.4 -> 8.0; the 7x7 one at batch 5, from host memory, 19.5 -> 19.0)
+    asm volatile("" ::"s"(a.in), "s"(a.wpk), "s"(a.in_off), "s"(a.in_pb), "s"(a.in_pf), "s"(a.in_py), "s"(a.IFM), "s"(a.IH), "s"(a.IW), "s"(a.sy), "s"(a.sx), "s"(a.py), "s"(a.px),
+                 "s"(a.row_groups), "s"(a.col_groups), "s"(a.total), "s"(a.div_rows.mul), "s"(a.div_rows.shift), "s"(a.div_cols.mul), "s"(a.div_cols.shift), "s"(a.wg_rows),
+                 "s"(a.wg_cols), "s"(a.lds_rows), "s"(a.pitch), "s"(a.xor_mask), "s"(gridDim.x));
     // neighbouring row groups on one die: they share image rows (the grid is a multiple of 8)
     const uint32_t wg = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (wg >= (uint32_t)a.total) return;
