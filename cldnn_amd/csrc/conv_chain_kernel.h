@@ -17,8 +17,9 @@
 // requests of a wave return in order, so one that goes to memory at the start of a granule also holds up every activation
 // requested behind it.
 //
-// What bounds it: nothing alone.  Without the requantisation the chain of three stages below takes 63 us instead of 73, without its
-// stores 64, with a residual that lies in L1 60; the waves wait for memory a third of the time.  So three stages go 16 pixels at a
+// What bounds it: memory first (batch 128: 2.0 x the bytes of a copy's best case, 4.1 to 4.8 TB/s), the vector ALU second.  Without the
+// requantisation the chain of three stages below takes 63 us instead of 71, without its stores 64, with a residual that lies in L1 60;
+// the waves wait for memory a third of the time.  So three stages go 16 pixels at a
 // time (NT == 1) in 128 registers: eight waves to a workgroup, four to a SIMD, where 32 pixels at a time leave two.  The weights are
 // read from LDS twice as often for it, a third of what LDS delivers.  64 -> 64 -> 256 + sum -> 64 at 56x56, batch 128: 77.9 us with
 // 32 pixels, 73.2 with 16, 68.4 with the residual ahead as well (32 pixels and the residual ahead: 70.5); batch 32: 25.6, 24.1, 22.9
