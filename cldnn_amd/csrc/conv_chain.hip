@@ -503,8 +503,8 @@ void launch_conv_chain(hipStream_t s, const ChainStageIn* st, const ChainPlan& p
     a.units = pl.units;
     a.vec_quads = (pl.lds_bytes - pl.units * 4096) / 16;
     a.granules = pl.granules;
-    a.gpw = pl.granules / (pl.grid * pl.waves), a.grem = pl.granules % (pl.grid * pl.waves);
-    a.div_waves = make_fast_div((uint32_t)pl.grid * (uint32_t)pl.waves);
+    a.gpw = pl.granules / pl.grid, a.grem = pl.granules % pl.grid;
+    a.div_wgs = make_fast_div((uint32_t)pl.grid);
     a.M = (uint32_t)pl.m_total;
     a.OHW = p0.OH * p0.OW, a.OW = p0.OW;
     a.div_ohw = make_fast_div((uint32_t)a.OHW), a.div_ow = make_fast_div((uint32_t)a.OW);

@@ -10,16 +10,16 @@
 // is never written (unless somebody else reads it) and never read back.
 //
 // Work split: persistent workgroups of INDEPENDENT waves.  All weights of all stages (a few tens of KB) and
-// the per-feature vectors are copied into LDS once per workgroup; after that a wave walks over its own range of
-// 16*NT-pixel granules without any barrier.  Feature counts are multiples of 64.  Stage 0 reads its activations straight from global memory, D K-steps
+// the per-feature vectors are copied into LDS once per workgroup; after that a wave walks over every fourth or eighth granule
+// (16*NT pixels) of its workgroup's range without any barrier.  Feature counts are multiples of 64.  Stage 0 reads its activations straight from global memory, D K-steps
 // ahead of their use, and the look-ahead runs across granule boundaries (as in the weights-stationary kernel).
 // The residual of stage 1 is asked for a whole granule ahead, each span's as soon as the previous granule has used its registers:
 // requests of a wave return in order, so one that goes to memory at the start of a granule also holds up every activation
 // requested behind it.
 //
-// What bounds it: memory first (batch 128: 2.0 x the bytes of a copy's best case, 4.1 to 4.8 TB/s), the vector ALU second.  Without the
-// requantisation the chain of three stages below takes 63 us instead of 71, without its stores 64, with a residual that lies in L1 60;
-// the waves wait for memory a third of the time.  So three stages go 16 pixels at a
+// What bounds it: memory (4.1 to 4.8 TB/s), then the vector ALU.  With more bytes to fetch than now (see the order of granules) the
+// chain of three stages below took 71 us, without the requantisation 63, without its stores 64, with a residual that lies in L1 60;
+// the waves waited for memory a third of the time.  So three stages go 16 pixels at a
 // time (NT == 1) in 128 registers: eight waves to a workgroup, four to a SIMD, where 32 pixels at a time leave two.  The weights are
 // read from LDS twice as often for it, a third of what LDS delivers.  64 -> 64 -> 256 + sum -> 64 at 56x56, batch 128: 77.9 us with
 // 32 pixels, 73.2 with 16, 68.4 with the residual ahead as well (32 pixels and the residual ahead: 70.5); batch 32: 25.6, 24.1, 22.9
@@ -55,8 +55,8 @@ struct ChainArgs {
     int32_t units;
     int32_t vec_quads;         // 16-byte pieces of per-feature vectors behind the units
     int32_t granules;          // ceil(M / (16 * NT))
-    int32_t gpw, grem;         // granules / waves of the grid and the remainder
-    FastDiv div_waves;         // wave w starts at granule w * gpw + (w * grem) / waves = floor(w * granules / waves)
+    int32_t gpw, grem;         // granules / workgroups and the remainder
+    FastDiv div_wgs;           // workgroup w starts at granule w * gpw + (w * grem) / workgroups = floor(w * granules / workgroups)
     uint32_t M;
     int32_t OHW, OW;
     FastDiv div_ohw, div_ow;
@@ -169,16 +169,19 @@ __global__ void __launch_bounds__(64 * chain_waves(NT), NT == 1 ? 4 : 1) conv_ch
     request_image(copied);
     step_fence();
 
-    // Every die gets one contiguous run of workgroups, every wave one contiguous range of granules: rows that
-    // share filter taps stay inside one die's L2.  (A shared counter that hands out granules one by one was tried:
+    // Every die gets one contiguous run of workgroups, every workgroup one contiguous range of granules, which its waves take in
+    // turn: rows that share filter taps are read at about the same time, by the waves of one workgroup, and come from memory once.
+    // (With a range of its own to every wave a row was read three times, 40 us apart: 226 and 176 MiB fetched of 123 at batch 128, now 141
+    // and 132; 81.4 -> 72.6 and 68.6 -> 64.9 us, batch 32 24.3 -> 23.2 and 23.2 -> 22.3.)
+    // (A shared counter that hands out granules one by one was tried:
     // device-scope atomics on a handful of addresses take about 0.2 us each, one after the other, which cost four
     // times what the better balance saved.)
+    constexpr int WAVES = chain_waves(NT);
     const int per_xcd = gridDim.x >> 3;  // the grid is a multiple of 8
     const uint32_t vb = (blockIdx.x & 7u) * (uint32_t)per_xcd + (blockIdx.x >> 3);
     // (a 64-bit division of two run-time values here costs every wave a few hundred instructions before its first request)
-    const uint32_t gw = vb * (uint32_t)chain_waves(NT) + (uint32_t)wave;
-    const int g_begin = (int)(gw * (uint32_t)a.gpw + a.div_waves.div(gw * (uint32_t)a.grem));
-    const int g1 = (int)((gw + 1) * (uint32_t)a.gpw + a.div_waves.div((gw + 1) * (uint32_t)a.grem));
+    const int g_begin = (int)(vb * (uint32_t)a.gpw + a.div_wgs.div(vb * (uint32_t)a.grem)) + wave;
+    const int g1 = (int)((vb + 1) * (uint32_t)a.gpw + a.div_wgs.div((vb + 1) * (uint32_t)a.grem));
 
     const v4i xm0 = {(int)s0.xor_mask, (int)s0.xor_mask, (int)s0.xor_mask, (int)s0.xor_mask};
     const v4i xm1 = {(int)s1.xor_mask, (int)s1.xor_mask, (int)s1.xor_mask, (int)s1.xor_mask};
@@ -251,8 +254,8 @@ __global__ void __launch_bounds__(64 * chain_waves(NT), NT == 1 ? 4 : 1) conv_ch
     store_image(copied);
     __syncthreads();  // weights and vectors are in LDS; no barrier after this point
 
-    for (int g = g_begin; g < g1; ++g) {
-        setup(g + 1, nxt);
+    for (int g = g_begin; g < g1; g += WAVES) {
+        setup(g + WAVES, nxt);
         // ---------------- stage 0: the spatial convolution, all SP0 spans at once
         v4i acc0[SP0 * 4][NT];
 #pragma unroll
