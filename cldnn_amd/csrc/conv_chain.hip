@@ -359,8 +359,8 @@ static void launch_dwchain(hipStream_t s, const ChainStageIn* st, const ChainPla
     a.U0 = pl.u32[0], a.KS = (a.U0 + 1) / 2, a.U2 = pl.stages > 2 ? pl.u32[2] : 0;
     a.w1 = a.U0 * 64, a.w2 = a.w1 + a.KS * pl.u32[1] * 128, a.vec = a.w2 + a.U2 * 128;
     a.n0 = pl.sp[0] * 64, a.n1 = pl.sp[1] * 64, a.n2 = pl.stages > 2 ? pl.sp[2] * 64 : 0;
-    a.gpw = pl.granules / (pl.grid * 4), a.grem = pl.granules % (pl.grid * 4);
-    a.div_waves = make_fast_div((uint32_t)pl.grid * 4u);
+    a.gpw = pl.granules / pl.grid, a.grem = pl.granules % pl.grid;
+    a.div_wgs = make_fast_div((uint32_t)pl.grid);
     a.M = (uint32_t)pl.m_total;
     a.OHW = p0.OH * p0.OW, a.OW = p0.OW;
     a.div_ohw = make_fast_div((uint32_t)a.OHW), a.div_ow = make_fast_div((uint32_t)a.OW);

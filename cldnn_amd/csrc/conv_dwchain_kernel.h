@@ -21,7 +21,9 @@
 // activations of the next unit (also across granules) requested while the present one is multiplied, all weights and
 // per-feature vectors in LDS.
 // MobileNet v2 at batch 32, kernel time before (spans of 64, one tap per product) and now: 112x112 32-16-96 47.1 -> 30.0 us,
-// 112x112 96-24-144 25.1 -> 18.1, 56x56 144-24-144 31.4 -> 22.1, 28x28 192-32-192 13.0 -> 9.8.
+// 112x112 96-24-144 25.1 -> 18.1, 56x56 144-24-144 31.4 -> 22.1, 28x28 192-32-192 13.0 -> 9.8; with the first granule's requests out
+// while the image is on its way to LDS 27.3, 16.9, 19.7 and 9.1.  The waves of a workgroup take its granules in turn, so that rows that
+// share filter taps are read at about the same time: nothing at batch 32, at batch 100 48.8 -> 44.5, 47.7 -> 45.4, 22.0 -> 20.4 us.
 #pragma once
 #include <type_traits>
 
@@ -36,8 +38,8 @@ struct DwChainArgs {
     const v4i* img;            // LDS image: depthwise weights [U0][64], fragments of stage 1 [KS][P1][2], of stage 2 [U2][2], vectors
     int32_t quads;             // its 16-byte pieces
     int32_t w1, w2, vec;       // where the fragments and the vectors start, in pieces
-    int32_t gpw, grem;         // granules / waves of the grid and the remainder
-    FastDiv div_waves;         // wave w starts at granule w * gpw + (w * grem) / waves = floor(w * granules / waves)
+    int32_t gpw, grem;         // granules / workgroups and the remainder
+    FastDiv div_wgs;           // workgroup w starts at granule w * gpw + (w * grem) / workgroups = floor(w * granules / workgroups)
     uint32_t M;
     int32_t OHW, OW;
     FastDiv div_ohw, div_ow;
@@ -88,9 +90,9 @@ __global__ void __launch_bounds__(256, EPI0 == EPI_KIND_FAST ? 2 : (P1 == 1 ? 4 
 
     const int per_xcd = gridDim.x >> 3;  // the grid is a multiple of 8
     const uint32_t vb = (blockIdx.x & 7u) * (uint32_t)per_xcd + (blockIdx.x >> 3);
-    const uint32_t gw = vb * 4u + (uint32_t)wave;
-    const int g_begin = (int)(gw * (uint32_t)a.gpw + a.div_waves.div(gw * (uint32_t)a.grem));
-    const int g_end = (int)((gw + 1) * (uint32_t)a.gpw + a.div_waves.div((gw + 1) * (uint32_t)a.grem));
+    // the workgroup's range, which its waves take in turn: rows that share filter taps are read at about the same time
+    const int g_begin = (int)(vb * (uint32_t)a.gpw + a.div_wgs.div(vb * (uint32_t)a.grem)) + wave;
+    const int g_end = (int)((vb + 1) * (uint32_t)a.gpw + a.div_wgs.div((vb + 1) * (uint32_t)a.grem));
     if (g_begin >= g_end) {
         store_image(copied);
         __syncthreads();
@@ -188,8 +190,8 @@ __global__ void __launch_bounds__(256, EPI0 == EPI_KIND_FAST ? 2 : (P1 == 1 ? 4 
     store_image(copied);
     __syncthreads();  // weights and vectors are in LDS; no barrier after this point
 
-    for (int g = g_begin; g < g_end; ++g) {
-        setup(g + 1, nxt);
+    for (int g = g_begin; g < g_end; g += 4) {
+        setup(g + 4, nxt);
         // residual of the projection (a fused sum): requested now, used after the whole depthwise stage
         int2 ev1[P1];
         v4i acc1[P1][2];
