@@ -65,11 +65,16 @@ struct KsplitArgs {
     Epilogue epi;
 };
 
-// look-ahead in K-steps: what 128 registers hold (16 waves of a workgroup = four per SIMD)
-template <int FT, int PT, int ADDR>
+// look-ahead in K-steps: what 128 registers hold (16 waves of a workgroup = four per SIMD).  32 x 64 tiles have eight waves, and above
+// 128 registers a CU holds one workgroup instead of two: with lanes' addresses, or two rows of a pooling window, three steps take 130 to
+// 135, two take 104 to 112.  256 -> 256, 3x3 at 14x14 without a border, three steps and two: batch 8 (224 workgroups) 5.34 and 5.26 us,
+// batch 16 9.05 and 7.12, batch 64 30.3 and 22.3; with its pooling, batch 8 4.60 and 4.48, batch 64 21.4 and 17.5.  The run-time form of
+// the epilogue keeps three: batch 1 6.03 and 6.60, batch 8 6.28 and 6.87.
+template <int FT, int PT, int ADDR, int EPI>
 constexpr int ksplit_depth()
 {
-    return FT * PT == 1 ? 8 : (FT * PT == 2 ? 6 : (FT * PT == 8 || ADDR == ADDR_LANES ? 3 : 4));
+    constexpr bool TWO = FT * PT == 8 && (EPI == EPI_KIND_POOL || (ADDR == ADDR_LANES && EPI != EPI_KIND_FAST));
+    return FT * PT == 1 ? 8 : (FT * PT == 2 ? 6 : (TWO ? 2 : FT * PT == 8 || ADDR == ADDR_LANES ? 3 : 4));
 }
 
 // Everything on the way to the stores, behind one wait.  (Fetched where it is first used it was two waits in front of the first
@@ -89,7 +94,7 @@ template <int FT, int PT, int ADDR, int EPI>
 __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(KsplitArgs a)
 {
     fetch_arguments(a);
-    constexpr int D = ksplit_depth<FT, PT, ADDR>();
+    constexpr int D = ksplit_depth<FT, PT, ADDR, EPI>();
     constexpr int SUB = 4 / FT;  // feature tiles per span of 64
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

@@ -1,0 +1,49 @@
+"""Kernels that rely on several waves a SIMD stay within the registers that allow them.
+
+From the metadata of the library's own gfx950 code objects; no GPU."""
+import functools
+import re
+import subprocess
+
+import pytest
+
+from test_mfma_wait_states import code_objects
+
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+GENERIC, RELU, FUSED, LINEAR, CLAMPQ, F32, POOL = 0, 2, 3, 4, 5, 7, 8  # EPI_KIND_*
+LANES = 1  # ADDR_LANES
+
+
+@functools.lru_cache(None)
+def resources(directory):
+    """mangled name -> (vector registers, bytes of scratch a lane)"""
+    found = {}
+    for i, image in enumerate(code_objects()):
+        path = directory / ("%d.elf" % i)
+        path.write_bytes(image)
+        notes = subprocess.run([READELF, "--notes", str(path)], stdout=subprocess.PIPE, check=True, text=True).stdout
+        for kernel in notes.split("  - .agpr_count:")[1:]:
+            value = {k: re.search(r"\.%s:\s+(\S+)" % k, kernel).group(1) for k in ("symbol", "vgpr_count", "private_segment_fixed_size")}
+            found[value["symbol"]] = int(value["vgpr_count"]), int(value["private_segment_fixed_size"])
+    return found
+
+
+def instances(name, *parameters):
+    """fragment of a mangled name: a template's integer (Li) and boolean (Lb) arguments"""
+    return name + "I" + "".join("L%c%dE" % ("b" if isinstance(p, bool) else "i", p) for p in parameters) + "E"
+
+
+CASES = (
+    # workgroups of 512 threads, two waves a SIMD: two of them share a CU
+    [("conv_ksplit_kernel", (4, 2, LANES, epi), 4) for epi in (GENERIC, RELU, FUSED, LINEAR, F32, POOL)]
+    + [("conv_ksplit_kernel", (4, 2, 0, epi), 4) for epi in (RELU, FUSED, LINEAR, F32, POOL)]
+)
+
+
+@pytest.mark.parametrize("name,parameters,waves", CASES, ids=lambda v: "_".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_registers_leave_the_waves_that_the_kernel_relies_on(tmp_path_factory, name, parameters, waves):
+    table = resources(tmp_path_factory.getbasetemp())
+    found = [v for k, v in table.items() if instances(name, *parameters) in k]
+    assert len(found) == 1, "%d kernels" % len(found)
+    registers, scratch = found[0]
+    assert 512 // (-(-registers // 8) * 8) >= waves and scratch == 0, "%d registers, %d bytes of scratch" % (registers, scratch)
