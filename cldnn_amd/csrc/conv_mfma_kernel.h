@@ -1414,16 +1414,25 @@ __global__ void __launch_bounds__(256) conv_stream_kernel(MfmaArgs a)
     const bool live = f0 < a.OFM;
     const int valid = a.OFM - f0;
 
-    // ---- requests: the weights first, whose addresses are there; the activations' take a while to compute
+    // ---- requests: the weights first, whose addresses are there; the activations' take a while to compute.  With the run-time
+    // epilogue, where that would take a third to half of the waves a SIMD has (256 -> 128 at 56x56, batch 64, 16 pixels to a wave: 84.0 us
+    // with the weights first, 68.7 behind; 128 -> 128, 32 pixels, 95.7 and 78.8), they come behind the activations: the compiler then
+    // walks the K-steps with few fragments at a time.
+    constexpr bool WEIGHTS_FIRST = EPI != EPI_KIND_GENERIC || KS == 1 || (KS == 2 && NT == 1);
     v4i fb[KS][NT], ev[NT], fa[KS][4], init[4];
-    const v4i* wsrc = a.wpk + (size_t)span * KS * 256 + kq * 64 + l16;
+    auto request_weights = [&] {
+        const v4i* wsrc = a.wpk + (size_t)span * KS * 256 + kq * 64 + l16;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
+        for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) fa[ks][mt] = wsrc[ks * 256 + mt * 16];
+            for (int mt = 0; mt < 4; ++mt) fa[ks][mt] = wsrc[ks * 256 + mt * 16];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) init[mt] = *reinterpret_cast<const v4i*>(a.acc_init + f0 + mt * 4);
-    step_fence();
+        for (int mt = 0; mt < 4; ++mt) init[mt] = *reinterpret_cast<const v4i*>(a.acc_init + f0 + mt * 4);
+    };
+    if constexpr (WEIGHTS_FIRST) {
+        request_weights();
+        step_fence();
+    }
 
     // tap offsets of this lane's K-chunks, computed instead of looked up (a table load would put a second
     // memory round trip in front of the activation loads)
@@ -1475,6 +1484,7 @@ __global__ void __launch_bounds__(256) conv_stream_kernel(MfmaArgs a)
             if (a.fe.fused) ev[nt] = *reinterpret_cast<const v4i*>((const int8_t*)a.eltw + e);
         }
     }
+    if constexpr (!WEIGHTS_FIRST) request_weights();
     LaneScales sc;
     if (live) load_scales<EPI>(a, f0, sc);
 

@@ -37,6 +37,8 @@ CASES = (
     # workgroups of 512 threads, two waves a SIMD: two of them share a CU
     [("conv_ksplit_kernel", (4, 2, LANES, epi), 4) for epi in (GENERIC, RELU, FUSED, LINEAR, F32, POOL)]
     + [("conv_ksplit_kernel", (4, 2, 0, epi), 4) for epi in (RELU, FUSED, LINEAR, F32, POOL)]
+    # a wave pays one trip to memory, which other waves cover
+    + [("conv_stream_kernel", p + (GENERIC,), waves) for p, waves in (((1, 2), 7), ((1, 4), 6), ((1, 8), 6), ((2, 2), 5), ((2, 4), 4), ((2, 8), 4))]
 )
 
 
