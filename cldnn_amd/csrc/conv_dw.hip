@@ -188,8 +188,10 @@ __global__ void __launch_bounds__(256) conv_dw3x3_kernel(DwArgs a)
 // against 25 and 400.  At that rate memory is the bound of large planes; a wave keeps its table in registers for `rounds`
 // sets of 64 pixels and requests the next set before it finishes the present one.  Small planes are bound by the launch and
 // the latency of one set: the prologue has no branch, or the compiler fetches the arguments in four turns, each behind the one before,
-// and the weights are asked for behind two of them, before the addresses of the activations are known (32 x 576 x 14x14, 3x3, queued
-// one behind the other: 5.02 -> 4.43 us a layer; 7 x 67 x 93x93, 5x5 at stride 2, 6.74 -> 5.98; 10 x 488 x 59x59 13.0 -> 12.3).
+// and the weights are asked for behind two of them, before the addresses of the activations are known (recorded, one behind the
+// other, with a branch in front of the requests and now: 32 x 576 x 14x14, 3x3, 5.0 and 4.8 us a layer, batch 1 2.74 and 2.49; 7 x 67 x
+// 93x93, 5x5 at stride 2, 7.1 and 6.4; 10 x 488 x 59x59, 5x5, 18.1 and 17.9).  A workgroup too many leaves behind its requests.  Without
+// that end the 5x5 forms were a wave a SIMD short: 64 x 256 x 56x56 49.3 us, 46.8 with it, 128 x 96 x 112x112 135.8 and 130.7.
 // Kernel time, 32 x 576 x 14x14, 3x3: 6.3 -> 5.3 us (1.4 us at the rate of a large copy and about 3 of launch); 8 x 512 x 28x28,
 // 5x5: 32.4 -> 6.5; 32 x 64 x 112x112, 5x5: 143 -> 26 (10.3 at the rate of a large copy), 3x3: 22.7 -> 18.4.
 template <int FY, int NB, int EPI>
@@ -198,7 +200,7 @@ __global__ void __launch_bounds__(256, 2) conv_dw_rows_kernel(DwArgs a)
     constexpr int S = FY * NB;
     // neighbouring chunks of a plane on one XCD (the grid is a multiple of 8): the rows they share are in its L2
     const uint32_t turn = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-    const bool spare = turn >= a.works;  // (no branch, or what is behind it would be fetched behind it)
+    const bool spare = turn >= a.works;  // (leaves behind its requests: what is behind a branch would be fetched behind it)
     const uint32_t work = spare ? 0u : turn;
     const uint32_t fs = a.div_chunks.div(work), chunk = work - fs * a.chunks;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, f0 = (int)fs * 16;
@@ -235,13 +237,15 @@ __global__ void __launch_bounds__(256, 2) conv_dw_rows_kernel(DwArgs a)
             for (int n = 0; n < NB; ++n)  // (positions past the row belong to pixels that do not exist, or to no tap)
                 x[j * NB + n] = *reinterpret_cast<const v4i*>(a.in + min(src + (uint32_t)j * tap_py + (uint32_t)n * 64u, a.in_last));
         const uint32_t ox = ox0 + (uint32_t)q;
-        ok = real && !spare && ox < (uint32_t)a.OW;
+        ok = real && ox < (uint32_t)a.OW;
         opos = b * (uint32_t)a.out_p.pb + oy * (uint32_t)a.out_p.py + ox * 16u;
         if constexpr (EPI == EPI_KIND_FAST)
             if (a.fe.fused && ok)
                 ev4 = *reinterpret_cast<const v4i*>(el + (b * (uint32_t)a.eltw_p.pb + oy * (uint32_t)(a.esy * (int)a.eltw_p.py) + ox * (uint32_t)(a.esx * 16)));
     };
     request(0);
+    step_fence();
+    if (spare) return;  // (with an end on the way the compiler keeps 16 registers less)
     int r = 0;
     do {
         v4i acc[4][1];
