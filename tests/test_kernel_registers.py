@@ -39,6 +39,8 @@ CASES = (
     + [("conv_ksplit_kernel", (4, 2, 0, epi), 4) for epi in (RELU, FUSED, LINEAR, F32, POOL)]
     # a wave pays one trip to memory, which other waves cover
     + [("conv_stream_kernel", p + (GENERIC,), waves) for p, waves in (((1, 2), 7), ((1, 4), 6), ((1, 8), 6), ((2, 2), 5), ((2, 4), 4), ((2, 8), 4))]
+    # 16 pixels x 64 features to a wave: what covers its waits is other waves
+    + [("conv_bdir_kernel", (64, 1, 1, False, epi), 4) for epi in (RELU, FUSED, LINEAR, F32, POOL)]
     # large planes are bound by memory
     + [("conv_dw_rows_kernel", (taps, blocks, epi), waves) for taps, blocks, waves in ((3, 2, 4), (5, 2, 4), (5, 3, 3)) for epi in (RELU, LINEAR, CLAMPQ)]
 )
