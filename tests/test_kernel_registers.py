@@ -1,13 +1,14 @@
-"""Kernels that rely on several waves a SIMD stay within the registers that allow them.
+"""Kernels that rely on several waves a SIMD stay within the registers that allow them, and one that is all latency requests its
+operands behind a single fetch of its arguments.
 
-From the metadata of the library's own gfx950 code objects; no GPU."""
+From the metadata and the disassembly of the library's own gfx950 code objects; no GPU."""
 import functools
 import re
 import subprocess
 
 import pytest
 
-from test_mfma_wait_states import code_objects
+from test_mfma_wait_states import code_objects, kernels
 
 READELF = "/opt/rocm/llvm/bin/llvm-readelf"
 GENERIC, RELU, FUSED, LINEAR, CLAMPQ, F32, POOL = 0, 2, 3, 4, 5, 7, 8  # EPI_KIND_*
@@ -53,3 +54,20 @@ def test_registers_leave_the_waves_that_the_kernel_relies_on(tmp_path_factory, n
     assert len(found) == 1, "%d kernels" % len(found)
     registers, scratch = found[0]
     assert 512 // (-(-registers // 8) * 8) >= waves and scratch == 0, "%d registers, %d bytes of scratch" % (registers, scratch)
+
+
+@pytest.mark.parametrize("epi", [RELU, LINEAR])
+def test_depthwise_requests_wait_for_the_arguments_once(tmp_path, epi):
+    wanted, found = instances("conv_dw3x3_kernel", epi), []
+    for i, image in enumerate(code_objects()):
+        if wanted.encode() in image:
+            path = tmp_path / ("%d.elf" % i)
+            path.write_bytes(image)
+            found += [code for name, code in kernels(str(path)).items() if wanted in name]
+    assert len(found) == 1, "%d kernels" % len(found)
+    waits = 0
+    for op, operands, _ in found[0]:
+        if op.startswith("global_load"):
+            break
+        waits += op == "s_waitcnt" and "lgkmcnt" in operands
+    assert waits == 1
