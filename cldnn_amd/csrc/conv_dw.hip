@@ -311,6 +311,7 @@ DwPlan dw_plan(const ConvProblem& p, bool fast_epilogue, int cus)
     const int64_t gx = (m + pl.block - 1) / pl.block;
     CHIP_REQUIRE(gx < (1ll << 31), CLDNN_HIP_UNSUPPORTED_SIZE, "convolution too large for one launch");
     pl.grid = (int)gx;  // of the accumulator probe as well
+    pl.one_round = gx * ((p.OFM + 15) / 16) <= 8ll * cus ? 1 : 0;
     pl.packed_bytes = (size_t)((p.OFM + 15) / 16) * p.FY * p.FX * 16;
     pl.mask_bytes = pl.packed_bytes * 4;
     return pl;
@@ -403,9 +404,15 @@ void launch_conv_dw(hipStream_t s, const ConvProblem& p, const DwPlan& pl, const
     }
     if (fast && masked && !raw) {
         a.div_ohw = make_fast_div((uint32_t)a.OHW), a.div_ow = make_fast_div((uint32_t)a.OW);
-        const bool plain = !fast->has_wqf && epi.calib && !fast->fused;
-        if (plain && fast->relu_folded) hipLaunchKernelGGL(conv_dw3x3_kernel<EPI_KIND_RELU>, grid, dim3(256), 0, s, a);
-        else if (plain && fast->act == CLDNN_HIP_ACT_NONE) hipLaunchKernelGGL(conv_dw3x3_kernel<EPI_KIND_LINEAR>, grid, dim3(256), 0, s, a);
+        const bool plain = epi.calib && !fast->fused;
+        // A clamp on the dequantised value has its branch-free form where the chip holds all workgroups at once.  (The run-time form was
+        // 1 to 10 % slower than before, with the division's branch.)  Stride 2, with the branch, without it, branch-free: 32 x 192 x 28x28 4.86,
+        // 4.90 and 3.92 us, 16 x 96 x 112x112 (1176 workgroups) 8.14, 8.78 and 7.44, 64 x 576 x 28x28 (1764) 11.1, 11.8 and 9.7.  With more
+        // the waves of the slower form run into each other less, and memory is the bound: 40 x 96 x 112x112 (2940) 15.6, 15.8 and 16.3, 128
+        // images 38.8, 39.3 and 43.6 (37.4 at the rate of a large copy).
+        if (plain && pl.one_round && fast->has_wqf && fast->iqf_one && fast->clamp_folded) hipLaunchKernelGGL(conv_dw3x3_kernel<EPI_KIND_CLAMPQ>, grid, dim3(256), 0, s, a);
+        else if (plain && !fast->has_wqf && fast->relu_folded) hipLaunchKernelGGL(conv_dw3x3_kernel<EPI_KIND_RELU>, grid, dim3(256), 0, s, a);
+        else if (plain && !fast->has_wqf && fast->act == CLDNN_HIP_ACT_NONE) hipLaunchKernelGGL(conv_dw3x3_kernel<EPI_KIND_LINEAR>, grid, dim3(256), 0, s, a);
         else hipLaunchKernelGGL(conv_dw3x3_kernel<EPI_KIND_FAST>, grid, dim3(256), 0, s, a);
         CHIP_CHECK(hipGetLastError());
         return;

@@ -187,6 +187,7 @@ struct DwPlan {
     int rows;           // the matrix-core kernel: its grid, workgroups to a slice, workgroups in all, sets of 64 pixels to a wave
     int grid_rows, chunks, works, rounds;
     size_t row_bytes;
+    int one_round;      // the chip holds all workgroups of the 3x3 kernel at once
 };
 DwPlan dw_plan(const ConvProblem& p, bool fast_epilogue, int cus);
 void dw_pack_weights(const ConvProblem& p, const int8_t* w, int8_t* packed);

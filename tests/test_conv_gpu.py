@@ -555,6 +555,24 @@ def test_depthwise_kernel(eng, shape, in_dt):
     assert_same(ro2, go2)
 
 
+@pytest.mark.parametrize("shape", [(1, 5, 3, 2), (3, 40, 19, 23), (2, 48, 589, 589), (2, 48, 595, 595)], ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("in_dt,top", [(np.uint8, 6.0), (np.int8, 6.0), (np.uint8, 7.0)], ids=["u8", "s8", "u8_past_the_range"])
+def test_depthwise_clamp_on_both_sides_of_a_full_chip(eng, shape, in_dt, top):
+    """3x3 at stride 2 with relu6: 2040 and 2082 workgroups lie on the two sides of the 2048 that the chip holds at once; a clamp to 7 times
+    127 / 6 leaves the range of int8, which the branch-free form refuses.  Integers behind the same rounding: the same bits."""
+    B, C, H, W = shape
+    x, w, bias, _, _ = problem(29, B, C, H, W, C, 3, 3, in_dt, groups=C)
+    r = np.random.default_rng(4)
+    wqf = (3.0 / (3 * (147.4 if in_dt == np.uint8 else 73.9) * 73.3) * r.uniform(0.5, 2, C)).astype(np.float32)
+    kw = dict(stride=(2, 2), pad=(1, 1), groups=C, out_dt="s8", act="clamp", act_m=0.0, act_n=top)
+    ref = rc.conv(x, w, bias, wqf=wqf, calib=np.full(C, 127 / 6, np.float32), **kw)
+    got, info = hip.conv_forward(eng, x, w, bias, wqf, np.full(C, 127 / 6, np.float32), fmt="fs_b_yx_fsv16", in_pad=(1, 1), want_info=True, **kw)
+    assert b"conv_dw3x3_kernel" in info.kernel_name and b"rows" not in info.kernel_name
+    assert_same(ref, got)
+    assert B * C < 100 or len(np.unique(ref)) > 100
+
+
+
 @pytest.mark.parametrize("shape", [(2, 3, 32, 32, 64, 7, 7, 2, 3), (1, 3, 20, 20, 32, 3, 3, 1, 1), (2, 3, 19, 21, 32, 3, 3, 2, 1),
                                    (1, 4, 9, 9, 16, 5, 5, 1, 2), (1, 1, 12, 12, 80, 3, 1, 1, 0)],
                          ids=lambda s: "x".join(map(str, s)))
