@@ -435,16 +435,17 @@ def test_wide_projections_are_chained_in_the_shared_form_only(eng, mid, proj, ex
     xin.close()
 
 
-@pytest.mark.parametrize("fused", [True, False], ids=["fused", "plain"])
+@pytest.mark.parametrize("eltw_dt", [np.int8, np.uint8, None], ids=["fused", "fused_u8", "plain"])
 @pytest.mark.parametrize("ifm", [192, 576, 960])
-def test_two_stage_chain_behind_a_wide_1x1(eng, ifm, fused):
+def test_two_stage_chain_behind_a_wide_1x1(eng, ifm, eltw_dt):
     """a reducing 1x1 (3, 9 or 15 K-steps) and the expansion behind it; the last granule of 32 pixels is not full"""
     r = np.random.default_rng(ifm)
     B, H, W = 3, 13, 11
     x = r.integers(0, 256, (B, ifm, H, W)).astype(np.uint8)
     xin = hip.upload(eng, x, "fs_b_yx_fsv16")
     l0, l1 = layer(r, ifm, 64, 1, np.uint8), layer(r, 64, 256, 1, np.int8)
-    e, ecal = r.integers(-128, 128, (B, 256, H, W)).astype(np.int8), r.uniform(0.25, 1.0, 256).astype(np.float32)
+    fused, lo = eltw_dt is not None, 0 if eltw_dt == np.uint8 else -128
+    e, ecal = r.integers(lo, lo + 256, (B, 256, H, W)).astype(eltw_dt or np.int8), r.uniform(0.25, 1.0, 256).astype(np.float32)
     ebuf = hip.upload(eng, e, "fs_b_yx_fsv16")
     kw = dict(bias_dt=hip.I32, has_wqf=True, has_calib=True)
     d0 = hip.conv_desc(xin.tensor, l0[0].shape, "s8", act="relu", **kw)
