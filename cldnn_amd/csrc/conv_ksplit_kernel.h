@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(FT * PT == 8 ? 512 : 1024) conv_ksplit_kernel(
     if constexpr (!EARLY) request_rest();
     lds_barrier();
     if (!live) return;
-    // the waves' sums of one fragment on top of `sum`: all reads on their way before the first is added
+    // the waves' sums of one fragment on top of `sum`, of 4, 8 or 16 waves (mfma_plan): all reads on their way before the first is added
     auto add_up = [&](const v4i* src, v4i sum) {
         auto add = [&](auto wc) {
             constexpr int W = decltype(wc)::value;

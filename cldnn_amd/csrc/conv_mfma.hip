@@ -442,6 +442,7 @@ MfmaPlan mfma_plan(const ConvProblem& p, int tile, int cus, bool forced)
         const int frags = pl.ks_ft * pl.ks_pt;
         pl.ks_waves = pl.ksteps >= 32 ? 16 : (pl.ksteps >= 8 ? 8 : 4);
         pl.ks_waves = std::max(std::min(pl.ks_waves, 64 / frags), frags);
+        CHIP_REQUIRE(pl.ks_waves == 4 || pl.ks_waves == 8 || pl.ks_waves == 16, CLDNN_HIP_ERROR, "the split-K kernel adds up 4, 8 or 16 partial sums");
         pl.ks_per = (pl.ksteps + pl.ks_waves - 1) / pl.ks_waves;
         const int64_t ftiles = (int64_t)pl.ofm_tiles * (4 / pl.ks_ft);
         pl.mtiles = (int)((pl.m_total + 16 * pl.ks_pt - 1) / (16 * pl.ks_pt));
