@@ -18,8 +18,8 @@
 //
 // How the offset of an activation fragment is found (ADDR):
 //   UNIFORM  the four k-chunks of a step are one tap and four slices of the bordered input: one scalar offset per step,
-//            walked with scalar counters.  A feature count that is not a multiple of 64 ends in a step that starts at the
-//            last four slices; the slices it repeats have zero weights.
+//            found by a lane each for 64 steps at once.  A feature count that is not a multiple of 64 ends in a step that starts
+//            at the last four slices; the slices it repeats have zero weights.
 //   LANES    anything else (fewer than four slices, no border): every lane computes tap and slice of its own chunk and
 //            checks the tap against the image where there is no border.
 //   GATHERED a fully_connected over a plane: the activations were put into fragment order by gemv_gather_kernel.
@@ -68,8 +68,9 @@ struct KsplitArgs {
 // look-ahead in K-steps: what 128 registers hold (16 waves of a workgroup = four per SIMD).  32 x 64 tiles have eight waves, and above
 // 128 registers a CU holds one workgroup instead of two: with lanes' addresses, or two rows of a pooling window, three steps take 130 to
 // 135, two take 104 to 112.  256 -> 256, 3x3 at 14x14 without a border, three steps and two: batch 8 (224 workgroups) 5.34 and 5.26 us,
-// batch 16 9.05 and 7.12, batch 64 30.3 and 22.3; with its pooling, batch 8 4.60 and 4.48, batch 64 21.4 and 17.5.  The run-time form of
-// the epilogue keeps three: batch 1 6.03 and 6.60, batch 8 6.28 and 6.87.
+// batch 16 9.05 and 7.12, batch 64 30.3 and 22.3; with its pooling, batch 8 4.60 and 4.48, batch 64 21.4 and 17.5.  Only a walk of many
+// steps on a CU of its own likes three better: 788 -> 142 at 9x9, batch 8 (15 steps a wave), 9.3 and 9.8.  The run-time form of the epilogue
+// keeps three: batch 1 6.03 and 6.60, batch 8 6.28 and 6.87.
 template <int FT, int PT, int ADDR, int EPI>
 constexpr int ksplit_depth()
 {

@@ -135,7 +135,10 @@ static int choose_lds_tile(const ConvProblem& p, int64_t m, int cus)
 }
 
 // Microseconds of a split-K tile and of the best tile kernel at sizes where neither fills the chip twice, fitted to sweeps
-// of 43 layers (batch 1 to 32, 1x1 to 5x5; both within 15 %).  A split-K workgroup brings (features + pixels) * K bytes to
+// of 43 layers (batch 1 to 32, 1x1 to 5x5; both within 15 % then).  The kernels have become faster since: over 90 layers drawn from 1 to 150
+// images, 3 to 480 K-steps and 8 to 1016 features a split-K tile takes 13 % less than this says in the mean (18 % rms), the best tile kernel
+// 5 % less (18 % rms).  The row that is chosen is 5.6 % above the best one in the mean, 0.7 % in the median; the large misses (20 to 50 %)
+// are split-K rows that are not chosen, for few K-steps above all, and streaming rows that are, where a weights-stationary one is faster.  A split-K workgroup brings (features + pixels) * K bytes to
 // its CU at 115 bytes a nanosecond after a start of 0.9 us; a tile kernel walks its K-steps in 0.165 us each, two workgroups
 // per CU at the same speed, and its split form halves the walk.
 static double ksplit_us(int64_t m, int ofm, int ksteps, int cus, int ft, int pt)
@@ -170,8 +173,9 @@ static void wsl_depth(int ksteps, int* depth, int* padded);
 // Microseconds of a row on an arbitrary shape with a border: start + K-steps * time of a step + output bytes.  A step takes
 // its latency (`step`) or, with several workgroups on a CU, its throughput (`load` times the workgroups per CU), whichever
 // is longer.  Fitted to timings of 270 layers drawn over 1 to 150 images, 3 to 480 K-steps and 8 to 1016 features
-// (within 10-14 % rms).  The table in choose_row was swept over the layers of three networks; picking by these costs
-// instead takes a layer drawn from that range from 11 % above its best row to 5 % (slices in fours), and from 9 % to 3 %.
+// (within 10-14 % rms then; with today's kernels 9 to 27 %, the weights-stationary rows, which are 20 % faster than it says, 25 to 31 %).  The table in
+// choose_row was swept over the layers of three networks; picking by these costs instead took a layer drawn from that range from 11 % above
+// its best row to 5 % (slices in fours), and from 9 % to 3 %; of 90 drawn ones it is 6.5 % and 4.2 % now.
 struct RowCost {
     int row;
     double start, step, load, per_mb;

@@ -1418,8 +1418,8 @@ __global__ void __launch_bounds__(256) conv_stream_kernel(MfmaArgs a)
 
     // ---- requests: the weights first, whose addresses are there; the activations' take a while to compute.  With the run-time
     // epilogue, where that would take a third to half of the waves a SIMD has (256 -> 128 at 56x56, batch 64, 16 pixels to a wave: 84.0 us
-    // with the weights first, 68.7 behind; 128 -> 128, 32 pixels, 95.7 and 78.8), they come behind the activations: the compiler then
-    // walks the K-steps with few fragments at a time.
+    // with the weights first, 68.7 behind; 128 -> 128, 32 pixels, 95.7 and 78.8, at batch 32, two rounds either way, 47.9 and 50.7), they
+    // come behind the activations: the compiler then walks the K-steps with few fragments at a time.
     constexpr bool WEIGHTS_FIRST = EPI != EPI_KIND_GENERIC || KS == 1 || (KS == 2 && NT == 1);
     v4i fb[KS][NT], ev[NT], fa[KS][4], init[4];
     auto request_weights = [&] {
