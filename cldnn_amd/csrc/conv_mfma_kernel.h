@@ -958,8 +958,10 @@ __global__ void __launch_bounds__(256 * KG) conv_bdir_kernel(MfmaArgs a)
     // register allocator makes of the prologue, and above 256 the kernel loses its second wave per SIMD (25 % slower):
     // five steps keep it clear of the limit.  So do seven for 16 pixels x 64 features: with eight it is 128 to 132 registers, and above 128
     // a SIMD has three waves instead of four (256 -> 256 at 28x28, batch 128, 34.8 us with 131 registers, 32.2 with 128, 31.0 with seven
-    // steps and 118; 3x3 over 64 at 56x56, batch 32, 14.0, 13.5 and 13.0; batch 4, where one wave a SIMD has work, 4.07, 4.13 and 3.99)
-    constexpr int D = LEAN ? 3 : BN == 128 && NT == 2 && KG == 1 ? 5 : BN == 64 && NT == 1 && KG == 1 && !LANES ? 7 : BDIR_PREFETCH_DISTANCE(A_LOADS + NT);
+    // steps and 118; 3x3 over 64 at 56x56, batch 32, 14.0, 13.5 and 13.0; batch 4, where one wave a SIMD has work, 4.07, 4.13 and 3.99).  K split
+    // over four groups is held to 128, and spilled inside the loop with eight (512 -> 512, 3x3 at 14x14, batch 16, 28.6 us, with a sum 31.6;
+    // with seven 20.1 and 20.9)
+    constexpr int D = LEAN ? 3 : BN == 128 && NT == 2 && KG == 1 ? 5 : BN == 64 && NT == 1 && (KG == 1 || KG == 4) && !LANES ? 7 : BDIR_PREFETCH_DISTANCE(A_LOADS + NT);
     constexpr int DA = D;
     v4i ra[DA][A_LOADS], rb[D][NT];
     auto load_a = [&](int ks, v4i (&xa)[A_LOADS]) {

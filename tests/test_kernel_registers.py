@@ -42,6 +42,8 @@ CASES = (
     + [("conv_stream_kernel", p + (GENERIC,), waves) for p, waves in (((1, 2), 7), ((1, 4), 6), ((1, 8), 6), ((2, 2), 5), ((2, 4), 4), ((2, 8), 4))]
     # 16 pixels x 64 features to a wave: what covers its waits is other waves
     + [("conv_bdir_kernel", (64, 1, 1, False, epi), 4) for epi in (RELU, FUSED, LINEAR, F32, POOL)]
+    # the same with K split over four groups: 16 waves in 128 registers
+    + [("conv_bdir_kernel", (64, 1, 4, False, epi), 4) for epi in (GENERIC, RELU, FUSED, LINEAR, F32, POOL)]
     # large planes are bound by memory
     + [("conv_dw_rows_kernel", (taps, blocks, epi), waves) for taps, blocks, waves in ((3, 2, 4), (5, 2, 4), (5, 3, 3)) for epi in (RELU, LINEAR, CLAMPQ)]
 )
