@@ -30,6 +30,10 @@
 // scalar counters, the epilogue's reads and a drain of the queue in front of the meeting): 3x3 256 -> 256 at 14x14 2.30 -> 1.99 us, 1x1
 // 1024 -> 256 2.09 -> 1.83, 3x3 512 -> 512 at 7x7 3.05 -> 2.75, 1x1 512 -> 128 at 28x28 1.96 -> 1.67; of these 0.45 pass until
 // the last workgroup has started and 0.6 to 0.8 until the operands are there; 4 or 8 waves instead of 16 change less than 0.1.
+// The price are 10 to 20 registers: with more than 96 a workgroup of sixteen waves does not start beside the finishing waves of the one
+// before.  With many workgroups to a CU that costs a tile of one to four fragments 3 to 10 %, 30 % under the run-time epilogue (256 -> 256,
+// 3x3 at 14x14, batch 48, 32 x 32 tiles: 25.9 -> 27.5 us).  Such sizes go to the 32 x 64 tile or to other kernels; only a tile
+// override brings them here.
 #pragma once
 #include "conv_mfma_kernel.h"
 
